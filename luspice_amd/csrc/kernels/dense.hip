@@ -314,15 +314,17 @@ __device__ __forceinline__ void tile_mm(const double *As, const double *Bs, int 
 
 // L21 = A21 U11^-1 (64-row tiles) and U12 = L11^-1 A12 (64-column tiles) as
 // tile products with the inverses from the diagonal kernel.
-__global__ void __launch_bounds__(256) dense_trsm_kernel(const DenseJob *jobs, const int *active, int p)
+__global__ void __launch_bounds__(256) dense_trsm_kernel(const DenseJob *jobs, const int *active, int p,
+                                                         const int2 *tiles)
 {
-    const DenseJob J = jobs[blockIdx.y];
+    const int2 tk = tiles[blockIdx.x];                 // (job, tile): only tiles that exist
+    const DenseJob J = jobs[tk.x];
     if (p >= J.T || (active && !active[J.mat])) return;
     const int b = min(kNb, J.T - p);
     const int rem = J.T - p - b;
     if (rem <= 0) return;
     const int ntile = (rem + kNb - 1) / kNb;
-    const int t = blockIdx.x;
+    const int t = tk.y;
     if (t >= 2 * ntile) return;
     extern __shared__ double lds[];
     double *As = lds;
@@ -460,20 +462,28 @@ __device__ __forceinline__ void acc_to_lds(double *Cs, const v4d (&acc)[2][2])
 //        then, once J.flag says the diagonal block is factored, turned into
 //        L21 = A21 U11^-1 and U12 = L11^-1 A12 with the inverses in W;
 //   the interior tiles (ti, tj >= 1): updated.
-// An edge tile only waits on tile 0 of its job, which comes first in the
+// An edge tile only waits on tile 0 of its job, which comes earlier in the
 // grid (dispatch order), so it is resident or done.  The wait is bounded
 // and raises the abort word if it gives up.
+//
+// The grid is a list of the (job, tile) pairs that exist in this panel, every
+// job's tile 0 first (the longest), then the edge tiles, then the interior.
+// A rectangular grid (jobs x the largest job's tiles) is mostly workgroups
+// that return at once, and each of them still takes 66 KB of LDS on a CU
+// before it can: on 420 blocks of T 64..705 that was 42 000 workgroups for
+// panel 0, of which 9 600 have a tile.
 __global__ void __launch_bounds__(256, 2) dense_gemm_kernel(const DenseJob *jobs, const int *active, int p,
-                                                            int *abort_word)
+                                                            int *abort_word, const int2 *tiles)
 {
-    const DenseJob J = jobs[blockIdx.y];
+    const int2 tk = tiles[blockIdx.x];
+    const DenseJob J = jobs[tk.x];
     if (p >= J.T || (active && !active[J.mat])) return;
     const int b = min(kNb, J.T - p);
     const int q0 = p + b;
     const int rem = J.T - q0;
     if (rem <= 0) return;
     const int nt = (rem + 63) / 64;
-    const int tile = blockIdx.x;
+    const int tile = tk.y;
     if (tile >= nt * nt) return;
     const int ni = nt - 1;
     int ti = 0, tj = 0;
@@ -610,34 +620,71 @@ __global__ void __launch_bounds__(256, 2) dense_gemm_kernel(const DenseJob *jobs
 }
 
 // ---------------------------------------------------------------------------
-// One wave per block column c: pivot test, scatter of the pattern slots into
-// the sparse factors, dense copy in storage precision.
+// Pivot test, scatter of the pattern slots into the sparse factors and dense
+// copy in storage precision.  One wave per item (job, column c, segment of
+// kFinishRows rows / slots); the first segment of a column tests its pivot.
+// kFinishRows / 64 loads of each kind are in flight per wave, so a segment
+// costs three dependent round trips (slot -> row and target, value, store)
+// whatever the column's length, and long columns spread over several waves.
+constexpr int kFinishRows = 512;
+constexpr int kFinishUnroll = kFinishRows / kWave;
+
 template <typename T>
-__global__ void __launch_bounds__(64) dense_finish_kernel(const DenseJob *jobs, const void *mats,
-                                                          const int *active, double ptol,
-                                                          double stol)
+__global__ void __launch_bounds__(256) dense_finish_kernel(const DenseJob *jobs, const void *mats,
+                                                           const int *active, double ptol,
+                                                           double stol, const int4 *items, int nitems)
 {
-    const DenseJob J = jobs[blockIdx.y];
-    const int c = blockIdx.x;
+    const int it = uniform((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
+    if (it >= nitems) return;
+    const int4 tk = items[it];
+    const DenseJob J = jobs[tk.x];
+    const int c = tk.y;
+    const int r0 = tk.z * kFinishRows;
     if (c >= J.T || (active && !active[J.mat])) return;
     const FactorDesc<T> M = ((const FactorDesc<T> *)mats)[J.mat];
-    const int lane = threadIdx.x;
+    const int lane = lane_id();
     const size_t ld = (size_t)J.T;
     const double *Sc = J.S + (size_t)c * ld;
     T *Fc = M.tail_F + (size_t)c * ld;
-    for (int r = lane; r < J.T; r += kWave) Fc[r] = from_f64<T>(Sc[r]);
     const int k = M.tail_k0 + c;
     const int64_t c0 = M.cp[k];
     const int m = (int)(M.cp[k + 1] - c0);
     const int dl = M.dp[k] - (int)c0;
-    for (int s = M.tail_ds[c] + lane; s < m; s += kWave) {
-        const T v = from_f64<T>(Sc[M.pos[c0 + s] - M.tail_k0]);
-        M.val[c0 + s] = v;
-        if (s < dl) M.urow[M.dst[c0 + s]] = v;
-        else if (s == dl) M.diag[k] = v;
-        else M.lrow[M.dst[c0 + s]] = v;
+    const int s0 = M.tail_ds[c] + r0;                  // m - tail_ds[c] <= T
+    {
+        double v[kFinishUnroll];
+        int ps[kFinishUnroll], ds[kFinishUnroll];
+#pragma unroll
+        for (int u = 0; u < kFinishUnroll; u++) {
+            const int r = r0 + u * kWave + lane;
+            v[u] = r < J.T ? Sc[r] : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < kFinishUnroll; u++) {
+            const int e = s0 + u * kWave + lane;
+            ps[u] = e < m ? M.pos[c0 + e] - M.tail_k0 : -1;
+            ds[u] = e < m ? M.dst[c0 + e] : 0;
+        }
+        double w[kFinishUnroll];
+#pragma unroll
+        for (int u = 0; u < kFinishUnroll; u++) w[u] = ps[u] >= 0 ? Sc[ps[u]] : 0.0;
+#pragma unroll
+        for (int u = 0; u < kFinishUnroll; u++) {
+            const int r = r0 + u * kWave + lane;
+            if (r < J.T) Fc[r] = from_f64<T>(v[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < kFinishUnroll; u++) {
+            if (ps[u] < 0) continue;
+            const int e = s0 + u * kWave + lane;
+            const T f = from_f64<T>(w[u]);
+            M.val[c0 + e] = f;
+            if (e < dl) M.urow[ds[u]] = f;
+            else if (e == dl) M.diag[k] = f;
+            else M.lrow[ds[u]] = f;
+        }
     }
-    if (lane == 0) {
+    if (lane == 0 && r0 == 0) {
         const double piv = Sc[c];
         const double lmax = __longlong_as_double((long long)J.colmax[c]);
         if (piv == 0.0) {
@@ -666,15 +713,17 @@ __global__ void __launch_bounds__(64) dense_finish_kernel(const DenseJob *jobs, 
 // ---------------------------------------------------------------------------
 // Forward solve, rows of the block: yp[k0 + r] = b[rowat] - L(k0 + r, :k0) y.
 template <typename T>
-__global__ void __launch_bounds__(256) tail_fwd_gather_kernel(const void *mats, const int *tails,
+__global__ void __launch_bounds__(256) tail_fwd_gather_kernel(const void *mats, const int2 *groups,
                                                               const long *voff, const int *active,
                                                               const double *b, const double *y, double *yp,
-                                                              const double *rs)
+                                                              const double *rs, const int *n_active)
 {
-    const int mi = tails[blockIdx.y];
+    if (n_active && uniform(ld_relaxed(n_active)) == 0) return;
+    const int2 tk = groups[blockIdx.x];                // (matrix, group of four rows)
+    const int mi = tk.x;
     if (active && !active[mi]) return;
     const TriDesc<T> M = ((const TriDesc<T> *)mats)[mi];
-    const int r = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int r = tk.y * 4 + (threadIdx.x >> 6);
     if (r >= M.tail_T) return;
     const int lane = lane_id();
     const int i = M.tail_k0 + r;
@@ -708,12 +757,14 @@ constexpr int kTailAcc = 6;                 // accumulator waves per workgroup
 constexpr int kTailSlice = (kNb + kTailAcc - 1) / kTailAcc;   // coupling columns per accumulator wave
 
 template <typename T, bool kLower>
-__global__ void __launch_bounds__(512) tail_trsv_kernel(const void *mats, const int *tails,
+__global__ void __launch_bounds__(512) tail_trsv_kernel(const void *mats, const int2 *pairs,
                                                         const long *voff, const int *active,
                                                         double *y, const double *yp, double *z, double *x,
-                                                        int *abort_word, const double *cs)
+                                                        int *abort_word, const double *cs, const int *n_active)
 {
-    const int mi = tails[blockIdx.y];
+    // nothing active: every workgroup returns before it takes a ticket
+    if (n_active && uniform(ld_relaxed(n_active)) == 0) return;
+    const int mi = pairs[blockIdx.x].x;                // as many workgroups per matrix as it has pairs
     const TriDesc<T> M = ((const TriDesc<T> *)mats)[mi];
     const int lane = lane_id();
     const int wv = threadIdx.x >> 6;
@@ -856,7 +907,7 @@ __global__ void __launch_bounds__(512) tail_trsv_kernel(const void *mats, const 
         // the last workgroup of this matrix re-arms its ticket counter
         if (threadIdx.x == 0) {
             const int fin = atomicAdd(&M.tail_ctr[1], 1);
-            if (fin == (int)gridDim.x - 1) {
+            if (fin == npair - 1) {
                 st_relaxed(&M.tail_ctr[0], 0);
                 st_relaxed(&M.tail_ctr[1], 0);
             }
@@ -881,62 +932,86 @@ hipError_t dense_set_lds()
 // whose T is below maxT the update kernel returns before its tiles once
 // p + 64 >= T, so each of its panels is factored exactly once.
 hipError_t launch_dense_lu(const DenseJob *jobs, int njobs, int maxT, const int *active, int *abort_word,
-                           hipStream_t st)
+                           const DenseGrid &G, hipStream_t st)
 {
     if (maxT <= 0) return hipSuccess;
     hipLaunchKernelGGL(dense_diag_kernel, dim3(njobs), dim3(256), kDiagLds, st, jobs, active, 0);
-    for (int p = 0; p < maxT; p += kNb) {
-        const int rem = maxT - p - min(kNb, maxT - p);
-        if (rem > 0) {
-            const int nt = (rem + kNb - 1) / kNb;
-            if (p == 0)
-                hipLaunchKernelGGL(dense_trsm_kernel, dim3(2 * nt, njobs), dim3(256), kGemmLds, st, jobs, active, p);
-            hipLaunchKernelGGL(dense_gemm_kernel, dim3(nt * nt, njobs), dim3(256), kGemmLds, st, jobs,
-                               active, p, abort_word);
-        }
+    if (G.ntrsm)
+        hipLaunchKernelGGL(dense_trsm_kernel, dim3(G.ntrsm), dim3(256), kGemmLds, st, jobs, active, 0, G.trsm);
+    for (size_t i = 0; i + 1 < G.panel.size(); i++) {
+        const long cnt = G.panel[i + 1] - G.panel[i];
+        hipLaunchKernelGGL(dense_gemm_kernel, dim3((unsigned)cnt), dim3(256), kGemmLds, st, jobs, active,
+                           (int)i * kNb, abort_word, G.gemm + G.panel[i]);
     }
     return hipGetLastError();
 }
 
-template <typename T>
-hipError_t launch_dense_finish(const DenseJob *jobs, int njobs, int maxT, const void *mats,
-                               const int *active, double ptol, double stol, hipStream_t st)
+// The lists behind the grids (see DenseGrid): jobs by falling T, so that the
+// longest ones start first.
+void dense_grid_lists(const std::vector<int> &T, const std::vector<int> &mat, DenseGridHost &H)
 {
-    hipLaunchKernelGGL(dense_finish_kernel<T>, dim3(maxT, njobs), dim3(64), 0, st, jobs, mats, active, ptol,
-                       stol);
-    return hipGetLastError();
+    const int nj = (int)T.size();
+    const int maxT = nj ? T[0] : 0;
+    H = DenseGridHost();
+    H.panel.push_back(0);
+    for (int p = 0; p + kNb < maxT; p += kNb) {
+        auto nt = [&](int j) { return T[j] > p + kNb ? (T[j] - p - kNb + kNb - 1) / kNb : 0; };
+        for (int j = 0; j < nj && nt(j); j++) H.gemm.push_back(make_int2(j, 0));
+        for (int j = 0; j < nj && nt(j); j++)
+            for (int t = 1; t <= 2 * (nt(j) - 1); t++) H.gemm.push_back(make_int2(j, t));
+        for (int j = 0; j < nj && nt(j); j++)
+            for (int t = 2 * (nt(j) - 1) + 1; t < nt(j) * nt(j); t++) H.gemm.push_back(make_int2(j, t));
+        if (p == 0)
+            for (int j = 0; j < nj && nt(j); j++)
+                for (int t = 0; t < 2 * nt(j); t++) H.trsm.push_back(make_int2(j, t));
+        H.panel.push_back((long)H.gemm.size());
+    }
+    for (int j = 0; j < nj; j++) {
+        for (int c = 0; c < T[j]; c++)
+            for (int g = 0; g * kFinishRows < T[j]; g++) H.finish.push_back(make_int4(j, c, g, 0));
+        for (int g = 0; g * 4 < T[j]; g++) H.gather.push_back(make_int2(mat[j], g));
+        for (int t = 0; t * 2 * kNb < T[j]; t++) H.trsv.push_back(make_int2(mat[j], t));
+    }
 }
-template hipError_t launch_dense_finish<float>(const DenseJob *, int, int, const void *, const int *, double, double, hipStream_t);
-template hipError_t launch_dense_finish<double>(const DenseJob *, int, int, const void *, const int *, double, double, hipStream_t);
-template hipError_t launch_dense_finish<__half>(const DenseJob *, int, int, const void *, const int *, double, double, hipStream_t);
 
 template <typename T>
-hipError_t launch_tail_solve(const void *mats, const int *tails, int ntails, int maxT, const long *voff,
-                             const int *active, const double *b, double *y, double *yp, double *z,
-                             double *x, bool forward, int *abort_word, const double *rs, const double *cs,
+hipError_t launch_dense_finish(const DenseJob *jobs, const void *mats, const int *active, double ptol, double stol,
+                               const DenseGrid &G, hipStream_t st)
+{
+    if (!G.nfinish) return hipSuccess;
+    hipLaunchKernelGGL(dense_finish_kernel<T>, dim3((G.nfinish + 3) / 4), dim3(256), 0, st, jobs, mats, active, ptol,
+                       stol, G.finish, G.nfinish);
+    return hipGetLastError();
+}
+template hipError_t launch_dense_finish<float>(const DenseJob *, const void *, const int *, double, double, const DenseGrid &, hipStream_t);
+template hipError_t launch_dense_finish<double>(const DenseJob *, const void *, const int *, double, double, const DenseGrid &, hipStream_t);
+template hipError_t launch_dense_finish<__half>(const DenseJob *, const void *, const int *, double, double, const DenseGrid &, hipStream_t);
+
+template <typename T>
+hipError_t launch_tail_solve(const void *mats, const DenseGrid &G, const long *voff, const int *active,
+                             const double *b, double *y, double *yp, double *z, double *x, bool forward,
+                             int *abort_word, const double *rs, const double *cs, const int *n_active,
                              hipStream_t st)
 {
-    const int nblk = (maxT + kNb - 1) / kNb;
-    const int npair = (nblk + 1) / 2;                   // two 64-row blocks per workgroup
     if (forward) {
-        hipLaunchKernelGGL(tail_fwd_gather_kernel<T>, dim3((maxT + 3) / 4, ntails), dim3(256), 0, st, mats,
-                           tails, voff, active, b, y, yp, rs);
-        hipLaunchKernelGGL((tail_trsv_kernel<T, true>), dim3(npair, ntails), dim3(512), 0, st, mats, tails,
-                           voff, active, y, yp, z, x, abort_word, cs);
+        hipLaunchKernelGGL(tail_fwd_gather_kernel<T>, dim3(G.ngather), dim3(256), 0, st, mats, G.gather, voff,
+                           active, b, y, yp, rs, n_active);
+        hipLaunchKernelGGL((tail_trsv_kernel<T, true>), dim3(G.ntrsv), dim3(512), 0, st, mats, G.trsv, voff,
+                           active, y, yp, z, x, abort_word, cs, n_active);
     } else {
-        hipLaunchKernelGGL((tail_trsv_kernel<T, false>), dim3(npair, ntails), dim3(512), 0, st, mats, tails,
-                           voff, active, y, yp, z, x, abort_word, cs);
+        hipLaunchKernelGGL((tail_trsv_kernel<T, false>), dim3(G.ntrsv), dim3(512), 0, st, mats, G.trsv, voff,
+                           active, y, yp, z, x, abort_word, cs, n_active);
     }
     return hipGetLastError();
 }
-template hipError_t launch_tail_solve<float>(const void *, const int *, int, int, const long *, const int *,
-                                              const double *, double *, double *, double *, double *, bool,
-                                              int *, const double *, const double *, hipStream_t);
-template hipError_t launch_tail_solve<double>(const void *, const int *, int, int, const long *, const int *,
-                                              const double *, double *, double *, double *, double *, bool,
-                                              int *, const double *, const double *, hipStream_t);
-template hipError_t launch_tail_solve<__half>(const void *, const int *, int, int, const long *, const int *,
-                                              const double *, double *, double *, double *, double *, bool,
-                                              int *, const double *, const double *, hipStream_t);
+template hipError_t launch_tail_solve<float>(const void *, const DenseGrid &, const long *, const int *, const double *,
+                                              double *, double *, double *, double *, bool, int *,
+                                              const double *, const double *, const int *, hipStream_t);
+template hipError_t launch_tail_solve<double>(const void *, const DenseGrid &, const long *, const int *, const double *,
+                                              double *, double *, double *, double *, bool, int *,
+                                              const double *, const double *, const int *, hipStream_t);
+template hipError_t launch_tail_solve<__half>(const void *, const DenseGrid &, const long *, const int *, const double *,
+                                              double *, double *, double *, double *, bool, int *,
+                                              const double *, const double *, const int *, hipStream_t);
 
 }  // namespace lsp

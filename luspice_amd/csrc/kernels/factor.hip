@@ -134,17 +134,30 @@ __device__ __forceinline__ bool run_gemv_unset(const T *val, XP x, const LSP_GLO
     return true;
 }
 
-// Marks the factor values of every active matrix unset (before a refactor);
-// blockIdx.y is the matrix.
+// Before a refactor: marks the factor values of the active matrices' columns
+// left of the dense block unset (the block's columns are never polled by
+// value), and resets every matrix's status words.  One workgroup per chunk
+// (matrix, kFillSlots slots); each matrix has at least one.  Kernels, not
+// memsets, so the whole refactor sequence stays capturable in a HIP graph.
 template <typename T>
-__global__ void __launch_bounds__(256) fill_unset_kernel(const FactorDesc<T> *mats, const int *active)
+__global__ void __launch_bounds__(256) fill_unset_kernel(const FactorDesc<T> *mats, const int *active,
+                                                         const int2 *chunks, int *abort_word, int *dbg)
 {
-    const int m = blockIdx.y;
-    if (active && !active[m]) return;
-    const FactorDesc<T> M = mats[m];
-    const long n = (long)M.cp[M.n];
-    const long stride = (long)gridDim.x * blockDim.x;
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) M.val[i] = Unset<T>::value();
+    const int2 ch = chunks[blockIdx.x];
+    const FactorDesc<T> M = mats[ch.x];
+    const int tid = threadIdx.x;
+    if (ch.y == 0 && tid < kMstat)
+        M.mstat[tid] = tid == 1 || tid == 2 || tid == 6 ? 0x7fffffff : 0;   // first-column words: none
+    if (blockIdx.x == 0) {
+        if (dbg && tid < 8) dbg[tid] = -1;
+        if (abort_word && tid == 0) *abort_word = 0;
+    }
+    if (active && !active[ch.x]) return;
+    const long n = (long)M.cp[M.tail_k0];
+    const long s0 = (long)ch.y * kFillSlots + tid;
+#pragma unroll
+    for (int u = 0; u < kFillSlots / 256; u++)
+        if (s0 + 256 * u < n) M.val[s0 + 256 * u] = Unset<T>::value();
 }
 
 // One column of the left-looking refactorization.  XP is the work vector's
@@ -428,26 +441,6 @@ __global__ void __launch_bounds__(256) refactor_kernel(FactorLaunch L)
     if (leave_queue(L.ctr, nq, L.total_waves)) advance_epoch(L.epoch, epoch);
 }
 
-// Per-matrix status words are reset by a kernel (not a memset) so the whole
-// refactor sequence stays capturable in a HIP graph.
-__global__ void reset_mstat_kernel(int *mstat, int nmat, int *abort_word, int *dbg)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (dbg && i < 8) dbg[i] = -1;
-    if (i < nmat) {
-        int *w = mstat + kMstat * i;
-        w[0] = 0;
-        w[1] = 0x7fffffff;
-        w[2] = 0x7fffffff;
-        w[3] = 0;
-        w[4] = 0;
-        w[5] = 0;
-        w[6] = 0x7fffffff;
-        w[7] = 0;
-    }
-    if (i == 0 && abort_word) *abort_word = 0;
-}
-
 }  // namespace lsp
 
 // ---------------------------------------------------------------------------
@@ -468,26 +461,16 @@ template hipError_t launch_refactor<double>(const FactorLaunch &, int, hipStream
 template hipError_t launch_refactor<__half>(const FactorLaunch &, int, hipStream_t);
 
 template <typename T>
-hipError_t launch_fill_unset(const void *mats, const int *active, int nmat, long max_slots, hipStream_t st)
+hipError_t launch_fill_unset(const void *mats, const int *active, const int2 *chunks, int nchunks, int *abort_word,
+                             int *dbg, hipStream_t st)
 {
-    const long want = (max_slots + 255) / 256;
-    const int bx = (int)std::max(1L, std::min(1024L, want));
-    hipLaunchKernelGGL(fill_unset_kernel<T>, dim3(bx, nmat), dim3(256), 0, st, (const FactorDesc<T> *)mats,
-                       active);
+    hipLaunchKernelGGL(fill_unset_kernel<T>, dim3(nchunks), dim3(256), 0, st, (const FactorDesc<T> *)mats, active,
+                       chunks, abort_word, dbg);
     return hipGetLastError();
 }
-template hipError_t launch_fill_unset<float>(const void *, const int *, int, long, hipStream_t);
-template hipError_t launch_fill_unset<double>(const void *, const int *, int, long, hipStream_t);
-template hipError_t launch_fill_unset<__half>(const void *, const int *, int, long, hipStream_t);
-
-hipError_t launch_reset_mstat(int *mstat, int nmat, int *abort_word, int *dbg, hipStream_t st)
-{
-    const int threads = 256;
-    const int blocks = (nmat + threads - 1) / threads;
-    hipLaunchKernelGGL(reset_mstat_kernel, dim3(blocks > 0 ? blocks : 1), dim3(threads), 0, st,
-                       mstat, nmat, abort_word, dbg);
-    return hipGetLastError();
-}
+template hipError_t launch_fill_unset<float>(const void *, const int *, const int2 *, int, int *, int *, hipStream_t);
+template hipError_t launch_fill_unset<double>(const void *, const int *, const int2 *, int, int *, int *, hipStream_t);
+template hipError_t launch_fill_unset<__half>(const void *, const int *, const int2 *, int, int *, int *, hipStream_t);
 
 template <typename T>
 hipError_t refactor_set_lds(int cap)

@@ -438,7 +438,7 @@ int Batch::set_active(const int *mask)
 // (an upper estimate used for admission; device_bytes() reports the actual).
 size_t Batch::estimate_device_bytes() const
 {
-    double n = 0, nnz = 0, slots = 0, rel = 0, nlu = 0, sell = 0, slices = 0, T = 0, T2 = 0;
+    double n = 0, nnz = 0, slots = 0, rel = 0, nlu = 0, sell = 0, slices = 0, T = 0, T2 = 0, lists = 0;
     double maxcol = 0;
     const double nc = (double)circ_.size();
     for (const auto &C : circ_) {
@@ -446,6 +446,8 @@ size_t Batch::estimate_device_bytes() const
         n += C.n; nnz += C.nnz; slots += (double)P.cp[C.n]; rel += (double)P.relp[C.n];
         nlu += (double)(P.n_l + P.n_u); sell += (double)C.sell.slots; slices += C.sell.nslices;
         T += P.tail_T; T2 += (double)P.tail_T * P.tail_T;
+        const double nt = (P.tail_T + 63) / 64;                           // update tiles of every panel, TRSM tiles
+        lists += nt * nt * nt / 3 + 2 * nt + 2.0 * P.tail_T * (1 + P.tail_T / 512) + P.tail_T / 4 + nt;
         maxcol = std::max(maxcol, (double)P.max_col);
     }
     const double m = std::max(1, opt_.ir_inner);
@@ -459,6 +461,7 @@ size_t Batch::estimate_device_bytes() const
     if (opt_.factor_shift > 0.0) b += 8 * n;                               // shifted diagonal entries
     b += 8 * T2 + 16 * T + 65536.0 * nc;                                   // dense block work
     b += 24 * n + 8 * slices + 16 * n;                                    // task lists, row packets
+    b += 8 * lists + 8 * (slots / kFillSlots + nc);                       // dense-block and fill work lists
     b += 64 * n + 8 * (2 * m + 1) * n;                                    // vectors, Krylov bases V and Z
     b += (4 + 8) * (slots + nlu + n + T2);                                 // fp32 + fp64 factor sets
     if (maxcol > std::max(1, opt_.lds_cap)) b += 256.0 * 8 * 4 * maxcol * 8;   // global column scratch
@@ -612,42 +615,64 @@ int Batch::upload_all()
         if (!d_done_ || !d_ctr_ || !d_abort_ || !d_mstat_ || !d_epoch_)
             return LSP_E_ALLOC;
     }
-    // dense trailing blocks
+    // dense trailing blocks, the jobs by falling order T
     {
-        std::vector<int> tds, tlc, tails;
+        std::vector<int> tds, tlc;
         std::vector<DenseJob> jobs;
         d_tailS_ = (double *)dalloc(nt2_tot_ * sizeof(double));
         d_colmax_ = (unsigned long long *)dalloc(nt_tot_ * sizeof(unsigned long long));
-        int ntail = 0;
-        for (const auto &C : circ_) ntail += C.plan.tail_T > 0;
-        d_tailW_ = (double *)dalloc((size_t)std::max(ntail, 1) * 2 * 64 * 64 * sizeof(double));
-        d_dflag_ = upload(std::vector<int>(std::max(ntail, 1), 0));
-        if (!d_tailS_ || !d_colmax_ || !d_tailW_ || !d_dflag_) return LSP_E_ALLOC;
+        std::vector<int> mat, order;
         for (int m = 0; m < nc; m++) {
-            const CircuitHost &C = circ_[m];
-            const LspPlan &P = C.plan;
+            const LspPlan &P = circ_[m].plan;
             tds.insert(tds.end(), P.tail_ds.begin(), P.tail_ds.end());
             tlc.insert(tlc.end(), P.tail_lcut.begin(), P.tail_lcut.end());
-            if (P.tail_T > 0) {
-                DenseJob J{};
-                J.S = d_tailS_ + C.o_t2;
-                J.W = d_tailW_ + jobs.size() * 2 * 64 * 64;
-                J.colmax = d_colmax_ + C.o_t;
-                J.flag = d_dflag_ + jobs.size();
-                J.T = P.tail_T;
-                J.mat = m;
-                jobs.push_back(J);
-                tails.push_back(m);
-                max_tail_T_ = std::max(max_tail_T_, P.tail_T);
-            }
+            if (P.tail_T > 0) mat.push_back(m);
         }
-        njobs_ = (int)jobs.size();
+        std::stable_sort(mat.begin(), mat.end(),
+                         [&](int a, int b) { return circ_[a].plan.tail_T > circ_[b].plan.tail_T; });
+        njobs_ = (int)mat.size();
+        d_tailW_ = (double *)dalloc((size_t)std::max(njobs_, 1) * 2 * 64 * 64 * sizeof(double));
+        d_dflag_ = upload(std::vector<int>(std::max(njobs_, 1), 0));
+        if (!d_tailS_ || !d_colmax_ || !d_tailW_ || !d_dflag_) return LSP_E_ALLOC;
+        for (int m : mat) {
+            const CircuitHost &C = circ_[m];
+            DenseJob J{};
+            J.S = d_tailS_ + C.o_t2;
+            J.W = d_tailW_ + jobs.size() * 2 * 64 * 64;
+            J.colmax = d_colmax_ + C.o_t;
+            J.flag = d_dflag_ + jobs.size();
+            J.T = C.plan.tail_T;
+            J.mat = m;
+            jobs.push_back(J);
+            order.push_back(J.T);
+        }
+        max_tail_T_ = njobs_ ? order[0] : 0;
+        DenseGridHost H;
+        dense_grid_lists(order, mat, H);
+        dgrid_.gemm = upload(H.gemm);
+        dgrid_.trsm = upload(H.trsm);
+        dgrid_.finish = upload(H.finish);
+        dgrid_.gather = upload(H.gather);
+        dgrid_.trsv = upload(H.trsv);
+        dgrid_.panel = H.panel;
+        dgrid_.ntrsm = (int)H.trsm.size();
+        dgrid_.nfinish = (int)H.finish.size();
+        dgrid_.ngather = (int)H.gather.size();
+        dgrid_.ntrsv = (int)H.trsv.size();
         d_tail_ds_ = upload(tds);
         d_tail_lcut_ = upload(tlc);
         d_djobs_ = upload(jobs);
-        d_tails_ = upload(tails);
         d_tail_ctr_ = upload(std::vector<int>(4 * nc, 0));
-        if (!d_tail_ds_ || !d_tail_lcut_ || !d_djobs_ || !d_tails_ || !d_tail_ctr_)
+        std::vector<int2> fill;
+        for (int m = 0; m < nc; m++) {
+            const LspPlan &P = circ_[m].plan;
+            const long slots = std::max<long>(1, P.cp[P.tail_k0]);
+            for (long c = 0; c * kFillSlots < slots; c++) fill.push_back(make_int2(m, (int)c));
+        }
+        d_fillchunk_ = upload(fill);
+        nfillchunk_ = (int)fill.size();
+        if (!d_tail_ds_ || !d_tail_lcut_ || !d_djobs_ || !d_tail_ctr_ || !d_fillchunk_ || !dgrid_.gemm ||
+            !dgrid_.trsm || !dgrid_.finish || !dgrid_.gather || !dgrid_.trsv)
             return LSP_E_ALLOC;
         if (njobs_) {
             rc = check(dense_set_lds(), "dense lds attr");
@@ -981,20 +1006,16 @@ int Batch::refactor_t(FactorSet<T> &fs, const int *d_active)
     L.ptol = opt_.refactor_ptol;
     L.stol = opt_.repivot == 3 ? opt_.pivot_tol : 0.0;
     L.dbg = d_dbg_;
-    rc = check(launch_reset_mstat(d_mstat_, (int)circ_.size(), d_abort_, d_dbg_, stream_), "reset");
-    if (rc) return rc;
-    long max_slots = 0;
-    for (const auto &C : circ_) max_slots = std::max(max_slots, (long)C.plan.cp[C.n]);
-    rc = check(launch_fill_unset<T>(fs.fdesc, d_active, (int)circ_.size(), max_slots, stream_), "unset");
+    rc = check(launch_fill_unset<T>(fs.fdesc, d_active, d_fillchunk_, nfillchunk_, d_abort_, d_dbg_, stream_), "unset");
     if (rc) return rc;
     if (!capturing_) (void)hipEventRecord(ev_[0], stream_);   // the persistent kernel alone, from here
     rc = check(launch_refactor<T>(L, fblocks_, stream_), "refactor launch");
     if (!capturing_) (void)hipEventRecord(ev_[1], stream_);      // the persistent kernel alone
     if (!rc && njobs_) {
-        rc = check(launch_dense_lu(d_djobs_, njobs_, max_tail_T_, d_active, d_abort_, stream_), "dense lu");
+        rc = check(launch_dense_lu(d_djobs_, njobs_, max_tail_T_, d_active, d_abort_, dgrid_, stream_), "dense lu");
         if (!rc)
-            rc = check(launch_dense_finish<T>(d_djobs_, njobs_, max_tail_T_, fs.fdesc, d_active,
-                                              opt_.refactor_ptol, L.stol, stream_), "dense finish");
+            rc = check(launch_dense_finish<T>(d_djobs_, fs.fdesc, d_active, opt_.refactor_ptol, L.stol, dgrid_,
+                                              stream_), "dense finish");
     }
     if (!capturing_) (void)hipEventRecord(ev_[5], stream_);      // + dense trailing block
     return rc;
@@ -1263,15 +1284,13 @@ int Batch::trisolve_t(FactorSet<T> &fs, const double *d_b, double *d_x, const in
     int rc = check(launch_solve_unset(Lf, ntot_, stream_), "solve unset");
     if (!rc) rc = check(launch_trisolve_half<T>(Lf, true, tblocks_f_, stream_), "trisolve fwd");
     if (!rc && njobs_)
-        rc = check(launch_tail_solve<T>(fs.tdesc, d_tails_, njobs_, max_tail_T_, d_voff_, d_active, d_b,
-                                        d_ty_, d_typ_, d_tz_, d_x, true, d_abort_ + 1, Lf.rs, Lf.cs,
-                                        stream_),
+        rc = check(launch_tail_solve<T>(fs.tdesc, dgrid_, d_voff_, d_active, d_b, d_ty_, d_typ_, d_tz_, d_x, true,
+                                        d_abort_ + 1, Lf.rs, Lf.cs, d_nact, stream_),
                    "tail fwd");
     if (!capturing_) (void)hipEventRecord(ev_[4], stream_);
     if (!rc && njobs_)
-        rc = check(launch_tail_solve<T>(fs.tdesc, d_tails_, njobs_, max_tail_T_, d_voff_, d_active, d_b,
-                                        d_ty_, d_typ_, d_tz_, d_x, false, d_abort_ + 1, Lf.rs, Lf.cs,
-                                        stream_),
+        rc = check(launch_tail_solve<T>(fs.tdesc, dgrid_, d_voff_, d_active, d_b, d_ty_, d_typ_, d_tz_, d_x, false,
+                                        d_abort_ + 1, Lf.rs, Lf.cs, d_nact, stream_),
                    "tail bwd");
     if (!rc) rc = check(launch_trisolve_half<T>(Lb, false, tblocks_b_, stream_), "trisolve bwd");
     if (!capturing_) (void)hipEventRecord(ev_[3], stream_);

@@ -104,12 +104,15 @@ struct DeviceArrays {
     int nq_f_ = 1, nq_t_ = 1;                          // queue counters: refactor, solves
     long width_f_ = 0, width_tf_ = 0, width_tb_ = 0;   // widest merged level
     // dense trailing blocks
-    int *d_tail_ds_ = nullptr, *d_tail_lcut_ = nullptr, *d_tail_ctr_ = nullptr, *d_tails_ = nullptr;
+    int *d_tail_ds_ = nullptr, *d_tail_lcut_ = nullptr, *d_tail_ctr_ = nullptr;
     double *d_tailS_ = nullptr;
     unsigned long long *d_colmax_ = nullptr;
     int *d_dflag_ = nullptr;                   // per dense job: the last diagonal block factored
     DenseJob *d_djobs_ = nullptr;
     int njobs_ = 0, max_tail_T_ = 0;
+    DenseGrid dgrid_;                          // work lists of the dense-block launches
+    int2 *d_fillchunk_ = nullptr;              // (matrix, chunk) of the unset fill
+    int nfillchunk_ = 0;
     long nt_tot_ = 0, nt2_tot_ = 0;
     long nfw_tot_ = 0, nbw_tot_ = 0;     // row tasks of the sparse solves
     FactorSet<float> f32_;
