@@ -10,20 +10,13 @@
 //
 // Refactorization (fixed pivot order; no pivot search, as in the sparse part):
 //   the persistent refactor kernel applies every column outside the block and
-//   leaves S = A22 - L21 U12 (fp64, column-major T x T).  Then, for the
-//   64-column panels p:
-//     dense_diag_kernel   (panel 0) S[p:p+64, p:p+64] = L11 \ U11, and
-//                         L11^-1, U11^-1
-//     dense_trsm_kernel   (panel 0) L21 = A21 U11^-1 (64-row tiles) and
-//                         U12 = L11^-1 A12 (64-column tiles), as tile products
-//     dense_gemm_kernel   S22 -= L21 U12 (64x64 tiles, fp64 matrix cores); its
-//                         first tile then factors the next panel's diagonal
-//                         block, and the next panel's L21 / U12 tiles wait
-//                         for it and multiply by its inverses, so each later
-//                         panel costs one launch
-//   dense_finish_kernel  applies the pivot test (|pivot| >= ptol max_i |x_i|,
-//   i.e. ptol * max |L(:,c)| <= 1), scatters the block into the sparse factor
-//   arrays and writes a dense copy in storage precision for the solves.
+//   leaves S = A22 - L21 U12 (fp64, column-major T x T).  Then
+//     dense_lu_kernel     factors every block of the batch in one launch, as a
+//                         dataflow of 64 x 64 tiles (see there)
+//     dense_pivot_kernel  applies the pivot test (|pivot| >= ptol max_i |x_i|,
+//                         i.e. ptol * max |L(:,c)| <= 1) and copies the diagonal
+//   The factor of the block stays dense: in S itself for fp64 storage (tail_F
+//   is S then), else in tail_F, which the tiles fill as they become final.
 // Structural zeros stay exactly zero (every product that reaches them has a
 // structurally zero factor), so the sparse pattern is reproduced.
 //
@@ -37,13 +30,15 @@
 // accumulating each finished block's contribution as it arrives.  Blocks
 // hand over their values as the sparse solves do: y and z are unset before
 // the solve and a waiting block polls the values themselves.
+#include <algorithm>
+
 #include "common.hpp"
 #include "launch.hpp"
 
 namespace lsp {
 
 constexpr int kNb = 64;            // panel width
-constexpr int kBsLd = 65;          // padded leading dimension of the GEMM B tile
+constexpr int kTile = kNb * kNb;   // doubles per packed tile
 
 __device__ __forceinline__ unsigned long long dbits(double v)
 {
@@ -59,653 +54,471 @@ __device__ __forceinline__ double bcast(double v, int src)
     return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
 }
 
-// ---------------------------------------------------------------------------
-// Diagonal block: LU of the 64x64 block and the inverses of both factors,
-// blocked by 16-column sub-panels (256 threads).  Thread (r, s) = (tid % 16,
-// tid / 16) keeps elements (r + 16a, s + 16b), a, b < 4, of A, of X = L^-1
-// and of Y = U^-1 in registers; a partial last block is padded with identity
-// rows and columns.  For each sub-panel k (columns k0 = 16k .. k0 + 15):
-//   1. the owners publish, in LDS, the panel columns (rows >= k0), the block
-//      row [R | I | A12] (R: rows k0.. of X left of k0; A12: rows k0.. of A
-//      right of the panel) and delta - Yacc over the panel columns;
-//   2. wave 0 factors the 64 x 16 panel, one row per lane: step c broadcasts
-//      the pivot row by readlane, every lane below it forms l = A(i, c) / p
-//      (times the reciprocal) and updates its row -- the same operations, in
-//      the same order, as the unblocked right-looking elimination, so the
-//      factor is the same bit for bit;
-//   3. wave 1 applies L11^-1 to the block row, one column per lane: D R, D =
-//      L11^-1 and U12 = L11^-1 A12 in one forward substitution; wave 2 solves
-//      V U11 = delta - Yacc, one row per lane, for the panel columns of Y;
-//   4. every thread takes its final panel values and applies the rank-16
-//      updates: A22 -= L21 U12, the rows of X below the panel -= L21 [D R | D]
-//      (X <- M_k^-1 X for the elementary block factor M_k of L), and
-//      Yacc(:, right of the panel) += V U12.
-// Four barriers per sub-panel instead of one per column.  Outputs: L\U over
-// the block in S, L^-1 (unit lower) and U^-1 (upper) into the job's
-// workspace W (column-major, leading dimension 64), and the column maxima of
-// |L| for the pivot test.
-constexpr int kDgLs = 80;                  // row stride of the panel and delta - Yacc buffers
-constexpr int kDgRs = 68;                  // row stride of the block-row buffer
-constexpr int kDgLp = 0;                   // [16][80]: A(i, k0 + q) at q * 80 + i
-constexpr int kDgRow = 16 * kDgLs;         // [16][68]: block row at q * 68 + j
-constexpr int kDgW = kDgRow + 16 * kDgRs;  // [16][80]: delta - Yacc(i, k0 + q), then V, at q * 80 + i
-constexpr int kDgRp = kDgW + 16 * kDgLs;   // [16]: pivot reciprocals of the sub-panel
-constexpr size_t kDiagLds = sizeof(double) * (kDgRp + 16);
-
-__device__ __forceinline__ double max16(double v)
+// Maxima of 16 non-negative values over the lanes that differ in the four
+// lane bits from `top` (8 or 32) down: each step keeps half of the values and
+// exchanges the other half.  Returns value i's maximum in the lanes whose
+// four bits spell i.
+template <int H>
+__device__ __forceinline__ void max_halve(double (&a)[16], int lane, int off)
 {
+    const bool up = lane & off;
 #pragma unroll
-    for (int off = 8; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, kWave));
-    return v;
-}
-
-// The block body, run by all 256 threads of a workgroup: panel p of job J,
-// its input read from src (column-major, leading dimension lds: the block in
-// S itself, or a copy in LDS that the caller has made visible with a
-// barrier); sm is kDiagLds bytes of LDS, which may overlap src.
-__device__ __forceinline__ void diag_block(const DenseJob &J, int p, const double *src, size_t lds, double *sm)
-{
-    const int tid = threadIdx.x;
-    const int r = tid & 15, s = tid >> 4;
-    const int lane = tid & 63, wid = tid >> 6;
-    const int b = min(kNb, J.T - p);
-    const size_t ld = (size_t)J.T;
-    double *Sp = J.S + (size_t)p * ld + p;
-    double A[4][4], X[4][4], Y[4][4];
-#pragma unroll
-    for (int a = 0; a < 4; a++) {
-        const int i = r + 16 * a;
-#pragma unroll
-        for (int bb = 0; bb < 4; bb++) {
-            const int j = s + 16 * bb;
-            const double v = src[(size_t)min(j, b - 1) * lds + min(i, b - 1)];
-            A[a][bb] = (i < b && j < b) ? v : (i == j ? 1.0 : 0.0);
-            X[a][bb] = 0.0;
-            Y[a][bb] = 0.0;
-        }
-    }
-    __syncthreads();                                   // src read by every thread: sm may overlap it
-    double *Lp = sm + kDgLp, *Rw = sm + kDgRow, *Wv = sm + kDgW, *Rp = sm + kDgRp;
-#pragma unroll
-    for (int kb = 0; kb < 4; kb++) {
-        const int k0 = 16 * kb;
-        // 1. publish
-#pragma unroll
-        for (int a = kb; a < 4; a++) Lp[s * kDgLs + r + 16 * a] = A[a][kb];
-#pragma unroll
-        for (int bb = 0; bb < 4; bb++)
-            Rw[r * kDgRs + s + 16 * bb] = bb < kb ? X[kb][bb] : bb == kb ? (r == s ? 1.0 : 0.0) : A[kb][bb];
-#pragma unroll
-        for (int a = 0; a <= kb; a++) Wv[s * kDgLs + r + 16 * a] = (a == kb && r == s ? 1.0 : 0.0) - Y[a][kb];
-        __syncthreads();
-        // 2. panel LU on wave 0 (rows above k0 are read and left alone)
-        if (wid == 0) {
-            double v[16];
-#pragma unroll
-            for (int q = 0; q < 16; q++) v[q] = Lp[q * kDgLs + lane];
-#pragma unroll
-            for (int q = 0; q < 16; q++) {
-                const int c = k0 + q;
-                const double rp = 1.0 / bcast(v[q], c);
-                const double l = lane > c ? v[q] * rp : 0.0;
-                if (lane > c) v[q] = l;
-#pragma unroll
-                for (int j = q + 1; j < 16; j++) v[j] = fma(-l, bcast(v[j], c), v[j]);
-                if (lane == 0) Rp[q] = rp;
-            }
-            if (lane >= k0) {
-#pragma unroll
-                for (int q = 0; q < 16; q++) Lp[q * kDgLs + lane] = v[q];
-            }
-        }
-        __syncthreads();
-        // 3. triangular solves with the panel's diagonal block; the next
-        //    column of L11 / row of U11 is loaded while the current one is used
-        if (wid == 1) {
-            double w[16], lc[2][16];
-#pragma unroll
-            for (int q = 0; q < 16; q++) w[q] = Rw[q * kDgRs + lane];
-#pragma unroll
-            for (int q = 1; q < 16; q++) lc[0][q] = Lp[k0 + q];
-#pragma unroll
-            for (int qp = 0; qp < 15; qp++) {
-                if (qp + 1 < 15) {
-#pragma unroll
-                    for (int q = qp + 2; q < 16; q++) lc[(qp + 1) & 1][q] = Lp[(qp + 1) * kDgLs + k0 + q];
-                }
-#pragma unroll
-                for (int q = qp + 1; q < 16; q++) w[q] = fma(-lc[qp & 1][q], w[qp], w[q]);
-            }
-#pragma unroll
-            for (int q = 0; q < 16; q++) Rw[q * kDgRs + lane] = w[q];
-        } else if (wid == 2) {
-            if (lane < k0 + 16) {                      // rows below hold no V
-                double w[16], uc[2][16], rq[2];
-#pragma unroll
-                for (int q = 0; q < 16; q++) w[q] = Wv[q * kDgLs + lane];
-                rq[0] = Rp[0];
-#pragma unroll
-                for (int j = 1; j < 16; j++) uc[0][j] = Lp[j * kDgLs + k0];
-#pragma unroll
-                for (int q = 0; q < 16; q++) {
-                    if (q + 1 < 16) {
-                        rq[(q + 1) & 1] = Rp[q + 1];
-#pragma unroll
-                        for (int j = q + 2; j < 16; j++) uc[(q + 1) & 1][j] = Lp[j * kDgLs + k0 + q + 1];
-                    }
-                    w[q] = w[q] * rq[q & 1];
-#pragma unroll
-                    for (int j = q + 1; j < 16; j++) w[j] = fma(-w[q], uc[q & 1][j], w[j]);
-                }
-#pragma unroll
-                for (int q = 0; q < 16; q++) Wv[q * kDgLs + lane] = w[q];
-            }
-        }
-        __syncthreads();
-        // 4. final panel values, then the rank-16 updates (operands of step
-        //    q + 1 loaded while step q is applied)
-#pragma unroll
-        for (int a = kb; a < 4; a++) A[a][kb] = Lp[s * kDgLs + r + 16 * a];
-#pragma unroll
-        for (int bb = 0; bb < 4; bb++) {
-            const double v = Rw[r * kDgRs + s + 16 * bb];
-            if (bb <= kb) X[kb][bb] = v;
-            else A[kb][bb] = v;
-        }
-#pragma unroll
-        for (int a = 0; a <= kb; a++) Y[a][kb] = Wv[s * kDgLs + r + 16 * a];
-        if (kb < 3) {
-            double lq[2][4], rq[2][4], vq[2][4];
-#pragma unroll
-            for (int a = kb + 1; a < 4; a++) lq[0][a] = Lp[r + 16 * a];
-#pragma unroll
-            for (int bb = 0; bb < 4; bb++) rq[0][bb] = Rw[s + 16 * bb];
-#pragma unroll
-            for (int a = 0; a <= kb; a++) vq[0][a] = Wv[r + 16 * a];
-#pragma unroll
-            for (int q = 0; q < 16; q++) {
-                const int cb = q & 1, nb = cb ^ 1;
-                if (q + 1 < 16) {
-#pragma unroll
-                    for (int a = kb + 1; a < 4; a++) lq[nb][a] = Lp[(q + 1) * kDgLs + r + 16 * a];
-#pragma unroll
-                    for (int bb = 0; bb < 4; bb++) rq[nb][bb] = Rw[(q + 1) * kDgRs + s + 16 * bb];
-#pragma unroll
-                    for (int a = 0; a <= kb; a++) vq[nb][a] = Wv[(q + 1) * kDgLs + r + 16 * a];
-                }
-#pragma unroll
-                for (int a = kb + 1; a < 4; a++)
-#pragma unroll
-                    for (int bb = 0; bb < 4; bb++) {
-                        if (bb > kb) A[a][bb] = fma(-lq[cb][a], rq[cb][bb], A[a][bb]);
-                        else X[a][bb] = fma(-lq[cb][a], rq[cb][bb], X[a][bb]);
-                    }
-#pragma unroll
-                for (int a = 0; a <= kb; a++)
-#pragma unroll
-                    for (int bb = kb + 1; bb < 4; bb++) Y[a][bb] = fma(vq[cb][a], rq[cb][bb], Y[a][bb]);
-            }
-        }
-        __syncthreads();                               // LDS reads done before the next sub-panel's writes
-    }
-    double *W = J.W;
-#pragma unroll
-    for (int a = 0; a < 4; a++) {
-        const int i = r + 16 * a;
-#pragma unroll
-        for (int bb = 0; bb < 4; bb++) {
-            const int j = s + 16 * bb;
-            if (i < b && j < b) Sp[(size_t)j * ld + i] = A[a][bb];
-            // W is read by other workgroups of the same update launch
-            st_coherent(&W[j * kNb + i], i > j ? X[a][bb] : (i == j ? 1.0 : 0.0));
-            st_coherent(&W[kNb * kNb + j * kNb + i], i <= j ? Y[a][bb] : 0.0);
-        }
-    }
-    // column maxima of |L| inside the block: the 16 threads of one s are
-    // consecutive lanes of one wave
-#pragma unroll
-    for (int bb = 0; bb < 4; bb++) {
-        const int j = s + 16 * bb;
-        double am = 0.0;
-#pragma unroll
-        for (int a = 0; a < 4; a++) {
-            const int i = r + 16 * a;
-            if (i > j && i < b) am = fmax(am, fabs(A[a][bb]));
-        }
-        am = max16(am);
-        if (r == 0 && j < b) atomicMax(&J.colmax[p + j], dbits(am));
+    for (int i = 0; i < H; i++) {
+        const double other = __shfl_xor(up ? a[i] : a[H + i], off, kWave);
+        a[i] = fmax(up ? a[H + i] : a[i], other);
     }
 }
-
-__global__ void __launch_bounds__(256) dense_diag_kernel(const DenseJob *jobs, const int *active, int p)
+__device__ __forceinline__ double max_scatter16(double (&a)[16], int lane, int top)
 {
-    extern __shared__ double lds[];
-    const DenseJob J = jobs[blockIdx.x];
-    if (p >= J.T || (active && !active[J.mat])) return;
-    if (threadIdx.x == 0) st_relaxed(J.flag, 0);      // no later panel final yet (read by the next launches)
-    diag_block(J, p, J.S + (size_t)p * J.T + p, (size_t)J.T, lds);
+    max_halve<8>(a, lane, top);
+    max_halve<4>(a, lane, top >> 1);
+    max_halve<2>(a, lane, top >> 2);
+    max_halve<1>(a, lane, top >> 3);
+    return a[0];
 }
 
-// ---------------------------------------------------------------------------
-// 64x64x64 tile product on 256 threads: thread (ty, tx) = (tid % 16, tid / 16)
-// accumulates rows ty + 16 i and columns tx + 16 j (i, j < 4) of As * Bs,
-// As[k*64 + i] = left(i, k), Bs[k*65 + j] = right(k, j).  Consecutive lanes
-// read consecutive LDS words.
-constexpr size_t kGemmLds = sizeof(double) * (kNb * 64 + kNb * kBsLd);
-static_assert(kDiagLds <= kGemmLds, "tile 0 of the update factors the next diagonal block in its own LDS");
-
-__device__ __forceinline__ void tile_mm(const double *As, const double *Bs, int kmax, double (&acc)[4][4])
-{
-    const int tid = threadIdx.x;
-    const int ty = tid & 15, tx = tid >> 4;
-#pragma unroll 4
-    for (int k = 0; k < kmax; k++) {
-        double a[4], bb[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) a[i] = As[k * 64 + ty + 16 * i];
-#pragma unroll
-        for (int j = 0; j < 4; j++) bb[j] = Bs[k * kBsLd + tx + 16 * j];
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int j = 0; j < 4; j++) acc[i][j] = fma(a[i], bb[j], acc[i][j]);
-    }
-}
-
-// L21 = A21 U11^-1 (64-row tiles) and U12 = L11^-1 A12 (64-column tiles) as
-// tile products with the inverses from the diagonal kernel.
-__global__ void __launch_bounds__(256) dense_trsm_kernel(const DenseJob *jobs, const int *active, int p,
-                                                         const int2 *tiles)
-{
-    const int2 tk = tiles[blockIdx.x];                 // (job, tile): only tiles that exist
-    const DenseJob J = jobs[tk.x];
-    if (p >= J.T || (active && !active[J.mat])) return;
-    const int b = min(kNb, J.T - p);
-    const int rem = J.T - p - b;
-    if (rem <= 0) return;
-    const int ntile = (rem + kNb - 1) / kNb;
-    const int t = tk.y;
-    if (t >= 2 * ntile) return;
-    extern __shared__ double lds[];
-    double *As = lds;
-    double *Bs = lds + kNb * 64;
-    const int tid = threadIdx.x;
-    const size_t ld = (size_t)J.T;
-    const double *W = J.W;
-    const bool lower = t < ntile;
-    const int r0 = p + b + t * kNb;                    // L21 tile rows
-    const int c0 = p + b + (t - ntile) * kNb;          // U12 tile columns
-    {
-        double va[16], vb[16];
-#pragma unroll
-        for (int u = 0; u < 16; u++) {
-            const int e = tid + 256 * u;
-            const int k = e >> 6, i = e & 63;
-            if (lower) {
-                const int rr = r0 + i;
-                va[u] = (rr < J.T && k < b) ? J.S[(size_t)(p + k) * ld + rr] : 0.0;
-                vb[u] = W[kNb * kNb + i * kNb + k];                     // U^-1(k, i)
-            } else {
-                va[u] = W[k * kNb + i];                                 // L^-1(i, k)
-                const int cc = c0 + k;                                  // column k of the tile, row i
-                vb[u] = (cc < J.T && i < b) ? J.S[(size_t)cc * ld + p + i] : 0.0;
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < 16; u++) {
-            const int e = tid + 256 * u;
-            const int k = e >> 6, i = e & 63;
-            As[k * 64 + i] = va[u];
-            if (lower) Bs[k * kBsLd + i] = vb[u];
-            else Bs[i * kBsLd + k] = vb[u];
-        }
-    }
-    __syncthreads();
-    double acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc[i][j] = 0.0;
-    tile_mm(As, Bs, kNb, acc);
-    const int ty = tid & 15, tx = tid >> 4;
-    if (lower) {
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int c = tx + 16 * j;
-            double am = 0.0;
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int rr = r0 + ty + 16 * i;
-                if (rr < J.T && c < b) {
-                    J.S[(size_t)(p + c) * ld + rr] = acc[i][j];
-                    am = fmax(am, fabs(acc[i][j]));
-                }
-            }
-            am = max16(am);
-            if (ty == 0 && c < b) atomicMax(&J.colmax[p + c], dbits(am));
-        }
-    } else {
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int cc = c0 + tx + 16 * j;
-            if (cc >= J.T) continue;
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int rr = ty + 16 * i;
-                if (rr < b) J.S[(size_t)cc * ld + p + rr] = acc[i][j];
-            }
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------
-// S22 -= L21 U12 on 64x64 tiles with fp64 matrix cores.  Wave w computes the
-// 32x32 quadrant (rows 32 (w & 1), columns 32 (w >> 1)) as 2x2 products of
-// v_mfma_f64_16x16x4f64, whose operands and result sit in the lanes as
-//   A(i, k): lane i + 16k      B(k, j): lane j + 16k
-//   D(i, j): lane j + 16 (i % 4), register i / 4.
-// K (the panel width) is zero-padded to a multiple of 4 in LDS.  The result
-// goes through LDS so that the read-modify-write of S runs down columns.
 typedef double v4d __attribute__((ext_vector_type(4)));
 
-// acc = As * Bs over k < kmax (a multiple of 4), As[k*64 + i], Bs[k*65 + j]
-__device__ __forceinline__ void mfma_tile(const double *As, const double *Bs, int kmax, v4d (&acc)[2][2])
-{
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, w = tid >> 6;
-    const int rb = (w & 1) * 32, cb = (w >> 1) * 32;
-    const int li = lane & 15, lk = lane >> 4;
-#pragma unroll
-    for (int x = 0; x < 2; x++)
-#pragma unroll
-        for (int y = 0; y < 2; y++) acc[x][y] = (v4d){0.0, 0.0, 0.0, 0.0};
-    for (int k4 = 0; k4 < kmax; k4 += 4) {
-        const int k = k4 + lk;
-        double av[2], bv[2];
-#pragma unroll
-        for (int x = 0; x < 2; x++) av[x] = As[k * 64 + rb + 16 * x + li];
-#pragma unroll
-        for (int y = 0; y < 2; y++) bv[y] = Bs[k * kBsLd + cb + 16 * y + li];
-#pragma unroll
-        for (int x = 0; x < 2; x++)
-#pragma unroll
-            for (int y = 0; y < 2; y++) acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[x], bv[y], acc[x][y], 0, 0, 0);
-    }
-}
-
-// The product to Cs[j*65 + i] (the caller has finished reading As / Bs if
-// they overlap Cs).
-__device__ __forceinline__ void acc_to_lds(double *Cs, const v4d (&acc)[2][2])
-{
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, w = tid >> 6;
-    const int rb = (w & 1) * 32, cb = (w >> 1) * 32;
-    const int li = lane & 15, lk = lane >> 4;
-#pragma unroll
-    for (int x = 0; x < 2; x++)
-#pragma unroll
-        for (int y = 0; y < 2; y++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int i = rb + 16 * x + 4 * r + lk;
-                const int j = cb + 16 * y + li;
-                Cs[j * kBsLd + i] = acc[x][y][r];
-            }
-}
-
-// Update launch for panel p (columns p .. q0 - 1, q0 = p + 64): tile (ti, tj)
-// of the trailing matrix from (q0, q0).  Tiles go in the order
-//   (0, 0), the next panel's diagonal block: updated, then factored here
-//        (look-ahead, while the other tiles run), W written agent-coherent,
-//        and J.flag set to q0 / 64;
-//   the next panel's edge tiles, column (ti, 0) and row (0, tj): updated,
-//        then, once J.flag says the diagonal block is factored, turned into
-//        L21 = A21 U11^-1 and U12 = L11^-1 A12 with the inverses in W;
-//   the interior tiles (ti, tj >= 1): updated.
-// An edge tile only waits on tile 0 of its job, which comes earlier in the
-// grid (dispatch order), so it is resident or done.  The wait is bounded
-// and raises the abort word if it gives up.
+// ---------------------------------------------------------------------------
+// Diagonal block: LU of a 64 x 64 block held by the four waves of a workgroup,
+// wave w its columns 16w .. 16w + 15 as the matrix cores leave them
+// (acc[x][e]: row 16x + 4e + lane / 16, column 16w + lane % 16).
+// v_mfma_f64_16x16x4f64 takes four columns of L and four rows of U, and a
+// register e of acc[x] is those four rows as its right operand, so the block is
+// factored in groups of four columns:
+//   * wave k factors its own 16 columns: per group it turns the four columns to
+//     one row per lane through LDS, eliminates them (the pivot row broadcast by
+//     readlane, l = A(i, q) / p through the pivot's reciprocal), and updates its
+//     other columns on the matrix cores: the group's rows become U = (4 x 4
+//     unit-lower inverse) acc, the rows below lose L U;
+//   * one barrier, then the waves w > k apply the four groups the same way and
+//     wave k + 1 goes on at once;
+//   * wave k meanwhile stores what the panel's other tiles need.
+// The panel's other tiles solve with L (or U^T) from the left by the same
+// groups, from two operand tiles W: at 64 c + r the entry L (r, c), negated
+// below the 4 x 4 diagonal blocks and the blocks' inverses on them; at
+// 4096 + 64 c + r the same of U^T.
 //
-// The grid is a list of the (job, tile) pairs that exist in this panel, every
-// job's tile 0 first (the longest), then the edge tiles, then the interior.
-// A rectangular grid (jobs x the largest job's tiles) is mostly workgroups
-// that return at once, and each of them still takes 66 KB of LDS on a CU
-// before it can: on 420 blocks of T 64..705 that was 42 000 workgroups for
-// panel 0, of which 9 600 have a tile.
-__global__ void __launch_bounds__(256, 2) dense_gemm_kernel(const DenseJob *jobs, const int *active, int p,
-                                                            int *abort_word, const int2 *tiles)
+// Bound by the chain of 64 pivots and by one wave's instruction issue: a group
+// (four reciprocals, two trips through LDS, two dependent products) takes
+// 0.85 us.  Per block, in the launch below on one MI355X, T = 720: 17 us, against
+// 21 us with 16-column eliminations on one wave (15 broadcasts and updates a
+// step) and 19 us with both 64 x 64 inverses carried along on the vector units.
+constexpr int kDgLd = 66;                  // column stride of a panel in LDS (two lanes per bank)
+constexpr int kDgPanel = 16 * kDgLd;       // panel: A(i, k0 + q) at q * kDgLd + i
+constexpr int kDgInv = 128;                // per group: L4^-1(i, k) at 4k + i, U4^-1(k, j) at 16 + 4k + j
+constexpr int kDgBuf = kDgPanel + kDgInv;  // two buffers: panel k + 1 is written while k is read
+constexpr size_t kDiagLds = sizeof(double) * 2 * kDgBuf;
+
+// Rows 4e .. 4e + 3 of block t become U = (inverse operand) t, the rows below
+// them lose L u; a is the group's operand of this block (rows 4e .. 4e + 3 the
+// 4 x 4 inverse, below them -L, above them anything).  Returns U as operand.
+__device__ __forceinline__ double group_solve(double a, v4d &t, int e, int li)
 {
-    const int2 tk = tiles[blockIdx.x];
-    const DenseJob J = jobs[tk.x];
-    if (p >= J.T || (active && !active[J.mat])) return;
-    const int b = min(kNb, J.T - p);
-    const int q0 = p + b;
-    const int rem = J.T - q0;
-    if (rem <= 0) return;
-    const int nt = (rem + 63) / 64;
-    const int tile = tk.y;
-    if (tile >= nt * nt) return;
-    const int ni = nt - 1;
-    int ti = 0, tj = 0;
-    if (tile > 2 * ni) {
-        ti = 1 + (tile - 1 - 2 * ni) % ni;
-        tj = 1 + (tile - 1 - 2 * ni) / ni;
-    } else if (tile > ni) {
-        tj = tile - ni;
-    } else {
-        ti = tile;
-    }
-    const int edge = tile == 0 ? 0 : tj == 0 ? 1 : ti == 0 ? 2 : 0;   // 1: L21 tile, 2: U12 tile
-    const int r0 = q0 + ti * 64;
-    const int c0 = q0 + tj * 64;
-    extern __shared__ double lds[];
-    double *As = lds;                                  // As[k*64 + i] = L21(r0+i, p+k)
-    double *Bs = lds + kNb * 64;                       // Bs[k*65 + j] = U12(p+k, c0+j)
-    const int tid = threadIdx.x;
-    const size_t ld = (size_t)J.T;
-    const int b4 = (b + 3) & ~3;
-    // 16 elements per thread of each operand; all loads are issued before
-    // the first LDS store so they are in flight together
-    {
-        double va[16], vb[16];
+    const v4d zero = (v4d){0.0, 0.0, 0.0, 0.0};
+    const double u = __builtin_amdgcn_mfma_f64_16x16x4f64((li >> 2) == e ? a : 0.0, t[e], zero, 0, 0, 0)[e];
+    t[e] = u;
+    if (e < 3) t = __builtin_amdgcn_mfma_f64_16x16x4f64((li >> 2) > e ? a : 0.0, u, t, 0, 0, 0);
+    return u;
+}
+
+// Leaves L\U of the wave's own panel in v (row lane >= 16w, column 16w + q) and
+// its U blocks above the panel in acc[x], x < w.
+__device__ __forceinline__ void diag_block(double *Wg, double *sm_, int wv, int lane_, v4d (&acc)[4], double (&v)[16])
+{
+    LSP_LDS double *sm = (LSP_LDS double *)sm_;
+    LSP_GLOBAL double *W = gp(Wg);
+#pragma unroll 1
+    for (int kb = 0; kb < 4; kb++) {
+        int lane = lane_;                       // opaque per panel: nothing lane-dependent is hoisted (and spilled)
+        asm volatile("" : "+v"(lane));
+        const int li = lane & 15, lk = lane >> 4;
+        LSP_LDS double *pn = sm + (kb & 1) * kDgBuf, *iv = pn + kDgPanel;
+        const int k0 = 16 * kb;
+        // acc[y] is row block (kb + y) % 4: the panel's own block is acc[0]
+        // throughout (the blocks rotate below), the rows below it acc[1 .. 3 - kb]
+        // (all operands are read before the first product; those past the
+        // block's end are not used)
+        auto apply = [&](int e, double inv) {
+            double a[4];
 #pragma unroll
-        for (int u = 0; u < 16; u++) {
-            const int e = tid + 256 * u;
-            const int k = e >> 6, i = e & 63;            // A: column k, row i
-            const int rr = r0 + i;
-            va[u] = (rr < J.T && k < b) ? J.S[(size_t)(p + k) * ld + rr] : 0.0;
-            const int c = c0 + k;                         // B: column k of the tile, row i of the panel
-            vb[u] = (c < J.T && i < b) ? J.S[(size_t)c * ld + p + i] : 0.0;
+            for (int y = 0; y < 4; y++) a[y] = -pn[(4 * e + lk) * kDgLd + k0 + 16 * y + li];
+            const double u = group_solve((li >> 2) == e ? inv : a[0], acc[0], e, li);
+#pragma unroll
+            for (int y = 1; y < 4; y++)
+                if (kb + y < 4) acc[y] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[y], u, acc[y], 0, 0, 0);
+            return u;
+        };
+        if (wv == kb) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int c = k0 + 4 * e;
+                if ((li >> 2) == e) {
+#pragma unroll
+                    for (int y = 0; y < 4; y++)
+                        if (kb + y < 4) {
+#pragma unroll
+                            for (int r = 0; r < 4; r++) pn[li * kDgLd + k0 + 16 * y + 4 * r + lk] = acc[y][r];
+                        }
+                }
+                wave_fence();
+                double *g = v + 4 * e;                  // the group's columns, row lane
+#pragma unroll
+                for (int q = 0; q < 4; q++) g[q] = pn[(4 * e + q) * kDgLd + lane];
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const double lq = lane > c + q ? g[q] * (1.0 / bcast(g[q], c + q)) : 0.0;
+                    if (lane > c + q) g[q] = lq;
+#pragma unroll
+                    for (int j = q + 1; j < 4; j++) g[j] = fma(-lq, bcast(g[j], c + q), g[j]);
+                }
+#pragma unroll
+                for (int q = 0; q < 4; q++) pn[(4 * e + q) * kDgLd + lane] = g[q];
+                // L4^-1 (li % 4, lk): column lk by substitution in every lane
+                double y[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    y[i] = lk == i ? 1.0 : 0.0;
+#pragma unroll
+                    for (int m = 0; m < i; m++) y[i] = fma(-bcast(g[m], c + i), y[m], y[i]);
+                }
+                const double inv = (li & 2) ? ((li & 1) ? y[3] : y[2]) : ((li & 1) ? y[1] : y[0]);
+                if (li < 4) iv[32 * e + 4 * lk + li] = inv;
+                wave_fence();
+                if (e < 3) apply(e, inv);
+            }
         }
-#pragma unroll
-        for (int u = 0; u < 16; u++) {
-            const int e = tid + 256 * u;
-            const int k = e >> 6, i = e & 63;
-            As[k * 64 + i] = va[u];
-            Bs[i * kBsLd + k] = vb[u];
-        }
-    }
-    __syncthreads();
-    v4d acc[2][2];
-    mfma_tile(As, Bs, b4, acc);
-    __syncthreads();                                   // As/Bs reads done: reuse LDS for the product
-    double *Cs = lds;                                  // Cs[j*65 + i]
-    acc_to_lds(Cs, acc);
-    __syncthreads();
-    double cv[16];
-#pragma unroll
-    for (int u = 0; u < 16; u++) {
-        const int e = tid + 256 * u;
-        const int j = e >> 6, i = e & 63;
-        const int rr = r0 + i, c = c0 + j;
-        cv[u] = (rr < J.T && c < J.T) ? J.S[(size_t)c * ld + rr] : 0.0;
-    }
-#pragma unroll
-    for (int u = 0; u < 16; u++) {
-        const int e = tid + 256 * u;
-        const int j = e >> 6, i = e & 63;
-        const int rr = r0 + i, c = c0 + j;
-        const double v = cv[u] - Cs[j * kBsLd + i];
-        cv[u] = v;
-        if (!edge && rr < J.T && c < J.T) J.S[(size_t)c * ld + rr] = v;
-        if (tile == 0) Cs[j * kBsLd + i] = v;           // element read by this thread alone above
-    }
-    if (tile == 0) {
-        // the next panel's diagonal block is final (every earlier panel's
-        // update has reached it): factor it while the other tiles run
         __syncthreads();
-        diag_block(J, q0, Cs, kBsLd, lds);
-        store_complete();                              // this wave's W stores acknowledged
-        __syncthreads();
-        if (tid == 0) st_relaxed(J.flag, q0 / kNb);
-        return;
-    }
-    if (!edge) return;
-    // Edge tile of the next panel: the updated tile in LDS as the operand it
-    // will be (L21: left, As layout; U12: right, Bs layout), then the wait
-    // for the diagonal block's inverses.
-    __syncthreads();                                   // Cs reads done
+        if (wv == kb) {
+            // operand tiles, while the others update
 #pragma unroll
-    for (int u = 0; u < 16; u++) {
-        const int e = tid + 256 * u;
-        const int j = e >> 6, i = e & 63;
-        if (edge == 1) As[j * 64 + i] = cv[u];         // left(i, k = j)
-        else Bs[i * kBsLd + j] = cv[u];                // right(k = i, j)
-    }
-    int ok = 1;
-    if (tid < kWave)
-        ok = wave_wait(tid == 0 ? J.flag : nullptr, q0 / kNb, abort_word, nullptr, -1, kSolveBackoff);
-    if (!__syncthreads_and(ok)) return;
-    const double *W = J.W;
-    {
-        double wv[16];
+            for (int q = 0; q < 16; q++) {
+                const int e = q >> 2, i = lane - k0;
+                if (lane >= k0 + 4 * e)
+                    st_coherent((double *)&W[(k0 + q) * kNb + lane],
+                                i < 4 * e + 4 ? (double)iv[32 * e + 4 * (q & 3) + (i & 3)] : -v[q]);
+            }
+            // U4^-1 of group lane % 4, row by row
+            {
+                const int e = lane & 3;
+                const LSP_LDS double *d = pn + 4 * e * kDgLd + k0 + 4 * e;
+                double rp[4];
 #pragma unroll
-        for (int u = 0; u < 16; u++) wv[u] = ld_coherent_val(&W[(edge == 1 ? kNb * kNb : 0) + tid + 256 * u]);
+                for (int k = 0; k < 4; k++) rp[k] = 1.0 / d[k * kDgLd + k];
 #pragma unroll
-        for (int u = 0; u < 16; u++) {
-            const int e = tid + 256 * u;
-            const int j = e >> 6, k = e & 63;
-            if (edge == 1) Bs[k * kBsLd + j] = wv[u];  // U11^-1(k, j)
-            else As[e] = wv[u];                        // L11^-1(i = k, j): As[j*64 + i]
+                for (int k = 0; k < 4; k++) {
+                    double z[4];
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        z[j] = j < k ? 0.0 : rp[k];
+                        if (j > k) {
+                            double t = 0.0;
+#pragma unroll
+                            for (int m = k; m < j; m++) t = fma(z[m], d[j * kDgLd + m], t);
+                            z[j] = -t * rp[j];
+                        }
+                        if (lane < 4) iv[32 * e + 16 + 4 * k + j] = z[j];
+                    }
+                }
+                wave_fence();
+            }
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if ((li >> 2) >= e)
+                    st_coherent((double *)&W[kTile + (k0 + 4 * e + lk) * kNb + k0 + li],
+                                (li >> 2) == e ? (double)iv[32 * e + 16 + 4 * lk + (li & 3)]
+                                               : -(double)pn[li * kDgLd + k0 + 4 * e + lk]);
+        } else if (wv > kb) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const double u = apply(e, iv[32 * e + 4 * lk + (li & 3)]);
+                st_coherent((double *)&W[kTile + (k0 + 4 * e + lk) * kNb + 16 * wv + li], -u);
+            }
         }
-    }
-    __syncthreads();
-    mfma_tile(As, Bs, kNb, acc);
-    __syncthreads();
-    acc_to_lds(Cs, acc);
-    __syncthreads();
-    // the panel's columns (L21) or rows (U12) of this tile, and |L| maxima
-    double am[16];
-#pragma unroll
-    for (int u = 0; u < 16; u++) {
-        const int e = tid + 256 * u;
-        const int j = e >> 6, i = e & 63;
-        const int rr = r0 + i, c = c0 + j;
-        const double v = Cs[j * kBsLd + i];
-        const bool in = rr < J.T && c < J.T;
-        if (in) J.S[(size_t)c * ld + rr] = v;
-        am[u] = in ? fabs(v) : 0.0;
-    }
-    if (edge == 1) {
-        // column j = e >> 6 = tid / 64 + 4u: a wave holds 64 rows of one column
-#pragma unroll
-        for (int u = 0; u < 16; u++) {
-            double m = am[u];
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off, kWave));
-            const int j = (tid >> 6) + 4 * u;
-            if ((tid & 63) == 0) atomicMax(&J.colmax[q0 + j], dbits(m));
-        }
+        const v4d first = acc[0];
+        acc[0] = acc[1];
+        acc[1] = acc[2];
+        acc[2] = acc[3];
+        acc[3] = first;
     }
 }
 
 // ---------------------------------------------------------------------------
-// Pivot test, scatter of the pattern slots into the sparse factors and dense
-// copy in storage precision.  One wave per item (job, column c, segment of
-// kFinishRows rows / slots); the first segment of a column tests its pivot.
-// kFinishRows / 64 loads of each kind are in flight per wave, so a segment
-// costs three dependent round trips (slot -> row and target, value, store)
-// whatever the column's length, and long columns spread over several waves.
-constexpr int kFinishRows = 512;
-constexpr int kFinishUnroll = kFinishRows / kWave;
+// The block's LU in one persistent launch over every job of the batch.
+//
+// Tile (i, j) is one task, done once: it subtracts its products
+// L(i, p) U(p, j), p < q = min(i, j), from S in registers as the operand tiles
+// become final, then
+//   i == j  factors the 64 x 64 block and publishes its inverses (diag_block),
+//   i > j   solves with U(q, q): a tile of L,
+//   i < j   solves with L(q, q): a tile of U,
+// and publishes its flag.  Workgroups of four waves take tasks from a queue
+// ordered by the panels that remain (longest block first, then by q), so a
+// task only waits on tasks handed out before it, which running workgroups
+// hold: the schedule cannot deadlock at any occupancy.  Waits are bounded.
+//
+// What bounds it: on one large block the chain from diagonal block to diagonal
+// block (27 us a panel: the block 17, its edge tiles' solve 3, two hand-offs
+// through memory 2, the next block's last product 4); on many blocks the
+// workgroups that wait in such chains.  One launch per panel, each updating the
+// whole trailing matrix, took 41 us a panel and read and wrote every trailing
+// tile once a panel.  T = 1853: 1.25 -> 0.83 ms; T = 720: 0.45 -> 0.31 ms; 420
+// blocks of T 64..705, with the former pass that scattered the block into the
+// sparse factors: 1.53 -> 0.72 ms.
+//
+// fp64 matrix cores, v_mfma_f64_16x16x4f64; operands and result sit in the
+// lanes as
+//   A(i, k): lane i + 16k      B(k, j): lane j + 16k
+//   D(i, j): lane j + 16 (i % 4), register i / 4,
+// so a D block fed back as B is the same value in the same lane: register r
+// of D holds the rows 4r .. 4r + 3 that step r of the next product needs.  A
+// wave therefore keeps all 64 rows of 16 columns, and the final solve with
+// the diagonal block needs no LDS and no barrier.  A tile of L is computed
+// transposed, which makes both kinds the same code: with r, c the result's
+// row and column, U has (r, c) = (i, j) and takes L from the left, L has
+// (r, c) = (j, i) and takes U from the left.  Final tiles go to a packed copy,
+// element (r, c) at 64 r + c, which is the layout both operands of a later
+// product are read in (coalesced, no line shared between tiles); L is stored
+// negated there, so that the matrix cores subtract.
+constexpr int kStage = 4;                  // k-steps of operands per register stage
 
-template <typename T>
-__global__ void __launch_bounds__(256) dense_finish_kernel(const DenseJob *jobs, const void *mats,
-                                                           const int *active, double ptol,
-                                                           double stol, const int4 *items, int nitems)
-{
-    const int it = uniform((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
-    if (it >= nitems) return;
-    const int4 tk = items[it];
-    const DenseJob J = jobs[tk.x];
-    const int c = tk.y;
-    const int r0 = tk.z * kFinishRows;
-    if (c >= J.T || (active && !active[J.mat])) return;
-    const FactorDesc<T> M = ((const FactorDesc<T> *)mats)[J.mat];
-    const int lane = lane_id();
-    const size_t ld = (size_t)J.T;
-    const double *Sc = J.S + (size_t)c * ld;
-    T *Fc = M.tail_F + (size_t)c * ld;
-    const int k = M.tail_k0 + c;
-    const int64_t c0 = M.cp[k];
-    const int m = (int)(M.cp[k + 1] - c0);
-    const int dl = M.dp[k] - (int)c0;
-    const int s0 = M.tail_ds[c] + r0;                  // m - tail_ds[c] <= T
+// One register stage of a product: kStage steps of both operands.
+struct TileStage {
+    double a[kStage][4], b[kStage];
+    __device__ __forceinline__ void load(const double *X, const double *Y, int s0, int wv, int li, int lk)
     {
-        double v[kFinishUnroll];
-        int ps[kFinishUnroll], ds[kFinishUnroll];
+        const LSP_GLOBAL double *xp = gp(X) + (4 * s0 + lk) * kNb + li;
+        const LSP_GLOBAL double *yp = gp(Y) + (4 * s0 + lk) * kNb + 16 * wv + li;
 #pragma unroll
-        for (int u = 0; u < kFinishUnroll; u++) {
-            const int r = r0 + u * kWave + lane;
-            v[u] = r < J.T ? Sc[r] : 0.0;
-        }
+        for (int s = 0; s < kStage; s++) {
 #pragma unroll
-        for (int u = 0; u < kFinishUnroll; u++) {
-            const int e = s0 + u * kWave + lane;
-            ps[u] = e < m ? M.pos[c0 + e] - M.tail_k0 : -1;
-            ds[u] = e < m ? M.dst[c0 + e] : 0;
-        }
-        double w[kFinishUnroll];
-#pragma unroll
-        for (int u = 0; u < kFinishUnroll; u++) w[u] = ps[u] >= 0 ? Sc[ps[u]] : 0.0;
-#pragma unroll
-        for (int u = 0; u < kFinishUnroll; u++) {
-            const int r = r0 + u * kWave + lane;
-            if (r < J.T) Fc[r] = from_f64<T>(v[u]);
-        }
-#pragma unroll
-        for (int u = 0; u < kFinishUnroll; u++) {
-            if (ps[u] < 0) continue;
-            const int e = s0 + u * kWave + lane;
-            const T f = from_f64<T>(w[u]);
-            M.val[c0 + e] = f;
-            if (e < dl) M.urow[ds[u]] = f;
-            else if (e == dl) M.diag[k] = f;
-            else M.lrow[ds[u]] = f;
+            for (int x = 0; x < 4; x++) a[s][x] = ld_coherent_val(xp, (uint32_t)(4 * s * kNb + 16 * x));
+            b[s] = ld_coherent_val(yp, (uint32_t)(4 * s * kNb));
         }
     }
-    if (lane == 0 && r0 == 0) {
-        const double piv = Sc[c];
-        const double lmax = __longlong_as_double((long long)J.colmax[c]);
-        if (piv == 0.0) {
-            atomicMin(&M.mstat[2], k);
-        } else if (!(ptol * lmax <= 1.0)) {
-            atomicAdd(&M.mstat[0], 1);
-            atomicMin(&M.mstat[1], k);
-        }
-        const double vmax = sizeof(T) == 2 ? 65504.0 : sizeof(T) == 4 ? 3.4028234663852886e38 : 1.0e308;
-        if (!(fabs(piv) <= vmax) || !(lmax <= vmax)) atomicAdd(&M.mstat[3], 1);
-        if (stol > 0.0) {
-            // splu's choice on these values, in units of |pivot|: the other
-            // candidates are the multipliers L(r, c), r > c, of the block
-            const int dpos = M.dpos[k];
-            const double md = dpos > k ? fabs(Sc[dpos - M.tail_k0]) : -1.0;
-            const int v = piv == 0.0 ? (lmax > 0.0 ? 1 : 0)
-                                     : splu_pivot_verdict(dpos == k, 1.0, lmax, md, stol);
-            if (v) {
-                atomicAdd(&M.mstat[v == 1 ? 4 : 5], 1);
-                atomicMin(&M.mstat[6], k);
+    __device__ __forceinline__ void apply(v4d (&acc)[4]) const
+    {
+#pragma unroll
+        for (int s = 0; s < kStage; s++)
+#pragma unroll
+            for (int x = 0; x < 4; x++) acc[x] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s][x], b[s], acc[x], 0, 0, 0);
+    }
+};
+
+template <typename T>
+__global__ void __launch_bounds__(256, 2) dense_lu_kernel(const DenseJob *jobs, const void *mats, const int *active,
+                                                          const int4 *tasks, int ntask, int *ctr, int *epoch_word,
+                                                          int *abort_word)
+{
+    extern __shared__ double lds[];
+    __shared__ int s_t;
+    const int epoch = read_epoch(epoch_word);
+    for (;;) {
+        // opaque per task: the compiler would otherwise hoist every lane
+        // address of the body out of the loop and spill them
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        const int lane = tid & (kWave - 1), wv = uniform(tid >> 6);
+        const int li = lane & 15, lk = lane >> 4;
+        // one ticket per workgroup; an abort is seen by all its waves or none
+        if (tid == 0) s_t = aborted(abort_word) ? ntask : wave_ticket(ctr);
+        __syncthreads();
+        const int t = uniform(s_t);
+        __syncthreads();
+        if (t >= ntask) break;
+        const int4 tk = tasks[t];
+        const DenseJob J = jobs[tk.x];
+        if (active && !active[J.mat]) continue;
+        T *F = ((const FactorDesc<T> *)mats)[J.mat].tail_F;
+        const int ti = tk.y, tj = tk.z;
+        const int q = min(ti, tj);
+        const bool low = ti > tj;                       // a tile of L: (r, c) = (j, i)
+        const int nt = J.nt;
+        const size_t ld = (size_t)J.T;
+        const int *ready = J.flag;
+        // the result's rows r come from tile row / column q, its columns c from the other index
+        const int r0 = q * kNb, c0 = (low ? ti : tj) * kNb;
+        const int c = c0 + 16 * wv + li;
+        // S(i, j) at rs * r + cs * c; rows and columns past T are zero (a
+        // diagonal block's are the identity's)
+        const size_t rs = low ? ld : 1, cs = low ? 1 : ld;
+        v4d acc[4];
+#pragma unroll
+        for (int x = 0; x < 4; x++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int r = r0 + 16 * x + 4 * e + lk;
+                const double v = gp(J.S)[rs * min(r, J.T - 1) + cs * min(c, J.T - 1)];
+                acc[x][e] = r < J.T && c < J.T ? v : (ti == tj && r == c ? 1.0 : 0.0);
             }
+        // operand tiles of product p: X left (rows r), Y right (columns c)
+        const int xs = low ? nt : 1, xo = low ? q : q * nt;           // L(q, p) or U(p, q)
+        const int ys = low ? 1 : nt, yo = low ? ti * nt : tj;         // U(p, j) or L(i, p)
+        int ok = 1;
+        for (int p0 = 0; p0 < q && ok; p0 += kWave / 2) {
+            // lanes 2p, 2p + 1: the flags of product p's two tiles
+            const int np = min(kWave / 2, q - p0);
+            const int p = p0 + (lane >> 1);
+            const int *flag = p < q ? &ready[(lane & 1) ? ys * p + yo : xs * p + xo] : nullptr;
+            int seen = flag == nullptr;
+            for (int done = 0, have = 0; done < np;) {
+                const int pre = wave_wait_prefix(flag, epoch, abort_word, seen, have, 2 * np, nullptr, -1, kSolveBackoff);
+                if (pre < 0) {
+                    ok = 0;
+                    break;
+                }
+                have = pre;
+                const int np1 = (pre >> 1) - done;      // products ready now
+                if (np1 <= 0) continue;
+                const int pb = p0 + done;
+                auto xt = [&](int n) { return J.P + (size_t)(xs * (pb + n) + xo) * kTile; };
+                auto yt = [&](int n) { return J.P + (size_t)(ys * (pb + n) + yo) * kTile; };
+                static_assert(4 * kStage == 16, "a product is four stages");
+                TileStage s0, s1;
+                s0.load(xt(0), yt(0), 0, wv, li, lk);
+                for (int n = 0; n < np1; n++) {
+                    // each product is summed by itself and added once: one
+                    // rounding at the magnitude of S per 64 terms, not 64
+                    v4d t[4];
+#pragma unroll
+                    for (int x = 0; x < 4; x++) t[x] = (v4d){0.0, 0.0, 0.0, 0.0};
+                    s1.load(xt(n), yt(n), kStage, wv, li, lk);
+                    s0.apply(t);
+                    s0.load(xt(n), yt(n), 2 * kStage, wv, li, lk);
+                    s1.apply(t);
+                    s1.load(xt(n), yt(n), 3 * kStage, wv, li, lk);
+                    s0.apply(t);
+                    if (n + 1 < np1) s0.load(xt(n + 1), yt(n + 1), 0, wv, li, lk);
+                    s1.apply(t);
+#pragma unroll
+                    for (int x = 0; x < 4; x++) acc[x] += t[x];
+                }
+                done = pre >> 1;
+            }
+        }
+        if (ti == tj) {
+            if (!__syncthreads_and(ok)) continue;
+            double v[16];
+            diag_block(J.W + (size_t)q * 2 * kTile, lds, wv, lane, acc, v);
+            store_complete();
+            __syncthreads();
+            if (tid == 0) st_relaxed(&J.flag[(size_t)q * (nt + 1)], epoch);
+            // what only later launches read: the factor in place and in
+            // storage precision, and the column maxima of |L|
+            auto put = [&](int r, int cc, double f) {
+                if (r < J.T && cc < J.T) {
+                    gp(J.S)[ld * cc + r] = f;
+                    if constexpr (sizeof(T) != 8) st_g(&F[ld * cc + r], from_f64<T>(f));
+                }
+            };
+            double am[16];
+#pragma unroll
+            for (int e = 0; e < 16; e++) am[e] = lane > 16 * wv + e && r0 + lane < J.T ? fabs(v[e]) : 0.0;
+            double mx = max_scatter16(am, lane, 32);    // lanes 4e .. 4e + 3: column e
+            mx = fmax(mx, __shfl_xor(mx, 2, kWave));
+            mx = fmax(mx, __shfl_xor(mx, 1, kWave));
+            const int mc = r0 + 16 * wv + (lane >> 2);
+            if ((lane & 3) == 0 && mc < J.T) atomicMax(&J.colmax[mc], dbits(mx));
+            if (lane >= 16 * wv) {
+#pragma unroll
+                for (int e = 0; e < 16; e++) put(r0 + lane, r0 + 16 * wv + e, v[e]);
+            }
+#pragma unroll
+            for (int x = 0; x < 3; x++)
+                if (x < wv) {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) put(r0 + 16 * x + 4 * e + lk, c, acc[x][e]);
+                }
+            continue;
+        }
+        // the panel's triangle from the left, by groups of four rows
+        ok = ok && wave_wait(lane == 0 ? &ready[(size_t)q * (nt + 1)] : nullptr, epoch, abort_word, nullptr, -1,
+                             kSolveBackoff);
+        if (ok) {
+            const LSP_GLOBAL double *wp = gp(J.W) + (size_t)q * 2 * kTile + (low ? kTile : 0) + lk * kNb + li;
+            double w[16][4];
+#pragma unroll
+            for (int s = 0; s < 16; s++)
+#pragma unroll
+                for (int x = s / 4; x < 4; x++) w[s][x] = ld_coherent_val(wp, (uint32_t)(4 * s * kNb + 16 * x));
+#pragma unroll
+            for (int s = 0; s < 16; s++) {
+                const double u = group_solve(w[s][s / 4], acc[s / 4], s % 4, li);
+#pragma unroll
+                for (int x = s / 4 + 1; x < 4; x++)
+                    acc[x] = __builtin_amdgcn_mfma_f64_16x16x4f64(w[s][x], u, acc[x], 0, 0, 0);
+            }
+            double *Pt = J.P + (size_t)(ti * nt + tj) * kTile;
+#pragma unroll
+            for (int x = 0; x < 4; x++)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    st_coherent(&Pt[(16 * x + 4 * e + lk) * kNb + 16 * wv + li], low ? -acc[x][e] : acc[x][e]);
+            store_complete();
+        }
+        if (!__syncthreads_and(ok)) continue;
+        if (tid == 0) st_relaxed(&J.flag[(size_t)ti * nt + tj], epoch);
+        // what only later launches read: the factor in place and in storage
+        // precision, and the column maxima of |L| for the pivot test
+        // (rows opaque again, or the first loads' addresses stay live)
+        int rl = r0 + lk;
+        asm volatile("" : "+v"(rl));
+        double am[16];
+#pragma unroll
+        for (int x = 0; x < 4; x++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int r = rl + 16 * x + 4 * e;
+                const bool in = r < J.T && c < J.T;
+                am[4 * x + e] = in ? fabs(acc[x][e]) : 0.0;
+                if (in) {
+                    const size_t at = rs * r + cs * c;
+                    gp(J.S)[at] = acc[x][e];
+                    if constexpr (sizeof(T) != 8) st_g(&F[at], from_f64<T>(acc[x][e]));
+                }
+            }
+        if (low) {
+            const double mx = max_scatter16(am, lane, 8);   // lane li: register li's row of the result
+            const int r = rl + 4 * li;
+            if (r < J.T) atomicMax(&J.colmax[r], dbits(mx));
+        }
+    }
+    if (threadIdx.x < kWave && leave_queue(ctr, 1, (int)gridDim.x)) advance_epoch(epoch_word, epoch);
+}
+
+// ---------------------------------------------------------------------------
+// One thread per block column: pivot test and the diagonal of the factors.
+template <typename T>
+__global__ void __launch_bounds__(256) dense_pivot_kernel(const DenseJob *jobs, const void *mats, const int *active,
+                                                          double ptol, double stol, const int2 *items)
+{
+    const int2 tk = items[blockIdx.x];
+    const DenseJob J = jobs[tk.x];
+    const int c = tk.y * 256 + (int)threadIdx.x;
+    if (c >= J.T || (active && !active[J.mat])) return;
+    const FactorDesc<T> M = ((const FactorDesc<T> *)mats)[J.mat];
+    const double *Sc = J.S + (size_t)c * (size_t)J.T;
+    const int k = M.tail_k0 + c;
+    const double piv = Sc[c];
+    const double lmax = __longlong_as_double((long long)J.colmax[c]);
+    M.diag[k] = from_f64<T>(piv);
+    if (piv == 0.0) {
+        atomicMin(&M.mstat[2], k);
+    } else if (!(ptol * lmax <= 1.0)) {
+        atomicAdd(&M.mstat[0], 1);
+        atomicMin(&M.mstat[1], k);
+    }
+    const double vmax = sizeof(T) == 2 ? 65504.0 : sizeof(T) == 4 ? 3.4028234663852886e38 : 1.0e308;
+    if (!(fabs(piv) <= vmax) || !(lmax <= vmax)) atomicAdd(&M.mstat[3], 1);
+    if (stol > 0.0) {
+        // splu's choice on these values, in units of |pivot|: the other
+        // candidates are the multipliers L(r, c), r > c, of the block
+        const int dpos = M.dpos[k];
+        const double md = dpos > k ? fabs(Sc[dpos - M.tail_k0]) : -1.0;
+        const int v = piv == 0.0 ? (lmax > 0.0 ? 1 : 0) : splu_pivot_verdict(dpos == k, 1.0, lmax, md, stol);
+        if (v) {
+            atomicAdd(&M.mstat[v == 1 ? 4 : 5], 1);
+            atomicMin(&M.mstat[6], k);
         }
     }
 }
@@ -918,74 +731,63 @@ __global__ void __launch_bounds__(512) tail_trsv_kernel(const void *mats, const 
 // ---------------------------------------------------------------------------
 // host launchers
 // ---------------------------------------------------------------------------
-hipError_t dense_set_lds()
+template <typename T>
+hipError_t launch_dense_lu(const DenseJob *jobs, const void *mats, const int *active, const DenseGrid &G, int *ctr,
+                           int *epoch, int *abort_word, int blocks, double ptol, double stol, hipStream_t st)
 {
-    hipError_t e = hipFuncSetAttribute((const void *)dense_gemm_kernel,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGemmLds);
-    if (e != hipSuccess) return e;
-    return hipFuncSetAttribute((const void *)dense_trsm_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)kGemmLds);
-}
-
-// Panel 0's diagonal block has a launch of its own; every later diagonal
-// block is factored by tile 0 of the preceding trailing update.  For a job
-// whose T is below maxT the update kernel returns before its tiles once
-// p + 64 >= T, so each of its panels is factored exactly once.
-hipError_t launch_dense_lu(const DenseJob *jobs, int njobs, int maxT, const int *active, int *abort_word,
-                           const DenseGrid &G, hipStream_t st)
-{
-    if (maxT <= 0) return hipSuccess;
-    hipLaunchKernelGGL(dense_diag_kernel, dim3(njobs), dim3(256), kDiagLds, st, jobs, active, 0);
-    if (G.ntrsm)
-        hipLaunchKernelGGL(dense_trsm_kernel, dim3(G.ntrsm), dim3(256), kGemmLds, st, jobs, active, 0, G.trsm);
-    for (size_t i = 0; i + 1 < G.panel.size(); i++) {
-        const long cnt = G.panel[i + 1] - G.panel[i];
-        hipLaunchKernelGGL(dense_gemm_kernel, dim3((unsigned)cnt), dim3(256), kGemmLds, st, jobs, active,
-                           (int)i * kNb, abort_word, G.gemm + G.panel[i]);
-    }
+    hipLaunchKernelGGL(dense_lu_kernel<T>, dim3(std::min(blocks, G.nlu)), dim3(256), kDiagLds, st, jobs, mats, active,
+                       G.lu, G.nlu, ctr, epoch, abort_word);
+    hipLaunchKernelGGL(dense_pivot_kernel<T>, dim3(G.npivot), dim3(256), 0, st, jobs, mats, active, ptol, stol,
+                       G.pivot);
     return hipGetLastError();
 }
+template hipError_t launch_dense_lu<float>(const DenseJob *, const void *, const int *, const DenseGrid &, int *, int *,
+                                           int *, int, double, double, hipStream_t);
+template hipError_t launch_dense_lu<double>(const DenseJob *, const void *, const int *, const DenseGrid &, int *, int *,
+                                           int *, int, double, double, hipStream_t);
+template hipError_t launch_dense_lu<__half>(const DenseJob *, const void *, const int *, const DenseGrid &, int *, int *,
+                                           int *, int, double, double, hipStream_t);
 
 // The lists behind the grids (see DenseGrid): jobs by falling T, so that the
 // longest ones start first.
 void dense_grid_lists(const std::vector<int> &T, const std::vector<int> &mat, DenseGridHost &H)
 {
     const int nj = (int)T.size();
-    const int maxT = nj ? T[0] : 0;
     H = DenseGridHost();
-    H.panel.push_back(0);
-    for (int p = 0; p + kNb < maxT; p += kNb) {
-        auto nt = [&](int j) { return T[j] > p + kNb ? (T[j] - p - kNb + kNb - 1) / kNb : 0; };
-        for (int j = 0; j < nj && nt(j); j++) H.gemm.push_back(make_int2(j, 0));
-        for (int j = 0; j < nj && nt(j); j++)
-            for (int t = 1; t <= 2 * (nt(j) - 1); t++) H.gemm.push_back(make_int2(j, t));
-        for (int j = 0; j < nj && nt(j); j++)
-            for (int t = 2 * (nt(j) - 1) + 1; t < nt(j) * nt(j); t++) H.gemm.push_back(make_int2(j, t));
-        if (p == 0)
-            for (int j = 0; j < nj && nt(j); j++)
-                for (int t = 0; t < 2 * nt(j); t++) H.trsm.push_back(make_int2(j, t));
-        H.panel.push_back((long)H.gemm.size());
+    // Tiles by the panels that remain from theirs on.  Of one panel: the
+    // diagonal blocks, then the previous panel's other tiles (ready by now;
+    // put right after their own diagonal block they would hold a workgroup
+    // each while it is factored), then the two tiles the next diagonal block
+    // waits for.
+    const int most = nj ? (T[0] + kNb - 1) / kNb : 0;
+    auto panels = [&](int left, auto put) {
+        for (int j = 0; j < nj; j++) {
+            const int nt = (T[j] + kNb - 1) / kNb;
+            if (nt < left) break;                        // smaller blocks start later
+            put(j, nt, nt - left);
+        }
+    };
+    for (int left = most; left >= 0; left--) {
+        panels(left, [&](int j, int nt, int q) { if (q < nt) H.lu.push_back(make_int4(j, q, q, 0)); });
+        panels(left + 1, [&](int j, int nt, int q) {
+            for (int i = q + 2; i < nt; i++) {
+                H.lu.push_back(make_int4(j, i, q, 0));
+                H.lu.push_back(make_int4(j, q, i, 0));
+            }
+        });
+        panels(left, [&](int j, int nt, int q) {
+            if (q + 1 < nt) {
+                H.lu.push_back(make_int4(j, q + 1, q, 0));
+                H.lu.push_back(make_int4(j, q, q + 1, 0));
+            }
+        });
     }
     for (int j = 0; j < nj; j++) {
-        for (int c = 0; c < T[j]; c++)
-            for (int g = 0; g * kFinishRows < T[j]; g++) H.finish.push_back(make_int4(j, c, g, 0));
+        for (int c = 0; c * 256 < T[j]; c++) H.pivot.push_back(make_int2(j, c));
         for (int g = 0; g * 4 < T[j]; g++) H.gather.push_back(make_int2(mat[j], g));
         for (int t = 0; t * 2 * kNb < T[j]; t++) H.trsv.push_back(make_int2(mat[j], t));
     }
 }
-
-template <typename T>
-hipError_t launch_dense_finish(const DenseJob *jobs, const void *mats, const int *active, double ptol, double stol,
-                               const DenseGrid &G, hipStream_t st)
-{
-    if (!G.nfinish) return hipSuccess;
-    hipLaunchKernelGGL(dense_finish_kernel<T>, dim3((G.nfinish + 3) / 4), dim3(256), 0, st, jobs, mats, active, ptol,
-                       stol, G.finish, G.nfinish);
-    return hipGetLastError();
-}
-template hipError_t launch_dense_finish<float>(const DenseJob *, const void *, const int *, double, double, const DenseGrid &, hipStream_t);
-template hipError_t launch_dense_finish<double>(const DenseJob *, const void *, const int *, double, double, const DenseGrid &, hipStream_t);
-template hipError_t launch_dense_finish<__half>(const DenseJob *, const void *, const int *, double, double, const DenseGrid &, hipStream_t);
 
 template <typename T>
 hipError_t launch_tail_solve(const void *mats, const DenseGrid &G, const long *voff, const int *active,

@@ -56,7 +56,7 @@ struct FactorDesc {
     const int *tail_ds;     // tail_T: sparse dependencies of tail column c
     double *tail_S;         // tail_T^2 fp64 work block, column-major
     unsigned long long *tail_colmax;   // tail_T: max |L(i,c)| as bit patterns
-    T *tail_F;              // tail_T^2 factor copy in storage precision
+    T *tail_F;              // tail_T^2 factor in storage precision (tail_S itself for fp64)
     int n;
     int tail_k0;
     int tail_T;
@@ -92,14 +92,18 @@ struct TriDesc {
     int pad_;
 };
 
-// One dense trailing block to factor (fp64 work, fixed pivot order).
+// One dense trailing block to factor (fp64 work, fixed pivot order), nt x nt
+// tiles of 64 x 64.
 struct DenseJob {
     double *S;              // T x T, column-major, leading dimension T
-    double *W;              // 2 x 64 x 64 workspace: inverses of the current diagonal block
+    double *P;              // nt * nt packed tiles: the final tiles of L and U as operands
+    double *W;              // per panel 2 x 64 x 64: its diagonal block's factors as operands (dense.hip)
     unsigned long long *colmax;
-    int *flag;              // panel whose diagonal block (and W) is final, during an update launch
+    int *flag;              // nt * nt: epoch of the launch that made the tile final
     int T;
+    int nt;
     int mat;                // matrix index (descriptor, mstat, active mask)
+    int pad_;
 };
 
 // SELL-C-sigma SpMV with C = 64 (one wave per slice, one lane per row).

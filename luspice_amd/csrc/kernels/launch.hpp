@@ -101,29 +101,23 @@ hipError_t launch_fill_unset(const void *mats, const int *active, const int2 *ch
                              int *dbg, hipStream_t st);
 
 // dense trailing blocks (dense.hip)
-hipError_t dense_set_lds();
 // Grids of the dense-block kernels as lists of the work items that exist, so
 // that blocks of uneven order in one batch launch no empty workgroups.  Jobs
 // are numbered by falling T.
 struct DenseGridHost {
-    std::vector<int2> gemm, trsm;        // (job, tile): update tiles panel by panel; panel 0's TRSM tiles
-    std::vector<long> panel;             // first entry of each panel in gemm, and the end
-    std::vector<int4> finish;            // (job, column, segment)
+    std::vector<int4> lu;                // (job, tile row, tile column) in dependency order
+    std::vector<int2> pivot;             // (job, group of 256 columns)
     std::vector<int2> gather, trsv;      // (matrix, group of 4 rows), (matrix, pair of 64-row blocks)
 };
 struct DenseGrid {
-    const int2 *gemm = nullptr, *trsm = nullptr;
-    const int4 *finish = nullptr;
-    const int2 *gather = nullptr, *trsv = nullptr;
-    std::vector<long> panel;
-    int ntrsm = 0, nfinish = 0, ngather = 0, ntrsv = 0;
+    const int4 *lu = nullptr;
+    const int2 *pivot = nullptr, *gather = nullptr, *trsv = nullptr;
+    int nlu = 0, npivot = 0, ngather = 0, ntrsv = 0;
 };
 void dense_grid_lists(const std::vector<int> &T, const std::vector<int> &mat, DenseGridHost &H);
-hipError_t launch_dense_lu(const DenseJob *jobs, int njobs, int maxT, const int *active, int *abort_word,
-                           const DenseGrid &G, hipStream_t st);
 template <typename T>
-hipError_t launch_dense_finish(const DenseJob *jobs, const void *mats, const int *active, double ptol, double stol,
-                               const DenseGrid &G, hipStream_t st);
+hipError_t launch_dense_lu(const DenseJob *jobs, const void *mats, const int *active, const DenseGrid &G, int *ctr,
+                           int *epoch, int *abort_word, int blocks, double ptol, double stol, hipStream_t st);
 template <typename T>
 hipError_t launch_tail_solve(const void *mats, const DenseGrid &G, const long *voff, const int *active,
                              const double *b, double *y, double *yp, double *z, double *x, bool forward,

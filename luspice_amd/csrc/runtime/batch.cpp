@@ -267,7 +267,9 @@ int Batch::ensure_factor_set(FactorSet<T> &fs)
     fs.lrow = (T *)dalloc(nl_tot_ * sizeof(T));
     fs.urow = (T *)dalloc(nu_tot_ * sizeof(T));
     fs.diag = (T *)dalloc(ntot_ * sizeof(T));
-    fs.tailF = (T *)dalloc(nt2_tot_ * sizeof(T));
+    // fp64 factors of the dense blocks stay where they were computed
+    if constexpr (std::is_same<T, double>::value) fs.tailF = d_tailS_;
+    else fs.tailF = (T *)dalloc(nt2_tot_ * sizeof(T));
     if (!fs.val || !fs.lrow || !fs.urow || !fs.diag || !fs.tailF) return LSP_E_ALLOC;
     const int nc = (int)circ_.size();
     std::vector<FactorDesc<T>> fd(nc);
@@ -438,7 +440,7 @@ int Batch::set_active(const int *mask)
 // (an upper estimate used for admission; device_bytes() reports the actual).
 size_t Batch::estimate_device_bytes() const
 {
-    double n = 0, nnz = 0, slots = 0, rel = 0, nlu = 0, sell = 0, slices = 0, T = 0, T2 = 0, lists = 0;
+    double n = 0, nnz = 0, slots = 0, rel = 0, nlu = 0, sell = 0, slices = 0, T = 0, T2 = 0, lists = 0, tiles = 0;
     double maxcol = 0;
     const double nc = (double)circ_.size();
     for (const auto &C : circ_) {
@@ -446,8 +448,9 @@ size_t Batch::estimate_device_bytes() const
         n += C.n; nnz += C.nnz; slots += (double)P.cp[C.n]; rel += (double)P.relp[C.n];
         nlu += (double)(P.n_l + P.n_u); sell += (double)C.sell.slots; slices += C.sell.nslices;
         T += P.tail_T; T2 += (double)P.tail_T * P.tail_T;
-        const double nt = (P.tail_T + 63) / 64;                           // update tiles of every panel, TRSM tiles
-        lists += nt * nt * nt / 3 + 2 * nt + 2.0 * P.tail_T * (1 + P.tail_T / 512) + P.tail_T / 4 + nt;
+        const double nt = (P.tail_T + 63) / 64;                           // tiles, their packed copies and inverses
+        lists += 2 * nt * nt + P.tail_T / 4 + 8 * nt;
+        tiles += nt * nt + 2 * nt;
         maxcol = std::max(maxcol, (double)P.max_col);
     }
     const double m = std::max(1, opt_.ir_inner);
@@ -459,11 +462,11 @@ size_t Batch::estimate_device_bytes() const
     if (opt_.krylov_spmv == 2) b += 2 * sell;                              // FP16 SELL values
     b += 16 * nnz + 24 * n + 16 * (nc + 1);                               // Ruiz: row/col, scaled values, scales
     if (opt_.factor_shift > 0.0) b += 8 * n;                               // shifted diagonal entries
-    b += 8 * T2 + 16 * T + 65536.0 * nc;                                   // dense block work
+    b += 8 * T2 + 16 * T + 8.0 * 64 * 64 * tiles;                          // dense block work
     b += 24 * n + 8 * slices + 16 * n;                                    // task lists, row packets
     b += 8 * lists + 8 * (slots / kFillSlots + nc);                       // dense-block and fill work lists
     b += 64 * n + 8 * (2 * m + 1) * n;                                    // vectors, Krylov bases V and Z
-    b += (4 + 8) * (slots + nlu + n + T2);                                 // fp32 + fp64 factor sets
+    b += (4 + 8) * (slots + nlu + n) + 4 * T2;                             // fp32 + fp64 factor sets
     if (maxcol > std::max(1, opt_.lds_cap)) b += 256.0 * 8 * 4 * maxcol * 8;   // global column scratch
     return (size_t)(1.05 * b) + (1u << 20);
 }
@@ -605,7 +608,7 @@ int Batch::upload_all()
         std::vector<int> zeros(ntot_, 0);
         d_done_ = upload(zeros);
         std::vector<int> z6(8, 0);
-        std::vector<int> zq(3 * kQueueInts, 0);    // refactor, forward, backward queue blocks
+        std::vector<int> zq(4 * kQueueInts, 0);    // refactor, forward, backward, dense-block queue blocks
         d_ctr_ = upload(zq); d_abort_ = upload(z6);
         std::vector<int> e1(4, 1);                 // epochs start at 1, flags at 0
         d_epoch_ = upload(e1);
@@ -631,32 +634,41 @@ int Batch::upload_all()
         std::stable_sort(mat.begin(), mat.end(),
                          [&](int a, int b) { return circ_[a].plan.tail_T > circ_[b].plan.tail_T; });
         njobs_ = (int)mat.size();
-        d_tailW_ = (double *)dalloc((size_t)std::max(njobs_, 1) * 2 * 64 * 64 * sizeof(double));
-        d_dflag_ = upload(std::vector<int>(std::max(njobs_, 1), 0));
-        if (!d_tailS_ || !d_colmax_ || !d_tailW_ || !d_dflag_) return LSP_E_ALLOC;
+        size_t ntile = 0, npanel = 0;
+        for (int m : mat) {
+            const size_t nt = (circ_[m].plan.tail_T + 63) / 64;
+            ntile += nt * nt;
+            npanel += nt;
+        }
+        d_tailW_ = (double *)dalloc(npanel * 2 * 64 * 64 * sizeof(double));
+        d_tailP_ = (double *)dalloc(ntile * 64 * 64 * sizeof(double));
+        d_dflag_ = upload(std::vector<int>(ntile, 0));
+        if (!d_tailS_ || !d_colmax_ || !d_tailW_ || !d_tailP_ || !d_dflag_) return LSP_E_ALLOC;
+        ntile = npanel = 0;
         for (int m : mat) {
             const CircuitHost &C = circ_[m];
             DenseJob J{};
-            J.S = d_tailS_ + C.o_t2;
-            J.W = d_tailW_ + jobs.size() * 2 * 64 * 64;
-            J.colmax = d_colmax_ + C.o_t;
-            J.flag = d_dflag_ + jobs.size();
             J.T = C.plan.tail_T;
+            J.nt = (J.T + 63) / 64;
+            J.S = d_tailS_ + C.o_t2;
+            J.P = d_tailP_ + ntile * 64 * 64;
+            J.W = d_tailW_ + npanel * 2 * 64 * 64;
+            J.colmax = d_colmax_ + C.o_t;
+            J.flag = d_dflag_ + ntile;
             J.mat = m;
             jobs.push_back(J);
             order.push_back(J.T);
+            ntile += (size_t)J.nt * J.nt;
+            npanel += J.nt;
         }
-        max_tail_T_ = njobs_ ? order[0] : 0;
         DenseGridHost H;
         dense_grid_lists(order, mat, H);
-        dgrid_.gemm = upload(H.gemm);
-        dgrid_.trsm = upload(H.trsm);
-        dgrid_.finish = upload(H.finish);
+        dgrid_.lu = upload(H.lu);
+        dgrid_.pivot = upload(H.pivot);
         dgrid_.gather = upload(H.gather);
         dgrid_.trsv = upload(H.trsv);
-        dgrid_.panel = H.panel;
-        dgrid_.ntrsm = (int)H.trsm.size();
-        dgrid_.nfinish = (int)H.finish.size();
+        dgrid_.nlu = (int)H.lu.size();
+        dgrid_.npivot = (int)H.pivot.size();
         dgrid_.ngather = (int)H.gather.size();
         dgrid_.ntrsv = (int)H.trsv.size();
         d_tail_ds_ = upload(tds);
@@ -671,13 +683,9 @@ int Batch::upload_all()
         }
         d_fillchunk_ = upload(fill);
         nfillchunk_ = (int)fill.size();
-        if (!d_tail_ds_ || !d_tail_lcut_ || !d_djobs_ || !d_tail_ctr_ || !d_fillchunk_ || !dgrid_.gemm ||
-            !dgrid_.trsm || !dgrid_.finish || !dgrid_.gather || !dgrid_.trsv)
+        if (!d_tail_ds_ || !d_tail_lcut_ || !d_djobs_ || !d_tail_ctr_ || !d_fillchunk_ || !dgrid_.lu ||
+            !dgrid_.pivot || !dgrid_.gather || !dgrid_.trsv)
             return LSP_E_ALLOC;
-        if (njobs_) {
-            rc = check(dense_set_lds(), "dense lds attr");
-            if (rc) return rc;
-        }
     }
     d_ain_ = (double *)dalloc(nnz_tot_ * sizeof(double));
     // Ruiz equilibration for FP16 factor storage: per-entry circuit-local
@@ -1012,10 +1020,9 @@ int Batch::refactor_t(FactorSet<T> &fs, const int *d_active)
     rc = check(launch_refactor<T>(L, fblocks_, stream_), "refactor launch");
     if (!capturing_) (void)hipEventRecord(ev_[1], stream_);      // the persistent kernel alone
     if (!rc && njobs_) {
-        rc = check(launch_dense_lu(d_djobs_, njobs_, max_tail_T_, d_active, d_abort_, dgrid_, stream_), "dense lu");
-        if (!rc)
-            rc = check(launch_dense_finish<T>(d_djobs_, fs.fdesc, d_active, opt_.refactor_ptol, L.stol, dgrid_,
-                                              stream_), "dense finish");
+        // two 4-wave workgroups per CU (the kernel's register budget)
+        rc = check(launch_dense_lu<T>(d_djobs_, fs.fdesc, d_active, dgrid_, d_ctr_ + 3 * kQueueInts, d_epoch_ + 1,
+                                      d_abort_, 2 * cu_count_, opt_.refactor_ptol, L.stol, stream_), "dense lu");
     }
     if (!capturing_) (void)hipEventRecord(ev_[5], stream_);      // + dense trailing block
     return rc;
@@ -1786,6 +1793,22 @@ int Batch::export_factors(int c, int *pinv, int *Lp, int *Li, double *Lx, int *U
         for (long i = 0; i < ns; i++) v[i] = (double)__half2float(f[i]);
     }
     if (rc) return rc;
+    if (P.tail_T > 0) {
+        // the block's own entries live in its dense factor only
+        const size_t t2 = (size_t)P.tail_T * P.tail_T;
+        auto fetch = [&](auto *dev, auto conv) {
+            std::vector<std::decay_t<decltype(*dev)>> h(t2);
+            const int r = check(hipMemcpy(h.data(), dev + C.o_t2, t2 * sizeof(*dev), hipMemcpyDeviceToHost), "export");
+            for (int k = P.tail_k0; !r && k < C.n; k++)
+                for (long s = P.cp[k] + P.tail_ds[k - P.tail_k0]; s < P.cp[k + 1]; s++)
+                    v[s] = conv(h[(size_t)(k - P.tail_k0) * P.tail_T + (P.pos[s] - P.tail_k0)]);
+            return r;
+        };
+        if (cur_prec_ == LSP_PREC_FP64) rc = fetch(f64_.tailF, [](double x) { return x; });
+        else if (cur_prec_ == LSP_PREC_FP32) rc = fetch(f32_.tailF, [](float x) { return (double)x; });
+        else rc = fetch(f16_.tailF, [](__half x) { return (double)__half2float(x); });
+        if (rc) return rc;
+    }
     if (pinv) std::copy(P.pinv.begin(), P.pinv.end(), pinv);
     long l = 0, u = 0;
     for (int k = 0; k < C.n; k++) {

@@ -74,7 +74,7 @@ struct DeviceArrays {
     int *d_snend_ = nullptr, *d_ru_ = nullptr, *d_fcut_ = nullptr, *d_bcut_ = nullptr;
     int *d_dpos_ = nullptr;              // per column: position of the diagonal row q[k]
     int *d_fpk_ = nullptr, *d_bpk_ = nullptr, *d_twide_ = nullptr;
-    double *d_tailW_ = nullptr;
+    double *d_tailW_ = nullptr, *d_tailP_ = nullptr;   // diagonal-block inverses, packed tiles
     // Ruiz equilibration (FP16 factor storage)
     int *d_arow_ = nullptr, *d_acol_ = nullptr;
     long *d_raoff_ = nullptr, *d_rvoff_ = nullptr;
@@ -107,9 +107,9 @@ struct DeviceArrays {
     int *d_tail_ds_ = nullptr, *d_tail_lcut_ = nullptr, *d_tail_ctr_ = nullptr;
     double *d_tailS_ = nullptr;
     unsigned long long *d_colmax_ = nullptr;
-    int *d_dflag_ = nullptr;                   // per dense job: the last diagonal block factored
+    int *d_dflag_ = nullptr;                   // per tile of every dense job: epoch of the launch that made it final
     DenseJob *d_djobs_ = nullptr;
-    int njobs_ = 0, max_tail_T_ = 0;
+    int njobs_ = 0;
     DenseGrid dgrid_;                          // work lists of the dense-block launches
     int2 *d_fillchunk_ = nullptr;              // (matrix, chunk) of the unset fill
     int nfillchunk_ = 0;
