@@ -146,6 +146,10 @@ __device__ __forceinline__ void advance_epoch(int *counter, int epoch)
     st_relaxed(counter, epoch < 0x3fffffff ? epoch + 1 : 1);
 }
 
+// A launch queued ahead of a decision made on the device: it does nothing
+// when the word an earlier launch counted is not zero.
+__device__ __forceinline__ bool gated(const int *gate) { return gate && uniform(ld_relaxed(gate)) != 0; }
+
 __device__ __forceinline__ bool aborted(const int *abort_word)
 {
     return uniform(ld_relaxed(abort_word)) != 0;

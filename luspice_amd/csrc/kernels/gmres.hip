@@ -7,237 +7,320 @@
 // crossings per inner iteration (:595-615); here every vector operation and
 // the small Hessenberg/Givens work stay on the device.
 //
-// Orthogonalisation is classical Gram-Schmidt applied twice (CGS2): each pass
-// is one block-dot h = V^T w and one update w -= V h, so a pass costs two
-// launches instead of 2(j+1) dependent reductions; two passes give the same
-// O(eps) loss of orthogonality as the reference's two-pass modified
-// Gram-Schmidt.
+// Orthogonalisation is classical Gram-Schmidt applied twice (CGS2); two passes
+// give the same O(eps) loss of orthogonality as the reference's two-pass
+// modified Gram-Schmidt.
+//
+// What bounds it: launches.  At n <= 1e5 every vector fits the caches and each
+// kernel is near the cost of a launch (about 4 us), so the work is laid out for
+// few of them.  Reductions are two-stage and deterministic; the second stage
+// has no launch of its own, every workgroup that needs a sum adds its matrix's
+// partial sums itself (in the same order, so all agree).  One inner iteration
+// is the preconditioner's solves and four launches:
+//   sell_block_kernel (spmv.hip)  w = A z, partial V^T w
+//   orth_kernel<first>            h = V^T w, w -= V h, partial V^T w
+//   orth_kernel<second>           h = V^T w, w -= V h, partial w^T w
+//   basis_kernel                  V_{j+1} = w / ||w||, Givens step, and the
+//                                 solves' work values of the next iteration set
+//                                 to the unset marker
+// and a cycle adds two (residual with its norm; start_kernel) and one at its
+// end (update_kernel: back substitution and x += Z y).  With one launch per
+// operation an iteration took thirteen beside the solves.  Whole Newton steps
+// (refactor and solve): 200 unknowns 0.65 -> 0.38 ms, 1020 unknowns with fp32
+// factors 0.97 -> 0.65 ms, 512 circuits with fp32 factors 7.77 -> 7.42 ms.
 //
 // Batch layout: vectors of matrix m live at voff[m] .. voff[m]+n_m in arenas
-// of length ntot; basis vector i is V + i*ntot.  Reductions are two-stage and
-// deterministic: row chunks (matrix, r0, r1) write per-chunk partial sums,
-// then one thread per (matrix, i) adds them in chunk order.  Matrices whose
-// act[m] == 0 are skipped by every kernel.
+// of length ntot; basis vector i is V + i*ntot.  One workgroup per row chunk
+// (matrix, r0, r1).  Matrices whose act[m] == 0 are skipped; a matrix's first
+// workgroup (its lead) keeps its Hessenberg, rotations and state, and may clear
+// act[m] in a launch whose other workgroups still read it: either value leaves
+// a finished matrix's solution alone.
 #include "common.hpp"
 #include "launch.hpp"
 
 namespace lsp {
 
+constexpr int kKrT = 256;               // threads per workgroup
+constexpr int kKrW = kKrT / kWave;
 
+// Sum over the workgroup, in every thread.
 __device__ __forceinline__ double block_sum(double v, double *red)
 {
     v = wave_sum(v);
-    const int w = threadIdx.x >> 6;
-    if (lane_id() == 0) red[w] = v;
+    if (lane_id() == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
-    double s = 0.0;
-    if (threadIdx.x == 0) {
-        for (int i = 0; i < (int)(blockDim.x >> 6); i++) s += red[i];
-    }
+    const double s = red[0] + red[1] + red[2] + red[3];
     __syncthreads();
     return s;
 }
 
-// partial[c][i] = sum over chunk c of V_i * w  (i = 0..nv-1); with V == w and
-// nv == 1 this is the squared norm.
-__global__ void __launch_bounds__(256) chunk_dots_kernel(KrylovArgs K, const double *V, const double *w, int nv)
+// Sum of p[stride * c] over c in [c0, c1), by one wave, in every lane.
+__device__ __forceinline__ double wave_partials(const double *p, long stride, int c0, int c1)
 {
-    __shared__ double red[4];
-    const int c = blockIdx.x;
-    const int4 ch = K.chunks[c];
+    double s = 0.0;
+    for (int c = c0 + lane_id(); c < c1; c += kWave) s += p[stride * c];
+    return wave_sum(s);
+}
+
+// conv, abort word and active counts before a solve.
+__global__ void __launch_bounds__(kKrT) solve_init_kernel(int *conv, int nmat, int *abort_word, int *nact)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < nmat && conv) conv[i] = 0;
+    if (i == 0 && abort_word) *abort_word = 0;
+    if (i < kNact) nact[i] = 0;
+}
+
+// Sets the solves' work values of one row to the unset marker.
+__device__ __forceinline__ void unset_row(const UnsetArgs &U, long i)
+{
+    const double u = Unset<double>::value();
+    U.y[i] = u;
+    U.yp[i] = u;
+    U.z[i] = u;
+    U.zp[i] = u;
+}
+
+// Cycle start: ||r|| (and on the first cycle ||b||) from the residual's
+// partial sums, the outer convergence test, V_0 = r / ||r||.
+__global__ void __launch_bounds__(kKrT) start_kernel(KrylovArgs K, const double *r, int cyc, double *hist,
+                                                     const int *gate, UnsetArgs U)
+{
+    __shared__ double s2[2];
+    if (gated(gate)) return;
+    const bool first = cyc == 0;
+    const int4 ch = K.chunks[blockIdx.x];
+    const int m = ch.x;
+    const bool lead = ch.y == 0;
+    if (K.conv[m]) {                            // skipped; the lead says so
+        if (lead && threadIdx.x == 0) {
+            K.act[m] = 0;
+            K.cycled[m] = 0;
+            if (first) K.jfin[m] = 0;
+        }
+        return;
+    }
+    const int wv = threadIdx.x >> 6;
+    if (wv < 2) {
+        const double s = wave_partials(K.spartial + wv, 2, K.sbeg[m], K.sbeg[m + 1]);
+        if (lane_id() == 0) s2[wv] = s;
+    }
+    __syncthreads();
+    const double beta = sqrt(s2[0]);
+    const double nb = first ? sqrt(s2[1]) : K.nb[m];
+    const double rel = beta / nb;
+    const bool done = rel <= K.outer_tol || !(beta > 0.0);
+    if (lead && threadIdx.x == 0) {
+        K.beta[m] = beta;
+        if (first) K.nb[m] = nb;
+        if (m == 0) hist[cyc & 1] = nb > 0 ? rel : beta;
+        K.cycled[m] = 0;
+        if (first) K.jfin[m] = 0;               // later cycles: basis_kernel's count, once it runs
+        K.act[m] = done ? 0 : 1;
+        if (done) K.conv[m] = 1;
+        else {
+            K.g[(long)m * (K.mmax + 1)] = beta;
+            atomicAdd(&K.nact[nact_word(cyc, 0)], 1);
+        }
+    }
+    if (done) return;
+    const long vo = K.voff[m];
+    for (int i = ch.y + threadIdx.x; i < ch.z; i += kKrT) {
+        K.V[vo + i] = r[vo + i] / beta;
+        unset_row(U, vo + i);
+    }
+}
+
+// One orthogonalisation pass of column j: h_i = V_i^T w from the partial sums,
+// w -= sum h_i V_i over the chunk, and the next partial sums: V_i^T w after the
+// first pass, w^T w after the second.  pin holds `pstride` sums per part,
+// parts pbeg[m] .. pbeg[m + 1).
+constexpr int kOrthTile = 256;          // basis vectors whose coefficients are in LDS at a time
+template <bool kFirst>
+__global__ void __launch_bounds__(kKrT) orth_kernel(KrylovArgs K, int j, const double *pin, const int *pbeg,
+                                                    int pstride)
+{
+    __shared__ double h[kOrthTile], red[kOrthTile * kKrW];
+    const int4 ch = K.chunks[blockIdx.x];
+    const int m = ch.x;
+    // the next iteration's active count, read by nobody before basis_kernel adds to it
+    if (kFirst && blockIdx.x == 0 && threadIdx.x == 0) K.nact[nact_word(0, j + 1)] = 0;
+    if (!K.act[m]) return;
+    const int nv = j + 1;
+    const int wv = threadIdx.x >> 6;
+    const int p0 = pbeg[m], p1 = pbeg[m + 1];
+    const long vo = K.voff[m];
+    double *w = K.w + vo;
+    const double *V = K.V + vo;
+    double *H = K.H + (long)m * (K.mmax + 1) * K.mmax;
+    double *out = K.partial + (long)blockIdx.x * (K.mmax + 1);
+    constexpr int kRows = 2;                    // rows per thread and pass (a chunk of 512 in one pass)
+    double ww = 0.0;
+    for (int r0 = ch.y; r0 < ch.z; r0 += kRows * kKrT) {
+        double a[kRows];
+        int r[kRows];
+#pragma unroll
+        for (int t = 0; t < kRows; t++) {
+            r[t] = r0 + t * kKrT + (int)threadIdx.x;
+            a[t] = r[t] < ch.z ? w[r[t]] : 0.0;
+        }
+        for (int t0 = 0; t0 < nv; t0 += kOrthTile) {
+            const int nt = min(kOrthTile, nv - t0);
+            __syncthreads();                    // the tile before has been read
+            for (int i = wv; i < nt; i += kKrW) {
+                const double s = wave_partials(pin + t0 + i, pstride, p0, p1);
+                if (lane_id() == 0) h[i] = s;
+            }
+            __syncthreads();
+            if (ch.y == 0 && r0 == 0)
+                for (int i = threadIdx.x; i < nt; i += kKrT) {
+                    if (kFirst) H[(long)(t0 + i) * K.mmax + j] = h[i];
+                    else H[(long)(t0 + i) * K.mmax + j] += h[i];
+                }
+            for (int i = 0; i < nt; i++) {
+                const double hi = h[i];
+#pragma unroll
+                for (int t = 0; t < kRows; t++)
+                    if (r[t] < ch.z) a[t] -= hi * V[(long)(t0 + i) * K.ntot + r[t]];
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < kRows; t++)
+            if (r[t] < ch.z) w[r[t]] = a[t];
+        if (kFirst) {
+            for (int t0 = 0; t0 < nv; t0 += kOrthTile) {
+                const int nt = min(kOrthTile, nv - t0);
+                __syncthreads();
+                for (int i = 0; i < nt; i++) {
+                    double s = 0.0;
+#pragma unroll
+                    for (int t = 0; t < kRows; t++)
+                        if (r[t] < ch.z) s += V[(long)(t0 + i) * K.ntot + r[t]] * a[t];
+                    s = wave_sum(s);
+                    if (lane_id() == 0) red[i * kKrW + wv] = s;
+                }
+                __syncthreads();
+                for (int i = threadIdx.x; i < nt; i += kKrT) {
+                    const double s = red[i * kKrW] + red[i * kKrW + 1] + red[i * kKrW + 2] + red[i * kKrW + 3];
+                    out[t0 + i] = r0 == ch.y ? s : out[t0 + i] + s;
+                }
+            }
+        } else {
+#pragma unroll
+            for (int t = 0; t < kRows; t++) ww += a[t] * a[t];
+        }
+    }
+    if (!kFirst) {
+        ww = block_sum(ww, red);
+        if (threadIdx.x == 0) K.pnorm[blockIdx.x] = ww;
+    }
+}
+
+// V_i^T w for i <= j over one chunk (more basis vectors than the product's
+// kernel takes along).
+__global__ void __launch_bounds__(kKrT) chunk_dots_kernel(KrylovArgs K, int nv)
+{
+    __shared__ double red[kKrW];
+    const int4 ch = K.chunks[blockIdx.x];
     if (!K.act[ch.x]) return;
     const long vo = K.voff[ch.x];
     for (int i = 0; i < nv; i++) {
-        const double *vi = V + (long)i * K.ntot + vo;
+        const double *vi = K.V + (long)i * K.ntot + vo;
         double s = 0.0;
-        for (int r = ch.y + threadIdx.x; r < ch.z; r += blockDim.x) s += vi[r] * w[vo + r];
+        for (int r = ch.y + threadIdx.x; r < ch.z; r += kKrT) s += vi[r] * K.w[vo + r];
         s = block_sum(s, red);
-        if (threadIdx.x == 0) K.partial[(long)c * (K.mmax + 1) + i] = s;
+        if (threadIdx.x == 0) K.partial2[(long)blockIdx.x * (K.mmax + 1) + i] = s;
     }
 }
 
-// out[m*(mmax+1)+i] = sum of partials (mode 0: store, mode 1: add into H
-// column j and hcol, mode 2: sqrt into hn)
-// One wave per (matrix, i): lanes stride over the matrix's chunks, then a
-// wave sum (a single thread walking hundreds of chunks took ~46 us on c1).
-__global__ void __launch_bounds__(64) reduce_partials_kernel(KrylovArgs K, int nv, int mode, int j, double *out)
+// End of inner iteration j: V_{j+1} = w / ||w||, the work values of the next
+// solves unset; the lead does the Givens step and ends the matrix's cycle when
+// its residual estimate is small enough.
+__global__ void __launch_bounds__(kKrT) basis_kernel(KrylovArgs K, int j, UnsetArgs U)
 {
-    const int t = blockIdx.x;
-    const int m = t / nv, i = t % nv;
-    if (m >= K.nmat || !K.act[m]) return;
-    double s = 0.0;
-    for (int c = K.cbeg[m] + (int)threadIdx.x; c < K.cbeg[m + 1]; c += kWave)
-        s += K.partial[(long)c * (K.mmax + 1) + i];
-    s = wave_sum(s);
-    if (threadIdx.x != 0) return;
-    if (mode == 0) {
-        out[(long)m * (K.mmax + 1) + i] = s;
-    } else if (mode == 1) {
-        K.hcol[(long)m * (K.mmax + 1) + i] = s;
-        K.H[(long)m * (K.mmax + 1) * K.mmax + (long)i * K.mmax + j] += s;
-    } else {
-        out[m] = sqrt(s);
+    __shared__ double s_hn;
+    const int4 ch = K.chunks[blockIdx.x];
+    const int m = ch.x;
+    if (!K.act[m]) return;
+    if (threadIdx.x < kWave) {
+        const double s = wave_partials(K.pnorm, 1, K.cbeg[m], K.cbeg[m + 1]);
+        if (threadIdx.x == 0) s_hn = sqrt(s);
     }
-}
-
-// w -= sum_{i<nv} hcol[i] V_i
-__global__ void __launch_bounds__(256) chunk_update_kernel(KrylovArgs K, const double *V, double *w, int nv)
-{
-    const int c = blockIdx.x;
-    const int4 ch = K.chunks[c];
-    if (!K.act[ch.x]) return;
-    const long vo = K.voff[ch.x];
-    const double *h = K.hcol + (long)ch.x * (K.mmax + 1);
-    for (int r = ch.y + threadIdx.x; r < ch.z; r += blockDim.x) {
-        double acc = w[vo + r];
-        for (int i = 0; i < nv; i++) acc -= h[i] * V[(long)i * K.ntot + vo + r];
-        w[vo + r] = acc;
-    }
-}
-
-// dst = src * (1/den[m]) per matrix (dst may alias src); den from beta or hn
-__global__ void __launch_bounds__(256) chunk_scale_kernel(KrylovArgs K, const double *src, double *dst,
-                                                          const double *den)
-{
-    const int c = blockIdx.x;
-    const int4 ch = K.chunks[c];
-    if (!K.act[ch.x]) return;
-    const long vo = K.voff[ch.x];
-    const double d = den[ch.x];
-    for (int r = ch.y + threadIdx.x; r < ch.z; r += blockDim.x) dst[vo + r] = src[vo + r] / d;
-}
-
-// Cycle start: outer convergence test on beta, reset H and g.
-// One workgroup per matrix: every thread reads the same state and takes the
-// same branch; the Hessenberg and g are cleared by all threads together.
-__global__ void __launch_bounds__(128) start_cycle_kernel(KrylovArgs K, int *n_active)
-{
-    const int m = blockIdx.x;
-    if (m >= K.nmat) return;
-    const bool lead = threadIdx.x == 0;
-    const bool conv = K.conv[m] != 0;
-    const double rel = K.beta[m] / K.nb[m];
-    const bool done = !conv && (rel <= K.outer_tol || !(K.beta[m] > 0.0));
-    __syncthreads();                            // every thread has read conv before it changes
-    if (lead) {
-        K.cycled[m] = 0;
-        K.jfin[m] = 0;
-        K.act[m] = conv || done ? 0 : 1;
-        if (done) K.conv[m] = 1;
-    }
-    if (conv || done) return;
-    double *H = K.H + (long)m * (K.mmax + 1) * K.mmax;
-    for (long t = threadIdx.x; t < (long)(K.mmax + 1) * K.mmax; t += blockDim.x) H[t] = 0.0;
-    double *g = K.g + (long)m * (K.mmax + 1);
-    for (int t = threadIdx.x; t <= K.mmax; t += blockDim.x) g[t] = t == 0 ? K.beta[m] : 0.0;
-    if (lead) atomicAdd(n_active, 1);
-}
-
-// Givens step for column j; sets act = 0 when the cycle ends for matrix m.
-__global__ void givens_kernel(KrylovArgs K, int j, int *n_active)
-{
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= K.nmat || !K.act[m]) return;
+    __syncthreads();
+    const double hn = s_hn;
+    const long vo = K.voff[m];
     const int mm = K.mmax;
+    for (int i = ch.y + threadIdx.x; i < ch.z; i += kKrT) {
+        K.V[(long)(j + 1) * K.ntot + vo + i] = K.w[vo + i] / hn;
+        unset_row(U, vo + i);
+    }
+    if (ch.y != 0 || threadIdx.x != 0) return;
     double *H = K.H + (long)m * (mm + 1) * mm;
     double *cs = K.cs + (long)m * mm, *sn = K.sn + (long)m * mm;
     double *g = K.g + (long)m * (mm + 1);
-    const double hn = K.hn[m];
-    H[(long)(j + 1) * mm + j] = hn;
+    double a = H[j];                            // column j under the earlier rotations
     for (int i = 0; i < j; i++) {
-        const double t0 = H[(long)i * mm + j];
-        const double t1 = H[(long)(i + 1) * mm + j];
-        H[(long)i * mm + j] = cs[i] * t0 + sn[i] * t1;
-        H[(long)(i + 1) * mm + j] = -sn[i] * t0 + cs[i] * t1;
+        const double b = H[(long)(i + 1) * mm + j];
+        H[(long)i * mm + j] = cs[i] * a + sn[i] * b;
+        a = -sn[i] * a + cs[i] * b;
     }
-    const double a = H[(long)j * mm + j], c = H[(long)(j + 1) * mm + j];
-    const double r = sqrt(a * a + c * c);
-    cs[j] = r > 0 ? a / r : 1.0;
-    sn[j] = r > 0 ? c / r : 0.0;
+    const double r = sqrt(a * a + hn * hn);
+    const double c = r > 0 ? a / r : 1.0, s = r > 0 ? hn / r : 0.0;
+    cs[j] = c;
+    sn[j] = s;
     H[(long)j * mm + j] = r;
-    H[(long)(j + 1) * mm + j] = 0.0;
-    g[j + 1] = -sn[j] * g[j];
-    g[j] = cs[j] * g[j];
+    const double gj = g[j];
+    const double gn = -s * gj;
+    g[j + 1] = gn;
+    g[j] = c * gj;
     K.jfin[m] = j + 1;
     K.cycled[m] = 1;
-    const bool done = fabs(g[j + 1]) / K.nb[m] <= K.inner_tol || hn < 1e-14 || j + 1 >= mm;
+    const bool done = fabs(gn) / K.nb[m] <= K.inner_tol || hn < 1e-14 || j + 1 >= mm;
     if (done) K.act[m] = 0;
-    else atomicAdd(n_active, 1);
+    else atomicAdd(&K.nact[nact_word(0, j + 1)], 1);
 }
 
-// y = R^-1 g over the first jfin columns; re-activates matrices that cycled
-// so the following combine / preconditioner / update launches see them.
-__global__ void backsolve_kernel(KrylovArgs K)
+constexpr int kYLds = 2048;
+
+// End of a cycle: y = R^-1 g over the matrix's steps, x += sum y_i Z_i.
+__global__ void __launch_bounds__(kKrT) update_kernel(KrylovArgs K, const double *Z, double *x, const int *gate)
 {
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= K.nmat) return;
-    if (!K.cycled[m]) { K.act[m] = 0; return; }
+    __shared__ double ylds[kYLds];
+    if (gated(gate)) return;
+    const int4 ch = K.chunks[blockIdx.x];
+    const int m = ch.x;
+    if (!K.cycled[m]) return;
     const int mm = K.mmax, jf = K.jfin[m];
+    // very long cycles: the matrix's workgroups all write the same y
+    double *y = jf <= kYLds ? ylds : K.yv + (long)m * mm;
     const double *H = K.H + (long)m * (mm + 1) * mm;
     const double *g = K.g + (long)m * (mm + 1);
-    double *y = K.yv + (long)m * mm;
-    for (int i = jf - 1; i >= 0; i--) {
-        double s = g[i];
-        for (int t = i + 1; t < jf; t++) s -= H[(long)i * mm + t] * y[t];
-        y[i] = s / H[(long)i * mm + i];
+    if (jf <= kWave) {
+        // lane t holds row t: subtract column i once y_i is known
+        if (threadIdx.x < kWave) {
+            const int t = threadIdx.x;
+            double s = t < jf ? g[t] : 0.0;
+            for (int i = jf - 1; i >= 0; i--) {
+                const double col = t <= i ? H[(long)t * mm + i] : 0.0;
+                const double yi = bcast_f64(s, i) / bcast_f64(col, i);
+                if (t == i) y[i] = yi;
+                if (t < i) s -= col * yi;
+            }
+        }
+    } else if (threadIdx.x == 0) {
+        for (int i = jf - 1; i >= 0; i--) {
+            double s = g[i];
+            for (int t = i + 1; t < jf; t++) s -= H[(long)i * mm + t] * y[t];
+            y[i] = s / H[(long)i * mm + i];
+        }
     }
-    K.act[m] = 1;
-}
-
-// t = V y (first jfin basis vectors)
-__global__ void __launch_bounds__(256) chunk_combine_kernel(KrylovArgs K, const double *V, double *t)
-{
-    const int c = blockIdx.x;
-    const int4 ch = K.chunks[c];
-    if (!K.act[ch.x]) return;
-    const long vo = K.voff[ch.x];
-    const int jf = K.jfin[ch.x];
-    const double *y = K.yv + (long)ch.x * K.mmax;
-    for (int r = ch.y + threadIdx.x; r < ch.z; r += blockDim.x) {
+    __syncthreads();
+    const long vo = K.voff[m];
+    for (int r = ch.y + threadIdx.x; r < ch.z; r += kKrT) {
         double acc = 0.0;
-        for (int i = 0; i < jf; i++) acc += y[i] * V[(long)i * K.ntot + vo + r];
-        t[vo + r] = acc;
+        for (int i = 0; i < jf; i++) acc += y[i] * Z[(long)i * K.ntot + vo + r];
+        x[vo + r] += acc;
     }
-}
-
-// x += z for matrices in the update phase
-__global__ void __launch_bounds__(256) chunk_axpy_kernel(KrylovArgs K, double *x, const double *z)
-{
-    const int c = blockIdx.x;
-    const int4 ch = K.chunks[c];
-    if (!K.act[ch.x]) return;
-    const long vo = K.voff[ch.x];
-    for (int r = ch.y + threadIdx.x; r < ch.z; r += blockDim.x) x[vo + r] += z[vo + r];
-}
-
-// x = v on active matrices
-__global__ void __launch_bounds__(256) chunk_fill_kernel(KrylovArgs K, double *x, double v)
-{
-    const int c = blockIdx.x;
-    const int4 ch = K.chunks[c];
-    if (!K.act[ch.x]) return;
-    const long vo = K.voff[ch.x];
-    for (int r = ch.y + threadIdx.x; r < ch.z; r += blockDim.x) x[vo + r] = v;
-}
-
-// Set act for every not-yet-converged matrix (used before the outer residual)
-__global__ void activate_kernel(KrylovArgs K)
-{
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m < K.nmat) K.act[m] = K.conv[m] ? 0 : 1;
-}
-
-// act = 1 for all (final residual evaluation, b-norms)
-__global__ void set_all_active_kernel(KrylovArgs K, int v)
-{
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m < K.nmat) K.act[m] = v;
-}
-
-__global__ void zero_kernel(double *p, long n)
-{
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0.0;
 }
 
 __global__ void zero_int_kernel(int *p, long n)
@@ -255,71 +338,40 @@ __global__ void copy_kernel(const double *src, double *dst, long n)
 // ---------------------------------------------------------------------------
 static inline int nb_for(long n, int t) { return (int)((n + t - 1) / t); }
 
-hipError_t k_chunk_dots(const KrylovArgs &K, const double *V, const double *w, int nv, hipStream_t s)
+hipError_t k_solve_init(int *conv, int nmat, int *abort_word, int *nact, hipStream_t s)
 {
-    hipLaunchKernelGGL(chunk_dots_kernel, dim3(K.nchunks), dim3(256), 0, s, K, V, w, nv);
+    hipLaunchKernelGGL(solve_init_kernel, dim3(nb_for(nmat > kNact ? nmat : kNact, kKrT)), dim3(kKrT), 0, s, conv,
+                       nmat, abort_word, nact);
     return hipGetLastError();
 }
-hipError_t k_reduce(const KrylovArgs &K, int nv, int mode, int j, double *out, hipStream_t s)
+hipError_t k_start(const KrylovArgs &K, const double *r, int cyc, double *hist, const int *gate,
+                   const UnsetArgs &U, hipStream_t s)
 {
-    const int tot = K.nmat * nv;
-    hipLaunchKernelGGL(reduce_partials_kernel, dim3(tot > 0 ? tot : 1), dim3(kWave), 0, s, K, nv, mode, j, out);
+    hipLaunchKernelGGL(start_kernel, dim3(K.nchunks), dim3(kKrT), 0, s, K, r, cyc, hist, gate, U);
     return hipGetLastError();
 }
-hipError_t k_chunk_update(const KrylovArgs &K, const double *V, double *w, int nv, hipStream_t s)
+hipError_t k_chunk_dots(const KrylovArgs &K, int nv, hipStream_t s)
 {
-    hipLaunchKernelGGL(chunk_update_kernel, dim3(K.nchunks), dim3(256), 0, s, K, V, w, nv);
+    hipLaunchKernelGGL(chunk_dots_kernel, dim3(K.nchunks), dim3(kKrT), 0, s, K, nv);
     return hipGetLastError();
 }
-hipError_t k_chunk_scale(const KrylovArgs &K, const double *src, double *dst, const double *den, hipStream_t s)
+hipError_t k_orth(const KrylovArgs &K, int j, bool first, hipStream_t s)
 {
-    hipLaunchKernelGGL(chunk_scale_kernel, dim3(K.nchunks), dim3(256), 0, s, K, src, dst, den);
+    const dim3 g(K.nchunks), t(kKrT);
+    if (!first) hipLaunchKernelGGL(orth_kernel<false>, g, t, 0, s, K, j, K.partial, K.cbeg, K.mmax + 1);
+    else if (j < kSpmvDots)                     // sums from the product's kernel
+        hipLaunchKernelGGL(orth_kernel<true>, g, t, 0, s, K, j, K.spartial, K.sbeg, kSpmvDots);
+    else hipLaunchKernelGGL(orth_kernel<true>, g, t, 0, s, K, j, K.partial2, K.cbeg, K.mmax + 1);
     return hipGetLastError();
 }
-hipError_t k_start_cycle(const KrylovArgs &K, int *n_active, hipStream_t s)
+hipError_t k_basis(const KrylovArgs &K, int j, const UnsetArgs &U, hipStream_t s)
 {
-    hipLaunchKernelGGL(start_cycle_kernel, dim3(K.nmat > 0 ? K.nmat : 1), dim3(128), 0, s, K, n_active);
+    hipLaunchKernelGGL(basis_kernel, dim3(K.nchunks), dim3(kKrT), 0, s, K, j, U);
     return hipGetLastError();
 }
-hipError_t k_givens(const KrylovArgs &K, int j, int *n_active, hipStream_t s)
+hipError_t k_update(const KrylovArgs &K, const double *Z, double *x, const int *gate, hipStream_t s)
 {
-    hipLaunchKernelGGL(givens_kernel, dim3(nb_for(K.nmat, 128)), dim3(128), 0, s, K, j, n_active);
-    return hipGetLastError();
-}
-hipError_t k_backsolve(const KrylovArgs &K, hipStream_t s)
-{
-    hipLaunchKernelGGL(backsolve_kernel, dim3(nb_for(K.nmat, 128)), dim3(128), 0, s, K);
-    return hipGetLastError();
-}
-hipError_t k_chunk_combine(const KrylovArgs &K, const double *V, double *t, hipStream_t s)
-{
-    hipLaunchKernelGGL(chunk_combine_kernel, dim3(K.nchunks), dim3(256), 0, s, K, V, t);
-    return hipGetLastError();
-}
-hipError_t k_chunk_axpy(const KrylovArgs &K, double *x, const double *z, hipStream_t s)
-{
-    hipLaunchKernelGGL(chunk_axpy_kernel, dim3(K.nchunks), dim3(256), 0, s, K, x, z);
-    return hipGetLastError();
-}
-hipError_t k_chunk_fill(const KrylovArgs &K, double *x, double v, hipStream_t s)
-{
-    hipLaunchKernelGGL(chunk_fill_kernel, dim3(K.nchunks), dim3(256), 0, s, K, x, v);
-    return hipGetLastError();
-}
-hipError_t k_activate(const KrylovArgs &K, hipStream_t s)
-{
-    hipLaunchKernelGGL(activate_kernel, dim3(nb_for(K.nmat, 128)), dim3(128), 0, s, K);
-    return hipGetLastError();
-}
-hipError_t k_set_all_active(const KrylovArgs &K, int v, hipStream_t s)
-{
-    hipLaunchKernelGGL(set_all_active_kernel, dim3(nb_for(K.nmat, 128)), dim3(128), 0, s, K, v);
-    return hipGetLastError();
-}
-hipError_t k_zero(double *p, long n, hipStream_t s)
-{
-    if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(zero_kernel, dim3(nb_for(n, 256)), dim3(256), 0, s, p, n);
+    hipLaunchKernelGGL(update_kernel, dim3(K.nchunks), dim3(kKrT), 0, s, K, Z, x, gate);
     return hipGetLastError();
 }
 hipError_t k_zero_int(int *p, long n, hipStream_t s)

@@ -52,6 +52,16 @@ struct TriLaunch {
     int nq;                 // queue counters (1, 2 or 4) in the ctr block
 };
 
+// Active-circuit counts of a solve: one word per inner iteration in turn, two
+// (by the cycle's parity) for the count at a cycle's start.
+constexpr int kNact = 5;
+#ifdef __HIPCC__
+__host__ __device__
+#endif
+inline int nact_word(int cyc, int j) { return j == 0 ? 3 + (cyc & 1) : j % 3; }
+// Basis vectors whose dot products the product's kernel takes along.
+constexpr int kSpmvDots = 4;
+
 struct KrylovArgs {
     int nmat;
     int mmax;               // restart length m
@@ -60,21 +70,58 @@ struct KrylovArgs {
     const int4 *chunks;     // (matrix, r0, r1, 0)
     int nchunks;
     const int *cbeg;        // nmat+1 chunk ranges per matrix
-    double *partial;        // nchunks * (mmax+1)
+    const int *sbeg;        // nmat+1 ranges of the product's workgroups per matrix
+    double *V;              // basis, (mmax+1) * ntot
+    double *w;              // the vector being orthogonalised
+    double *spartial;       // sums of the product's workgroups (2 or kSpmvDots each)
+    double *partial;        // nchunks * (mmax+1): V^T w after the first pass
+    double *partial2;       // nchunks * (mmax+1): V^T w before it (more than kSpmvDots vectors)
+    double *pnorm;          // nchunks: w^T w
     double *H;              // nmat * (mmax+1) * mmax, H[i*mmax + j]
     double *cs, *sn;        // nmat * mmax
     double *g;              // nmat * (mmax+1)
     double *yv;             // nmat * mmax
     double *beta;           // nmat: ||r|| at cycle start
     double *nb;             // nmat: ||b||
-    double *hn;             // nmat: ||w|| of the current step
-    double *hcol;           // nmat * (mmax+1): scratch for one Arnoldi column
     int *act;               // nmat: 1 while the inner cycle runs
     int *jfin;              // nmat: inner steps taken in the cycle
     int *conv;              // nmat: 1 once the outer test passed
     int *cycled;            // nmat: 1 if the cycle produced an update
+    int *nact;              // kNact words
     double inner_tol, outer_tol;
 };
+
+// The solves' work values (position order).
+struct UnsetArgs {
+    double *y, *yp, *z, *zp;
+};
+
+// SELL products of the GMRES cycle (spmv.hip): one workgroup per four slices
+// of one matrix, with the sums the next kernel needs.
+enum SellMode {
+    kSellResidual = 1,      // y = b - A x; sums of y^2 and (first) b^2
+    kSellResidual0 = 2,     // the same for x = 0, which is written
+    kSellDots = 3           // y = A x; sums of V_i y, i < nv (nv <= kSpmvDots; 0: none)
+};
+struct SellArgs {
+    const int2 *blocks;     // (matrix, first slice)
+    int nblocks;
+    const int64_t *voff;
+    double *x;              // written by kSellResidual0 only
+    double *y;
+    const double *b;
+    const int *mask;        // per matrix: skipped unless mask[m] == run
+    int run;
+    const int *gate;        // see gated()
+    int *zero_word;         // cleared by the launch
+    double *partial;
+    const double *V;
+    long ntot;
+    int nv;
+    int first;
+};
+template <typename V>
+hipError_t launch_sell_block(const SellDesc<V> *mats, const SellArgs &A, SellMode mode, hipStream_t st);
 
 // One fused IR step over the circuits of a batch (irstep.hip).
 struct IrStepArgs {
@@ -143,20 +190,13 @@ hipError_t launch_gather_cast(long count, const int *idx, const double *in, Vout
                               hipStream_t st);
 
 // gmres.hip
-hipError_t k_chunk_dots(const KrylovArgs &K, const double *V, const double *w, int nv, hipStream_t s);
-hipError_t k_reduce(const KrylovArgs &K, int nv, int mode, int j, double *out, hipStream_t s);
-hipError_t k_chunk_update(const KrylovArgs &K, const double *V, double *w, int nv, hipStream_t s);
-hipError_t k_chunk_scale(const KrylovArgs &K, const double *src, double *dst, const double *den,
-                         hipStream_t s);
-hipError_t k_start_cycle(const KrylovArgs &K, int *n_active, hipStream_t s);
-hipError_t k_givens(const KrylovArgs &K, int j, int *n_active, hipStream_t s);
-hipError_t k_backsolve(const KrylovArgs &K, hipStream_t s);
-hipError_t k_chunk_combine(const KrylovArgs &K, const double *V, double *t, hipStream_t s);
-hipError_t k_chunk_axpy(const KrylovArgs &K, double *x, const double *z, hipStream_t s);
-hipError_t k_chunk_fill(const KrylovArgs &K, double *x, double v, hipStream_t s);
-hipError_t k_activate(const KrylovArgs &K, hipStream_t s);
-hipError_t k_set_all_active(const KrylovArgs &K, int v, hipStream_t s);
-hipError_t k_zero(double *p, long n, hipStream_t s);
+hipError_t k_solve_init(int *conv, int nmat, int *abort_word, int *nact, hipStream_t s);
+hipError_t k_start(const KrylovArgs &K, const double *r, int cyc, double *hist, const int *gate,
+                   const UnsetArgs &U, hipStream_t s);
+hipError_t k_chunk_dots(const KrylovArgs &K, int nv, hipStream_t s);
+hipError_t k_orth(const KrylovArgs &K, int j, bool first, hipStream_t s);
+hipError_t k_basis(const KrylovArgs &K, int j, const UnsetArgs &U, hipStream_t s);
+hipError_t k_update(const KrylovArgs &K, const double *Z, double *x, const int *gate, hipStream_t s);
 hipError_t k_zero_int(int *p, long n, hipStream_t s);
 hipError_t k_copy(const double *src, double *dst, long n, hipStream_t s);
 

@@ -19,7 +19,7 @@
 // csr_spmv_kernel: the reference's spmv_launch contract (one thread per row,
 //   256-thread blocks, y = A x in CSR order).
 #include "common.hpp"
-#include "desc.hpp"
+#include "launch.hpp"
 
 namespace lsp {
 
@@ -70,6 +70,92 @@ sell_spmv_kernel(const SellDesc<V> *mats, const int2 *tasks, int ntask,
     }
     y[vo + row] = b ? bi - s : s;
 }
+
+// The products of a GMRES cycle, one workgroup per four slices of one matrix;
+// the sums over its rows that the next kernel needs go along with them, which
+// saves a launch and a pass over the vectors each.  The row sums are those of
+// sell_spmv_kernel.
+template <typename V, int kMode>
+__global__ void __launch_bounds__(256) sell_block_kernel(const SellDesc<V> *mats, SellArgs A)
+{
+    __shared__ double red[4][kSpmvDots];
+    if (gated(A.gate)) return;
+    if (A.zero_word && blockIdx.x == 0 && threadIdx.x == 0) *A.zero_word = 0;
+    const int2 tk = A.blocks[blockIdx.x];
+    if (A.mask[tk.x] != A.run) return;
+    const SellDesc<V> M = mats[tk.x];
+    const int lane = lane_id();
+    const int wv = uniform((int)(threadIdx.x >> 6));
+    const int sl = tk.y + wv;
+    const int64_t vo = A.voff[tk.x];
+    const int k = sl * kWave + lane;
+    double sum[kSpmvDots] = {0.0, 0.0, 0.0, 0.0};
+    if (sl < M.nslices && k < M.n) {
+        const double *xm = A.x + vo;
+        const int len = M.rlen[k];
+        const int64_t base = M.off[sl] + lane;
+        const int row = M.perm[k];
+        const double bi = kMode == kSellDots ? 0.0 : A.b[vo + row];
+        double s = 0.0;
+        for (int j0 = 0; j0 < len; j0 += kSpmvBatch) {
+            V v[kSpmvBatch];
+            int c[kSpmvBatch];
+#pragma unroll
+            for (int u = 0; u < kSpmvBatch; u++) {
+                const int64_t e = base + (int64_t)min(j0 + u, len - 1) * kWave;
+                v[u] = M.val[e];
+                c[u] = M.col[e];
+            }
+            double xv[kSpmvBatch];
+#pragma unroll
+            for (int u = 0; u < kSpmvBatch; u++) xv[u] = kMode == kSellResidual0 ? 0.0 : xm[c[u]];
+#pragma unroll
+            for (int u = 0; u < kSpmvBatch; u++)
+                if (j0 + u < len) s += to_f64(v[u]) * xv[u];    // x = 0: a value that is not finite still shows
+        }
+        const double out = kMode == kSellDots ? s : bi - s;
+        A.y[vo + row] = out;
+        if constexpr (kMode == kSellResidual0) A.x[vo + row] = 0.0;
+        if constexpr (kMode == kSellDots) {
+#pragma unroll
+            for (int i = 0; i < kSpmvDots; i++)
+                if (i < A.nv) sum[i] = A.V[(long)i * A.ntot + vo + row] * out;
+        } else {
+            sum[0] = out * out;
+            if (A.first) sum[1] = bi * bi;
+        }
+    }
+    const int ns = kMode == kSellDots ? A.nv : 2;
+#pragma unroll
+    for (int i = 0; i < kSpmvDots; i++)
+        if (i < ns) {
+            const double t = wave_sum(sum[i]);
+            if (lane == 0) red[wv][i] = t;
+        }
+    __syncthreads();
+    const int i = threadIdx.x;
+    constexpr int kStride = kMode == kSellDots ? kSpmvDots : 2;
+    if (i < ns) A.partial[(long)blockIdx.x * kStride + i] = red[0][i] + red[1][i] + red[2][i] + red[3][i];
+}
+
+template <typename V>
+hipError_t launch_sell_block(const SellDesc<V> *mats, const SellArgs &A, SellMode mode, hipStream_t st)
+{
+    if (A.nblocks <= 0) return hipSuccess;
+    const dim3 g(A.nblocks), t(256);
+    if (mode == kSellDots) {
+        hipLaunchKernelGGL((sell_block_kernel<V, kSellDots>), g, t, 0, st, mats, A);
+    } else if constexpr (sizeof(V) == 8) {              // residuals are taken with the fp64 values
+        if (mode == kSellResidual) hipLaunchKernelGGL((sell_block_kernel<V, kSellResidual>), g, t, 0, st, mats, A);
+        else hipLaunchKernelGGL((sell_block_kernel<V, kSellResidual0>), g, t, 0, st, mats, A);
+    } else {
+        return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+template hipError_t launch_sell_block<double>(const SellDesc<double> *, const SellArgs &, SellMode, hipStream_t);
+template hipError_t launch_sell_block<float>(const SellDesc<float> *, const SellArgs &, SellMode, hipStream_t);
+template hipError_t launch_sell_block<__half>(const SellDesc<__half> *, const SellArgs &, SellMode, hipStream_t);
 
 __global__ void __launch_bounds__(256)
 csr_spmv_kernel(int n, const int *__restrict__ rowptr, const int *__restrict__ colidx,

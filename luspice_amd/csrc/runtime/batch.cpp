@@ -37,6 +37,7 @@ Batch::~Batch()
     if (graph_) (void)hipGraphDestroy(graph_);
     for (auto &m : mem_) if (m.p) (void)hipFree(m.p);
     if (h_pin_) (void)hipHostFree(h_pin_);
+    if (h_status_) (void)hipHostFree(h_status_);
     for (auto &e : ev_) if (e) (void)hipEventDestroy(e);
     if (own_stream_ && stream_) (void)hipStreamDestroy(stream_);
 }
@@ -73,19 +74,19 @@ void Batch::dfree(void *p)
 int Batch::alloc_krylov(int mm)
 {
     const int nc = (int)circ_.size();
-    for (void *p : {(void *)d_V_, (void *)d_Z_, (void *)d_partial_, (void *)d_H_, (void *)d_cs_, (void *)d_sn_,
-                    (void *)d_g_, (void *)d_yv_, (void *)d_hcol_})
+    for (void *p : {(void *)d_V_, (void *)d_Z_, (void *)d_partial_, (void *)d_partial2_, (void *)d_H_, (void *)d_cs_,
+                    (void *)d_sn_, (void *)d_g_, (void *)d_yv_})
         dfree(p);
     d_V_ = (double *)dalloc((size_t)(mm + 1) * ntot_ * 8);
     d_Z_ = (double *)dalloc((size_t)mm * ntot_ * 8);
     d_partial_ = (double *)dalloc((size_t)nchunks_ * (mm + 1) * 8);
+    d_partial2_ = (double *)dalloc((size_t)nchunks_ * (mm + 1) * 8);
     d_H_ = (double *)dalloc((size_t)nc * (mm + 1) * mm * 8);
     d_cs_ = (double *)dalloc((size_t)nc * mm * 8);
     d_sn_ = (double *)dalloc((size_t)nc * mm * 8);
     d_g_ = (double *)dalloc((size_t)nc * (mm + 1) * 8);
     d_yv_ = (double *)dalloc((size_t)nc * mm * 8);
-    d_hcol_ = (double *)dalloc((size_t)nc * (mm + 1) * 8);
-    if (!d_V_ || !d_Z_ || !d_partial_ || !d_H_ || !d_cs_ || !d_sn_ || !d_g_ || !d_yv_ || !d_hcol_)
+    if (!d_V_ || !d_Z_ || !d_partial_ || !d_partial2_ || !d_H_ || !d_cs_ || !d_sn_ || !d_g_ || !d_yv_)
         return LSP_E_ALLOC;
     mm_alloc_ = mm;
     return LSP_OK;
@@ -151,12 +152,12 @@ X *Batch::upload(const std::vector<X> &v)
     return d;
 }
 
-int Batch::sync_read_int(const int *d, int *h, int count)
+// Copies bytes [from, to) of the status block to its pinned host copy and waits.
+int Batch::read_status(size_t from, size_t to)
 {
-    int rc = check(hipMemcpyAsync(h, d, count * sizeof(int), hipMemcpyDeviceToHost, stream_),
-                   "read flags");
-    if (rc) return rc;
-    rc = check(hipStreamSynchronize(stream_), "sync");
+    int rc = check(hipMemcpyAsync(h_status_ + from, d_status_ + from, to - from, hipMemcpyDeviceToHost, stream_),
+                   "read status");
+    if (!rc) rc = check(hipStreamSynchronize(stream_), "sync");
     if (!rc) account_trisolve();
     return rc;
 }
@@ -607,15 +608,27 @@ int Batch::upload_all()
     {
         std::vector<int> zeros(ntot_, 0);
         d_done_ = upload(zeros);
+        const StatusLayout lay(nc);
+        d_status_ = (char *)dalloc(lay.end);
+        if (!d_status_) return LSP_E_ALLOC;
+        rc = check(hipMemset(d_status_, 0, lay.end), "status block");
+        if (rc) return rc;
+        d_mstat_ = (int *)(d_status_ + lay.mstat);
+        d_jfin_ = (int *)(d_status_ + lay.jfin);
+        d_abort_ = (int *)(d_status_ + lay.abort);
+        d_nact_ = (int *)(d_status_ + lay.nact);
+        d_hist_ = (double *)(d_status_ + lay.hist);
+        d_beta_ = (double *)(d_status_ + lay.beta);
+        d_nb_ = (double *)(d_status_ + lay.nb);
+        if (!h_status_ && hipHostMalloc((void **)&h_status_, lay.end, hipHostMallocDefault) != hipSuccess)
+            return LSP_E_ALLOC;
         std::vector<int> z6(8, 0);
         std::vector<int> zq(4 * kQueueInts, 0);    // refactor, forward, backward, dense-block queue blocks
-        d_ctr_ = upload(zq); d_abort_ = upload(z6);
+        d_ctr_ = upload(zq);
         std::vector<int> e1(4, 1);                 // epochs start at 1, flags at 0
         d_epoch_ = upload(e1);
-        std::vector<int> ms(kMstat * nc, 0);
-        d_mstat_ = upload(ms);
         d_dbg_ = upload(z6);
-        if (!d_done_ || !d_ctr_ || !d_abort_ || !d_mstat_ || !d_epoch_)
+        if (!d_done_ || !d_ctr_ || !d_epoch_ || !d_dbg_)
             return LSP_E_ALLOC;
     }
     // dense trailing blocks, the jobs by falling order T
@@ -886,15 +899,25 @@ int Batch::upload_all()
         d_voff_ = upload(voff);
         d_chunks_ = upload(chunks);
         d_cbeg_ = upload(cbeg);
+        std::vector<int2> sblock;
+        std::vector<int> sbeg(nc + 1, 0);
+        for (int m = 0; m < nc; m++) {
+            sbeg[m] = (int)sblock.size();
+            for (int sl = 0; sl < circ_[m].sell.nslices; sl += 4) sblock.push_back(make_int2(m, sl));
+        }
+        sbeg[nc] = nsblock_ = (int)sblock.size();
+        d_sblock_ = upload(sblock);
+        d_sbeg_ = upload(sbeg);
+        d_spartial_ = (double *)dalloc((size_t)nsblock_ * kSpmvDots * 8);
+        d_pnorm_ = (double *)dalloc((size_t)nchunks_ * 8);
+        if (!d_sblock_ || !d_sbeg_ || !d_spartial_ || !d_pnorm_) return LSP_E_ALLOC;
         rc = alloc_krylov(mm);
         if (rc) return rc;
-        d_beta_ = (double *)dalloc(nc * 8); d_nb_ = (double *)dalloc(nc * 8);
-        d_hn_ = (double *)dalloc(nc * 8);
-        d_act_ = (int *)dalloc(nc * 4); d_jfin_ = (int *)dalloc(nc * 4);
+        d_act_ = (int *)dalloc(nc * 4);
         d_conv_ = (int *)dalloc(nc * 4); d_cycled_ = (int *)dalloc(nc * 4);
-        d_nact_ = (int *)dalloc(16); d_subset_ = (int *)dalloc(nc * 4);
+        d_subset_ = (int *)dalloc(nc * 4);
         if (!d_b_ || !d_x_ || !d_r_ || !d_w_ || !d_z_ || !d_t_ || !d_ty_ || !d_tz_ || !d_typ_ || !d_tzp_ ||
-            !d_voff_ || !d_chunks_ || !d_cbeg_ || !d_act_)
+            !d_voff_ || !d_chunks_ || !d_cbeg_ || !d_act_ || !d_conv_ || !d_cycled_ || !d_subset_)
             return LSP_E_ALLOC;
         if (!h_pin_ && hipHostMalloc((void **)&h_pin_, 4096, hipHostMallocDefault) != hipSuccess)
             return LSP_E_ALLOC;
@@ -977,9 +1000,12 @@ KrylovArgs Batch::kargs() const
     K.chunks = d_chunks_;
     K.nchunks = nchunks_;
     K.cbeg = d_cbeg_;
-    K.partial = d_partial_;
+    K.sbeg = d_sbeg_;
+    K.V = d_V_;
+    K.w = d_w_;
+    K.spartial = d_spartial_; K.partial = d_partial_; K.partial2 = d_partial2_; K.pnorm = d_pnorm_;
     K.H = d_H_; K.cs = d_cs_; K.sn = d_sn_; K.g = d_g_; K.yv = d_yv_;
-    K.beta = d_beta_; K.nb = d_nb_; K.hn = d_hn_; K.hcol = d_hcol_;
+    K.beta = d_beta_; K.nb = d_nb_; K.nact = d_nact_;
     K.act = d_act_; K.jfin = d_jfin_; K.conv = d_conv_; K.cycled = d_cycled_;
     K.inner_tol = opt_.ir_inner_tol;
     K.outer_tol = opt_.ir_outer_tol;
@@ -1084,11 +1110,11 @@ int Batch::refactor_pass(int prec, const std::vector<int> *subset, std::vector<i
     rc = launch_refactor_prec(prec, d_active);
     if (rc) return rc;
     cur_prec_ = prec;
-    ms.assign((size_t)kMstat * circ_.size(), 0);
-    rc = check(hipMemcpyAsync(ms.data(), d_mstat_, ms.size() * 4, hipMemcpyDeviceToHost, stream_), "mstat");
-    if (!rc) rc = check(hipMemcpyAsync(h_pin_, d_abort_, 4, hipMemcpyDeviceToHost, stream_), "abort");
-    if (!rc) rc = check(hipStreamSynchronize(stream_), "refactor sync");
+    const StatusLayout lay = layout();
+    rc = read_status(0, lay.nact);                            // pivot status, abort words
     if (rc) return rc;
+    ms.assign(status<int>(lay.mstat), status<int>(lay.mstat) + (size_t)kMstat * circ_.size());
+    h_pin_[0] = status<int>(lay.abort)[0];
     float t_kernel = 0.0f, t_all = 0.0f;
     (void)hipEventElapsedTime(&t_kernel, ev_[0], ev_[1]);
     (void)hipEventElapsedTime(&t_all, ev_[0], ev_[5]);
@@ -1252,7 +1278,8 @@ int Batch::refactor(int prec, lsp_refactor_report *rep, const std::vector<int> *
 
 // ---------------------------------------------------------------------------
 template <typename T>
-int Batch::trisolve_t(FactorSet<T> &fs, const double *d_b, double *d_x, const int *d_active, const int *d_nact)
+int Batch::trisolve_t(FactorSet<T> &fs, const double *d_b, double *d_x, const int *d_active, const int *d_nact,
+                      bool unset)
 {
     if (!fs.ready) return LSP_E_ARG;
     TriLaunch Lf{};
@@ -1288,7 +1315,7 @@ int Batch::trisolve_t(FactorSet<T> &fs, const double *d_b, double *d_x, const in
     Lb.total_waves = tblocks_b_ * 4;
     Lb.nq = nq_t_;
     if (!capturing_) (void)hipEventRecord(ev_[2], stream_);
-    int rc = check(launch_solve_unset(Lf, ntot_, stream_), "solve unset");
+    int rc = unset ? check(launch_solve_unset(Lf, ntot_, stream_), "solve unset") : LSP_OK;
     if (!rc) rc = check(launch_trisolve_half<T>(Lf, true, tblocks_f_, stream_), "trisolve fwd");
     if (!rc && njobs_)
         rc = check(launch_tail_solve<T>(fs.tdesc, dgrid_, d_voff_, d_active, d_b, d_ty_, d_typ_, d_tz_, d_x, true,
@@ -1301,30 +1328,17 @@ int Batch::trisolve_t(FactorSet<T> &fs, const double *d_b, double *d_x, const in
                    "tail bwd");
     if (!rc) rc = check(launch_trisolve_half<T>(Lb, false, tblocks_b_, stream_), "trisolve bwd");
     if (!capturing_) (void)hipEventRecord(ev_[3], stream_);
-    tri_pending_ = true;
+    if (!capturing_) tri_pending_ = true;
     return rc;
 }
 
-int Batch::launch_trisolve_prec(int prec, const double *d_b, double *d_x, const int *active, const int *d_nact)
+int Batch::launch_trisolve_prec(int prec, const double *d_b, double *d_x, const int *active, const int *d_nact,
+                                bool unset)
 {
-    if (prec == LSP_PREC_FP32) return trisolve_t(f32_, d_b, d_x, active, d_nact);
-    if (prec == LSP_PREC_FP64) return trisolve_t(f64_, d_b, d_x, active, d_nact);
-    if (prec == LSP_PREC_FP16) return trisolve_t(f16_, d_b, d_x, active, d_nact);
+    if (prec == LSP_PREC_FP32) return trisolve_t(f32_, d_b, d_x, active, d_nact, unset);
+    if (prec == LSP_PREC_FP64) return trisolve_t(f64_, d_b, d_x, active, d_nact, unset);
+    if (prec == LSP_PREC_FP16) return trisolve_t(f16_, d_b, d_x, active, d_nact, unset);
     return LSP_E_ARG;
-}
-
-// Arnoldi product w = A z with the value precision chosen by krylov_spmv
-// (fp64 accumulation in every case; the residual always uses launch_spmv64)
-int Batch::launch_spmv_krylov(const double *d_xv, double *d_y, const int *active)
-{
-    const int64_t *vo = (const int64_t *)d_voff_;
-    if (opt_.krylov_spmv == 1)
-        return check(launch_sell_spmv<float>(d_sdesc32_, d_stask_, nstask_, vo, d_xv, d_y, nullptr, active,
-                                             stream_), "spmv32");
-    if (opt_.krylov_spmv == 2)
-        return check(launch_sell_spmv<__half>(d_sdesc16_, d_stask_, nstask_, vo, d_xv, d_y, nullptr, active,
-                                              stream_), "spmv16");
-    return launch_spmv64(d_xv, d_y, nullptr, active);
 }
 
 int Batch::launch_spmv64(const double *d_xv, double *d_y, const double *d_bv, const int *active)
@@ -1404,100 +1418,127 @@ int Batch::spmv(const double *x, double *y, bool on_device, int prec)
 }
 
 // ---------------------------------------------------------------------------
+// r = b - A x with its norm, and the start of cycle `cyc`: convergence test,
+// first basis vector, the solves' work values unset.
+int Batch::launch_residual(const KrylovArgs &K, const double *d_b, double *d_x, int cyc, bool x_is_zero,
+                           const int *gate)
+{
+    SellArgs A{};
+    A.blocks = d_sblock_;
+    A.nblocks = nsblock_;
+    A.voff = (const int64_t *)d_voff_;
+    A.x = d_x;
+    A.y = d_r_;
+    A.b = d_b;
+    A.mask = d_conv_;
+    A.run = 0;
+    A.gate = gate;
+    A.zero_word = d_nact_ + nact_word(cyc, 0);
+    A.partial = d_spartial_;
+    A.first = cyc == 0;
+    int rc = check(launch_sell_block<double>(d_sdesc64_, A, x_is_zero ? kSellResidual0 : kSellResidual, stream_),
+                   "residual");
+    return rc ? rc : check(k_start(K, d_r_, cyc, d_hist_, gate, unset_args(), stream_), "cycle start");
+}
+
+// Inner iteration j: z = M^-1 V_j, w = A z, two orthogonalisation passes, the
+// next basis vector.  The product's value precision is chosen by krylov_spmv
+// (fp64 accumulation in every case; the residual always takes the fp64
+// values).  Z_j = M^-1 V_j is kept, so the update x += M^-1 (V y) = Z y needs
+// no further solve (the flexible-GMRES form of right preconditioning).
+int Batch::launch_inner(const KrylovArgs &K, int prec, int j, const int *d_nact)
+{
+    double *Zj = d_Z_ + (long)j * ntot_;
+    int rc = launch_trisolve_prec(prec, d_V_ + (long)j * ntot_, Zj, d_act_, d_nact, false);
+    if (rc) return rc;
+    SellArgs A{};
+    A.blocks = d_sblock_;
+    A.nblocks = nsblock_;
+    A.voff = (const int64_t *)d_voff_;
+    A.x = Zj;
+    A.y = d_w_;
+    A.mask = d_act_;
+    A.run = 1;
+    A.partial = d_spartial_;
+    A.V = d_V_;
+    A.ntot = ntot_;
+    A.nv = j < kSpmvDots ? j + 1 : 0;
+    if (opt_.krylov_spmv == 1) rc = check(launch_sell_block<float>(d_sdesc32_, A, kSellDots, stream_), "spmv32");
+    else if (opt_.krylov_spmv == 2) rc = check(launch_sell_block<__half>(d_sdesc16_, A, kSellDots, stream_), "spmv16");
+    else rc = check(launch_sell_block<double>(d_sdesc64_, A, kSellDots, stream_), "spmv");
+    if (!rc && j >= kSpmvDots) rc = check(k_chunk_dots(K, j + 1, stream_), "dots");
+    if (!rc) rc = check(k_orth(K, j, true, stream_), "orth");
+    if (!rc) rc = check(k_orth(K, j, false, stream_), "orth");
+    return rc ? rc : check(k_basis(K, j, unset_args(), stream_), "basis");
+}
+
 int Batch::gmres_ir(const double *d_bv, double *d_xv, int prec, const std::vector<char> *subset,
                     lsp_solve_report *rep, bool keep_x)
 {
     const KrylovArgs K = kargs();
     const int nc = (int)circ_.size();
     const int mm = K.mmax;
+    const StatusLayout lay = layout();
     hipStream_t s = stream_;
     int rc;
 #define LSP_TRY(expr) do { rc = (expr); if (rc) return rc; } while (0)
 #define LSP_HIP(expr, what) LSP_TRY(check((expr), what))
     // conv = 1 for circuits outside the subset, 0 inside; x = 0 inside
     // unless keep_x (x then holds a first iterate, e.g. after fused steps)
-    {
+    if (subset) {
         std::vector<int> cv(nc, 0);
-        if (subset) for (int m = 0; m < nc; m++) cv[m] = (*subset)[m] ? 0 : 1;
+        for (int m = 0; m < nc; m++) cv[m] = (*subset)[m] ? 0 : 1;
         LSP_HIP(hipMemcpyAsync(d_conv_, cv.data(), nc * 4, hipMemcpyHostToDevice, s), "conv");
         LSP_HIP(hipStreamSynchronize(s), "sync");
     }
-    LSP_HIP(k_activate(K, s), "activate");
-    LSP_HIP(k_chunk_dots(K, d_bv, d_bv, 1, s), "dots");
-    LSP_HIP(k_reduce(K, 1, 2, 0, d_nb_, s), "reduce");
-    if (!keep_x) LSP_HIP(k_chunk_fill(K, d_xv, 0.0, s), "zero x");
+    LSP_HIP(k_solve_init(subset ? nullptr : d_conv_, nc, d_abort_ + 1, d_nact_, s), "solve init");
+    LSP_TRY(launch_residual(K, d_bv, d_xv, 0, !keep_x, nullptr));
     int outer_used = 0, inner_total = 0;
     res_hist0_.clear();
-    for (int outer = 0; outer < opt_.ir_outer; outer++) {
-        LSP_HIP(k_activate(K, s), "activate");
-        LSP_TRY(launch_spmv64(d_xv, d_r_, d_bv, d_act_));
-        LSP_HIP(k_chunk_dots(K, d_r_, d_r_, 1, s), "dots");
-        LSP_HIP(k_reduce(K, 1, 2, 0, d_beta_, s), "reduce");
-        LSP_HIP(k_zero_int(d_nact_, 1, s), "zero");
-        LSP_HIP(k_start_cycle(K, d_nact_, s), "start");
-        {
-            double bn[2];
-            LSP_HIP(hipMemcpyAsync(bn, d_beta_, 8, hipMemcpyDeviceToHost, s), "beta0");
-            LSP_HIP(hipMemcpyAsync(bn + 1, d_nb_, 8, hipMemcpyDeviceToHost, s), "nb0");
-            LSP_TRY(sync_read_int(d_nact_, h_pin_, 1));
-            res_hist0_.push_back(bn[1] > 0 ? bn[0] / bn[1] : bn[0]);
-        }
-        if (h_pin_[0] == 0) break;
-        outer_used++;
-        LSP_HIP(k_chunk_scale(K, d_r_, d_V_, d_beta_, s), "scale");
-        // Z_j = M^-1 V_j is kept, so the update x += M^-1 (V y) = Z y needs
-        // no further solve (the flexible-GMRES form of right preconditioning)
+    const int *nact = status<int>(lay.nact);
+    const double *hist = status<double>(lay.hist);
+    bool done = false;
+    for (int cyc = 0; !done;) {
         for (int j = 0; j < mm; j++) {
-            double *Vj = d_V_ + (long)j * ntot_;
-            double *Zj = d_Z_ + (long)j * ntot_;
-            LSP_TRY(launch_trisolve_prec(prec, Vj, Zj, d_act_));
-            LSP_TRY(launch_spmv_krylov(Zj, d_w_, d_act_));
-            for (int pass = 0; pass < 2; pass++) {
-                LSP_HIP(k_chunk_dots(K, d_V_, d_w_, j + 1, s), "dots");
-                LSP_HIP(k_reduce(K, j + 1, 1, j, nullptr, s), "reduce");
-                LSP_HIP(k_chunk_update(K, d_V_, d_w_, j + 1, s), "update");
+            LSP_TRY(launch_inner(K, prec, j, j == 0 ? d_nact_ + nact_word(cyc, 0) : nullptr));
+            // the end of the cycle and the start of the next are queued at
+            // once and do nothing while a circuit is still iterating, so one
+            // host wait per iteration serves both
+            const int *gate = d_nact_ + nact_word(cyc, j + 1);
+            LSP_HIP(k_update(K, d_Z_, d_xv, gate, s), "update");
+            LSP_TRY(launch_residual(K, d_bv, d_xv, cyc + 1, false, gate));
+            LSP_TRY(read_status(lay.abort, lay.end));
+            if (status<int>(lay.abort)[1]) return LSP_E_DEVICE;
+            if (cyc == 0 && j == 0) {
+                res_hist0_.push_back(hist[0]);
+                if (nact[nact_word(0, 0)] == 0) {        // nothing to solve
+                    done = true;
+                    break;
+                }
+                outer_used++;
             }
-            LSP_HIP(k_chunk_dots(K, d_w_, d_w_, 1, s), "dots");
-            LSP_HIP(k_reduce(K, 1, 2, 0, d_hn_, s), "reduce");
-            LSP_HIP(k_chunk_scale(K, d_w_, d_V_ + (long)(j + 1) * ntot_, d_hn_, s), "scale");
-            LSP_HIP(k_zero_int(d_nact_, 1, s), "zero");
-            LSP_HIP(k_givens(K, j, d_nact_, s), "givens");
             inner_total++;
-            LSP_TRY(sync_read_int(d_nact_, h_pin_, 1));
-            if (h_pin_[0] == 0) break;
+            if (nact[nact_word(cyc, j + 1)] == 0) break;
         }
-        LSP_HIP(k_backsolve(K, s), "backsolve");
-        LSP_HIP(k_chunk_combine(K, d_Z_, d_t_, s), "combine");
-        LSP_HIP(k_chunk_axpy(K, d_xv, d_t_, s), "axpy");
+        if (done || ++cyc >= opt_.ir_outer) break;
+        res_hist0_.push_back(hist[cyc & 1]);
+        if (nact[nact_word(cyc, 0)] == 0) break;
+        outer_used++;
     }
-    // final true residual of every circuit in the subset
-    {
-        std::vector<int> am(nc, 1);
-        if (subset) for (int m = 0; m < nc; m++) am[m] = (*subset)[m] ? 1 : 0;
-        LSP_HIP(hipMemcpyAsync(d_act_, am.data(), nc * 4, hipMemcpyHostToDevice, s), "act");
-        LSP_TRY(launch_spmv64(d_xv, d_r_, d_bv, d_act_));
-        LSP_HIP(k_chunk_dots(K, d_r_, d_r_, 1, s), "dots");
-        LSP_HIP(k_reduce(K, 1, 2, 0, d_beta_, s), "reduce");
-        std::vector<double> beta(nc), nb(nc);
-        LSP_HIP(hipMemcpyAsync(beta.data(), d_beta_, nc * 8, hipMemcpyDeviceToHost, s), "beta");
-        LSP_HIP(hipMemcpyAsync(nb.data(), d_nb_, nc * 8, hipMemcpyDeviceToHost, s), "nb");
-        LSP_HIP(hipMemcpyAsync(h_pin_, d_abort_ + 1, 4, hipMemcpyDeviceToHost, s), "abort");
-        LSP_HIP(hipStreamSynchronize(s), "sync");
-        account_trisolve();
-        if (h_pin_[0]) return LSP_E_DEVICE;
-        lsp_solve_report r{};
-        r.outer = outer_used;
-        r.inner_total = inner_total;
-        for (int m = 0; m < nc; m++) {
-            if (subset && !(*subset)[m]) continue;
-            double rel = nb[m] > 0 ? beta[m] / nb[m] : beta[m];
-            if (!(rel == rel)) rel = INFINITY;
-            r.max_rel_res = std::max(r.max_rel_res, rel);
-            if (rel <= opt_.ir_outer_tol * 10 || rel <= 1e-9) r.converged++;
-        }
-        r.status = LSP_OK;
-        if (rep) *rep = r;
+    // every circuit's norms are those of its last residual
+    const double *beta = status<double>(lay.beta), *nb = status<double>(lay.nb);
+    lsp_solve_report r{};
+    r.outer = outer_used;
+    r.inner_total = inner_total;
+    for (int m = 0; m < nc; m++) {
+        if (subset && !(*subset)[m]) continue;
+        double rel = nb[m] > 0 ? beta[m] / nb[m] : beta[m];
+        if (!(rel == rel)) rel = INFINITY;
+        r.max_rel_res = std::max(r.max_rel_res, rel);
+        if (rel <= opt_.ir_outer_tol * 10 || rel <= 1e-9) r.converged++;
     }
+    r.status = LSP_OK;
+    if (rep) *rep = r;
 #undef LSP_TRY
 #undef LSP_HIP
     return LSP_OK;
@@ -1643,8 +1684,6 @@ int Batch::solve(const double *b, double *x, bool on_device, lsp_solve_report *r
         db = d_b_;
         dx = d_x_;
     }
-    rc = check(k_zero_int(d_abort_ + 1, 1, stream_), "abort reset");
-    if (rc) return rc;
     // the circuits solved: the set_active mask, else all
     const int nc = (int)circ_.size();
     std::vector<char> live;
@@ -1720,8 +1759,6 @@ int Batch::solve(const double *b, double *x, bool on_device, lsp_solve_report *r
             if (!rr.repivoted) cur_prec_ = keep;
             if (rc && rc != LSP_E_SINGULAR) return rc;
             r.singular_fallback = rr.singular_circuits;
-            rc = check(k_zero_int(d_abort_ + 1, 1, stream_), "abort reset");
-            if (rc) return rc;
             lsp_solve_report r2{};
             rc = gmres_ir(db, dx, LSP_PREC_FP64, &subc, &r2);
             if (rc) return rc;
@@ -1847,13 +1884,18 @@ int Batch::export_factors(int c, int *pinv, int *Lp, int *Li, double *Lx, int *U
 // arguments.  After the replay the host reads the reports once; a circuit
 // still above the tolerance is finished by the eager solve (restart from 0,
 // fp64 fallback as in solve()).
-constexpr int kGraphInner = 8;          // GMRES inner iterations recorded in the step graph
+// GMRES inner iterations recorded in the step graph.  A replay runs every
+// recorded launch, and an idle iteration costs about 35 us on a 512-circuit
+// batch (its solves exit at once, n_active == 0), so the graph holds one more
+// than a step with such factors usually takes (512 circuits: 1 with fp64
+// factors, 3 with fp32); circuits that need more go on eagerly from the
+// graph's iterate.
+static int graph_inner(int prec) { return prec == LSP_PREC_FP64 ? 2 : prec == LSP_PREC_FP32 ? 4 : 8; }
 
 int Batch::record_step(int prec)
 {
     const KrylovArgs K = kargs();
     const int nc = (int)circ_.size();
-    const int mm = K.mmax;
     hipStream_t s = stream_;
     const double *d_bv = d_b_;
     double *d_xv = d_x_;
@@ -1861,8 +1903,8 @@ int Batch::record_step(int prec)
 #define LSP_TRY(expr) do { rc = (expr); if (rc) return rc; } while (0)
 #define LSP_HIP(expr, what) LSP_TRY(check((expr), what))
     LSP_TRY(launch_refactor_prec(prec, nullptr));
-    LSP_HIP(k_zero_int(d_abort_ + 1, 1, s), "abort reset");
     if (use_fused(prec)) {
+        LSP_HIP(k_zero_int(d_abort_ + 1, 1, s), "abort reset");
         // fused Richardson steps: a converged circuit's later launches return
         // at once, so the recorded count only bounds the work
         LSP_HIP(k_zero_int(d_irconv_, nc, s), "conv");
@@ -1870,44 +1912,12 @@ int Batch::record_step(int prec)
         for (int j = 0; j < fused_steps(); j++) LSP_TRY(ir_launch_prec(prec, d_bv, d_xv, tol2, j == 0));
         return LSP_OK;
     }
-    LSP_HIP(k_zero_int(d_conv_, nc, s), "conv");
-    LSP_HIP(k_activate(K, s), "activate");
-    LSP_HIP(k_chunk_dots(K, d_bv, d_bv, 1, s), "dots");
-    LSP_HIP(k_reduce(K, 1, 2, 0, d_nb_, s), "reduce");
-    LSP_HIP(k_chunk_fill(K, d_xv, 0.0, s), "zero x");
-    LSP_HIP(k_activate(K, s), "activate");
-    LSP_TRY(launch_spmv64(d_xv, d_r_, d_bv, d_act_));
-    LSP_HIP(k_chunk_dots(K, d_r_, d_r_, 1, s), "dots");
-    LSP_HIP(k_reduce(K, 1, 2, 0, d_beta_, s), "reduce");
-    LSP_HIP(k_zero_int(d_nact_, 1, s), "zero");
-    LSP_HIP(k_start_cycle(K, d_nact_, s), "start");
-    LSP_HIP(k_chunk_scale(K, d_r_, d_V_, d_beta_, s), "scale");
-    // a replay runs every recorded iteration: record the few a step usually
-    // needs; an idle iteration's solves exit at once (n_active == 0)
-    const int mg = std::min(mm, kGraphInner);
-    for (int j = 0; j < mg; j++) {
-        double *Vj = d_V_ + (long)j * ntot_;
-        double *Zj = d_Z_ + (long)j * ntot_;
-        LSP_TRY(launch_trisolve_prec(prec, Vj, Zj, d_act_, d_nact_));
-        LSP_TRY(launch_spmv_krylov(Zj, d_w_, d_act_));
-        for (int pass = 0; pass < 2; pass++) {
-            LSP_HIP(k_chunk_dots(K, d_V_, d_w_, j + 1, s), "dots");
-            LSP_HIP(k_reduce(K, j + 1, 1, j, nullptr, s), "reduce");
-            LSP_HIP(k_chunk_update(K, d_V_, d_w_, j + 1, s), "update");
-        }
-        LSP_HIP(k_chunk_dots(K, d_w_, d_w_, 1, s), "dots");
-        LSP_HIP(k_reduce(K, 1, 2, 0, d_hn_, s), "reduce");
-        LSP_HIP(k_chunk_scale(K, d_w_, d_V_ + (long)(j + 1) * ntot_, d_hn_, s), "scale");
-        LSP_HIP(k_zero_int(d_nact_, 1, s), "zero");
-        LSP_HIP(k_givens(K, j, d_nact_, s), "givens");
-    }
-    LSP_HIP(k_backsolve(K, s), "backsolve");
-    LSP_HIP(k_chunk_combine(K, d_Z_, d_t_, s), "combine");
-    LSP_HIP(k_chunk_axpy(K, d_xv, d_t_, s), "axpy");
-    LSP_HIP(k_set_all_active(K, 1, s), "act");
-    LSP_TRY(launch_spmv64(d_xv, d_r_, d_bv, d_act_));
-    LSP_HIP(k_chunk_dots(K, d_r_, d_r_, 1, s), "dots");
-    LSP_HIP(k_reduce(K, 1, 2, 0, d_beta_, s), "reduce");
+    LSP_HIP(k_solve_init(d_conv_, nc, d_abort_ + 1, d_nact_, s), "solve init");
+    LSP_TRY(launch_residual(K, d_bv, d_xv, 0, true, nullptr));
+    const int mg = std::min(K.mmax, graph_inner(prec));
+    for (int j = 0; j < mg; j++) LSP_TRY(launch_inner(K, prec, j, d_nact_ + nact_word(0, j)));
+    LSP_HIP(k_update(K, d_Z_, d_xv, nullptr, s), "update");
+    LSP_TRY(launch_residual(K, d_bv, d_xv, 1, false, nullptr));
 #undef LSP_TRY
 #undef LSP_HIP
     return LSP_OK;
@@ -1956,25 +1966,25 @@ int Batch::graph_step(int prec, lsp_refactor_report *rrep, lsp_solve_report *sre
     cur_prec_ = prec;
     const int nc = (int)circ_.size();
     const bool fused = use_fused(prec);
-    std::vector<int> ms(kMstat * nc), jf(nc), cv(nc, 0);
+    const int mg = std::min(std::max(1, opt_.ir_inner), graph_inner(prec));   // as recorded
+    const StatusLayout lay = layout();
+    std::vector<int> cv(nc, 0);
     std::vector<double> beta(nc), nb(nc);
-    int ab[2] = {0, 0};
-    rc = check(hipMemcpyAsync(ms.data(), d_mstat_, ms.size() * 4, hipMemcpyDeviceToHost, stream_), "mstat");
     if (fused) {
         // squared residual norms of the last step each circuit ran
-        if (!rc) rc = check(hipMemcpyAsync(beta.data(), d_rn2_, nc * 8, hipMemcpyDeviceToHost, stream_), "rn2");
+        rc = check(hipMemcpyAsync(beta.data(), d_rn2_, nc * 8, hipMemcpyDeviceToHost, stream_), "rn2");
         if (!rc) rc = check(hipMemcpyAsync(nb.data(), d_bn2_, nc * 8, hipMemcpyDeviceToHost, stream_), "bn2");
         if (!rc) rc = check(hipMemcpyAsync(cv.data(), d_irconv_, nc * 4, hipMemcpyDeviceToHost, stream_), "conv");
-    } else {
-        if (!rc) rc = check(hipMemcpyAsync(beta.data(), d_beta_, nc * 8, hipMemcpyDeviceToHost, stream_), "beta");
-        if (!rc) rc = check(hipMemcpyAsync(nb.data(), d_nb_, nc * 8, hipMemcpyDeviceToHost, stream_), "nb");
-        if (!rc) rc = check(hipMemcpyAsync(jf.data(), d_jfin_, nc * 4, hipMemcpyDeviceToHost, stream_), "jfin");
     }
-    if (!rc) rc = check(hipMemcpyAsync(h_pin_, d_abort_, 8, hipMemcpyDeviceToHost, stream_), "abort");
-    if (!rc) rc = check(hipStreamSynchronize(stream_), "graph sync");
+    if (!rc) rc = read_status(0, fused ? lay.nact : lay.end);
     if (rc) return rc;
-    ab[0] = h_pin_[0];
-    ab[1] = h_pin_[1];
+    if (!fused) {
+        beta.assign(status<double>(lay.beta), status<double>(lay.beta) + nc);
+        nb.assign(status<double>(lay.nb), status<double>(lay.nb) + nc);
+    }
+    const std::vector<int> ms(status<int>(lay.mstat), status<int>(lay.mstat) + (size_t)kMstat * nc);
+    const std::vector<int> jf(status<int>(lay.jfin), status<int>(lay.jfin) + nc);
+    const int ab[2] = {status<int>(lay.abort)[0], status<int>(lay.abort)[1]};
     stats_.graph_steps++;
     lsp_refactor_report r{};
     r.first_bad_circuit = -1;
@@ -2031,7 +2041,24 @@ int Batch::graph_step(int prec, lsp_refactor_report *rrep, lsp_solve_report *sre
     sr.inner_total = fused ? fused_steps() : jmax;
     sr.converged = conv;
     sr.status = LSP_OK;
-    if (conv < nc || r.status != LSP_OK) {
+    bool finished = conv == nc && r.status == LSP_OK;
+    if (!fused && r.status == LSP_OK && status<int>(lay.nact)[nact_word(0, mg)] != 0) {
+        // circuits that had not met the inner tolerance after the recorded
+        // iterations go on from the graph's iterate
+        std::vector<char> rest(nc, 0);
+        for (int m = 0; m < nc; m++) rest[m] = !(beta[m] <= opt_.ir_outer_tol * nb[m]);
+        lsp_solve_report rg{};
+        rc = gmres_ir(d_b_, d_x_, prec, &rest, &rg, true);
+        if (rc) return rc;
+        sr.outer += rg.outer;
+        sr.inner_total += rg.inner_total;
+        sr.converged = nc - (int)std::count(rest.begin(), rest.end(), 1) + rg.converged;
+        sr.max_rel_res = rg.max_rel_res;
+        for (int m = 0; m < nc; m++)
+            if (!rest[m] && nb[m] > 0) sr.max_rel_res = std::max(sr.max_rel_res, beta[m] / nb[m]);
+        finished = sr.converged == nc;
+    }
+    if (!finished) {
         // finish eagerly (rare): full IR from x = 0 with the fp64 fallback
         lsp_solve_report s2{};
         rc = solve(d_b_, d_x_, true, &s2);

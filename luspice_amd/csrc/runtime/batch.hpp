@@ -93,8 +93,8 @@ struct DeviceArrays {
     int nstask_ = 0;
     int *d_ctr_ = nullptr;               // [0..1] factor, [2..3] fwd, [4..5] bwd
     int *d_epoch_ = nullptr;             // epoch counters: [0] factor, [1] fwd, [2] bwd
-    int *d_abort_ = nullptr;             // [0] factor, [1] trisolve
-    int *d_mstat_ = nullptr;             // kMstat per circuit
+    int *d_abort_ = nullptr;             // [0] factor, [1] trisolve (in the status block)
+    int *d_mstat_ = nullptr;             // kMstat per circuit (in the status block)
     int *d_dbg_ = nullptr;               // first stuck wait of the refactor
     long long *d_timeline_ = nullptr;    // optional refactor timeline (LSP_REFACTOR_TIMELINE)
     long long *d_tri_tl_ = nullptr;      // optional trisolve timeline (LSP_TRISOLVE_TIMELINE)
@@ -123,21 +123,45 @@ struct DeviceArrays {
            *d_z_ = nullptr, *d_t_ = nullptr, *d_ty_ = nullptr, *d_tz_ = nullptr, *d_typ_ = nullptr,
            *d_tzp_ = nullptr, *d_V_ = nullptr,
            *d_Z_ = nullptr;
+    int2 *d_sblock_ = nullptr;           // (matrix, first slice) of the GMRES products' workgroups
+    int *d_sbeg_ = nullptr;              // nmat+1 ranges of them per matrix
+    int nsblock_ = 0;
     long *d_voff_ = nullptr;
     int4 *d_chunks_ = nullptr;
     int *d_cbeg_ = nullptr;
     int nchunks_ = 0;
-    double *d_partial_ = nullptr, *d_H_ = nullptr, *d_cs_ = nullptr, *d_sn_ = nullptr,
-           *d_g_ = nullptr, *d_yv_ = nullptr, *d_beta_ = nullptr, *d_nb_ = nullptr,
-           *d_hn_ = nullptr, *d_hcol_ = nullptr;
-    int *d_act_ = nullptr, *d_jfin_ = nullptr, *d_conv_ = nullptr, *d_cycled_ = nullptr,
-        *d_nact_ = nullptr, *d_subset_ = nullptr;
+    double *d_partial_ = nullptr, *d_partial2_ = nullptr, *d_spartial_ = nullptr, *d_pnorm_ = nullptr,
+           *d_H_ = nullptr, *d_cs_ = nullptr, *d_sn_ = nullptr, *d_g_ = nullptr, *d_yv_ = nullptr;
+    int *d_act_ = nullptr, *d_conv_ = nullptr, *d_cycled_ = nullptr, *d_subset_ = nullptr;
+    // what the host reads after a refactor or solve, in one block (StatusLayout)
+    char *d_status_ = nullptr;
+    int *d_jfin_ = nullptr, *d_nact_ = nullptr;
+    double *d_hist_ = nullptr, *d_beta_ = nullptr, *d_nb_ = nullptr;
     // fused IR step: rows below the dense block by level, and per-circuit state
     int *d_frow_ = nullptr, *d_flvp_ = nullptr, *d_brow_ = nullptr, *d_blvp_ = nullptr;
     int *d_irconv_ = nullptr;
     double *d_rn2_ = nullptr, *d_bn2_ = nullptr;
     int ir_lds_n_ = 0;                   // doubles of LDS for the work vector (0: not set up)
 };
+
+// Byte offsets of the status block: everything the host looks at after a
+// refactor, a solve or a step graph, so that one copy to pinned memory brings
+// it (a refactor reads the front, a solve the back, a step all of it).
+struct StatusLayout {
+    size_t mstat, jfin, abort, nact, hist, beta, nb, end;
+    explicit StatusLayout(int nc)
+    {
+        mstat = 0;
+        jfin = mstat + sizeof(int) * (size_t)kMstat * nc;
+        abort = (jfin + sizeof(int) * (size_t)nc + 7) & ~(size_t)7;
+        nact = abort + 8 * sizeof(int);
+        hist = nact + 8 * sizeof(int);
+        beta = hist + 2 * sizeof(double);
+        nb = beta + sizeof(double) * (size_t)nc;
+        end = nb + sizeof(double) * (size_t)nc;
+    }
+};
+static_assert(kNact <= 8, "active counts in the status block");
 
 class Batch : private DeviceArrays {
 public:
@@ -196,9 +220,9 @@ public:
     // One fused step on the given vectors for every circuit (no convergence
     // skip); rel_res gets ||b - A x|| / ||b|| before the update, per circuit.
     int ir_step(const double *b, double *x, bool on_device, double *rel_res);
+    // unset: the solves' work values are to be set to the unset marker first
     int launch_trisolve_prec(int prec, const double *d_b, double *d_x, const int *active,
-                             const int *d_nact = nullptr);
-    int launch_spmv_krylov(const double *d_xv, double *d_y, const int *active);
+                             const int *d_nact = nullptr, bool unset = true);
     int launch_spmv64(const double *d_x, double *d_y, const double *d_b, const int *active);
     hipStream_t stream() const { return stream_; }
     int cur_prec() const { return cur_prec_; }
@@ -216,13 +240,19 @@ private:
     void release_device();
     template <typename T> int refactor_t(FactorSet<T> &fs, const int *d_active);
     template <typename T> int trisolve_t(FactorSet<T> &fs, const double *d_b, double *d_x,
-                                         const int *d_active, const int *d_nact = nullptr);
+                                         const int *d_active, const int *d_nact, bool unset);
+    // pieces of the GMRES launch sequence, shared by the eager solve and the step graph
+    int launch_residual(const KrylovArgs &K, const double *d_b, double *d_x, int cyc, bool x_is_zero, const int *gate);
+    int launch_inner(const KrylovArgs &K, int prec, int j, const int *d_nact);
+    int read_status(size_t from, size_t to);
+    template <typename X> const X *status(size_t off) const { return (const X *)(h_status_ + off); }
+    StatusLayout layout() const { return StatusLayout((int)circ_.size()); }
+    UnsetArgs unset_args() const { return UnsetArgs{d_ty_, d_typ_, d_tz_, d_tzp_}; }
     void *dalloc(size_t bytes);
     void dfree(void *p);
     int alloc_krylov(int mm);
     template <typename X> X *upload(const std::vector<X> &v);
     int check(hipError_t e, const char *what);
-    int sync_read_int(const int *d, int *h, int count);
     KrylovArgs kargs() const;
     void account_trisolve();
 
@@ -241,6 +271,7 @@ private:
     int graph_prec_ = -1;
     bool capturing_ = false;
     int *h_pin_ = nullptr;               // pinned host words for flag reads
+    char *h_status_ = nullptr;           // pinned copy of the status block
     const char *refactor_tl_path_ = nullptr;   // LSP_REFACTOR_TIMELINE, read at creation
     const char *trisolve_tl_path_ = nullptr;   // LSP_TRISOLVE_TIMELINE, read at creation
     hipEvent_t ev_[6] = {};
