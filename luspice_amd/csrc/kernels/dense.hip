@@ -308,7 +308,7 @@ struct TileStage {
 template <typename T>
 __global__ void __launch_bounds__(256, 2) dense_lu_kernel(const DenseJob *jobs, const void *mats, const int *active,
                                                           const int4 *tasks, int ntask, int *ctr, int *epoch_word,
-                                                          int *abort_word)
+                                                          int *abort_word, long long *tick1)
 {
     extern __shared__ double lds[];
     __shared__ int s_t;
@@ -483,7 +483,10 @@ __global__ void __launch_bounds__(256, 2) dense_lu_kernel(const DenseJob *jobs, 
             if (r < J.T) atomicMax(&J.colmax[r], dbits(mx));
         }
     }
-    if (threadIdx.x < kWave && leave_queue(ctr, 1, (int)gridDim.x)) advance_epoch(epoch_word, epoch);
+    if (threadIdx.x < kWave && leave_queue(ctr, 1, (int)gridDim.x)) {
+        advance_epoch(epoch_word, epoch);
+        *tick1 = (long long)wall_clock64();
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -573,10 +576,12 @@ template <typename T, bool kLower>
 __global__ void __launch_bounds__(512) tail_trsv_kernel(const void *mats, const int2 *pairs,
                                                         const long *voff, const int *active,
                                                         double *y, const double *yp, double *z, double *x,
-                                                        int *abort_word, const double *cs, const int *n_active)
+                                                        int *abort_word, const double *cs, const int *n_active,
+                                                        long long *tick0)
 {
     // nothing active: every workgroup returns before it takes a ticket
     if (n_active && uniform(ld_relaxed(n_active)) == 0) return;
+    if (tick0 && blockIdx.x == 0 && threadIdx.x == 0) *tick0 = (long long)wall_clock64();
     const int mi = pairs[blockIdx.x].x;                // as many workgroups per matrix as it has pairs
     const TriDesc<T> M = ((const TriDesc<T> *)mats)[mi];
     const int lane = lane_id();
@@ -733,20 +738,21 @@ __global__ void __launch_bounds__(512) tail_trsv_kernel(const void *mats, const 
 // ---------------------------------------------------------------------------
 template <typename T>
 hipError_t launch_dense_lu(const DenseJob *jobs, const void *mats, const int *active, const DenseGrid &G, int *ctr,
-                           int *epoch, int *abort_word, int blocks, double ptol, double stol, hipStream_t st)
+                           int *epoch, int *abort_word, long long *tick1, int blocks, double ptol, double stol,
+                           hipStream_t st)
 {
     hipLaunchKernelGGL(dense_lu_kernel<T>, dim3(std::min(blocks, G.nlu)), dim3(256), kDiagLds, st, jobs, mats, active,
-                       G.lu, G.nlu, ctr, epoch, abort_word);
+                       G.lu, G.nlu, ctr, epoch, abort_word, tick1);
     hipLaunchKernelGGL(dense_pivot_kernel<T>, dim3(G.npivot), dim3(256), 0, st, jobs, mats, active, ptol, stol,
                        G.pivot);
     return hipGetLastError();
 }
 template hipError_t launch_dense_lu<float>(const DenseJob *, const void *, const int *, const DenseGrid &, int *, int *,
-                                           int *, int, double, double, hipStream_t);
+                                           int *, long long *, int, double, double, hipStream_t);
 template hipError_t launch_dense_lu<double>(const DenseJob *, const void *, const int *, const DenseGrid &, int *, int *,
-                                           int *, int, double, double, hipStream_t);
+                                           int *, long long *, int, double, double, hipStream_t);
 template hipError_t launch_dense_lu<__half>(const DenseJob *, const void *, const int *, const DenseGrid &, int *, int *,
-                                           int *, int, double, double, hipStream_t);
+                                           int *, long long *, int, double, double, hipStream_t);
 
 // The lists behind the grids (see DenseGrid): jobs by falling T, so that the
 // longest ones start first.
@@ -793,27 +799,30 @@ template <typename T>
 hipError_t launch_tail_solve(const void *mats, const DenseGrid &G, const long *voff, const int *active,
                              const double *b, double *y, double *yp, double *z, double *x, bool forward,
                              int *abort_word, const double *rs, const double *cs, const int *n_active,
-                             hipStream_t st)
+                             long long *tick0, hipStream_t st)
 {
     if (forward) {
         hipLaunchKernelGGL(tail_fwd_gather_kernel<T>, dim3(G.ngather), dim3(256), 0, st, mats, G.gather, voff,
                            active, b, y, yp, rs, n_active);
         hipLaunchKernelGGL((tail_trsv_kernel<T, true>), dim3(G.ntrsv), dim3(512), 0, st, mats, G.trsv, voff,
-                           active, y, yp, z, x, abort_word, cs, n_active);
+                           active, y, yp, z, x, abort_word, cs, n_active, (long long *)nullptr);
     } else {
         hipLaunchKernelGGL((tail_trsv_kernel<T, false>), dim3(G.ntrsv), dim3(512), 0, st, mats, G.trsv, voff,
-                           active, y, yp, z, x, abort_word, cs, n_active);
+                           active, y, yp, z, x, abort_word, cs, n_active, tick0);
     }
     return hipGetLastError();
 }
 template hipError_t launch_tail_solve<float>(const void *, const DenseGrid &, const long *, const int *, const double *,
                                               double *, double *, double *, double *, bool, int *,
-                                              const double *, const double *, const int *, hipStream_t);
+                                              const double *, const double *, const int *, long long *,
+                                              hipStream_t);
 template hipError_t launch_tail_solve<double>(const void *, const DenseGrid &, const long *, const int *, const double *,
                                               double *, double *, double *, double *, bool, int *,
-                                              const double *, const double *, const int *, hipStream_t);
+                                              const double *, const double *, const int *, long long *,
+                                              hipStream_t);
 template hipError_t launch_tail_solve<__half>(const void *, const DenseGrid &, const long *, const int *, const double *,
                                               double *, double *, double *, double *, bool, int *,
-                                              const double *, const double *, const int *, hipStream_t);
+                                              const double *, const double *, const int *, long long *,
+                                              hipStream_t);
 
 }  // namespace lsp

@@ -20,6 +20,16 @@ enum : int {
 // cache line each, and the count of waves finished.
 constexpr int kQueueInts = 128;
 
+// Wall-clock ticks the kernels leave in the status block: the device times of
+// the launches, without event records between them (each record drained the
+// stream and left a gap of 5-7 us).
+enum : int {
+    kTickFactor0 = 0, kTickFactor1 = 1,  // refactor: first workgroup in, last wave out
+    kTickDense1 = 2,                     // dense blocks done (the refactor's end when there are none)
+    kTickFwd0 = 3, kTickBwd0 = 4, kTickBwd1 = 5,   // solves: forward start, backward start, end
+    kTicks = 8
+};
+
 // Status words per matrix written by the refactor (FactorDesc::mstat).
 constexpr int kMstat = 8;
 

@@ -402,6 +402,7 @@ __global__ void __launch_bounds__(256) refactor_kernel(FactorLaunch L)
     LSP_GLOBAL double *xg = gp(L.scratch) + ((long)blockIdx.x * waves_per_block + wv) * L.scratch_stride;
     const FactorDesc<T> *mats = (const FactorDesc<T> *)L.mats;
     const int epoch = read_epoch(L.epoch);
+    if (blockIdx.x == 0 && threadIdx.x == 0) L.ticks[kTickFactor0] = (long long)wall_clock64();
 
     const int nq = queue_count(L.nq);
     const int q = queue_index(nq);
@@ -438,7 +439,10 @@ __global__ void __launch_bounds__(256) refactor_kernel(FactorLaunch L)
         }
     }
     // the last wave out re-arms the queue and advances the epoch
-    if (leave_queue(L.ctr, nq, L.total_waves)) advance_epoch(L.epoch, epoch);
+    if (leave_queue(L.ctr, nq, L.total_waves)) {
+        advance_epoch(L.epoch, epoch);
+        L.ticks[kTickFactor1] = L.ticks[kTickDense1] = (long long)wall_clock64();
+    }
 }
 
 }  // namespace lsp

@@ -29,6 +29,7 @@ struct FactorLaunch {
     long long *timeline;    // optional, 4 per task (100 MHz wall clock): start, flag
                             // published (end for a dense-block column), end of the
                             // last dependency wait, column
+    long long *ticks;       // kTick*: start and end of the launch
     int poll_backoff;       // dependency polls back off to at most poll_backoff + 1 sleeps
     int nq;                 // queue counters (1, 2 or 4) in the ctr block
 };
@@ -45,6 +46,7 @@ struct TriLaunch {
     const double *rs, *cs;  // optional row / column scales (Ruiz): b_s = R b, x = C z
     const int *n_active;    // optional: when *n_active == 0 no circuit is active, tasks are skipped
     long long *timeline;    // optional diagnostic, 2 per task: ticket granted, task finished
+    long long *tick0, *tick1;   // optional: start and end of the launch (kTick*)
     int ntask;
     int *ctr;               // kQueueInts: queue counters, waves finished
     int *abort_word;
@@ -164,12 +166,13 @@ struct DenseGrid {
 void dense_grid_lists(const std::vector<int> &T, const std::vector<int> &mat, DenseGridHost &H);
 template <typename T>
 hipError_t launch_dense_lu(const DenseJob *jobs, const void *mats, const int *active, const DenseGrid &G, int *ctr,
-                           int *epoch, int *abort_word, int blocks, double ptol, double stol, hipStream_t st);
+                           int *epoch, int *abort_word, long long *tick1, int blocks, double ptol, double stol,
+                           hipStream_t st);
 template <typename T>
 hipError_t launch_tail_solve(const void *mats, const DenseGrid &G, const long *voff, const int *active,
                              const double *b, double *y, double *yp, double *z, double *x, bool forward,
                              int *abort_word, const double *rs, const double *cs, const int *n_active,
-                             hipStream_t st);
+                             long long *tick0, hipStream_t st);
 
 // trisolve.hip
 template <typename T>

@@ -397,6 +397,7 @@ __device__ __forceinline__ void trisolve_body(const TriLaunch &L)
     // Every wave of the grid reads the same count (written by an earlier
     // launch) and returns at once: no ticket and no finish count.
     if (L.n_active && uniform(ld_relaxed(L.n_active)) == 0) return;
+    if (L.tick0 && blockIdx.x == 0 && threadIdx.x == 0) *L.tick0 = (long long)wall_clock64();
     const int nq = queue_count(L.nq);
     for (;;) {
         const int t = next_task(L.ctr, nq);
@@ -410,7 +411,8 @@ __device__ __forceinline__ void trisolve_body(const TriLaunch &L)
             L.timeline[2L * t + 1] = (long long)wall_clock64();
         }
     }
-    leave_queue(L.ctr, nq, L.total_waves);             // the last wave out re-arms the queue
+    // the last wave out re-arms the queue
+    if (leave_queue(L.ctr, nq, L.total_waves) && L.tick1) *L.tick1 = (long long)wall_clock64();
 }
 
 template <typename T>
@@ -424,12 +426,14 @@ __global__ void __launch_bounds__(256) trisolve_bwd_kernel(TriLaunch L)
     trisolve_body<T, false>(L);
 }
 
-// Sets the solve's work values (y, yp, z, zp) to the unset marker; skipped
-// when no circuit is active (the solves then return at once as well).
+// Sets the solve's work values (y, yp, z, zp) to the unset marker and clears
+// the abort word; skipped when no circuit is active (the solves then return at
+// once as well).
 __global__ void __launch_bounds__(256) solve_unset_kernel(double *y, double *yp, double *z, double *zp, long n,
-                                                          const int *n_active)
+                                                          const int *n_active, int *abort_word)
 {
     if (n_active && uniform(ld_relaxed(n_active)) == 0) return;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *abort_word = 0;
     const double u = Unset<double>::value();
     for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += (long)gridDim.x * 256L) {
         y[i] = u;
@@ -443,7 +447,7 @@ hipError_t launch_solve_unset(const TriLaunch &L, long n, hipStream_t st)
 {
     const long blocks = std::max(1L, std::min(4096L, (n + 255) / 256));
     hipLaunchKernelGGL(solve_unset_kernel, dim3((unsigned)blocks), dim3(256), 0, st, L.y, L.yp, L.z, L.zp, n,
-                       L.n_active);
+                       L.n_active, L.abort_word);
     return hipGetLastError();
 }
 

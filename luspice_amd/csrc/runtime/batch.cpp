@@ -38,7 +38,6 @@ Batch::~Batch()
     for (auto &m : mem_) if (m.p) (void)hipFree(m.p);
     if (h_pin_) (void)hipHostFree(h_pin_);
     if (h_status_) (void)hipHostFree(h_status_);
-    for (auto &e : ev_) if (e) (void)hipEventDestroy(e);
     if (own_stream_ && stream_) (void)hipStreamDestroy(stream_);
 }
 
@@ -163,20 +162,16 @@ int Batch::read_status(size_t from, size_t to)
 }
 
 // Adds the device time of the last forward/backward trisolve pair to the
-// running statistics; called after a stream synchronisation, when its events
-// are complete.
+// running statistics; called once the host has its ticks.
 void Batch::account_trisolve()
 {
     if (!tri_pending_) return;
-    float a = 0, b = 0;
-    if (hipEventElapsedTime(&a, ev_[2], ev_[4]) == hipSuccess &&
-        hipEventElapsedTime(&b, ev_[4], ev_[3]) == hipSuccess) {
-        t_fwd_ = a;
-        t_bwd_ = b;
-        stats_.fwd_ms += a;
-        stats_.bwd_ms += b;
-        stats_.tri_count++;
-    }
+    const long long *t = status<long long>(layout().ticks);
+    t_fwd_ = (float)((double)(t[kTickBwd0] - t[kTickFwd0]) * ms_per_tick_);
+    t_bwd_ = (float)((double)(t[kTickBwd1] - t[kTickBwd0]) * ms_per_tick_);
+    stats_.fwd_ms += t_fwd_;
+    stats_.bwd_ms += t_bwd_;
+    stats_.tri_count++;
     tri_pending_ = false;
 }
 
@@ -493,6 +488,9 @@ int Batch::upload_all()
     rc = check(hipGetDeviceProperties(&prop, dev), "hipGetDeviceProperties");
     if (rc) return rc;
     cu_count_ = prop.multiProcessorCount;
+    int khz = 0;
+    if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) == hipSuccess && khz > 0)
+        ms_per_tick_ = 1.0 / khz;
     if (!stream_) {
         rc = check(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking), "stream");
         if (rc) return rc;
@@ -615,6 +613,7 @@ int Batch::upload_all()
         if (rc) return rc;
         d_mstat_ = (int *)(d_status_ + lay.mstat);
         d_jfin_ = (int *)(d_status_ + lay.jfin);
+        d_ticks_ = (long long *)(d_status_ + lay.ticks);
         d_abort_ = (int *)(d_status_ + lay.abort);
         d_nact_ = (int *)(d_status_ + lay.nact);
         d_hist_ = (double *)(d_status_ + lay.hist);
@@ -922,11 +921,6 @@ int Batch::upload_all()
         if (!h_pin_ && hipHostMalloc((void **)&h_pin_, 4096, hipHostMallocDefault) != hipSuccess)
             return LSP_E_ALLOC;
     }
-    for (auto &e : ev_) {
-        if (e) continue;
-        rc = check(hipEventCreate(&e), "event");
-        if (rc) return rc;
-    }
     // initial SELL values
     rc = check(launch_gather_cast<double>(nsell_tot_, d_ssrc_, d_ain_, d_sval64_, stream_), "gather");
     if (!rc) rc = check(launch_gather_cast<float>(nsell_tot_, d_ssrc_, d_ain_, d_sval32_, stream_), "gather");
@@ -1040,17 +1034,15 @@ int Batch::refactor_t(FactorSet<T> &fs, const int *d_active)
     L.ptol = opt_.refactor_ptol;
     L.stol = opt_.repivot == 3 ? opt_.pivot_tol : 0.0;
     L.dbg = d_dbg_;
+    L.ticks = d_ticks_;
     rc = check(launch_fill_unset<T>(fs.fdesc, d_active, d_fillchunk_, nfillchunk_, d_abort_, d_dbg_, stream_), "unset");
     if (rc) return rc;
-    if (!capturing_) (void)hipEventRecord(ev_[0], stream_);   // the persistent kernel alone, from here
     rc = check(launch_refactor<T>(L, fblocks_, stream_), "refactor launch");
-    if (!capturing_) (void)hipEventRecord(ev_[1], stream_);      // the persistent kernel alone
     if (!rc && njobs_) {
         // two 4-wave workgroups per CU (the kernel's register budget)
         rc = check(launch_dense_lu<T>(d_djobs_, fs.fdesc, d_active, dgrid_, d_ctr_ + 3 * kQueueInts, d_epoch_ + 1,
-                                      d_abort_, 2 * cu_count_, opt_.refactor_ptol, L.stol, stream_), "dense lu");
+                                      d_abort_, d_ticks_ + kTickDense1, 2 * cu_count_, opt_.refactor_ptol, L.stol, stream_), "dense lu");
     }
-    if (!capturing_) (void)hipEventRecord(ev_[5], stream_);      // + dense trailing block
     return rc;
 }
 
@@ -1115,10 +1107,10 @@ int Batch::refactor_pass(int prec, const std::vector<int> *subset, std::vector<i
     if (rc) return rc;
     ms.assign(status<int>(lay.mstat), status<int>(lay.mstat) + (size_t)kMstat * circ_.size());
     h_pin_[0] = status<int>(lay.abort)[0];
-    float t_kernel = 0.0f, t_all = 0.0f;
-    (void)hipEventElapsedTime(&t_kernel, ev_[0], ev_[1]);
-    (void)hipEventElapsedTime(&t_all, ev_[0], ev_[5]);
-    t_refactor_ = t_all;
+    const long long *tk = status<long long>(lay.ticks);
+    const double t_kernel = (double)(tk[kTickFactor1] - tk[kTickFactor0]) * ms_per_tick_;
+    const double t_all = (double)(tk[kTickDense1] - tk[kTickFactor0]) * ms_per_tick_;
+    t_refactor_ = (float)t_all;
     stats_.refactor_ms += t_kernel;
     stats_.dense_ms += t_all - t_kernel;
     stats_.refactor_count++;
@@ -1307,27 +1299,27 @@ int Batch::trisolve_t(FactorSet<T> &fs, const double *d_b, double *d_x, const in
         if (!d_tri_tl_) d_tri_tl_ = (long long *)dalloc((size_t)(nfw_tot_ + nbw_tot_) * 2 * sizeof(long long));
         Lf.timeline = d_tri_tl_;
     }
+    Lf.tick0 = d_ticks_ + kTickFwd0;
     TriLaunch Lb = Lf;
+    Lb.tick0 = njobs_ ? nullptr : d_ticks_ + kTickBwd0;      // the dense blocks' upper solve starts it
+    Lb.tick1 = d_ticks_ + kTickBwd1;
     Lb.timeline = Lf.timeline ? Lf.timeline + 2 * nfw_tot_ : nullptr;
     Lb.task = d_bwtask_;
     Lb.ntask = (int)nbw_tot_;
     Lb.ctr = d_ctr_ + 2 * kQueueInts;
     Lb.total_waves = tblocks_b_ * 4;
     Lb.nq = nq_t_;
-    if (!capturing_) (void)hipEventRecord(ev_[2], stream_);
     int rc = unset ? check(launch_solve_unset(Lf, ntot_, stream_), "solve unset") : LSP_OK;
     if (!rc) rc = check(launch_trisolve_half<T>(Lf, true, tblocks_f_, stream_), "trisolve fwd");
     if (!rc && njobs_)
         rc = check(launch_tail_solve<T>(fs.tdesc, dgrid_, d_voff_, d_active, d_b, d_ty_, d_typ_, d_tz_, d_x, true,
-                                        d_abort_ + 1, Lf.rs, Lf.cs, d_nact, stream_),
+                                        d_abort_ + 1, Lf.rs, Lf.cs, d_nact, nullptr, stream_),
                    "tail fwd");
-    if (!capturing_) (void)hipEventRecord(ev_[4], stream_);
     if (!rc && njobs_)
         rc = check(launch_tail_solve<T>(fs.tdesc, dgrid_, d_voff_, d_active, d_b, d_ty_, d_typ_, d_tz_, d_x, false,
-                                        d_abort_ + 1, Lf.rs, Lf.cs, d_nact, stream_),
+                                        d_abort_ + 1, Lf.rs, Lf.cs, d_nact, d_ticks_ + kTickBwd0, stream_),
                    "tail bwd");
     if (!rc) rc = check(launch_trisolve_half<T>(Lb, false, tblocks_b_, stream_), "trisolve bwd");
-    if (!capturing_) (void)hipEventRecord(ev_[3], stream_);
     if (!capturing_) tri_pending_ = true;
     return rc;
 }
@@ -1359,18 +1351,15 @@ int Batch::trisolve(const double *b, double *x, bool on_device)
         db = d_b_;
         dx = d_x_;
     }
-    rc = check(k_zero_int(d_abort_ + 1, 1, stream_), "abort reset");
-    if (rc) return rc;
     rc = launch_trisolve_prec(cur_prec_, db, dx, nullptr);
     if (rc) return rc;
     if (!on_device) {
         rc = check(hipMemcpyAsync(x, d_x_, ntot_ * 8, hipMemcpyDeviceToHost, stream_), "x");
         if (rc) return rc;
     }
-    rc = check(hipMemcpyAsync(h_pin_, d_abort_ + 1, 4, hipMemcpyDeviceToHost, stream_), "abort");
-    if (!rc) rc = check(hipStreamSynchronize(stream_), "sync");
+    const StatusLayout lay = layout();
+    rc = read_status(lay.ticks, lay.nact);
     if (rc) return rc;
-    account_trisolve();
     const char *tl_path = trisolve_tl_path_;
     if (tl_path && d_tri_tl_) {
         // [nfw, nbw] (int64), forward then backward task lists (int32 x 2 per
@@ -1390,7 +1379,7 @@ int Batch::trisolve(const double *b, double *x, bool on_device)
             fclose(f);
         }
     }
-    return h_pin_[0] ? LSP_E_DEVICE : LSP_OK;
+    return status<int>(lay.abort)[1] ? LSP_E_DEVICE : LSP_OK;
 }
 
 int Batch::spmv(const double *x, double *y, bool on_device, int prec)
@@ -1507,7 +1496,7 @@ int Batch::gmres_ir(const double *d_bv, double *d_xv, int prec, const std::vecto
             const int *gate = d_nact_ + nact_word(cyc, j + 1);
             LSP_HIP(k_update(K, d_Z_, d_xv, gate, s), "update");
             LSP_TRY(launch_residual(K, d_bv, d_xv, cyc + 1, false, gate));
-            LSP_TRY(read_status(lay.abort, lay.end));
+            LSP_TRY(read_status(lay.ticks, lay.end));
             if (status<int>(lay.abort)[1]) return LSP_E_DEVICE;
             if (cyc == 0 && j == 0) {
                 res_hist0_.push_back(hist[0]);

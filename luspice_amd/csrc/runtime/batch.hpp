@@ -62,6 +62,7 @@ struct FactorSet {                       // per storage precision
 struct DeviceArrays {
     long ntot_ = 0, nnz_tot_ = 0;
     int cu_count_ = 0;
+    double ms_per_tick_ = 1e-5;          // of the device wall clock
     int mm_alloc_ = 0;
     // structure (device)
     int64_t *d_cp_ = nullptr, *d_relp_ = nullptr, *d_soff_ = nullptr;
@@ -136,6 +137,7 @@ struct DeviceArrays {
     // what the host reads after a refactor or solve, in one block (StatusLayout)
     char *d_status_ = nullptr;
     int *d_jfin_ = nullptr, *d_nact_ = nullptr;
+    long long *d_ticks_ = nullptr;
     double *d_hist_ = nullptr, *d_beta_ = nullptr, *d_nb_ = nullptr;
     // fused IR step: rows below the dense block by level, and per-circuit state
     int *d_frow_ = nullptr, *d_flvp_ = nullptr, *d_brow_ = nullptr, *d_blvp_ = nullptr;
@@ -148,12 +150,13 @@ struct DeviceArrays {
 // refactor, a solve or a step graph, so that one copy to pinned memory brings
 // it (a refactor reads the front, a solve the back, a step all of it).
 struct StatusLayout {
-    size_t mstat, jfin, abort, nact, hist, beta, nb, end;
+    size_t mstat, jfin, ticks, abort, nact, hist, beta, nb, end;
     explicit StatusLayout(int nc)
     {
         mstat = 0;
         jfin = mstat + sizeof(int) * (size_t)kMstat * nc;
-        abort = (jfin + sizeof(int) * (size_t)nc + 7) & ~(size_t)7;
+        ticks = (jfin + sizeof(int) * (size_t)nc + 7) & ~(size_t)7;
+        abort = ticks + sizeof(long long) * kTicks;
         nact = abort + 8 * sizeof(int);
         hist = nact + 8 * sizeof(int);
         beta = hist + 2 * sizeof(double);
@@ -274,7 +277,6 @@ private:
     char *h_status_ = nullptr;           // pinned copy of the status block
     const char *refactor_tl_path_ = nullptr;   // LSP_REFACTOR_TIMELINE, read at creation
     const char *trisolve_tl_path_ = nullptr;   // LSP_TRISOLVE_TIMELINE, read at creation
-    hipEvent_t ev_[6] = {};
     float t_refactor_ = 0, t_fwd_ = 0, t_bwd_ = 0;
     bool tri_pending_ = false;
     std::vector<double> res_hist0_;      // ||r||/||b|| of circuit 0 at each restart
