@@ -82,7 +82,7 @@ struct LspPlan {
     // dependency levels of the factorization (U pattern, level.c semantics)
     std::vector<int> level;               // n
     int nlevels = 0;
-    std::vector<int> ftask;               // columns sorted by (level, k)
+    std::vector<int> ftask;               // columns in refactor task order
     // row-wise copies for the row-gather trisolve
     std::vector<int> lrp, lci;            // L strictly lower, CSR by position
     std::vector<int> urp, uci;            // U strictly upper, CSR by position
@@ -126,14 +126,16 @@ struct LspPlan {
     int tail_T = 0;
     std::vector<int> tail_ds;             // T: U slots of tail column k0+c with pos < k0
     std::vector<int> tail_lcut;           // T: first lci index of tail row k0+r with col >= k0
-    std::vector<int> fkey;                // n: ordering key of column k's refactor task
+    std::vector<int> fkey;                // n: ordering key of column k's refactor task (rises
+                                          // along every dependency, counts back from the
+                                          // circuit's last level)
     int64_t tail_updates = 0;             // updates moved into the dense block
 };
 
 // Chooses the dense trailing block: the largest T in [min_T, max_T] whose
 // pattern density nnz(block) / T^2 is at least min_density (no tail when none
-// qualifies or max_T <= 0).  Rebuilds ftask (sparse columns by level, tail
-// columns keyed after their sparse dependencies), fwd_task / bwd_task (rows
+// qualifies or max_T <= 0).  Rebuilds ftask and fkey (each column a fixed lead
+// ahead of the last level that does not delay the end), fwd_task / bwd_task (rows
 // below k0 only, backward levels recomputed with the tail rows solved first)
 // and the tail maps.  Returns T.
 int lsp_plan_set_tail(LspPlan &P, int min_T, int max_T, double min_density);

@@ -7,11 +7,11 @@
 // pattern fixed by the CPU symbolic analysis, the way a Newton refactor reuses
 // them.  The reference launches one kernel per level
 // (bench/test_lu_wave.cu:200-217, src/mp/multiblock_lu.cu:423-431); here one
-// persistent launch walks every level of every matrix in the batch.
+// persistent launch walks every column of every matrix in the batch.
 //
 // Mapping to CDNA4
-//   * one wave64 per column task; tasks come from a global queue in level
-//     order, so a task only waits on tasks handed out earlier, which are held
+//   * one wave64 per column task; tasks come from a global queue in an
+//     order that rises along every dependency, so a task only waits on tasks handed out earlier, which are held
 //     by running waves: the schedule cannot deadlock whatever the occupancy;
 //   * the column's working vector x (fp64) lives in LDS when it fits
 //     (cap doubles per wave), else in a per-wave global scratch slice;

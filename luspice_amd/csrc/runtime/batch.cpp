@@ -5,7 +5,7 @@
 //   patterns, A scatter map, update map, levels, row-wise copies) and the
 //   SELL-C-64 layout.  Then every structure array of every circuit is
 //   concatenated into one device arena and the per-circuit descriptors are
-//   written.  Task lists of all circuits are merged by level so that one
+//   written.  Task lists of all circuits are merged by their keys so that one
 //   persistent launch advances every circuit's dependency front at once.
 // refactor(): value repack for SpMV + one persistent refactor launch.
 // solve(): fp64 GMRES-IR, every vector on the device; the host reads one
@@ -786,7 +786,7 @@ int Batch::upload_all()
         nstask_ = (int)st.size();
         if (!d_sdesc64_ || !d_sdesc32_ || !d_stask_) return LSP_E_ALLOC;
     }
-    // merged task lists: (level, circuit, index)
+    // merged task lists: (key, circuit, index)
     {
         auto merge = [&](auto key_of, auto order_of, long &width) {
             std::vector<std::pair<long, int2>> all;
