@@ -77,6 +77,12 @@ struct LspPlan {
     // holds the local slot in k of every row of L(:, e-1).
     std::vector<int64_t> relp;            // n+1
     std::vector<uint16_t> rel;            // local slots (max_col <= 65535)
+    // Per dependency (the first U slots of column k: all of them, or those left
+    // of the dense block), from depp[k] on: its first L slot (low word), the
+    // length of its run's last L column (low half of the high word) and the
+    // columns of the run after it (high half).
+    std::vector<int> depp;                // n+1
+    std::vector<uint64_t> dep;
     int64_t n_segments = 0;               // runs over all columns
     int max_col = 0;                      // max column pattern length
     // dependency levels of the factorization (U pattern, level.c semantics)
@@ -153,9 +159,11 @@ void lsp_ruiz_scales(int n, long nnz, const int *row, const int *col, const doub
 
 // Build the plan from A (q-order CSC, values only used for nothing here) and
 // the symbolic factors.  src_index maps each q-CSC entry to the caller's value
-// order (nullptr = identity).  Returns 0 ok, <0 on an inconsistent structure.
+// order (nullptr = identity).  A caller that goes on to lsp_plan_set_tail, which
+// builds the segments anew, passes segments = false.  Returns 0 ok, <0 on an
+// inconsistent structure.
 int lsp_build_plan(int n, const int *Ap, const int *Ai, const int *src_index,
-                   const LspGpLu &F, const int *q, LspPlan &P);
+                   const LspGpLu &F, const int *q, LspPlan &P, bool segments = true);
 
 // ---------------------------------------------------------------------------
 // SELL-C-sigma layout of A in original row/column order (sell.cpp)

@@ -146,7 +146,7 @@ static void sort_by_level(const std::vector<int> &lv, int nlv, std::vector<int> 
 }
 
 int lsp_build_plan(int n, const int *Ap, const int *Ai, const int *src_index,
-                   const LspGpLu &F, const int *q, LspPlan &P)
+                   const LspGpLu &F, const int *q, LspPlan &P, bool segments)
 {
     P = LspPlan();
     if (n >= kTriWideBase / 2) return -1;        // row task codes 2i + 1 stay below the block codes
@@ -289,7 +289,7 @@ int lsp_build_plan(int n, const int *Ap, const int *Ai, const int *src_index,
     P.tail_k0 = n;
     P.tail_T = 0;
     P.fkey = P.level;
-    return lsp_plan_build_segments(P);
+    return segments ? lsp_plan_build_segments(P) : 0;
 }
 
 static void plan_tri_supernodes(LspPlan &P);
@@ -319,6 +319,9 @@ int lsp_plan_build_segments(LspPlan &P)
     std::vector<int> where(n, -1), owner(n, -1);
     P.relp.assign(n + 1, 0);
     P.rel.clear();
+    P.depp.assign(n + 1, 0);
+    P.dep.clear();
+    P.dep.reserve(P.n_u);
     P.n_segments = 0;
     for (int k = 0; k < n; k++) {
         const int64_t c0 = P.cp[k];
@@ -327,21 +330,24 @@ int lsp_plan_build_segments(LspPlan &P)
             owner[P.pos[s]] = k;
         }
         const int ndep = k < k0 ? P.dp[k] - (int)c0 : P.tail_ds[k - k0];
-        for (int t = 0; t < ndep; t++) {
+        for (int t = 0; t < ndep;) {
             const int j = P.pos[c0 + t];
             const int e = std::min(P.snend[j], k);
-            const bool last = t + 1 == ndep || P.pos[c0 + t + 1] != j + 1 ||
-                              std::min(P.snend[P.pos[c0 + t + 1]], k) != e;
-            if (!last) continue;
-            if (j != e - 1) return -10;            // run stops inside its supernode
+            const int w = e - j;                       // columns of the run
+            if (t + w > ndep || P.pos[c0 + t + w - 1] != e - 1) return -10;   // run stops inside its supernode
+            const uint64_t nl = (uint64_t)(uint16_t)llen(e - 1) << 32;
+            for (int i = 0; i < w; i++)
+                P.dep.push_back((uint64_t)(uint32_t)(P.dp[j + i] + 1) | nl | (uint64_t)(w - 1 - i) << 48);
             P.n_segments++;
-            for (int64_t s = P.dp[j] + 1; s < P.cp[j + 1]; s++) {
+            for (int64_t s = P.dp[e - 1] + 1; s < P.cp[e]; s++) {
                 const int ps = P.pos[s];
-                if (owner[ps] != k) return -8;     // fill outside the pattern
+                if (owner[ps] != k) return -8;         // fill outside the pattern
                 P.rel.push_back((uint16_t)where[ps]);
             }
+            t += w;
         }
         P.relp[k + 1] = (int64_t)P.rel.size();
+        P.depp[k + 1] = (int)P.dep.size();
     }
     plan_tri_supernodes(P);
     return 0;
@@ -513,18 +519,22 @@ constexpr int kTaskLead = 32;
 static void order_factor_tasks(LspPlan &P)
 {
     const int n = P.n;
-    std::vector<int> h(n, 0), early(n, 0);      // longest chain after / before the column
+    std::vector<int> h(n, 0), at(n);            // longest chain after each column
     int top = 0;
     for (int k = n - 1; k >= 0; k--) {
-        top = std::max(top, h[k]);
+        const int hk = h[k] + 1;
+        top = std::max(top, hk - 1);
         const int64_t e = k < P.tail_k0 ? P.dp[k] : P.cp[k] + P.tail_ds[k - P.tail_k0];
-        for (int64_t s = P.cp[k]; s < e; s++) h[P.pos[s]] = std::max(h[P.pos[s]], h[k] + 1);
+        for (int64_t s = P.cp[k]; s < e; s++) h[P.pos[s]] = std::max(h[P.pos[s]], hk);
     }
-    std::vector<int> at(n);
     for (int k = 0; k < n; k++) {
-        const int64_t e = k < P.tail_k0 ? P.dp[k] : P.cp[k] + P.tail_ds[k - P.tail_k0];
-        for (int64_t s = P.cp[k]; s < e; s++) early[k] = std::max(early[k], early[P.pos[s]] + 1);
-        at[k] = std::max(early[k], top - h[k] - kTaskLead);
+        int early = P.level[k];
+        if (k >= P.tail_k0) {                   // no dependency inside the block
+            early = 0;
+            const int64_t e = P.cp[k] + P.tail_ds[k - P.tail_k0];
+            for (int64_t s = P.cp[k]; s < e; s++) early = std::max(early, P.level[P.pos[s]] + 1);
+        }
+        at[k] = std::max(early, top - h[k] - kTaskLead);
         P.fkey[k] = at[k] - top;
     }
     sort_by_level(at, top + 1, P.ftask);

@@ -26,6 +26,10 @@ namespace lsp {
 // device arrays through LSP_GLOBAL pointers and LDS through LSP_LDS pointers.
 #define LSP_GLOBAL __attribute__((address_space(1)))
 #define LSP_LDS __attribute__((address_space(3)))
+// Memory that nothing writes while the kernel runs, read at wave-uniform
+// addresses: scalar loads, which need no wait for the vector loads in flight.
+#define LSP_CONST __attribute__((address_space(4)))
+template <typename T> __device__ __forceinline__ const LSP_CONST T *kp(const T *p) { return (const LSP_CONST T *)p; }
 template <typename T> __device__ __forceinline__ LSP_GLOBAL T *gp(T *p) { return (LSP_GLOBAL T *)p; }
 template <typename T> __device__ __forceinline__ const LSP_GLOBAL T *gp(const T *p)
 {
@@ -216,6 +220,17 @@ template <> __device__ __forceinline__ __half ld_plain<__half>(const LSP_GLOBAL 
 {
     return __ushort_as_half(((const LSP_GLOBAL unsigned short *)base)[i]);
 }
+// The same for an element less than 2^28 away: the offset in bytes stays in 32
+// bits, so the load takes its base from SGPRs and one offset register instead
+// of a 64-bit address.
+template <typename T> __device__ __forceinline__ const LSP_GLOBAL T *near_el(const LSP_GLOBAL T *base, uint32_t i)
+{
+    return (const LSP_GLOBAL T *)((const LSP_GLOBAL char *)base + (uint32_t)(i * (uint32_t)sizeof(T)));
+}
+template <typename T> __device__ __forceinline__ T ld_coherent_near(const LSP_GLOBAL T *base, uint32_t i)
+{
+    return ld_coherent_val(near_el(base, i), 0u);
+}
 template <bool kCoherent, typename T>
 __device__ __forceinline__ T ld_val(const LSP_GLOBAL T *base, uint32_t i)
 {
@@ -312,13 +327,14 @@ __device__ __forceinline__ int wave_wait_prefix(const int *flag, int epoch, int 
     int seen = epoch;
     int backoff = 0;
     for (int round = 0;; round++) {
+        const unsigned long long miss = ~__ballot(ok);
+        const int p = miss ? min(nd, (int)__builtin_ctzll(miss)) : nd;
+        if (p > have) return p;
         if (!ok) {
             seen = ld_relaxed(flag);
             ok = seen == epoch;
         }
-        const unsigned long long miss = ~__ballot(ok);
-        const int p = miss ? min(nd, (int)__builtin_ctzll(miss)) : nd;
-        if (p > have) return p;
+        if (round == 0) continue;               // the first look comes before the first sleep
         if ((round & 15) == 15 && aborted(abort_word)) return -1;
         if (round > kRoundLimit) {
             if (!ok && atomicCAS(abort_word, 0, kErrSpin) == 0 && dbg) {
@@ -465,9 +481,8 @@ constexpr int kTri = kWave - 1;         // triangle steps held in registers (64-
 // masked), so the chain waits on registers only; a caller may load them
 // (load_triangle) before it waits for the right-hand side.
 template <int NT, bool kCoherent = true, typename T>
-__device__ __forceinline__ void load_triangle(const T *val, int lb, int ta, int tb, T (&tv)[NT])
+__device__ __forceinline__ void load_triangle(const T *val, int lb, int ta, int tb, T (&tv)[NT], int lane = lane_id())
 {
-    const int lane = lane_id();
     const int bw = tb - ta;
 #pragma unroll
     for (int q = 0; q < NT; q++) {
@@ -475,13 +490,12 @@ __device__ __forceinline__ void load_triangle(const T *val, int lb, int ta, int 
         const int tp = ta + qq;
         const int base = __builtin_amdgcn_readlane(lb, tp);
         const int off = min(max(lane - tp - 1, 0), bw - qq - 2);
-        tv[q] = ld_val<kCoherent>(gp(val) + (uint32_t)base, (uint32_t)off);
+        tv[q] = ld_val<kCoherent>(near_el(gp(val) + (uint32_t)base, (uint32_t)off), 0u);
     }
 }
 template <int NT, typename T>
-__device__ __forceinline__ double apply_triangle(const T (&tv)[NT], double xc, int ta, int tb)
+__device__ __forceinline__ double apply_triangle(const T (&tv)[NT], double xc, int ta, int tb, int lane = lane_id())
 {
-    const int lane = lane_id();
 #pragma unroll
     for (int q = 0; q < NT; q++) {
         const int tp = min(ta + q, kWave - 1);
@@ -492,11 +506,11 @@ __device__ __forceinline__ double apply_triangle(const T (&tv)[NT], double xc, i
     return xc;
 }
 template <int NT, bool kCoherent = true, typename T>
-__device__ __forceinline__ double run_triangle(const T *val, double xc, int lb, int ta, int tb)
+__device__ __forceinline__ double run_triangle(const T *val, double xc, int lb, int ta, int tb, int lane = lane_id())
 {
     T tv[NT];
-    load_triangle<NT, kCoherent>(val, lb, ta, tb, tv);
-    return apply_triangle<NT>(tv, xc, ta, tb);
+    load_triangle<NT, kCoherent>(val, lb, ta, tb, tv, lane);
+    return apply_triangle<NT>(tv, xc, ta, tb, lane);
 }
 // Upper triangular solve of a block of bw rows held one per lane (row t of
 // the block in lane t): column q' of the block's U is U(j_t, j_q') =

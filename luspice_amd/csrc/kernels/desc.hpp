@@ -40,19 +40,32 @@ constexpr int kTriPacket = 1 << 30;
 constexpr int kTriWide = 1 << 29;
 constexpr int kTriPacketLane = 4;
 
+// One task of the refactor, as the kernel reads it: what it needs to start
+// a column's loads, so that they depend on one record and not on a chain of
+// pointers.
+struct FactorTask {
+    int mat, k;             // matrix, column
+    int c0;                 // first slot
+    int a0, na;             // A(:, k): first entry, count
+    int d0;                 // first dependency record
+    long long u;            // segment-map cursor
+    uint16_t m, dl;         // slots, local slot of the diagonal
+    uint16_t ndep;          // dependencies (U slots; left of the dense block)
+    uint16_t tail;          // 1: a column of the dense trailing block
+    int pad_;
+};
+
 // Numeric refactorization over the static column patterns.
 template <typename T>
 struct FactorDesc {
     const int64_t *cp;      // n+1 slot pointers
-    const int *dp;          // n diagonal slots (absolute)
     const int *pos;         // slot -> row position
-    const int *aptr;        // n+1 q-order CSC pointers of A
     const int *asrc;        // A entry -> input value index
     const int *aslot;       // A entry -> local slot (-1 skipped duplicate)
     const double *ain;      // input values (fp64, caller order)
-    const int64_t *relp;    // n+1 segment-map pointers
     const uint16_t *rel;    // segment maps: local slots of each run's last L rows
-    const int *snend;       // n: one past the last column of j's supernode
+    const uint64_t *dep;    // dependency records: first L slot; length of the run's
+                            // last L column (16 bits), columns of the run after it
     const int *dst;         // slot -> index in lrow / urow / diag
     const int *dpos;        // n: position of the diagonal row q[k] (pinv[q[k]])
     T *val;                 // column storage of L and U

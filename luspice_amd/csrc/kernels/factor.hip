@@ -15,9 +15,12 @@
 //     by running waves: the schedule cannot deadlock whatever the occupancy;
 //   * the column's working vector x (fp64) lives in LDS when it fits
 //     (cap doubles per wave), else in a per-wave global scratch slice;
+//   * a task is one record and a dependency one more, so a column's loads are
+//     a chain of four round trips (record; dependency records and A's entries;
+//     flags and A's values; L), not ten through pointer arrays;
 //   * dependencies are fetched 64 at a time (one lane per dependency) and
 //     applied in order, by supernode segment, as soon as a leading group of
-//     their flags has been seen; rows below a segment are reached through
+//     their flags has been seen; inside the last run, by their values; rows below a segment are reached through
 //     16-bit local slot indices precomputed by the plan, so no search and no
 //     atomics touch x;
 //   * the finished column's L part is stored with agent-coherent stores and
@@ -27,6 +30,7 @@
 //     max-reduction) and the stores read only after the launch (U, diagonal,
 //     row-wise copies) follow the flag.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.hpp"
 #include "launch.hpp"
@@ -44,9 +48,8 @@ constexpr int kGemvBatch = 16;          // L values in flight per GEMV row pass
 // keeps G * B loads outstanding; every row is updated once.
 template <int G, int B, typename T, typename XP>
 __device__ __forceinline__ void run_gemv(const T *val, XP x, const LSP_GLOBAL uint16_t *map, int64_t u, double xc,
-                                         int lb, int ta, int tb, int tri, int R, int s0)
+                                         int lb, int ta, int tb, int tri, int R, int s0, int lane)
 {
-    const int lane = lane_id();
     const int bw = tb - ta;
     for (int i0 = 0; i0 < R; i0 += G * kWave) {
         int i[G], slot[G];
@@ -61,7 +64,7 @@ __device__ __forceinline__ void run_gemv(const T *val, XP x, const LSP_GLOBAL ui
         // same order measured slower, 3.55 -> 3.70 ms, so they load after)
         if constexpr (sizeof(T) == 8) {
 #pragma unroll
-            for (int g = 0; g < G; g++) slot[g] = i[g] < tri ? s0 + tb + i[g] : (int)map[u + (i[g] - tri)];
+            for (int g = 0; g < G; g++) slot[g] = i[g] < tri ? s0 + tb + i[g] : (int)*near_el(map + u, (uint32_t)(i[g] - tri));
         }
         for (int q0 = 0; q0 < bw; q0 += B) {
             T v[B][G];
@@ -70,7 +73,7 @@ __device__ __forceinline__ void run_gemv(const T *val, XP x, const LSP_GLOBAL ui
                 const int tp = ta + min(q0 + h, bw - 1);
                 const int base = __builtin_amdgcn_readlane(lb, tp) + (tb - tp - 1);
 #pragma unroll
-                for (int g = 0; g < G; g++) v[h][g] = ld_coherent_val(gp(val) + (uint32_t)base, (uint32_t)i[g]);
+                for (int g = 0; g < G; g++) v[h][g] = ld_coherent_near(gp(val) + (uint32_t)base, (uint32_t)i[g]);
             }
 #pragma unroll
             for (int h = 0; h < B; h++) {
@@ -81,40 +84,51 @@ __device__ __forceinline__ void run_gemv(const T *val, XP x, const LSP_GLOBAL ui
                 }
             }
         }
+        if constexpr (sizeof(T) != 8) {
 #pragma unroll
-        for (int g = 0; g < G; g++) {
-            if (i0 + g * kWave + lane < R) {
-                if constexpr (sizeof(T) != 8) slot[g] = i[g] < tri ? s0 + tb + i[g] : (int)map[u + (i[g] - tri)];
-                x[slot[g]] -= acc[g];
-            }
+            for (int g = 0; g < G; g++) slot[g] = i[g] < tri ? s0 + tb + i[g] : (int)*near_el(map + u, (uint32_t)(i[g] - tri));
         }
+        // (all reads of a pass before its writes: its rows are distinct slots,
+        // which the compiler cannot know, and one LDS round trip serves them all)
+        double xv[G];
+#pragma unroll
+        for (int g = 0; g < G; g++) xv[g] = x[slot[g]];
+#pragma unroll
+        for (int g = 0; g < G; g++)
+            if (i0 + g * kWave + lane < R) x[slot[g]] = xv[g] - acc[g];
     }
 }
 
-// The rows below a single-column part whose column j has not been seen
-// published: the values of L(:, j) are loaded until none is unset (the
-// values array holds the unset marker before the launch, and every value is
-// written once, as a whole), then applied as run_gemv would.  Used for the
-// last dependency of a column when it is the column just before it (the
-// critical chain of a supernode), which saves the producer's store
-// acknowledgement and the flag round trip.  Returns false when abandoned.
+// The rows below one dependency whose column has not been seen published: the
+// values of L(:, j) are loaded until none is unset (the values array holds the
+// unset marker before the launch, and every value is written once, as a
+// whole), then applied as run_gemv would.  Used in a column's last run (the
+// critical chain inside a supernode), which saves the producer's store
+// acknowledgement and the flag round trip.  Row i is slot row0 + i for i < tri,
+// map[u + i - tri] past that.  The lanes' unseen flags are looked at once, in
+// the shadow of the values.  Returns false when abandoned.
 template <int G, typename T, typename XP>
-__device__ __forceinline__ bool run_gemv_unset(const T *val, XP x, const LSP_GLOBAL uint16_t *map, int64_t u,
-                                               double xj, int base, int R, int *abort_word)
+__device__ __forceinline__ bool dep_unset(const T *val, XP x, const LSP_GLOBAL uint16_t *map, int64_t u, double xj,
+                                          int base, int row0, int tri, int R, const int *flag, int epoch, int &ok,
+                                          int *abort_word, int lane)
 {
-    const int lane = lane_id();
+    constexpr int H = G < 4 ? G : 4;            // chunks applied at a time
     for (int i0 = 0; i0 < R; i0 += G * kWave) {
-        int i[G], slot[G];
+        int slot[G];
         T v[G];
+        // the rows' slots do not depend on the column's values: they are read
+        // while those are polled, not after they arrive
 #pragma unroll
-        for (int g = 0; g < G; g++) i[g] = min(i0 + g * kWave + lane, R - 1);
-        // the rows' slots do not depend on the predecessor: their loads are
-        // in flight while its values are polled, not after they arrive
-#pragma unroll
-        for (int g = 0; g < G; g++) slot[g] = (int)map[u + i[g]];
+        for (int g = 0; g < G; g++) {
+            const int i = min(i0 + g * kWave + lane, R - 1);
+            slot[g] = i < tri ? row0 + i : (int)*near_el(map + u, (uint32_t)(i - tri));
+        }
+        int seen = ok;
+        if (i0 == 0 && !ok) seen = ld_relaxed(flag) == epoch;
         for (int round = 0;; round++) {
 #pragma unroll
-            for (int g = 0; g < G; g++) v[g] = ld_coherent_val(gp(val) + (uint32_t)base, (uint32_t)i[g]);
+            for (int g = 0; g < G; g++)
+                v[g] = ld_coherent_near(gp(val) + (uint32_t)base, (uint32_t)min(i0 + g * kWave + lane, R - 1));
             bool miss = false;
 #pragma unroll
             for (int g = 0; g < G; g++) miss |= Unset<T>::is(v[g]);
@@ -124,11 +138,17 @@ __device__ __forceinline__ bool run_gemv_unset(const T *val, XP x, const LSP_GLO
                 atomicCAS(abort_word, 0, kErrSpin);
                 return false;
             }
-            __builtin_amdgcn_s_sleep(2);
+            __builtin_amdgcn_s_sleep(1);
         }
+        ok = seen;
 #pragma unroll
-        for (int g = 0; g < G; g++) {
-            if (i0 + g * kWave + lane < R) x[slot[g]] -= to_f64(v[g]) * xj;
+        for (int g0 = 0; g0 < G; g0 += H) {
+            double xv[H];
+#pragma unroll
+            for (int h = 0; h < H; h++) xv[h] = x[slot[g0 + h]];
+#pragma unroll
+            for (int h = 0; h < H; h++)
+                if (i0 + (g0 + h) * kWave + lane < R) x[slot[g0 + h]] = xv[h] - to_f64(v[g0 + h]) * xj;
         }
     }
     return true;
@@ -160,6 +180,23 @@ __global__ void __launch_bounds__(256) fill_unset_kernel(const FactorDesc<T> *ma
         if (s0 + 256 * u < n) M.val[s0 + 256 * u] = Unset<T>::value();
 }
 
+// Runs of at most kSmallCols columns with at most 64 rows below, taken up to
+// kPack at a time: the loads of all of them (triangle, values, map) are in
+// flight together, one round trip instead of two per run, and they are then
+// applied in order.  Most runs of a circuit's columns are of this kind (85 to
+// 90 % on circuits of 100 to 5000 unknowns).  Together with the task records
+// and a register budget of 4 waves per SIMD: refactor of 512 such circuits
+// 3686 -> 2505 us (fp64), 3493 -> 2601 us (fp32); kPack = 1: 2630, 2645 us.
+constexpr int kPack = 3;
+constexpr int kSmallCols = 4;
+template <int N> using Int = std::integral_constant<int, N>;
+// Ready dependencies of a column's last run from which on they are applied
+// together instead of one by one (2 to 12 measured the same).  Values instead
+// of flags in the last run: refactor of one circuit of 200 / 1020 / 4999
+// unknowns 149 / 161 / 336 -> 120 / 124 / 255 us (fp64), of a 316 x 316 grid
+// 2993 -> 2580 us, where a link's 12 row chunks bound the chain.
+constexpr int kBulk = 3;
+
 // One column of the left-looking refactorization.  XP is the work vector's
 // pointer type: an LSP_LDS pointer when the column fits the wave's LDS slice,
 // an LSP_GLOBAL scratch pointer otherwise.
@@ -176,54 +213,82 @@ __global__ void __launch_bounds__(256) fill_unset_kernel(const FactorDesc<T> *ma
 // Columns outside any supernode are runs of length 1.  Slots are taken 64 at
 // a time; each lane fetches the metadata and waits on the flag of one slot.
 template <typename T, typename XP>
-__device__ void factor_column(const FactorDesc<T> &M, int k, XP x,
+__device__ void factor_column(const LSP_CONST FactorDesc<T> *M, const LSP_CONST FactorTask *tk, XP x,
                               int epoch, int *abort_word, double ptol, double stol, int *dbg, long long *tw,
                               int backoff, int *tctr, TicketReq &treq)
 {
+    // chunks of 64 rows per pass of dep_unset (316 x 316 grid with 4 / 8 / 12 / 16:
+    // 2781 / 2410 / 2584 / 2819 us fp32; a global x costs registers)
+    constexpr bool kLds = std::is_same<XP, LSP_LDS double *>::value;
+    constexpr int kWide = kLds ? 8 : 4;
     const int lane = lane_id();
-    const LSP_GLOBAL int64_t *cp = gp(M.cp);
-    const LSP_GLOBAL int *dp = gp(M.dp);
-    const LSP_GLOBAL int *pos = gp(M.pos);
-    const LSP_GLOBAL int *snend = gp(M.snend);
-    const LSP_GLOBAL uint16_t *map = gp(M.rel);
-    const int64_t c0 = cp[k];
-    const int m = (int)(cp[k + 1] - c0);
-    const int dl = dp[k] - (int)c0;            // local slot of the diagonal
+    const int k = tk->k;
+    const int c0 = tk->c0;
+    const int m = tk->m;
+    const int dl = tk->dl;                     // local slot of the diagonal
+    const int ndep = tk->ndep;
+    const bool tail = tk->tail;
+    const LSP_GLOBAL int *pos = gp(M->pos) + c0;
+    const LSP_GLOBAL uint64_t *dep = gp(M->dep) + tk->d0;
+    const LSP_GLOBAL uint16_t *map = gp(M->rel);
+    T *const val = M->val;
+    int *const done = M->done;
 
-    for (int i = lane; i < m; i += kWave) x[i] = 0.0;
-    wave_fence();
+    // everything the column's record points at, in flight together: the first
+    // dependencies' records and the entries of A(:, k)
+    int j = -2, ok = 1;
+    uint64_t dr = 0;
     {
-        const LSP_GLOBAL int *aslot = gp(M.aslot);
-        const LSP_GLOBAL int *asrc = gp(M.asrc);
-        const LSP_GLOBAL double *ain = gp(M.ain);
-        const int a1 = gp(M.aptr)[k + 1];
-        for (int p = gp(M.aptr)[k] + lane; p < a1; p += kWave) {
+        int as = -1;
+        double av = 0.0;
+        const int na = tk->na;
+        const LSP_GLOBAL int *aslot = gp(M->aslot) + tk->a0;
+        const LSP_GLOBAL int *asrc = gp(M->asrc) + tk->a0;
+        const LSP_GLOBAL double *ain = gp(M->ain);
+        int src = 0;
+        if (lane < na) {
+            as = aslot[lane];
+            src = asrc[lane];
+        }
+        if (lane < ndep) {
+            j = pos[lane];
+            dr = dep[lane];
+        }
+        for (int i = lane; i < m; i += kWave) x[i] = 0.0;
+        wave_fence();
+        if (as >= 0) av = ain[src];
+        if (lane < ndep) ok = ld_relaxed(done + j) == epoch;
+        for (int p = lane + kWave; p < na; p += kWave) {
             const int s = aslot[p];
             if (s >= 0) x[s] = ain[asrc[p]];
         }
+        if (as >= 0) x[as] = av;
+        wave_fence();
     }
-    wave_fence();
 
     // A column of the dense trailing block applies only its dependencies
     // outside the block (a prefix of its U slots); the block itself is
     // factored densely afterwards.
-    const bool tail = k >= M.tail_k0;
-    const int ndep = tail ? gp(M.tail_ds)[k - M.tail_k0] : dl;
-    int64_t u = gp(M.relp)[k];                 // map cursor
+    long long u = tk->u;                       // map cursor
     for (int s0 = 0; s0 < ndep; s0 += kWave) {
         const int nd = min(kWave, ndep - s0);
-        int j = -2, e = -2, lb = 0, nl = 0;
-        const int *flag = nullptr;
-        if (lane < nd) {
-            j = pos[c0 + s0 + lane];
-            e = min(snend[j], k);
-            lb = dp[j] + 1;                    // first L slot of column j
-            nl = (int)(cp[e] - dp[e - 1]) - 1; // |L(:, e-1)|
-            flag = &M.done[j];
+        if (s0 > 0) {
+            j = -2;
+            dr = 0;
+            ok = 1;
+            if (lane < nd) {
+                j = pos[s0 + lane];
+                dr = dep[s0 + lane];
+                ok = 0;
+            }
         }
+        const int *flag = lane < nd ? done + j : nullptr;
+        const int lb = (int)(uint32_t)dr;                // first L slot of column j
+        const int nl = (int)((uint32_t)(dr >> 32) & 0xffffu);   // length of its run's last L column
+        const int after = (int)(dr >> 48);               // columns of its run after it
         const int jp = __shfl_up(j, 1, kWave);
-        const int ep = __shfl_up(e, 1, kWave);
-        const bool head = lane < nd && (lane == 0 || j != jp + 1 || e != ep);
+        const int ap = __shfl_up(after, 1, kWave);
+        const bool head = lane < nd && (lane == 0 || j != jp + 1 || after != ap - 1);
         const unsigned long long heads = __ballot(head);
         double xc = lane < nd ? (double)x[s0 + lane] : 0.0;
         // Dependencies are applied as soon as a leading group of the chunk's
@@ -232,21 +297,28 @@ __device__ void factor_column(const FactorDesc<T> &M, int k, XP x,
         // the others while that one is still being factored, and then only
         // the predecessor's column.  A run that continues past the ready
         // prefix is cut there; its later rows stay in the rows below.
-        int ok = flag == nullptr;
-        // the last dependency is the column just before this one, alone in
-        // its part (the chain step inside a supernode): its values are
-        // checked directly instead of its flag
-        const bool chain_last = s0 + nd == ndep && __builtin_amdgcn_readlane(j, nd - 1) == k - 1;
+        // Inside the column's last run the dependencies come one by one, a
+        // chain step apart: while fewer than kBulk of them are ready, each is
+        // applied by its values as they appear (dep_unset), without the flag.
         for (int have = 0; have < nd;) {
-            if (chain_last && have == nd - 1) {
-                const int lbj = __builtin_amdgcn_readlane(lb, nd - 1);
-                const int nlj = __builtin_amdgcn_readlane(nl, nd - 1);
-                const double xj = bcast_f64(xc, nd - 1);
-                if (!run_gemv_unset<8>(M.val, x, map, u, xj, lbj, nlj, abort_word)) return;
-                u += nlj;
+            const int aft = __builtin_amdgcn_readlane(after, have);
+            const unsigned long long wait = ~(__ballot(ok) >> have);    // (lanes past nd count as ready)
+            if (s0 + have + aft + 1 == ndep && wait && __builtin_ctzll(wait) < kBulk) {
+                int lane = lane_id();                // opaque, as below
+                asm volatile("" : "+v"(lane));
+                const int base = __builtin_amdgcn_readlane(lb, have);
+                const int R = aft + __builtin_amdgcn_readlane(nl, have);
+                const double xj = bcast_f64(xc, have);
+                const auto direct = [&](auto g) {
+                    return dep_unset<decltype(g)::value>(val, x, map, u, xj, base, s0 + have + 1, aft, R, flag, epoch,
+                                                         ok, abort_word, lane);
+                };
+                if (!(R <= kWave ? direct(Int<1>()) : R <= 4 * kWave ? direct(Int<4>()) : direct(Int<kWide>()))) return;
+                if (aft == 0) u += R;
                 wave_fence();
-                have = nd;
-                break;
+                have++;
+                if (lane >= have && lane < nd) xc = x[s0 + lane];
+                continue;
             }
             const int p = wave_wait_prefix(flag, epoch, abort_word, ok, have, nd, dbg, k, backoff);
             if (p < 0) return;                                      // aborted; kernel drains
@@ -254,24 +326,103 @@ __device__ void factor_column(const FactorDesc<T> &M, int k, XP x,
             unsigned long long hs = (heads & ~((1ull << have) - 1)) | (1ull << have);
             if (p < kWave) hs &= (1ull << p) - 1;
             while (hs) {
+                // opaque per step: nothing lane-dependent is hoisted out of the
+                // loops (and held in registers through them)
+                int lane = lane_id();
+                asm volatile("" : "+v"(lane));
                 const int ta = __builtin_ctzll(hs);
-                hs &= hs - 1;
-                const int tb = hs ? __builtin_ctzll(hs) : p;
+                const unsigned long long hn = hs & (hs - 1);
+                const int tb = hn ? __builtin_ctzll(hn) : p;
                 const int bw = tb - ta;
-                const int jl = __builtin_amdgcn_readlane(e, ta) - 1;        // last column of the run
-                const int tri = jl - __builtin_amdgcn_readlane(j, tb - 1);  // run rows after this part
+                const int tri = __builtin_amdgcn_readlane(after, tb - 1);   // run rows after this part
                 const int nlast = __builtin_amdgcn_readlane(nl, ta);
+                const int R = tri + nlast;                // rows below the part
+                if (bw <= kSmallCols && R <= kWave) {
+                    // this run and the next ones while they are small
+                    int pa[kPack], pb[kPack], pR[kPack], slot[kPack];
+                    T tv[kPack][kSmallCols - 1], v[kPack][kSmallCols];
+                    int np = 0;
+                    bool small = true;
+#pragma unroll
+                    for (int r = 0; r < kPack; r++) {
+                        pa[r] = pb[r] = pR[r] = 0;
+                        slot[r] = 0;            // (set on every path, or the compiler carries
+#pragma unroll                                  //  last round's values through the loop)
+                        for (int q = 0; q < kSmallCols; q++) v[r][q] = T(0);
+#pragma unroll
+                        for (int q = 0; q < kSmallCols - 1; q++) tv[r][q] = T(0);
+                        if (small && hs) {
+                            const int a = __builtin_ctzll(hs);
+                            const unsigned long long h = hs & (hs - 1);
+                            const int b = h ? __builtin_ctzll(h) : p;
+                            const int w = b - a;
+                            const int tr = __builtin_amdgcn_readlane(after, b - 1);
+                            const int nr = __builtin_amdgcn_readlane(nl, a);
+                            small = w <= kSmallCols && tr + nr <= kWave;
+                            if (small) {
+                                pa[r] = a;
+                                pb[r] = b;
+                                pR[r] = tr + nr;
+                                if (pR[r] > 0) {
+                                    const int i = min(lane, pR[r] - 1);
+                                    slot[r] = i < tr ? s0 + b + i : (int)*near_el(map + u, (uint32_t)(i - tr));
+#pragma unroll
+                                    for (int q = 0; q < kSmallCols; q++)
+                                        if (q < w) {
+                                            const int base = __builtin_amdgcn_readlane(lb, a + q) + (w - q - 1);
+                                            v[r][q] = ld_coherent_near(gp(val) + (uint32_t)base, (uint32_t)i);
+                                        }
+                                }
+#pragma unroll
+                                for (int q = 0; q < kSmallCols - 1; q++)
+                                    if (q < w - 1) {
+                                        const int base = __builtin_amdgcn_readlane(lb, a + q);
+                                        const int off = min(max(lane - a - q - 1, 0), w - q - 2);
+                                        tv[r][q] = ld_coherent_near(gp(val) + (uint32_t)base, (uint32_t)off);
+                                    }
+                                if (tr == 0) u += nr;
+                                hs = h;
+                                np = r + 1;
+                            }
+                        }
+                    }
+#pragma unroll
+                    for (int r = 0; r < kPack; r++) {
+                        if (r < np) {
+                            const int w = pb[r] - pa[r];
+#pragma unroll
+                            for (int q = 0; q < kSmallCols - 1; q++)
+                                if (q < w - 1) {
+                                    const int tp = pa[r] + q;
+                                    const double nx = fma(-to_f64(tv[r][q]), bcast_f64(xc, tp), xc);
+                                    xc = (lane > tp && lane < pb[r]) ? nx : xc;
+                                }
+                            if (w > 1 && lane >= pa[r] && lane < pb[r]) x[s0 + lane] = xc;
+                            if (pR[r] > 0) {
+                                double acc = 0.0;
+#pragma unroll
+                                for (int q = 0; q < kSmallCols; q++)
+                                    if (q < w) acc = fma(to_f64(v[r][q]), bcast_f64(xc, pa[r] + q), acc);
+                                if (lane < pR[r]) x[slot[r]] -= acc;
+                                wave_fence();
+                                if (lane >= pb[r] && lane < nd) xc = x[s0 + lane];   // later lanes of this chunk
+                            }
+                        }
+                    }
+                    wave_fence();
+                    continue;
+                }
+                hs = hn;
                 if (bw > 1) {
                     if (bw <= 9) {
-                        xc = run_triangle<8>(M.val, xc, lb, ta, tb);
-                    } else if constexpr (sizeof(T) == 8) {
-                        // fp64 values: 16 triangle columns in registers at a
-                        // time (the same steps in the same order), which keeps
-                        // the kernel at 3 waves per SIMD instead of 2
-                        for (int t0 = ta; t0 < tb - 1; t0 += 16) xc = run_triangle<16>(M.val, xc, lb, t0, tb);
+                        xc = run_triangle<8>(val, xc, lb, ta, tb, lane);
                     } else {
-                        if (bw <= 25) xc = run_triangle<24>(M.val, xc, lb, ta, tb);
-                        else xc = run_triangle<kTri>(M.val, xc, lb, ta, tb);
+                        // 16 (fp64 values) or 24 triangle columns in registers
+                        // at a time (the same steps in the same order), for the
+                        // register budget of 4 waves per SIMD
+                        constexpr int kPart = sizeof(T) == 8 ? 16 : 24;
+                        for (int t0 = ta; t0 < tb - 1; t0 += kPart)
+                            xc = run_triangle<kPart>(val, xc, lb, t0, tb, lane);
                     }
                 }
                 if (lane >= ta && lane < tb) x[s0 + lane] = xc;
@@ -280,21 +431,22 @@ __device__ void factor_column(const FactorDesc<T> &M, int k, XP x,
                 // (about 32 loads in flight: a narrow part, such as the single
                 // column that ends a critical chain step, covers more rows
                 // per round trip)
-                const int R = tri + nlast;
                 // (fp64 values: half the columns in flight per pass, for the
-                // register budget of 3 waves per SIMD)
+                // register budget of 4 waves per SIMD)
                 constexpr int kB8 = sizeof(T) == 8 ? 4 : 8;
-                if (bw >= 8) {
-                    if (R > 2 * kWave) run_gemv<4, kB8>(M.val, x, map, u, xc, lb, ta, tb, tri, R, s0);
-                    else run_gemv<1, kGemvBatch>(M.val, x, map, u, xc, lb, ta, tb, tri, R, s0);
+                if constexpr (!kLds) {
+                    run_gemv<4, 4>(val, x, map, u, xc, lb, ta, tb, tri, R, s0, lane);
+                } else if (bw >= 8) {
+                    if (R > 2 * kWave) run_gemv<4, kB8>(val, x, map, u, xc, lb, ta, tb, tri, R, s0, lane);
+                    else run_gemv<1, kGemvBatch>(val, x, map, u, xc, lb, ta, tb, tri, R, s0, lane);
                 } else if (R <= kWave) {
-                    run_gemv<1, 8>(M.val, x, map, u, xc, lb, ta, tb, tri, R, s0);
+                    run_gemv<1, 8>(val, x, map, u, xc, lb, ta, tb, tri, R, s0, lane);
                 } else if (bw == 1) {
-                    run_gemv<8, 1>(M.val, x, map, u, xc, lb, ta, tb, tri, R, s0);
+                    run_gemv<8, 1>(val, x, map, u, xc, lb, ta, tb, tri, R, s0, lane);
                 } else if (bw <= 4) {
-                    run_gemv<sizeof(T) == 8 ? 4 : 8, 4>(M.val, x, map, u, xc, lb, ta, tb, tri, R, s0);
+                    run_gemv<4, 4>(val, x, map, u, xc, lb, ta, tb, tri, R, s0, lane);
                 } else {
-                    run_gemv<4, kB8>(M.val, x, map, u, xc, lb, ta, tb, tri, R, s0);
+                    run_gemv<4, kB8>(val, x, map, u, xc, lb, ta, tb, tri, R, s0, lane);
                 }
                 if (tri == 0) u += nlast;
                 wave_fence();
@@ -304,21 +456,23 @@ __device__ void factor_column(const FactorDesc<T> &M, int k, XP x,
         }
         wave_fence();
     }
-
+    T *const cv = val + c0;
     if (tail) {
         // U entries above the block are final; the rest of the column is the
         // Schur-complement column S(:, c) = A22(:, c) - L21 U12(:, c).
-        const int c = k - M.tail_k0;
+        const LSP_GLOBAL int *dst = gp(M->dst) + c0;
+        const int k0 = M->tail_k0, c = k - k0, T_ = M->tail_T;
+        T *const urow = M->urow;
         for (int i = lane; i < ndep; i += kWave) {
             const T v = from_f64<T>(x[i]);
-            st_g(&M.val[c0 + i], v);
-            st_g(&M.urow[gp(M.dst)[c0 + i]], v);
+            st_g(&cv[i], v);
+            st_g(&urow[dst[i]], v);
         }
-        LSP_GLOBAL double *Sc = gp(M.tail_S) + (size_t)c * (size_t)M.tail_T;
-        for (int r = lane; r < M.tail_T; r += kWave) Sc[r] = 0.0;
+        LSP_GLOBAL double *Sc = gp(M->tail_S) + (size_t)c * (size_t)T_;
+        for (int r = lane; r < T_; r += kWave) Sc[r] = 0.0;
         wave_fence();                           // same-address stores of one wave stay ordered
-        for (int s = ndep + lane; s < m; s += kWave) Sc[pos[c0 + s] - M.tail_k0] = x[s];
-        if (lane == 0) gp(M.tail_colmax)[c] = 0ull;
+        for (int s = ndep + lane; s < m; s += kWave) Sc[pos[s] - k0] = x[s];
+        if (lane == 0) gp(M->tail_colmax)[c] = 0ull;
         return;
     }
 
@@ -328,72 +482,91 @@ __device__ void factor_column(const FactorDesc<T> &M, int k, XP x,
     // after the flag, off the dependency chain.
     const double piv = x[dl];
     const double rpiv = 1.0 / piv;             // one division; L = x * (1 / pivot)
-    for (int i = dl + 1 + lane; i < m; i += kWave) st_coherent(&M.val[c0 + i], from_f64<T>(x[i] * rpiv));
+    for (int i0 = dl + 1 + lane; i0 < m; i0 += 4 * kWave) {
+        double xi[4];
+#pragma unroll
+        for (int h = 0; h < 4; h++) xi[h] = x[min(i0 + h * kWave, m - 1)];
+#pragma unroll
+        for (int h = 0; h < 4; h++)
+            if (i0 + h * kWave < m) st_coherent(&cv[i0 + h * kWave], from_f64<T>(xi[h] * rpiv));
+    }
     store_complete();
     if (tw) tw[1] = (long long)wall_clock64();  // timeline: flag published
-    if (lane == 0) st_relaxed(&M.done[k], epoch);
+    if (lane == 0) st_relaxed(&done[k], epoch);
     // The wave's next ticket is requested now: what follows waits on no
     // other wave, so the ticket is not held behind a dependency, and the
-    // atomic's round trip overlaps the bookkeeping.  fp64 storage only: with
-    // fp32 / FP16 storage the held request raised the kernel to 193 VGPRs
-    // and the fp32 refactor ran 4 % slower on c1 (fp64: 3.30 -> 3.24 ms,
-    // 512-circuit Newton batch +8 %).
-    if constexpr (sizeof(T) == 8) treq = ticket_issue(tctr);
+    // atomic's round trip overlaps the bookkeeping.
+    treq = ticket_issue(tctr);
 
+    // U, the diagonal and the row-wise copies, four slots per lane at a time
+    // (their targets' loads in flight together), and the pivot test's maximum
     // a stored value must be finite in the storage type (65504 for FP16)
     const double vmax = sizeof(T) == 2 ? 65504.0 : sizeof(T) == 4 ? 3.4028234663852886e38 : 1.0e308;
     double amax = 0.0;
     int nonfinite = 0;
-    for (int i = dl + 1 + lane; i < m; i += kWave) {
-        const double a = fabs(x[i]);
-        amax = fmax(amax, a);
-        nonfinite |= !(a <= 1.0e308) || !(a <= vmax * fabs(piv));
+    {
+        const LSP_GLOBAL int *dst = gp(M->dst) + c0;
+        T *const lrow = M->lrow, *const urow = M->urow, *const diag = M->diag;
+        const double lmax = vmax * fabs(piv);
+        for (int i0 = lane; i0 < m; i0 += 4 * kWave) {
+            int d[4];
+#pragma unroll
+            for (int h = 0; h < 4; h++) d[h] = dst[min(i0 + h * kWave, m - 1)];
+#pragma unroll
+            for (int h = 0; h < 4; h++) {
+                const int i = i0 + h * kWave;
+                if (i < m) {
+                    const double xi = x[i];
+                    const double a = fabs(xi);
+                    if (i > dl) {
+                        amax = fmax(amax, a);
+                        nonfinite |= !(a <= 1.0e308) || !(a <= lmax);
+                        st_g(&lrow[d[h]], from_f64<T>(xi * rpiv));
+                    } else {
+                        nonfinite |= !(a <= vmax);
+                        const T v = from_f64<T>(xi);
+                        st_g(&cv[i], v);
+                        st_g(i < dl ? &urow[d[h]] : &diag[k], v);
+                    }
+                }
+            }
+        }
     }
-    for (int i = lane; i < dl; i += kWave) nonfinite |= !(fabs(x[i]) <= vmax);
     amax = wave_max(amax);
-    nonfinite = __any(nonfinite) || !(fabs(piv) <= vmax);
+    nonfinite = __any(nonfinite);
+    int *const mstat = M->mstat;
     if (lane == 0) {
         if (piv == 0.0) {
-            atomicMin(&M.mstat[2], k);
+            atomicMin(&mstat[2], k);
         } else if (!(fabs(piv) >= ptol * amax)) {
-            atomicAdd(&M.mstat[0], 1);
-            atomicMin(&M.mstat[1], k);
+            atomicAdd(&mstat[0], 1);
+            atomicMin(&mstat[1], k);
         }
-        if (nonfinite) atomicAdd(&M.mstat[3], 1);
+        if (nonfinite) atomicAdd(&mstat[3], 1);
     }
     if (stol > 0.0) {
         // would splu (tol = stol) pick this pivot on these values?
-        const int dpos = gp(M.dpos)[k];
+        const int dpos = gp(M->dpos)[k];
         double dv = -1.0;
         if (dpos > k) {
             for (int i = dl + 1 + lane; i < m; i += kWave)
-                if (pos[c0 + i] == dpos) dv = fabs(x[i]);
+                if (pos[i] == dpos) dv = fabs(x[i]);
             dv = wave_max(dv);
         }
         if (lane == 0) {
             const int v = splu_pivot_verdict(dpos == k, fabs(piv), amax, dv, stol);
             if (v) {
-                atomicAdd(&M.mstat[v == 1 ? 4 : 5], 1);
-                atomicMin(&M.mstat[6], k);
+                atomicAdd(&mstat[v == 1 ? 4 : 5], 1);
+                atomicMin(&mstat[6], k);
             }
         }
     }
-    const LSP_GLOBAL int *dst = gp(M.dst);
-    for (int i = lane; i < dl; i += kWave) {
-        const T v = from_f64<T>(x[i]);
-        st_g(&M.val[c0 + i], v);
-        st_g(&M.urow[dst[c0 + i]], v);
-    }
-    if (lane == 0) {
-        const T v = from_f64<T>(piv);
-        st_g(&M.val[c0 + dl], v);
-        st_g(&M.diag[k], v);
-    }
-    for (int i = dl + 1 + lane; i < m; i += kWave) st_g(&M.lrow[dst[c0 + i]], from_f64<T>(x[i] * rpiv));
 }
 
+// 4 waves per SIMD: 128 VGPRs (with 141 VGPRs, 3 waves, the fp32 refactor of 512
+// circuits took 3062 us instead of 2613).
 template <typename T>
-__global__ void __launch_bounds__(256) refactor_kernel(FactorLaunch L)
+__global__ void __launch_bounds__(256, 4) refactor_kernel(FactorLaunch L)
 {
     extern __shared__ double lds[];
     const int wv = threadIdx.x >> 6;
@@ -414,19 +587,19 @@ __global__ void __launch_bounds__(256) refactor_kernel(FactorLaunch L)
         const int t = (req.leader >= 0 ? ticket_take(req) : wave_ticket(qc)) * nq + q;
         req.leader = -1;
         if (t >= L.ntask) break;
-        if (aborted(L.abort_word)) continue;                  // drain
-        const int2 tk = L.task[t];
-        if (L.active && !L.active[tk.x]) continue;
-        const FactorDesc<T> M = mats[tk.x];
-        const int k = tk.y;
-        const int m = (int)(M.cp[k + 1] - M.cp[k]);
+        const int gone = ld_relaxed(L.abort_word);            // in flight with the record
+        const LSP_CONST FactorTask *tk = kp(L.task) + t;
+        const int mat = tk->mat, m = tk->m;
+        if (L.active && !kp(L.active)[mat]) continue;
+        if (uniform(gone)) continue;                          // drain
+        const LSP_CONST FactorDesc<T> *M = kp(mats) + mat;
         long long tw[2] = {0, 0};               // end of the last wait, flag published
         long long *wp = L.timeline ? tw : nullptr;
         const long long t0 = L.timeline ? (long long)wall_clock64() : 0;
         if (m <= L.cap) {
-            factor_column<T>(M, k, xl, epoch, L.abort_word, L.ptol, L.stol, L.dbg, wp, L.poll_backoff, qc, req);
+            factor_column<T>(M, tk, xl, epoch, L.abort_word, L.ptol, L.stol, L.dbg, wp, L.poll_backoff, qc, req);
         } else if (m <= L.scratch_stride) {
-            factor_column<T>(M, k, xg, epoch, L.abort_word, L.ptol, L.stol, L.dbg, wp, L.poll_backoff, qc, req);
+            factor_column<T>(M, tk, xg, epoch, L.abort_word, L.ptol, L.stol, L.dbg, wp, L.poll_backoff, qc, req);
         } else {
             if (lane_id() == 0) st_relaxed(L.abort_word, kErrCapacity);
         }
@@ -435,7 +608,7 @@ __global__ void __launch_bounds__(256) refactor_kernel(FactorLaunch L)
             r[0] = t0;
             r[1] = tw[1] ? tw[1] : (long long)wall_clock64();
             r[2] = tw[0];
-            r[3] = k;
+            r[3] = tk->k;
         }
     }
     // the last wave out re-arms the queue and advances the epoch

@@ -13,7 +13,7 @@ namespace lsp {
 
 struct FactorLaunch {
     const void *mats;       // FactorDesc<T>[nmat]
-    const int2 *task;       // (matrix, column) in task order
+    const FactorTask *task;
     const int *active;      // per-matrix mask (nullptr = all)
     int ntask;
     int *epoch;             // device epoch counter: read at start, bumped by the last wave

@@ -240,11 +240,11 @@ static int build_circuit(CircuitHost &C, const lsp_circuit_in &in, const lsp_opt
     }
     int rc = lsp_gp_factor(C.n, Ap.data(), Ai.data(), Ax.data(), C.q.data(), opt.pivot_tol, C.sym);
     if (rc != -1) return LSP_E_SINGULAR;
-    if (lsp_build_plan(C.n, Ap.data(), Ai.data(), src.data(), C.sym, C.q.data(), C.plan) != 0)
+    const int tmax = opt.tail_max == 0 ? 8192 : opt.tail_max;
+    if (lsp_build_plan(C.n, Ap.data(), Ai.data(), src.data(), C.sym, C.q.data(), C.plan, tmax <= 0) != 0)
         return LSP_E_STRUCTURE;
     if (C.plan.max_col > 65535) return LSP_E_CAPACITY;
     {
-        const int tmax = opt.tail_max == 0 ? 8192 : opt.tail_max;
         const double tden = opt.tail_density > 0 ? opt.tail_density : 0.5;
         if (tmax > 0 && lsp_plan_set_tail(C.plan, 64, tmax, tden) < 0) return LSP_E_STRUCTURE;
     }
@@ -275,17 +275,14 @@ int Batch::ensure_factor_set(FactorSet<T> &fs)
         const CircuitHost &C = circ_[m];
         FactorDesc<T> &F = fd[m];
         F.cp = d_cp_ + C.o_np1;
-        F.dp = d_dp_ + C.o_n;
         F.pos = d_pos_ + C.o_slot;
-        F.aptr = d_aptr_ + C.o_np1;
         F.asrc = d_asrc_ + C.o_a;
         F.aslot = d_aslot_ + C.o_a;
         // FP16 reads the Ruiz-scaled copy; a factor-only shift also factors that copy
         const bool own_copy = std::is_same<T, __half>::value || opt_.factor_shift > 0.0;
         F.ain = (own_copy ? d_ains_ : d_ain_) + C.aoff;
-        F.relp = d_relp_ + C.o_np1;
         F.rel = d_rel_ + C.o_rel;
-        F.snend = d_snend_ + C.o_n;
+        F.dep = d_dep_ + C.o_dep;
         F.dst = d_dst_ + C.o_slot;
         F.dpos = d_dpos_ + C.o_n;
         F.val = fs.val + C.o_slot;
@@ -315,7 +312,7 @@ int Batch::ensure_factor_set(FactorSet<T> &fs)
         D.n = C.n;
         D.tail_F = fs.tailF + C.o_t2;
         D.val = F.val;
-        D.dp = F.dp;
+        D.dp = d_dp_ + C.o_n;
         D.snend = d_snend_ + C.o_n;
         D.ru = d_ru_ + C.o_n;
         D.fcut = d_fcut_ + C.o_n;
@@ -436,12 +433,13 @@ int Batch::set_active(const int *mask)
 // (an upper estimate used for admission; device_bytes() reports the actual).
 size_t Batch::estimate_device_bytes() const
 {
-    double n = 0, nnz = 0, slots = 0, rel = 0, nlu = 0, sell = 0, slices = 0, T = 0, T2 = 0, lists = 0, tiles = 0;
+    double n = 0, nnz = 0, slots = 0, rel = 0, deps = 0, nlu = 0, sell = 0, slices = 0, T = 0, T2 = 0, lists = 0, tiles = 0;
     double maxcol = 0;
     const double nc = (double)circ_.size();
     for (const auto &C : circ_) {
         const LspPlan &P = C.plan;
         n += C.n; nnz += C.nnz; slots += (double)P.cp[C.n]; rel += (double)P.relp[C.n];
+        deps += (double)P.dep.size();
         nlu += (double)(P.n_l + P.n_u); sell += (double)C.sell.slots; slices += C.sell.nslices;
         T += P.tail_T; T2 += (double)P.tail_T * P.tail_T;
         const double nt = (P.tail_T + 63) / 64;                           // tiles, their packed copies and inverses
@@ -451,7 +449,7 @@ size_t Batch::estimate_device_bytes() const
     }
     const double m = std::max(1, opt_.ir_inner);
     double b = 0;
-    b += 16 * (n + nc) + 4 * n + 8 * slots + 4 * (n + nc) + 8 * nnz;     // cp relp dp pos dst aptr asrc aslot
+    b += 8 * (n + nc) + 4 * n + 8 * slots + 8 * nnz + 8 * deps;          // cp dp pos dst asrc aslot dep
     b += 8 * (n + nc) + 4 * nlu + 24 * n + 2 * rel;                       // lrp urp lci uci rowat q snend ru fcut bcut rel
     b += 8 * (slices + nc) + 8 * n + 8 * sell;                            // SELL structure
     b += 12 * n + 8 * nnz + 12 * sell;                                    // flags, values
@@ -459,7 +457,7 @@ size_t Batch::estimate_device_bytes() const
     b += 16 * nnz + 24 * n + 16 * (nc + 1);                               // Ruiz: row/col, scaled values, scales
     if (opt_.factor_shift > 0.0) b += 8 * n;                               // shifted diagonal entries
     b += 8 * T2 + 16 * T + 8.0 * 64 * 64 * tiles;                          // dense block work
-    b += 24 * n + 8 * slices + 16 * n;                                    // task lists, row packets
+    b += (sizeof(FactorTask) + 16) * n + 8 * slices + 16 * n;             // task lists, row packets
     b += 8 * lists + 8 * (slots / kFillSlots + nc);                       // dense-block and fill work lists
     b += 64 * n + 8 * (2 * m + 1) * n;                                    // vectors, Krylov bases V and Z
     b += (4 + 8) * (slots + nlu + n) + 4 * T2;                             // fp32 + fp64 factor sets
@@ -499,11 +497,11 @@ int Batch::upload_all()
 
     // ---- concatenate structures ----
     long o_np1 = 0, o_n = 0, o_slot = 0, o_a = 0, o_rel = 0, o_l = 0, o_u = 0, o_sl = 0,
-         o_slp1 = 0, o_ss = 0, o_t = 0, o_t2 = 0, o_fpk = 0, o_bpk = 0, o_tw = 0;
+         o_slp1 = 0, o_ss = 0, o_t = 0, o_t2 = 0, o_fpk = 0, o_bpk = 0, o_tw = 0, o_dep = 0;
     for (auto &C : circ_) {
         C.o_fpk = o_fpk; C.o_bpk = o_bpk; C.o_tw = o_tw;
         o_fpk += (long)C.plan.fpk.size(); o_bpk += (long)C.plan.bpk.size(); o_tw += (long)C.plan.twide.size();
-        C.o_np1 = o_np1; C.o_n = o_n; C.o_slot = o_slot; C.o_a = o_a; C.o_rel = o_rel;
+        C.o_np1 = o_np1; C.o_n = o_n; C.o_slot = o_slot; C.o_a = o_a; C.o_rel = o_rel; C.o_dep = o_dep;
         C.o_l = o_l; C.o_u = o_u; C.o_sl = o_sl; C.o_slp1 = o_slp1; C.o_ss = o_ss;
         C.o_t = o_t; C.o_t2 = o_t2;
         const long T = C.plan.tail_T;
@@ -511,27 +509,27 @@ int Batch::upload_all()
         C.voff = o_n;
         C.aoff = o_a;
         o_np1 += C.n + 1; o_n += C.n; o_slot += C.plan.cp[C.n]; o_a += C.nnz;
-        o_rel += C.plan.relp[C.n]; o_l += C.plan.n_l; o_u += C.plan.n_u;
+        o_rel += C.plan.relp[C.n]; o_dep += (long)C.plan.dep.size(); o_l += C.plan.n_l; o_u += C.plan.n_u;
         o_sl += C.sell.nslices; o_slp1 += C.sell.nslices + 1; o_ss += C.sell.slots;
     }
     ntot_ = o_n; nnz_tot_ = o_a; nslot_tot_ = o_slot; nl_tot_ = o_l; nu_tot_ = o_u;
     nsell_tot_ = o_ss;
     nt_tot_ = o_t; nt2_tot_ = o_t2;
     {
-        std::vector<int64_t> cp, relp, soff;
-        std::vector<int> dp, pos, aptr, asrc, aslot, dst, lrp, lci, urp, uci, rowat, q, snend, ru, fcut, bcut, fpk, bpk,
+        std::vector<int64_t> cp, soff;
+        std::vector<uint64_t> dep;
+        std::vector<int> dp, pos, asrc, aslot, dst, lrp, lci, urp, uci, rowat, q, snend, ru, fcut, bcut, fpk, bpk,
             twide;
         std::vector<int> dpos;
         std::vector<int> srlen, scol, sperm, ssrc;
         std::vector<uint16_t> rel;
-        cp.reserve(o_np1); relp.reserve(o_np1); rel.reserve(o_rel);
+        cp.reserve(o_np1); rel.reserve(o_rel); dep.reserve(o_dep);
         for (auto &C : circ_) {
             const LspPlan &P = C.plan;
             cp.insert(cp.end(), P.cp.begin(), P.cp.end());
-            relp.insert(relp.end(), P.relp.begin(), P.relp.end());
+            dep.insert(dep.end(), P.dep.begin(), P.dep.end());
             dp.insert(dp.end(), P.dp.begin(), P.dp.end());
             pos.insert(pos.end(), P.pos.begin(), P.pos.end());
-            aptr.insert(aptr.end(), P.aptr.begin(), P.aptr.end());
             asrc.insert(asrc.end(), P.asrc.begin(), P.asrc.end());
             aslot.insert(aslot.end(), P.aslot.begin(), P.aslot.end());
             dst.insert(dst.end(), P.dst.begin(), P.dst.end());
@@ -565,8 +563,8 @@ int Batch::upload_all()
             sperm.insert(sperm.end(), S.perm.begin(), S.perm.end());
             for (int s : S.src) ssrc.push_back(s >= 0 ? (int)(s + C.aoff) : -1);
         }
-        d_cp_ = upload(cp); d_relp_ = upload(relp); d_soff_ = upload(soff);
-        d_dp_ = upload(dp); d_pos_ = upload(pos); d_aptr_ = upload(aptr);
+        d_cp_ = upload(cp); d_dep_ = upload(dep); d_soff_ = upload(soff);
+        d_dp_ = upload(dp); d_pos_ = upload(pos);
         d_asrc_ = upload(asrc); d_aslot_ = upload(aslot); d_dst_ = upload(dst);
         d_lrp_ = upload(lrp); d_lci_ = upload(lci); d_urp_ = upload(urp); d_uci_ = upload(uci);
         d_rowat_ = upload(rowat); d_q_ = upload(q); d_rel_ = upload(rel); d_snend_ = upload(snend);
@@ -597,7 +595,7 @@ int Batch::upload_all()
             if (!d_frow_ || !d_flvp_ || !d_brow_ || !d_blvp_ || !d_irconv_ || !d_rn2_ || !d_bn2_)
                 return LSP_E_ALLOC;
         }
-        if (!d_cp_ || !d_relp_ || !d_soff_ || !d_dp_ || !d_pos_ || !d_aptr_ || !d_asrc_ ||
+        if (!d_cp_ || !d_dep_ || !d_soff_ || !d_dp_ || !d_pos_ || !d_asrc_ ||
             !d_aslot_ || !d_dst_ || !d_lrp_ || !d_lci_ || !d_urp_ || !d_uci_ || !d_rowat_ ||
             !d_q_ || !d_rel_ || !d_snend_ || !d_ru_ || !d_fcut_ || !d_bcut_ || !d_fpk_ || !d_bpk_ || !d_twide_ || !d_srlen_ || !d_scol_ || !d_sperm_ || !d_ssrc_)
             return LSP_E_ALLOC;
@@ -818,7 +816,25 @@ int Batch::upload_all()
                         width_tb_);
         nfw_tot_ = (long)tw.size();
         nbw_tot_ = (long)tb.size();
-        d_ftask_ = upload(tf); d_fwtask_ = upload(tw); d_bwtask_ = upload(tb);
+        std::vector<FactorTask> ft(tf.size());
+        for (size_t t = 0; t < tf.size(); t++) {
+            const LspPlan &P = circ_[tf[t].x].plan;
+            const int k = tf[t].y;
+            FactorTask &F = ft[t];
+            F = FactorTask{};
+            F.mat = tf[t].x;
+            F.k = k;
+            F.c0 = (int)P.cp[k];
+            F.a0 = P.aptr[k];
+            F.na = P.aptr[k + 1] - P.aptr[k];
+            F.d0 = P.depp[k];
+            F.u = P.relp[k];
+            F.m = (uint16_t)(P.cp[k + 1] - P.cp[k]);
+            F.dl = (uint16_t)(P.dp[k] - P.cp[k]);
+            F.ndep = (uint16_t)(P.depp[k + 1] - P.depp[k]);
+            F.tail = k >= P.tail_k0;
+        }
+        d_ftask_ = upload(ft); d_fwtask_ = upload(tw); d_bwtask_ = upload(tb);
         if (!d_ftask_ || !d_fwtask_ || !d_bwtask_) return LSP_E_ALLOC;
     }
     // persistent grids
@@ -1117,8 +1133,10 @@ int Batch::refactor_pass(int prec, const std::vector<int> *subset, std::vector<i
     if (refactor_tl_path_ && d_timeline_) {
         std::vector<long long> tl((size_t)ntot_ * 4);
         (void)hipMemcpy(tl.data(), d_timeline_, tl.size() * sizeof(long long), hipMemcpyDeviceToHost);
+        std::vector<FactorTask> ft(ntot_);
+        (void)hipMemcpy(ft.data(), d_ftask_, ntot_ * sizeof(FactorTask), hipMemcpyDeviceToHost);
         std::vector<int2> tk(ntot_);
-        (void)hipMemcpy(tk.data(), d_ftask_, ntot_ * sizeof(int2), hipMemcpyDeviceToHost);
+        for (long t = 0; t < ntot_; t++) tk[t] = make_int2(ft[t].mat, ft[t].k);
         if (FILE *f = fopen(refactor_tl_path_, "wb")) {
             fwrite(tl.data(), sizeof(long long), tl.size(), f);
             fwrite(tk.data(), sizeof(int2), tk.size(), f);

@@ -37,7 +37,7 @@ struct CircuitHost {
     long o_n = 0;                        // n sized arrays
     long o_slot = 0;                     // slot arrays
     long o_a = 0;                    // A-entry arrays
-    long o_rel = 0;                      // update map
+    long o_rel = 0, o_dep = 0;           // update map, dependency records
     long o_l = 0, o_u = 0;               // strict L / U entry arrays
     long o_sl = 0, o_slp1 = 0, o_ss = 0; // SELL slices, slices+1, slots
     long o_t = 0, o_t2 = 0;              // dense block: T, T^2
@@ -65,8 +65,9 @@ struct DeviceArrays {
     double ms_per_tick_ = 1e-5;          // of the device wall clock
     int mm_alloc_ = 0;
     // structure (device)
-    int64_t *d_cp_ = nullptr, *d_relp_ = nullptr, *d_soff_ = nullptr;
-    int *d_dp_ = nullptr, *d_pos_ = nullptr, *d_aptr_ = nullptr, *d_asrc_ = nullptr,
+    int64_t *d_cp_ = nullptr, *d_soff_ = nullptr;
+    uint64_t *d_dep_ = nullptr;
+    int *d_dp_ = nullptr, *d_pos_ = nullptr, *d_asrc_ = nullptr,
         *d_aslot_ = nullptr, *d_dst_ = nullptr, *d_lrp_ = nullptr, *d_lci_ = nullptr,
         *d_urp_ = nullptr, *d_uci_ = nullptr, *d_rowat_ = nullptr, *d_q_ = nullptr,
         *d_done_ = nullptr, *d_srlen_ = nullptr,
@@ -89,7 +90,8 @@ struct DeviceArrays {
     SellDesc<__half> *d_sdesc16_ = nullptr;
     SellDesc<double> *d_sdesc64_ = nullptr;
     SellDesc<float> *d_sdesc32_ = nullptr;
-    int2 *d_ftask_ = nullptr, *d_fwtask_ = nullptr, *d_bwtask_ = nullptr, *d_stask_ = nullptr;
+    FactorTask *d_ftask_ = nullptr;
+    int2 *d_fwtask_ = nullptr, *d_bwtask_ = nullptr, *d_stask_ = nullptr;
     long nslot_tot_ = 0, nl_tot_ = 0, nu_tot_ = 0, nsell_tot_ = 0;
     int nstask_ = 0;
     int *d_ctr_ = nullptr;               // [0..1] factor, [2..3] fwd, [4..5] bwd
