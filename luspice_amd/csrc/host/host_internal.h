@@ -152,6 +152,28 @@ int lsp_plan_set_tail(LspPlan &P, int min_T, int max_T, double min_density);
 // target pattern (both mean the symbolic pattern is not closed under fill).
 int lsp_plan_build_segments(LspPlan &P);
 
+// The solve of one circuit by one workgroup of kLocalWaves waves, its vector in
+// LDS: the tasks of fwd_task / bwd_task, level by level (a level's tasks read
+// rows of earlier levels only; a wide supernode's blocks take a level each),
+// dealt to the waves in turn.  Records of four ints:
+//   task    kind | g << 8 | count << 16, first record, level, passes
+//   kind 0  rows of g lanes each, `passes` passes of kTriPacketPerLane entries
+//           per lane; records (row, first entry, end, 1 = the supernode's own
+//           entries are left to its triangle)
+//   kind 1  triangles of supernodes of at most g rows, g lanes each; one
+//           record per lane (row, diagonal slot, supernode width, ru), width 0
+//           for a lane without a row
+//   kind 2  one 64-row block of a supernode's triangle, one record per lane
+//           (row, diagonal slot, block's rows, ru); block | width << 12 in the
+//           place of the passes
+constexpr int kLocalWaves = 16;
+struct LspLocalSolve {
+    std::vector<int> task, rec;           // four ints per task, in wave order / per record
+    std::vector<int> wave;                // kLocalWaves + 1: first task of each wave
+    int nlev = 0;
+};
+void lsp_plan_local_solve(const LspPlan &P, bool forward, LspLocalSolve &S);
+
 // Ruiz equilibration scales: after `sweeps` sweeps, R A C has every row and
 // column maximum close to 1 (used to pivot on the scaled matrix).
 void lsp_ruiz_scales(int n, long nnz, const int *row, const int *col, const double *val, int sweeps,

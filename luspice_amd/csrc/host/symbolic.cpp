@@ -503,6 +503,92 @@ static void plan_tri_supernodes(LspPlan &P)
 }
 
 // ---------------------------------------------------------------------------
+// one-workgroup solves
+// ---------------------------------------------------------------------------
+void lsp_plan_local_solve(const LspPlan &P, bool forward, LspLocalSolve &S)
+{
+    const std::vector<int> &task = forward ? P.fwd_task : P.bwd_task;
+    const std::vector<int> &key = forward ? P.fwd_key : P.bwd_key;
+    const std::vector<int> &pk = forward ? P.fpk : P.bpk;
+    S = LspLocalSolve();
+    std::vector<std::vector<int>> per(kLocalWaves);
+    int turn = 0, level = 0;
+    auto row_rec = [&](int code) {
+        const int i = code >> 1, part = code & 1;
+        S.rec.push_back(i);
+        S.rec.push_back(forward ? P.lrp[i] : part ? P.bcut[i] : P.urp[i]);
+        S.rec.push_back(forward ? (part ? P.fcut[i] : P.lrp[i + 1]) : P.urp[i + 1]);
+        S.rec.push_back(part);
+        const size_t z = S.rec.size();
+        return S.rec[z - 2] - S.rec[z - 3];          // entries
+    };
+    auto tri_recs = [&](int s, int g) {
+        const int w = P.snend[s] - s;
+        for (int l = 0; l < g; l++) {
+            const int row = s + std::min(l, w - 1);
+            S.rec.push_back(row);
+            S.rec.push_back(P.dp[row]);
+            S.rec.push_back(l < w ? w : 0);
+            S.rec.push_back(P.ru[row]);
+        }
+    };
+    auto deal = [&](int head, int first, int lev, int passes) {
+        std::vector<int> &v = per[turn++ % kLocalWaves];
+        v.insert(v.end(), {head, first, lev, passes});
+    };
+    for (size_t a = 0; a < task.size();) {
+        size_t b = a;
+        int blocks = 1;
+        for (; b < task.size() && key[b] == key[a]; b++) {
+            const int code = task[b], first = (int)(S.rec.size() / 4);
+            if (code >= kTriPacketBase) {
+                const int o = code - kTriPacketBase, cnt = pk[o + 1];
+                if (pk[o] > 0) {
+                    int ne = 0;
+                    for (int r = 0; r < cnt; r++) ne = std::max(ne, row_rec(pk[o + 2 + r]));
+                    const int per_pass = pk[o] * kTriPacketPerLane;
+                    deal(0 | pk[o] << 8 | cnt << 16, first, level, (ne + per_pass - 1) / per_pass);
+                } else {
+                    const int g = -pk[o], per_wave = 64 / g;
+                    for (int r = 0; r < cnt; r++) tri_recs(pk[o + 2 + r], g);
+                    for (int r = cnt; r < per_wave; r++)
+                        for (int l = 0; l < g; l++) S.rec.insert(S.rec.end(), {0, 0, 0, 0});
+                    deal(1 | g << 8 | cnt << 16, first, level, 1);
+                }
+            } else if (code < 0 || code >= kTriWideBase) {
+                const int s = code < 0 ? -code - 1 : P.twide[2 * (code - kTriWideBase)];
+                const int bk = code < 0 ? 0 : P.twide[2 * (code - kTriWideBase) + 1];
+                blocks = std::max(blocks, bk + 1);
+                const int w = P.snend[s] - s;
+                const int bw = std::min(64, w - 64 * bk), r0 = forward ? s + 64 * bk : s + w - 64 * bk - bw;
+                for (int l = 0; l < 64; l++) {
+                    const int row = r0 + std::min(l, bw - 1);
+                    S.rec.insert(S.rec.end(), {row, P.dp[row], bw, P.ru[row]});
+                }
+                deal(2 | 64 << 8 | 1 << 16, first, level + bk, bk | w << 12);
+            } else {
+                const int ne = row_rec(code);
+                deal(0 | 64 << 8 | 1 << 16, first, level, (ne + 64 * kTriPacketPerLane - 1) / (64 * kTriPacketPerLane));
+            }
+        }
+        level += blocks;
+        a = b;
+    }
+    S.nlev = level;
+    // a wide supernode's later blocks belong to later levels than tasks dealt
+    // after them: each wave's tasks in level order
+    for (int w = 0; w < kLocalWaves; w++) {
+        S.wave.push_back((int)(S.task.size() / 4));
+        std::vector<int> &v = per[w];
+        std::vector<int> idx(v.size() / 4);
+        for (size_t t = 0; t < idx.size(); t++) idx[t] = (int)t;
+        std::stable_sort(idx.begin(), idx.end(), [&](int x, int y) { return v[4 * x + 2] < v[4 * y + 2]; });
+        for (int t : idx) S.task.insert(S.task.end(), v.begin() + 4 * t, v.begin() + 4 * t + 4);
+    }
+    S.wave.push_back((int)(S.task.size() / 4));
+}
+
+// ---------------------------------------------------------------------------
 // dense trailing block
 // ---------------------------------------------------------------------------
 // Order of the refactor's tasks: each column kTaskLead levels before the last

@@ -40,6 +40,9 @@ constexpr int kTriPacket = 1 << 30;
 constexpr int kTriWide = 1 << 29;
 constexpr int kTriPacketLane = 4;
 
+// Waves of a one-workgroup solve (localsolve.hip).
+constexpr int kLocalSolveWaves = 16;
+
 // One task of the refactor, as the kernel reads it: what it needs to start
 // a column's loads, so that they depend on one record and not on a chain of
 // pointers.
@@ -109,6 +112,10 @@ struct TriDesc {
     const T *tail_F;        // tail_T^2, column-major, unit-L below / U on and above
     const int *tail_lcut;   // tail_T: end of the sparse part of L row tail_k0 + r
     int *tail_ctr;          // 4 ints: block ticket counter, exit counter, pad
+    // one-workgroup solve, forward and backward: first task per wave, tasks
+    // and records of four ints each, levels (null: solved by the task queue)
+    const int *lwave[2], *ltask[2], *lrec[2];
+    int lnlev[2];
     int n;
     int tail_k0;
     int tail_T;

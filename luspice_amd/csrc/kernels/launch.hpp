@@ -175,6 +175,10 @@ hipError_t launch_tail_solve(const void *mats, const DenseGrid &G, const long *v
                              long long *tick0, hipStream_t st);
 
 // trisolve.hip
+// Solves of the `count` circuits in `list`, one workgroup each, at most `rows`
+// unknowns per circuit (localsolve.hip).
+template <typename T>
+hipError_t launch_local_solve(const TriLaunch &L, bool forward, const int *list, int count, int rows, hipStream_t st);
 template <typename T>
 hipError_t launch_trisolve_half(const TriLaunch &L, bool forward, int blocks, hipStream_t st);
 hipError_t launch_solve_unset(const TriLaunch &L, long n, hipStream_t st);

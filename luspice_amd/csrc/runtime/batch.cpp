@@ -28,6 +28,11 @@ namespace lsp {
 
 static_assert(kTriPacket == ::kTriPacketBase && kTriPacketLane == ::kTriPacketPerLane,
               "packet layout of the plan and the solve kernel");
+static_assert(kLocalSolveWaves == ::kLocalWaves, "waves of a one-workgroup solve");
+
+// Circuits of at most this many unknowns may be solved by one workgroup each
+// (their vector is 64 KB of LDS).
+constexpr int kLocalRows = 8192;
 
 
 Batch::~Batch()
@@ -248,11 +253,31 @@ static int build_circuit(CircuitHost &C, const lsp_circuit_in &in, const lsp_opt
         const double tden = opt.tail_density > 0 ? opt.tail_density : 0.5;
         if (tmax > 0 && lsp_plan_set_tail(C.plan, 64, tmax, tden) < 0) return LSP_E_STRUCTURE;
     }
+    // (the solves read entry 0 of L and U where a lane has none)
+    if (C.n <= kLocalRows && C.plan.tail_k0 > 0 && C.plan.n_l > 0 && C.plan.n_u > 0)
+        for (int d = 0; d < 2; d++) lsp_plan_local_solve(C.plan, d == 0, C.local[d]);
     std::vector<int> rp, ci, rsrc;
     lsp_coo_to_csr(C.n, C.nnz, C.row.data(), C.col.data(), rp, ci, rsrc);
     if (lsp_build_sell(C.n, rp.data(), ci.data(), rsrc.data(), 64, opt.sell_sigma, C.sell) != 0)
         return LSP_E_STRUCTURE;
     return ir_level_lists(C);
+}
+
+// Which circuits' triangular solves are one workgroup's (localsolve.hip).  Per
+// pair of solves that takes 0.64 us a level or 0.16 us a task, whichever is
+// more; the task queue takes 0.95 us a level or, for all circuits together, 1 us
+// per 190 tasks.  Measured (fp64, us, one workgroup / queue): n = 200, 87 levels
+// and 124 tasks, 56 / 81; n = 1020, 88 and 285, 53 / 58; n = 4999, 160 and 1230,
+// 192 / 156; 512 circuits of 100 to 5000 unknowns, 165 000 tasks, 450 / 960.
+static void choose_local(std::vector<CircuitHost> &circ)
+{
+    auto tasks = [](const CircuitHost &C) { return (long)(C.plan.fwd_task.size() + C.plan.bwd_task.size()); };
+    long total = 0;
+    for (const CircuitHost &C : circ) total += tasks(C);
+    for (CircuitHost &C : circ) {
+        const long levels = C.local[0].nlev + C.local[1].nlev;
+        C.local_on = levels > 0 && tasks(C) <= std::max(6 * levels, total / 30);
+    }
 }
 
 template <typename T>
@@ -323,6 +348,12 @@ int Batch::ensure_factor_set(FactorSet<T> &fs)
         D.tail_ctr = d_tail_ctr_ + 4 * m;
         D.tail_k0 = C.plan.tail_k0;
         D.tail_T = C.plan.tail_T;
+        for (int d = 0; d < 2; d++) {
+            D.lwave[d] = d_lwave_ + C.o_lw[d];
+            D.ltask[d] = d_ltask_ + C.o_lt[d];
+            D.lrec[d] = d_lrec_ + C.o_lr[d];
+            D.lnlev[d] = C.local[d].nlev;
+        }
         IrDesc<T> &I = id[m];
         I.A.off = d_soff_ + C.o_slp1;
         I.A.rlen = d_srlen_ + C.o_n;
@@ -433,13 +464,14 @@ int Batch::set_active(const int *mask)
 // (an upper estimate used for admission; device_bytes() reports the actual).
 size_t Batch::estimate_device_bytes() const
 {
-    double n = 0, nnz = 0, slots = 0, rel = 0, deps = 0, nlu = 0, sell = 0, slices = 0, T = 0, T2 = 0, lists = 0, tiles = 0;
+    double n = 0, nnz = 0, slots = 0, rel = 0, deps = 0, local = 0, nlu = 0, sell = 0, slices = 0, T = 0, T2 = 0, lists = 0, tiles = 0;
     double maxcol = 0;
     const double nc = (double)circ_.size();
     for (const auto &C : circ_) {
         const LspPlan &P = C.plan;
         n += C.n; nnz += C.nnz; slots += (double)P.cp[C.n]; rel += (double)P.relp[C.n];
         deps += (double)P.dep.size();
+        for (const LspLocalSolve &S : C.local) local += (double)(S.task.size() + S.rec.size() + S.wave.size());
         nlu += (double)(P.n_l + P.n_u); sell += (double)C.sell.slots; slices += C.sell.nslices;
         T += P.tail_T; T2 += (double)P.tail_T * P.tail_T;
         const double nt = (P.tail_T + 63) / 64;                           // tiles, their packed copies and inverses
@@ -453,6 +485,7 @@ size_t Batch::estimate_device_bytes() const
     b += 8 * (n + nc) + 4 * nlu + 24 * n + 2 * rel;                       // lrp urp lci uci rowat q snend ru fcut bcut rel
     b += 8 * (slices + nc) + 8 * n + 8 * sell;                            // SELL structure
     b += 12 * n + 8 * nnz + 12 * sell;                                    // flags, values
+    b += 4 * local + 4 * nc;                                              // one-workgroup solves
     if (opt_.krylov_spmv == 2) b += 2 * sell;                              // FP16 SELL values
     b += 16 * nnz + 24 * n + 16 * (nc + 1);                               // Ruiz: row/col, scaled values, scales
     if (opt_.factor_shift > 0.0) b += 8 * n;                               // shifted diagonal entries
@@ -569,6 +602,28 @@ int Batch::upload_all()
         d_lrp_ = upload(lrp); d_lci_ = upload(lci); d_urp_ = upload(urp); d_uci_ = upload(uci);
         d_rowat_ = upload(rowat); d_q_ = upload(q); d_rel_ = upload(rel); d_snend_ = upload(snend);
         d_ru_ = upload(ru); d_fcut_ = upload(fcut); d_bcut_ = upload(bcut);
+        {
+            choose_local(circ_);
+            std::vector<int> lt, lr, lw, ll;
+            for (size_t m = 0; m < circ_.size(); m++) {
+                CircuitHost &C = circ_[m];
+                for (int d = 0; d < 2 && C.local_on; d++) {
+                    const LspLocalSolve &S = C.local[d];
+                    C.o_lt[d] = (long)lt.size(); C.o_lr[d] = (long)lr.size(); C.o_lw[d] = (long)lw.size();
+                    lt.insert(lt.end(), S.task.begin(), S.task.end());
+                    lr.insert(lr.end(), S.rec.begin(), S.rec.end());
+                    lw.insert(lw.end(), S.wave.begin(), S.wave.end());
+                }
+                if (!C.local_on) continue;
+                ll.push_back((int)m);
+                local_rows_ = std::max(local_rows_, C.n);
+            }
+            auto work = [&](int m) { return circ_[m].local[0].task.size() + circ_[m].local[1].task.size(); };
+            std::stable_sort(ll.begin(), ll.end(), [&](int a, int b) { return work(a) > work(b); });
+            nlocal_ = (int)ll.size();
+            d_ltask_ = upload(lt); d_lrec_ = upload(lr); d_lwave_ = upload(lw); d_llist_ = upload(ll);
+            if (!d_ltask_ || !d_lrec_ || !d_lwave_ || !d_llist_) return LSP_E_ALLOC;
+        }
         d_fpk_ = upload(fpk); d_bpk_ = upload(bpk); d_twide_ = upload(twide);
         d_srlen_ = upload(srlen); d_scol_ = upload(scol); d_sperm_ = upload(sperm);
         d_ssrc_ = upload(ssrc);
@@ -786,11 +841,12 @@ int Batch::upload_all()
     }
     // merged task lists: (key, circuit, index)
     {
-        auto merge = [&](auto key_of, auto order_of, long &width) {
+        auto merge = [&](auto key_of, auto order_of, long &width, bool solve) {
             std::vector<std::pair<long, int2>> all;
             all.reserve(ntot_);
             for (int m = 0; m < nc; m++) {
                 const LspPlan &P = circ_[m].plan;
+                if (solve && circ_[m].local_on) continue;
                 const std::vector<int> &ord = order_of(P);
                 for (size_t t = 0; t < ord.size(); t++) all.push_back({(long)key_of(P, t), make_int2(m, ord[t])});
             }
@@ -807,13 +863,13 @@ int Batch::upload_all()
         };
         auto tf = merge([](const LspPlan &P, size_t t) { return P.fkey[P.ftask[t]]; },
                         [](const LspPlan &P) -> const std::vector<int> & { return P.ftask; },
-                        width_f_);
+                        width_f_, false);
         auto tw = merge([](const LspPlan &P, size_t t) { return P.fwd_key[t]; },
                         [](const LspPlan &P) -> const std::vector<int> & { return P.fwd_task; },
-                        width_tf_);
+                        width_tf_, true);
         auto tb = merge([](const LspPlan &P, size_t t) { return P.bwd_key[t]; },
                         [](const LspPlan &P) -> const std::vector<int> & { return P.bwd_task; },
-                        width_tb_);
+                        width_tb_, true);
         nfw_tot_ = (long)tw.size();
         nbw_tot_ = (long)tb.size();
         std::vector<FactorTask> ft(tf.size());
@@ -861,19 +917,23 @@ int Batch::upload_all()
             per_cu = (int)std::max<size_t>(1, std::min<size_t>(8, lds_cu / lds));
         }
         // Waves beyond the widest dependency level only poll; size each
-        // persistent grid to about twice that width (4 waves per block).
-        auto blocks_for = [&](long width, long cap_blocks) {
-            long want = (2 * width + 3) / 4;
+        // persistent grid to about twice that width (4 waves per block), but to
+        // 128 blocks at least while there are tasks for them: a task held early
+        // has its loads done when its turn comes (refactor of 200 unknowns 125
+        // us with the width rule's few blocks, 103 with 128, 126 with 512;
+        // solve pair of 4999 unknowns 226 -> 218 us).
+        auto blocks_for = [&](long width, long tasks, long cap_blocks) {
+            long want = std::max((2 * width + 3) / 4, std::min(128L, (tasks + 3) / 4));
             return (int)std::max(1L, std::min(cap_blocks, want));
         };
-        fblocks_ = blocks_for(width_f_, (long)per_cu * cu_count_);
+        fblocks_ = blocks_for(width_f_, ntot_, (long)per_cu * cu_count_);
         // The solves' waves mostly hold a task that waits for its values:
         // one 4-wave block per CU keeps the queue ahead of the ready front
         // (c1 pair 0.950 -> 0.919 ms against the width rule alone, 512
         // circuits 27.4k -> 29.0k circuit steps/s; two blocks per CU and
         // more were slower on both).
-        tblocks_f_ = blocks_for(width_tf_, cu_count_);
-        tblocks_b_ = blocks_for(width_tb_, cu_count_);
+        tblocks_f_ = blocks_for(width_tf_, nfw_tot_, cu_count_);
+        tblocks_b_ = blocks_for(width_tb_, nbw_tot_, cu_count_);
         if (opt_.refactor_blocks > 0) fblocks_ = opt_.refactor_blocks;
         if (opt_.trisolve_blocks > 0) tblocks_f_ = tblocks_b_ = opt_.trisolve_blocks;
         // Wide grids split each task queue over 4 counters: one counter's
@@ -1213,6 +1273,7 @@ int Batch::repivot(const std::vector<int> &cands, int *changed)
         C.sym = std::move(fresh[i].sym);
         C.plan = std::move(fresh[i].plan);
         C.sell = std::move(fresh[i].sell);
+        for (int d = 0; d < 2; d++) C.local[d] = std::move(fresh[i].local[d]);
         C.frow = std::move(fresh[i].frow);
         C.flvp = std::move(fresh[i].flvp);
         C.brow = std::move(fresh[i].brow);
@@ -1327,8 +1388,14 @@ int Batch::trisolve_t(FactorSet<T> &fs, const double *d_b, double *d_x, const in
     Lb.ctr = d_ctr_ + 2 * kQueueInts;
     Lb.total_waves = tblocks_b_ * 4;
     Lb.nq = nq_t_;
+    // small circuits by one workgroup each, the others through the task queue
+    TriLaunch Sf = Lf, Sb = Lb;
+    if (nlocal_) Lf.tick0 = nullptr;
+    if (nlocal_) Lb.tick0 = nullptr;
     int rc = unset ? check(launch_solve_unset(Lf, ntot_, stream_), "solve unset") : LSP_OK;
-    if (!rc) rc = check(launch_trisolve_half<T>(Lf, true, tblocks_f_, stream_), "trisolve fwd");
+    if (!rc && nlocal_)
+        rc = check(launch_local_solve<T>(Sf, true, d_llist_, nlocal_, local_rows_, stream_), "local fwd");
+    if (!rc && (nfw_tot_ || !nlocal_)) rc = check(launch_trisolve_half<T>(Lf, true, tblocks_f_, stream_), "trisolve fwd");
     if (!rc && njobs_)
         rc = check(launch_tail_solve<T>(fs.tdesc, dgrid_, d_voff_, d_active, d_b, d_ty_, d_typ_, d_tz_, d_x, true,
                                         d_abort_ + 1, Lf.rs, Lf.cs, d_nact, nullptr, stream_),
@@ -1337,7 +1404,9 @@ int Batch::trisolve_t(FactorSet<T> &fs, const double *d_b, double *d_x, const in
         rc = check(launch_tail_solve<T>(fs.tdesc, dgrid_, d_voff_, d_active, d_b, d_ty_, d_typ_, d_tz_, d_x, false,
                                         d_abort_ + 1, Lf.rs, Lf.cs, d_nact, d_ticks_ + kTickBwd0, stream_),
                    "tail bwd");
-    if (!rc) rc = check(launch_trisolve_half<T>(Lb, false, tblocks_b_, stream_), "trisolve bwd");
+    if (!rc && nlocal_)
+        rc = check(launch_local_solve<T>(Sb, false, d_llist_, nlocal_, local_rows_, stream_), "local bwd");
+    if (!rc && (nbw_tot_ || !nlocal_)) rc = check(launch_trisolve_half<T>(Lb, false, tblocks_b_, stream_), "trisolve bwd");
     if (!capturing_) tri_pending_ = true;
     return rc;
 }

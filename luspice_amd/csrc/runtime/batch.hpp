@@ -31,6 +31,9 @@ struct CircuitHost {
     // fused IR step: rows below the dense block grouped by forward / backward
     // level (row lists padded to n entries; nlv + 1 level pointers each)
     std::vector<int> frow, flvp, brow, blvp;
+    LspLocalSolve local[2];              // one-workgroup solves forward / backward (few unknowns)
+    bool local_on = false;               // chosen for this circuit (choose_local)
+    long o_lt[2] = {0, 0}, o_lr[2] = {0, 0}, o_lw[2] = {0, 0};   // their tasks, records, wave starts
     long voff = 0, aoff = 0;             // vector / value arena offsets
     // offsets into the concatenated device arrays
     long o_np1 = 0;                      // n+1 sized arrays
@@ -75,6 +78,9 @@ struct DeviceArrays {
     uint16_t *d_rel_ = nullptr;
     int *d_snend_ = nullptr, *d_ru_ = nullptr, *d_fcut_ = nullptr, *d_bcut_ = nullptr;
     int *d_dpos_ = nullptr;              // per column: position of the diagonal row q[k]
+    int *d_ltask_ = nullptr, *d_lrec_ = nullptr, *d_lwave_ = nullptr;   // one-workgroup solves
+    int *d_llist_ = nullptr;             // their circuits, most tasks first
+    int nlocal_ = 0, local_rows_ = 0;    // count, most unknowns of one
     int *d_fpk_ = nullptr, *d_bpk_ = nullptr, *d_twide_ = nullptr;
     double *d_tailW_ = nullptr, *d_tailP_ = nullptr;   // diagonal-block inverses, packed tiles
     // Ruiz equilibration (FP16 factor storage)
