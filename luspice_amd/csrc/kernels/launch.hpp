@@ -175,6 +175,11 @@ hipError_t launch_tail_solve(const void *mats, const DenseGrid &G, const long *v
                              long long *tick0, hipStream_t st);
 
 // trisolve.hip
+// Stores `bytes` (a multiple of 4) at dst in pinned host memory, then seq at
+// *done (export.hip); ctr is zero before and after.
+hipError_t launch_export(const void *src, void *dst, size_t bytes, unsigned *ctr, unsigned long long *done,
+                         unsigned long long seq, hipStream_t st);
+
 // Solves of the `count` circuits in `list`, one workgroup each, at most `rows`
 // unknowns per circuit (localsolve.hip).
 template <typename T>

@@ -16,6 +16,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -43,6 +44,7 @@ Batch::~Batch()
     for (auto &m : mem_) if (m.p) (void)hipFree(m.p);
     if (h_pin_) (void)hipHostFree(h_pin_);
     if (h_status_) (void)hipHostFree(h_status_);
+    if (h_stage_) (void)hipHostFree(h_stage_);
     if (own_stream_ && stream_) (void)hipStreamDestroy(stream_);
 }
 
@@ -156,12 +158,46 @@ X *Batch::upload(const std::vector<X> &v)
     return d;
 }
 
+// Results of at most this many bytes go to the host by export_kernel; a larger
+// one is a copy, whose rate counts more than its latency.
+constexpr size_t kStageBytes = 256 * 1024;
+
+int Batch::finish(const void *src, void *pinned, size_t bytes)
+{
+    int rc = LSP_OK;
+    unsigned long long *const done = (unsigned long long *)(h_pin_ + 64);
+    if (bytes > kStageBytes || bytes % 4 || !h_pin_) {
+        rc = bytes ? check(hipMemcpyAsync(pinned, src, bytes, hipMemcpyDeviceToHost, stream_), "export") : LSP_OK;
+        return rc ? rc : check(hipStreamSynchronize(stream_), "sync");
+    }
+    const unsigned long long seq = ++done_seq_;
+    rc = check(launch_export(src, pinned, bytes, d_exp_, done, seq, stream_), "export");
+    if (rc) return rc;
+    // Polled for as long as a step takes; past that, and when an error keeps the
+    // word from ever coming, the runtime's own wait.
+    const auto t0 = std::chrono::steady_clock::now();
+    for (int spin = 1; __atomic_load_n(done, __ATOMIC_ACQUIRE) != seq; spin++)
+        if (spin % 256 == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(20))
+            return check(hipStreamSynchronize(stream_), "sync");
+    return LSP_OK;
+}
+
+int Batch::fetch(const double *d_v, double *v)
+{
+    const size_t bytes = (size_t)ntot_ * 8;
+    if (bytes > kStageBytes) {
+        const int rc = check(hipMemcpyAsync(v, d_v, bytes, hipMemcpyDeviceToHost, stream_), "fetch");
+        return rc ? rc : finish();
+    }
+    const int rc = finish(d_v, h_stage_, bytes);
+    if (!rc) std::memcpy(v, h_stage_, bytes);
+    return rc;
+}
+
 // Copies bytes [from, to) of the status block to its pinned host copy and waits.
 int Batch::read_status(size_t from, size_t to)
 {
-    int rc = check(hipMemcpyAsync(h_status_ + from, d_status_ + from, to - from, hipMemcpyDeviceToHost, stream_),
-                   "read status");
-    if (!rc) rc = check(hipStreamSynchronize(stream_), "sync");
+    const int rc = finish(d_status_ + from, h_status_ + from, to - from);
     if (!rc) account_trisolve();
     return rc;
 }
@@ -994,8 +1030,14 @@ int Batch::upload_all()
         if (!d_b_ || !d_x_ || !d_r_ || !d_w_ || !d_z_ || !d_t_ || !d_ty_ || !d_tz_ || !d_typ_ || !d_tzp_ ||
             !d_voff_ || !d_chunks_ || !d_cbeg_ || !d_act_ || !d_conv_ || !d_cycled_ || !d_subset_)
             return LSP_E_ALLOC;
-        if (!h_pin_ && hipHostMalloc((void **)&h_pin_, 4096, hipHostMallocDefault) != hipSuccess)
+        if (!h_pin_) {
+            if (hipHostMalloc((void **)&h_pin_, 4096, hipHostMallocDefault) != hipSuccess) return LSP_E_ALLOC;
+            std::memset(h_pin_, 0, 4096);
+        }
+        if (!h_stage_ && hipHostMalloc((void **)&h_stage_, kStageBytes, hipHostMallocDefault) != hipSuccess)
             return LSP_E_ALLOC;
+        d_exp_ = upload(std::vector<unsigned>(1, 0u));
+        if (!d_exp_) return LSP_E_ALLOC;
     }
     // initial SELL values
     rc = check(launch_gather_cast<double>(nsell_tot_, d_ssrc_, d_ain_, d_sval64_, stream_), "gather");
@@ -1441,7 +1483,7 @@ int Batch::trisolve(const double *b, double *x, bool on_device)
     rc = launch_trisolve_prec(cur_prec_, db, dx, nullptr);
     if (rc) return rc;
     if (!on_device) {
-        rc = check(hipMemcpyAsync(x, d_x_, ntot_ * 8, hipMemcpyDeviceToHost, stream_), "x");
+        rc = fetch(d_x_, x);
         if (rc) return rc;
     }
     const StatusLayout lay = layout();
@@ -1486,11 +1528,7 @@ int Batch::spmv(const double *x, double *y, bool on_device, int prec)
     else
         rc = launch_spmv64(dx, dy, nullptr, nullptr);
     if (rc) return rc;
-    if (!on_device) {
-        rc = check(hipMemcpyAsync(y, d_w_, ntot_ * 8, hipMemcpyDeviceToHost, stream_), "y");
-        if (rc) return rc;
-    }
-    return check(hipStreamSynchronize(stream_), "sync");
+    return on_device ? finish() : fetch(d_w_, y);
 }
 
 // ---------------------------------------------------------------------------
@@ -1856,8 +1894,7 @@ int Batch::solve(const double *b, double *x, bool on_device, lsp_solve_report *r
         }
     }
     if (!on_device) {
-        rc = check(hipMemcpyAsync(x, d_x_, ntot_ * 8, hipMemcpyDeviceToHost, stream_), "x");
-        if (!rc) rc = check(hipStreamSynchronize(stream_), "sync");
+        rc = fetch(d_x_, x);
         if (rc) return rc;
     }
     r.status = r.converged == nlive ? LSP_OK : LSP_E_NOT_CONVERGED;
@@ -2157,8 +2194,7 @@ int Batch::copy_vector(const double *p, bool to_rhs)
 {
     int rc = to_rhs ? check(hipMemcpyAsync(d_b_, p, ntot_ * 8, hipMemcpyDefault, stream_), "rhs")
                     : check(hipMemcpyAsync((void *)p, d_x_, ntot_ * 8, hipMemcpyDefault, stream_), "x");
-    if (!rc) rc = check(hipStreamSynchronize(stream_), "sync");
-    return rc;
+    return rc ? rc : finish();
 }
 
 int Batch::kernel_stats(lsp_kernel_stats *st, int reset)

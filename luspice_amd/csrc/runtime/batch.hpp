@@ -104,6 +104,7 @@ struct DeviceArrays {
     int *d_epoch_ = nullptr;             // epoch counters: [0] factor, [1] fwd, [2] bwd
     int *d_abort_ = nullptr;             // [0] factor, [1] trisolve (in the status block)
     int *d_mstat_ = nullptr;             // kMstat per circuit (in the status block)
+    unsigned *d_exp_ = nullptr;          // workgroups done of a running export
     int *d_dbg_ = nullptr;               // first stuck wait of the refactor
     long long *d_timeline_ = nullptr;    // optional refactor timeline (LSP_REFACTOR_TIMELINE)
     long long *d_tri_tl_ = nullptr;      // optional trisolve timeline (LSP_TRISOLVE_TIMELINE)
@@ -262,6 +263,10 @@ private:
     void *dalloc(size_t bytes);
     void dfree(void *p);
     int alloc_krylov(int mm);
+    // Waits for everything queued on the stream; small results (pinned targets)
+    // come along without a copy of their own.
+    int finish(const void *src = nullptr, void *pinned = nullptr, size_t bytes = 0);
+    int fetch(const double *d_v, double *v);     // a vector arena to the caller's memory, then as finish()
     template <typename X> X *upload(const std::vector<X> &v);
     int check(hipError_t e, const char *what);
     KrylovArgs kargs() const;
@@ -283,6 +288,8 @@ private:
     bool capturing_ = false;
     int *h_pin_ = nullptr;               // pinned host words for flag reads
     char *h_status_ = nullptr;           // pinned copy of the status block
+    char *h_stage_ = nullptr;            // pinned staging of a small solution (kStageBytes)
+    unsigned long long done_seq_ = 0;    // last number asked of export_kernel (stored at h_pin_ + 64)
     const char *refactor_tl_path_ = nullptr;   // LSP_REFACTOR_TIMELINE, read at creation
     const char *trisolve_tl_path_ = nullptr;   // LSP_TRISOLVE_TIMELINE, read at creation
     float t_refactor_ = 0, t_fwd_ = 0, t_bwd_ = 0;
