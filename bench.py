@@ -78,7 +78,7 @@ def measured_traffic(kernel):
 def tri_roofline(tri_b, tri_ms):
     """HBM roofline of one trisolve pair (forward and backward launches with
     their dense-block solves) on the fp32 factors: algorithmic bytes over the
-    pair's event time; traffic from the counter runs of both sparse launches."""
+    pair's time (ticks its kernels write); traffic from the counter runs of both sparse launches."""
     ach = tri_b / (tri_ms * 1e-3) / 1e9 if tri_ms > 0 else 0.0
     tf = measured_traffic("lsp::trisolve_fwd_kernel<float>")
     tb = measured_traffic("lsp::trisolve_bwd_kernel<float>")

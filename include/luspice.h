@@ -239,7 +239,7 @@ int  lsp_batch_graph_step(lsp_batch *b, int prec, lsp_refactor_report *rrep,
  * be host or device memory; the call returns when the copy is complete). */
 int  lsp_batch_set_rhs(lsp_batch *b, const double *rhs);
 int  lsp_batch_get_x(lsp_batch *b, double *x);
-/* Device time of the last refactor / trisolve launches (ms, hipEvent). */
+/* Device time of the last refactor / trisolve launches (ms, from ticks the kernels write). */
 int  lsp_batch_last_times(const lsp_batch *b, double *refactor_ms,
                           double *fwd_ms, double *bwd_ms);
 
