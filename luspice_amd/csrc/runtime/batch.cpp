@@ -325,9 +325,13 @@ int Batch::ensure_factor_set(FactorSet<T> &fs)
     fs.urow = (T *)dalloc(nu_tot_ * sizeof(T));
     fs.diag = (T *)dalloc(ntot_ * sizeof(T));
     // fp64 factors of the dense blocks stay where they were computed
-    if constexpr (std::is_same<T, double>::value) fs.tailF = d_tailS_;
+    fs.tailS = (double *)dalloc(nt2_tot_ * sizeof(double));
+    if constexpr (std::is_same<T, double>::value) fs.tailF = fs.tailS;
     else fs.tailF = (T *)dalloc(nt2_tot_ * sizeof(T));
-    if (!fs.val || !fs.lrow || !fs.urow || !fs.diag || !fs.tailF) return LSP_E_ALLOC;
+    std::vector<DenseJob> jobs = jobs_;
+    for (DenseJob &J : jobs) J.S = fs.tailS + circ_[J.mat].o_t2;
+    fs.djobs = upload(jobs);
+    if (!fs.val || !fs.lrow || !fs.urow || !fs.diag || !fs.tailS || !fs.tailF || !fs.djobs) return LSP_E_ALLOC;
     const int nc = (int)circ_.size();
     std::vector<FactorDesc<T>> fd(nc);
     std::vector<TriDesc<T>> td(nc);
@@ -354,7 +358,7 @@ int Batch::ensure_factor_set(FactorSet<T> &fs)
         F.mstat = d_mstat_ + kMstat * m;
         F.n = C.n;
         F.tail_ds = d_tail_ds_ + C.o_t;
-        F.tail_S = d_tailS_ + C.o_t2;
+        F.tail_S = fs.tailS + C.o_t2;
         F.tail_colmax = d_colmax_ + C.o_t;
         F.tail_F = fs.tailF + C.o_t2;
         F.tail_k0 = C.plan.tail_k0;
@@ -525,11 +529,11 @@ size_t Batch::estimate_device_bytes() const
     if (opt_.krylov_spmv == 2) b += 2 * sell;                              // FP16 SELL values
     b += 16 * nnz + 24 * n + 16 * (nc + 1);                               // Ruiz: row/col, scaled values, scales
     if (opt_.factor_shift > 0.0) b += 8 * n;                               // shifted diagonal entries
-    b += 8 * T2 + 16 * T + 8.0 * 64 * 64 * tiles;                          // dense block work
+    b += 16 * T + 8.0 * 64 * 64 * tiles;                                   // dense block work
     b += (sizeof(FactorTask) + 16) * n + 8 * slices + 16 * n;             // task lists, row packets
     b += 8 * lists + 8 * (slots / kFillSlots + nc);                       // dense-block and fill work lists
     b += 64 * n + 8 * (2 * m + 1) * n;                                    // vectors, Krylov bases V and Z
-    b += (4 + 8) * (slots + nlu + n) + 4 * T2;                             // fp32 + fp64 factor sets
+    b += (4 + 8) * (slots + nlu + n) + (8 + 4 + 8) * T2;                   // fp32 + fp64 factor sets
     if (maxcol > std::max(1, opt_.lds_cap)) b += 256.0 * 8 * 4 * maxcol * 8;   // global column scratch
     return (size_t)(1.05 * b) + (1u << 20);
 }
@@ -722,8 +726,6 @@ int Batch::upload_all()
     // dense trailing blocks, the jobs by falling order T
     {
         std::vector<int> tds, tlc;
-        std::vector<DenseJob> jobs;
-        d_tailS_ = (double *)dalloc(nt2_tot_ * sizeof(double));
         d_colmax_ = (unsigned long long *)dalloc(nt_tot_ * sizeof(unsigned long long));
         std::vector<int> mat, order;
         for (int m = 0; m < nc; m++) {
@@ -744,20 +746,19 @@ int Batch::upload_all()
         d_tailW_ = (double *)dalloc(npanel * 2 * 64 * 64 * sizeof(double));
         d_tailP_ = (double *)dalloc(ntile * 64 * 64 * sizeof(double));
         d_dflag_ = upload(std::vector<int>(ntile, 0));
-        if (!d_tailS_ || !d_colmax_ || !d_tailW_ || !d_tailP_ || !d_dflag_) return LSP_E_ALLOC;
+        if (!d_colmax_ || !d_tailW_ || !d_tailP_ || !d_dflag_) return LSP_E_ALLOC;
         ntile = npanel = 0;
         for (int m : mat) {
             const CircuitHost &C = circ_[m];
             DenseJob J{};
             J.T = C.plan.tail_T;
             J.nt = (J.T + 63) / 64;
-            J.S = d_tailS_ + C.o_t2;
             J.P = d_tailP_ + ntile * 64 * 64;
             J.W = d_tailW_ + npanel * 2 * 64 * 64;
             J.colmax = d_colmax_ + C.o_t;
             J.flag = d_dflag_ + ntile;
             J.mat = m;
-            jobs.push_back(J);
+            jobs_.push_back(J);
             order.push_back(J.T);
             ntile += (size_t)J.nt * J.nt;
             npanel += J.nt;
@@ -774,7 +775,6 @@ int Batch::upload_all()
         dgrid_.ntrsv = (int)H.trsv.size();
         d_tail_ds_ = upload(tds);
         d_tail_lcut_ = upload(tlc);
-        d_djobs_ = upload(jobs);
         d_tail_ctr_ = upload(std::vector<int>(4 * nc, 0));
         std::vector<int2> fill;
         for (int m = 0; m < nc; m++) {
@@ -784,7 +784,7 @@ int Batch::upload_all()
         }
         d_fillchunk_ = upload(fill);
         nfillchunk_ = (int)fill.size();
-        if (!d_tail_ds_ || !d_tail_lcut_ || !d_djobs_ || !d_tail_ctr_ || !d_fillchunk_ || !dgrid_.lu ||
+        if (!d_tail_ds_ || !d_tail_lcut_ || !d_tail_ctr_ || !d_fillchunk_ || !dgrid_.lu ||
             !dgrid_.pivot || !dgrid_.gather || !dgrid_.trsv)
             return LSP_E_ALLOC;
     }
@@ -1158,7 +1158,7 @@ int Batch::refactor_t(FactorSet<T> &fs, const int *d_active)
     rc = check(launch_refactor<T>(L, fblocks_, stream_), "refactor launch");
     if (!rc && njobs_) {
         // two 4-wave workgroups per CU (the kernel's register budget)
-        rc = check(launch_dense_lu<T>(d_djobs_, fs.fdesc, d_active, dgrid_, d_ctr_ + 3 * kQueueInts, d_epoch_ + 1,
+        rc = check(launch_dense_lu<T>(fs.djobs, fs.fdesc, d_active, dgrid_, d_ctr_ + 3 * kQueueInts, d_epoch_ + 1,
                                       d_abort_, d_ticks_ + kTickDense1, 2 * cu_count_, opt_.refactor_ptol, L.stol, stream_), "dense lu");
     }
     return rc;

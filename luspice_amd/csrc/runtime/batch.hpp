@@ -52,7 +52,13 @@ struct CircuitHost {
 template <typename T>
 struct FactorSet {                       // per storage precision
     T *val = nullptr, *lrow = nullptr, *urow = nullptr, *diag = nullptr;
-    T *tailF = nullptr;                  // dense trailing blocks, storage precision
+    // Dense trailing blocks: fp64 work block and factor in storage precision
+    // (the same memory for fp64).  Each set has its own work block: with a
+    // shared one, a refactor in another precision would overwrite the fp64
+    // factors that circuits outside its mask still solve with.
+    double *tailS = nullptr;
+    T *tailF = nullptr;
+    DenseJob *djobs = nullptr;           // device
     FactorDesc<T> *fdesc = nullptr;      // device
     TriDesc<T> *tdesc = nullptr;         // device
     IrDesc<T> *idesc = nullptr;          // device (fused IR step)
@@ -115,10 +121,9 @@ struct DeviceArrays {
     long width_f_ = 0, width_tf_ = 0, width_tb_ = 0;   // widest merged level
     // dense trailing blocks
     int *d_tail_ds_ = nullptr, *d_tail_lcut_ = nullptr, *d_tail_ctr_ = nullptr;
-    double *d_tailS_ = nullptr;
     unsigned long long *d_colmax_ = nullptr;
     int *d_dflag_ = nullptr;                   // per tile of every dense job: epoch of the launch that made it final
-    DenseJob *d_djobs_ = nullptr;
+    std::vector<DenseJob> jobs_;               // without their work blocks (ensure_factor_set)
     int njobs_ = 0;
     DenseGrid dgrid_;                          // work lists of the dense-block launches
     int2 *d_fillchunk_ = nullptr;              // (matrix, chunk) of the unset fill
