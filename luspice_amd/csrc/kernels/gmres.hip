@@ -97,6 +97,7 @@ __global__ void __launch_bounds__(kKrT) start_kernel(KrylovArgs K, const double 
             K.act[m] = 0;
             K.cycled[m] = 0;
             if (first) K.jfin[m] = 0;
+            if (m == 0) hist[cyc & 1] = K.nb[m] > 0 ? K.beta[m] / K.nb[m] : K.beta[m];   // its last residual
         }
         return;
     }

@@ -203,17 +203,21 @@ int Batch::read_status(size_t from, size_t to)
 }
 
 // Adds the device time of the last forward/backward trisolve pair to the
-// running statistics; called once the host has its ticks.
+// running statistics; called once the host has its ticks.  A pair that was
+// queued ahead of the convergence test and had nothing to do left the ticks of
+// an earlier one and is not counted.
 void Batch::account_trisolve()
 {
     if (!tri_pending_) return;
+    tri_pending_ = false;
     const long long *t = status<long long>(layout().ticks);
+    if (t[kTickBwd1] == tri_end_) return;
+    tri_end_ = t[kTickBwd1];
     t_fwd_ = (float)((double)(t[kTickBwd0] - t[kTickFwd0]) * ms_per_tick_);
     t_bwd_ = (float)((double)(t[kTickBwd1] - t[kTickBwd0]) * ms_per_tick_);
     stats_.fwd_ms += t_fwd_;
     stats_.bwd_ms += t_bwd_;
     stats_.tri_count++;
-    tri_pending_ = false;
 }
 
 // ---------------------------------------------------------------------------
@@ -1074,6 +1078,7 @@ void Batch::release_device()
     cur_prec_ = -1;
     uploaded_ = false;
     tri_pending_ = false;
+    tri_end_ = 0;                        // as the new status block's
 }
 
 int Batch::set_stream(hipStream_t s)

@@ -299,6 +299,7 @@ private:
     const char *trisolve_tl_path_ = nullptr;   // LSP_TRISOLVE_TIMELINE, read at creation
     float t_refactor_ = 0, t_fwd_ = 0, t_bwd_ = 0;
     bool tri_pending_ = false;
+    long long tri_end_ = 0;              // end tick of the last pair counted
     std::vector<double> res_hist0_;      // ||r||/||b|| of circuit 0 at each restart
     lsp_kernel_stats stats_{};
 };
