@@ -1616,7 +1616,8 @@ int Batch::gmres_ir(const double *d_bv, double *d_xv, int prec, const std::vecto
     res_hist0_.clear();
     const int *nact = status<int>(lay.nact);
     const double *hist = status<double>(lay.hist);
-    bool done = false;
+    bool done = opt_.ir_outer <= 0;                     // no cycle: the residual of x as it is
+    if (done) LSP_TRY(read_status(lay.ticks, lay.end));
     for (int cyc = 0; !done;) {
         for (int j = 0; j < mm; j++) {
             LSP_TRY(launch_inner(K, prec, j, j == 0 ? d_nact_ + nact_word(cyc, 0) : nullptr));
