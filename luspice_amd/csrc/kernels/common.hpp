@@ -286,7 +286,6 @@ __device__ __forceinline__ void wave_sync()
 // few hundred cycles with all lanes saturate the memory path the producers
 // need, and the factorization then crawls.  The caller issues one
 // acquire_fence() after a successful wait.
-constexpr int kRoundLimit = 1 << 21;
 
 __device__ __forceinline__ bool wave_wait(const int *flag, int epoch, int *abort_word,
                                           int *dbg = nullptr, int who2 = -1, int max_backoff = 7)
@@ -316,13 +315,29 @@ __device__ __forceinline__ bool wave_wait(const int *flag, int epoch, int *abort
     }
 }
 
+// Raises the abort word; the lane that was first writes down what it waited
+// for (seen: the flag's value, or kSeenUnset for a wait on values).
+__device__ __forceinline__ void give_up(int *abort_word, int *dbg, int j, int seen, int epoch, int round, int k)
+{
+    if (atomicCAS(abort_word, 0, kErrSpin) == 0 && dbg) {
+        dbg[0] = j;
+        dbg[1] = seen;
+        dbg[2] = epoch;
+        dbg[3] = round;
+        dbg[4] = k;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    }
+}
+
 // Wave-collective wait for a growing prefix of lanes: lane l < nd waits on
 // its flag (null = nothing to wait for); `ok` holds the lane's seen state
 // across calls and starts as (flag == null).  Returns the length p of the
 // leading run of lanes whose flags have all been seen, once p > have, or -1
-// when the wait was abandoned.  The result is wave-uniform.
+// when the wait was abandoned.  The result is wave-uniform.  dbg names the first
+// wait given up: column who2 on lane's column j.
 __device__ __forceinline__ int wave_wait_prefix(const int *flag, int epoch, int *abort_word, int &ok, int have,
-                                                int nd, int *dbg = nullptr, int who2 = -1, int max_backoff = 7)
+                                                int nd, int *dbg = nullptr, int who2 = -1, int max_backoff = 7,
+                                                int j = -1, int limit = kRoundLimit)
 {
     int seen = epoch;
     int backoff = 0;
@@ -336,14 +351,8 @@ __device__ __forceinline__ int wave_wait_prefix(const int *flag, int epoch, int 
         }
         if (round == 0) continue;               // the first look comes before the first sleep
         if ((round & 15) == 15 && aborted(abort_word)) return -1;
-        if (round > kRoundLimit) {
-            if (!ok && atomicCAS(abort_word, 0, kErrSpin) == 0 && dbg) {
-                dbg[1] = seen;
-                dbg[2] = epoch;
-                dbg[3] = round;
-                dbg[4] = who2;
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-            }
+        if (round > limit) {
+            if (!ok) give_up(abort_word, dbg, j, seen, epoch, round, who2);
             return -1;
         }
         for (int s = 0; s <= backoff; s++) __builtin_amdgcn_s_sleep(4);

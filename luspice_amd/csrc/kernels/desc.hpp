@@ -16,6 +16,11 @@ enum : int {
     kErrCapacity = 2,    // a column/row exceeded its scratch capacity
 };
 
+// Polls after which a wait gives up (seconds), and what the report says was
+// seen when the wait was for values and not for a flag.
+constexpr int kRoundLimit = 1 << 21;
+constexpr int kSeenUnset = -2;
+
 // Ints in one persistent kernel's queue block: up to 4 queue counters, a
 // cache line each, and the count of waves finished.
 constexpr int kQueueInts = 128;

@@ -110,7 +110,7 @@ __device__ __forceinline__ void run_gemv(const T *val, XP x, const LSP_GLOBAL ui
 template <int G, typename T, typename XP>
 __device__ __forceinline__ bool dep_unset(const T *val, XP x, const LSP_GLOBAL uint16_t *map, int64_t u, double xj,
                                           int base, int row0, int tri, int R, const int *flag, int epoch, int &ok,
-                                          int *abort_word, int lane)
+                                          int *abort_word, int lane, int *dbg, int j, int k, int limit)
 {
     constexpr int H = G < 4 ? G : 4;            // chunks applied at a time
     for (int i0 = 0; i0 < R; i0 += G * kWave) {
@@ -134,8 +134,8 @@ __device__ __forceinline__ bool dep_unset(const T *val, XP x, const LSP_GLOBAL u
             for (int g = 0; g < G; g++) miss |= Unset<T>::is(v[g]);
             if (!__any(miss)) break;
             if ((round & 15) == 15 && aborted(abort_word)) return false;
-            if (round > kRoundLimit) {
-                atomicCAS(abort_word, 0, kErrSpin);
+            if (round > limit) {
+                give_up(abort_word, dbg, j, kSeenUnset, epoch, round, k);
                 return false;
             }
             __builtin_amdgcn_s_sleep(1);
@@ -215,7 +215,7 @@ constexpr int kBulk = 3;
 template <typename T, typename XP>
 __device__ void factor_column(const LSP_CONST FactorDesc<T> *M, const LSP_CONST FactorTask *tk, XP x,
                               int epoch, int *abort_word, double ptol, double stol, int *dbg, long long *tw,
-                              int backoff, int *tctr, TicketReq &treq)
+                              int backoff, int limit, int *tctr, TicketReq &treq)
 {
     // chunks of 64 rows per pass of dep_unset (316 x 316 grid with 4 / 8 / 12 / 16:
     // 2781 / 2410 / 2584 / 2819 us fp32; a global x costs registers)
@@ -311,7 +311,8 @@ __device__ void factor_column(const LSP_CONST FactorDesc<T> *M, const LSP_CONST 
                 const double xj = bcast_f64(xc, have);
                 const auto direct = [&](auto g) {
                     return dep_unset<decltype(g)::value>(val, x, map, u, xj, base, s0 + have + 1, aft, R, flag, epoch,
-                                                         ok, abort_word, lane);
+                                                         ok, abort_word, lane, dbg,
+                                                         __builtin_amdgcn_readlane(j, have), k, limit);
                 };
                 if (!(R <= kWave ? direct(Int<1>()) : R <= 4 * kWave ? direct(Int<4>()) : direct(Int<kWide>()))) return;
                 if (aft == 0) u += R;
@@ -320,7 +321,7 @@ __device__ void factor_column(const LSP_CONST FactorDesc<T> *M, const LSP_CONST 
                 if (lane >= have && lane < nd) xc = x[s0 + lane];
                 continue;
             }
-            const int p = wave_wait_prefix(flag, epoch, abort_word, ok, have, nd, dbg, k, backoff);
+            const int p = wave_wait_prefix(flag, epoch, abort_word, ok, have, nd, dbg, k, backoff, j, limit);
             if (p < 0) return;                                      // aborted; kernel drains
             if (tw) tw[0] = (long long)wall_clock64();
             unsigned long long hs = (heads & ~((1ull << have) - 1)) | (1ull << have);
@@ -597,9 +598,11 @@ __global__ void __launch_bounds__(256, 4) refactor_kernel(FactorLaunch L)
         long long *wp = L.timeline ? tw : nullptr;
         const long long t0 = L.timeline ? (long long)wall_clock64() : 0;
         if (m <= L.cap) {
-            factor_column<T>(M, tk, xl, epoch, L.abort_word, L.ptol, L.stol, L.dbg, wp, L.poll_backoff, qc, req);
+            factor_column<T>(M, tk, xl, epoch, L.abort_word, L.ptol, L.stol, L.dbg, wp, L.poll_backoff, L.round_limit, qc,
+                             req);
         } else if (m <= L.scratch_stride) {
-            factor_column<T>(M, tk, xg, epoch, L.abort_word, L.ptol, L.stol, L.dbg, wp, L.poll_backoff, qc, req);
+            factor_column<T>(M, tk, xg, epoch, L.abort_word, L.ptol, L.stol, L.dbg, wp, L.poll_backoff, L.round_limit, qc,
+                             req);
         } else {
             if (lane_id() == 0) st_relaxed(L.abort_word, kErrCapacity);
         }

@@ -25,7 +25,8 @@ struct FactorLaunch {
     int total_waves;
     double ptol;
     double stol;            // > 0: also classify each pivot against splu's choice at this tol
-    int *dbg;               // 8 ints: first stuck wait (dep, seen, epoch, spins, column)
+    int *dbg;               // 8 ints: first wait given up (dep, seen, epoch, rounds, column)
+    int round_limit;        // a dependency wait gives up after this many polls
     long long *timeline;    // optional, 4 per task (100 MHz wall clock): start, flag
                             // published (end for a dense-block column), end of the
                             // last dependency wait, column

@@ -443,6 +443,7 @@ int Batch::prepare(const lsp_circuit_in *cin, int nc, const lsp_options *opt)
     if (opt_.ir_method < 0 || opt_.ir_method > 1 ||
         opt_.ir_fused_steps < 0 || opt_.refactor_fp64 < 0 || opt_.refactor_fp64 > 1)
         return LSP_E_ARG;
+    if (const char *r = getenv("LSP_REFACTOR_ROUNDS")) round_limit_ = std::max(0, atoi(r));   // tests of the give-up path
     refactor_tl_path_ = getenv("LSP_REFACTOR_TIMELINE");     // diagnostic dumps
     trisolve_tl_path_ = getenv("LSP_TRISOLVE_TIMELINE");
     circ_.resize(nc);
@@ -1157,6 +1158,7 @@ int Batch::refactor_t(FactorSet<T> &fs, const int *d_active)
     L.ptol = opt_.refactor_ptol;
     L.stol = opt_.repivot == 3 ? opt_.pivot_tol : 0.0;
     L.dbg = d_dbg_;
+    L.round_limit = round_limit_;
     L.ticks = d_ticks_;
     rc = check(launch_fill_unset<T>(fs.fdesc, d_active, d_fillchunk_, nfillchunk_, d_abort_, d_dbg_, stream_), "unset");
     if (rc) return rc;
@@ -1257,8 +1259,9 @@ int Batch::refactor_pass(int prec, const std::vector<int> *subset, std::vector<i
         if (dbg[0] >= 0 && dbg[0] < ntot_)
             (void)hipMemcpy(&flag_now, d_done_ + dbg[0], 4, hipMemcpyDeviceToHost);
         last_error = "refactor wait gave up: column " + std::to_string(dbg[4]) + " waiting on " +
-                     std::to_string(dbg[0]) + " saw " + std::to_string(dbg[1]) + " epoch " +
-                     std::to_string(dbg[2]) + " spins " + std::to_string(dbg[3]) +
+                     std::to_string(dbg[0]) +
+                     (dbg[1] == kSeenUnset ? " by its values" : " saw " + std::to_string(dbg[1])) + " epoch " +
+                     std::to_string(dbg[2]) + " polls " + std::to_string(dbg[3]) +
                      "; flag in memory after the launch: " + std::to_string(flag_now);
     }
     return LSP_OK;

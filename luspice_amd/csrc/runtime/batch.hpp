@@ -295,6 +295,7 @@ private:
     char *h_status_ = nullptr;           // pinned copy of the status block
     char *h_stage_ = nullptr;            // pinned staging of a small solution (kStageBytes)
     unsigned long long done_seq_ = 0;    // last number asked of export_kernel (stored at h_pin_ + 64)
+    int round_limit_ = kRoundLimit;            // LSP_REFACTOR_ROUNDS, read at creation
     const char *refactor_tl_path_ = nullptr;   // LSP_REFACTOR_TIMELINE, read at creation
     const char *trisolve_tl_path_ = nullptr;   // LSP_TRISOLVE_TIMELINE, read at creation
     float t_refactor_ = 0, t_fwd_ = 0, t_bwd_ = 0;
