@@ -14,8 +14,9 @@
 // What bounds it: launches.  At n <= 1e5 every vector fits the caches and each
 // kernel is near the cost of a launch (about 4 us), so the work is laid out for
 // few of them.  Reductions are two-stage and deterministic; the second stage
-// has no launch of its own, every workgroup that needs a sum adds its matrix's
-// partial sums itself (in the same order, so all agree).  One inner iteration
+// has no launch of its own while the parts are few (fold()): every workgroup
+// that needs a sum adds its matrix's partial sums itself (in the same order, so
+// all agree).  One inner iteration
 // is the preconditioner's solves and four launches:
 //   sell_block_kernel (spmv.hip)  w = A z, partial V^T w
 //   orth_kernel<first>            h = V^T w, w -= V h, partial V^T w
@@ -62,6 +63,18 @@ __device__ __forceinline__ double wave_partials(const double *p, long stride, in
     return wave_sum(s);
 }
 
+// Adds up each matrix's parts once, one wave per (matrix, sum), in the order in
+// which the consumers would: out[nv * m + i] is sum i of in's parts of matrix m.
+__global__ void __launch_bounds__(kWave) fold_kernel(const double *in, const int *pbeg, int pstride, int nv,
+                                                     const int *mask, int run, const int *gate, double *out)
+{
+    if (gated(gate)) return;
+    const int m = blockIdx.x / nv, i = blockIdx.x % nv;
+    if (mask[m] != run) return;
+    const double s = wave_partials(in + i, pstride, pbeg[m], pbeg[m + 1]);
+    if (threadIdx.x == 0) out[(long)m * nv + i] = s;
+}
+
 // conv, abort word and active counts before a solve.
 __global__ void __launch_bounds__(kKrT) solve_init_kernel(int *conv, int nmat, int *abort_word, int *nact)
 {
@@ -84,7 +97,8 @@ __device__ __forceinline__ void unset_row(const UnsetArgs &U, long i)
 // Cycle start: ||r|| (and on the first cycle ||b||) from the residual's
 // partial sums, the outer convergence test, V_0 = r / ||r||.
 __global__ void __launch_bounds__(kKrT) start_kernel(KrylovArgs K, const double *r, int cyc, double *hist,
-                                                     const int *gate, UnsetArgs U)
+                                                     const int *gate, UnsetArgs U, const double *pin,
+                                                     const int *pbeg)
 {
     __shared__ double s2[2];
     if (gated(gate)) return;
@@ -103,7 +117,7 @@ __global__ void __launch_bounds__(kKrT) start_kernel(KrylovArgs K, const double 
     }
     const int wv = threadIdx.x >> 6;
     if (wv < 2) {
-        const double s = wave_partials(K.spartial + wv, 2, K.sbeg[m], K.sbeg[m + 1]);
+        const double s = wave_partials(pin + wv, 2, pbeg[m], pbeg[m + 1]);
         if (lane_id() == 0) s2[wv] = s;
     }
     __syncthreads();
@@ -237,14 +251,15 @@ __global__ void __launch_bounds__(kKrT) chunk_dots_kernel(KrylovArgs K, int nv)
 // End of inner iteration j: V_{j+1} = w / ||w||, the work values of the next
 // solves unset; the lead does the Givens step and ends the matrix's cycle when
 // its residual estimate is small enough.
-__global__ void __launch_bounds__(kKrT) basis_kernel(KrylovArgs K, int j, UnsetArgs U)
+__global__ void __launch_bounds__(kKrT) basis_kernel(KrylovArgs K, int j, UnsetArgs U, const double *pin,
+                                                     const int *pbeg)
 {
     __shared__ double s_hn;
     const int4 ch = K.chunks[blockIdx.x];
     const int m = ch.x;
     if (!K.act[m]) return;
     if (threadIdx.x < kWave) {
-        const double s = wave_partials(K.pnorm, 1, K.cbeg[m], K.cbeg[m + 1]);
+        const double s = wave_partials(pin, 1, pbeg[m], pbeg[m + 1]);
         if (threadIdx.x == 0) s_hn = sqrt(s);
     }
     __syncthreads();
@@ -345,10 +360,36 @@ hipError_t k_solve_init(int *conv, int nmat, int *abort_word, int *nact, hipStre
                        nmat, abort_word, nact);
     return hipGetLastError();
 }
+
+// The sums a consumer is about to read: the parts as they are, or added up.
+struct Parts {
+    const double *p;
+    const int *beg;
+    int stride;
+};
+// Every workgroup of a consumer adds up all parts of its matrix (`reads` of them
+// over the batch, for each of nv sums), which grows with the square of a
+// circuit's size.  From kFoldLines cache lines on, a launch of its own adds them
+// up first, to the same sums bit for bit.  An iteration beside its solves, as
+// they are / added up first: n = 99 906 (196 chunks) 49 / 58 us over 3 iterations,
+// 67 / 73 over 20, 146 / 142 over 60; n = 250 000 (489 chunks) 68 / 79 over 3,
+// 209 / 180 over 60; chunks of 64 rows, n = 99 906 60 / 69 over 3, 136 / 97 over 20,
+// 372 / 183 over 60.  A launch costs 3.3 us, a million lines 1 to 3 us.
+constexpr double kFoldLines = 1.5e6;
+static Parts fold(const KrylovArgs &K, Parts in, int nv, long reads, const int *mask, int run, const int *gate,
+                  hipStream_t s)
+{
+    if ((double)reads * nv * (in.stride < 8 ? in.stride : 8) / 8 < kFoldLines) return in;
+    hipLaunchKernelGGL(fold_kernel, dim3((unsigned)(K.nmat * nv)), dim3(kWave), 0, s, in.p, in.beg, in.stride, nv, mask,
+                       run, gate, K.folded);
+    return Parts{K.folded, K.each, nv};
+}
+
 hipError_t k_start(const KrylovArgs &K, const double *r, int cyc, double *hist, const int *gate,
                    const UnsetArgs &U, hipStream_t s)
 {
-    hipLaunchKernelGGL(start_kernel, dim3(K.nchunks), dim3(kKrT), 0, s, K, r, cyc, hist, gate, U);
+    const Parts in = fold(K, Parts{K.spartial, K.sbeg, 2}, 2, K.sreads, K.conv, 0, gate, s);
+    hipLaunchKernelGGL(start_kernel, dim3(K.nchunks), dim3(kKrT), 0, s, K, r, cyc, hist, gate, U, in.p, in.beg);
     return hipGetLastError();
 }
 hipError_t k_chunk_dots(const KrylovArgs &K, int nv, hipStream_t s)
@@ -358,16 +399,18 @@ hipError_t k_chunk_dots(const KrylovArgs &K, int nv, hipStream_t s)
 }
 hipError_t k_orth(const KrylovArgs &K, int j, bool first, hipStream_t s)
 {
+    const bool prod = first && j < kSpmvDots;   // sums from the product's kernel
+    Parts in = prod ? Parts{K.spartial, K.sbeg, kSpmvDots} : Parts{first ? K.partial2 : K.partial, K.cbeg, K.mmax + 1};
+    in = fold(K, in, j + 1, prod ? K.sreads : K.creads, K.act, 1, nullptr, s);
     const dim3 g(K.nchunks), t(kKrT);
-    if (!first) hipLaunchKernelGGL(orth_kernel<false>, g, t, 0, s, K, j, K.partial, K.cbeg, K.mmax + 1);
-    else if (j < kSpmvDots)                     // sums from the product's kernel
-        hipLaunchKernelGGL(orth_kernel<true>, g, t, 0, s, K, j, K.spartial, K.sbeg, kSpmvDots);
-    else hipLaunchKernelGGL(orth_kernel<true>, g, t, 0, s, K, j, K.partial2, K.cbeg, K.mmax + 1);
+    if (first) hipLaunchKernelGGL(orth_kernel<true>, g, t, 0, s, K, j, in.p, in.beg, in.stride);
+    else hipLaunchKernelGGL(orth_kernel<false>, g, t, 0, s, K, j, in.p, in.beg, in.stride);
     return hipGetLastError();
 }
 hipError_t k_basis(const KrylovArgs &K, int j, const UnsetArgs &U, hipStream_t s)
 {
-    hipLaunchKernelGGL(basis_kernel, dim3(K.nchunks), dim3(kKrT), 0, s, K, j, U);
+    const Parts in = fold(K, Parts{K.pnorm, K.cbeg, 1}, 1, K.creads, K.act, 1, nullptr, s);
+    hipLaunchKernelGGL(basis_kernel, dim3(K.nchunks), dim3(kKrT), 0, s, K, j, U, in.p, in.beg);
     return hipGetLastError();
 }
 hipError_t k_update(const KrylovArgs &K, const double *Z, double *x, const int *gate, hipStream_t s)

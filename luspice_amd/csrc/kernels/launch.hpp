@@ -80,6 +80,9 @@ struct KrylovArgs {
     double *partial;        // nchunks * (mmax+1): V^T w after the first pass
     double *partial2;       // nchunks * (mmax+1): V^T w before it (more than kSpmvDots vectors)
     double *pnorm;          // nchunks: w^T w
+    double *folded;         // nmat * max(mmax+1, 2): sums added up by a launch of their own (gmres.hip)
+    const int *each;        // nmat+1: 0, 1, 2, .. (their parts: one per matrix)
+    long sreads, creads;    // sums over the matrices of chunks times product parts / chunk parts
     double *H;              // nmat * (mmax+1) * mmax, H[i*mmax + j]
     double *cs, *sn;        // nmat * mmax
     double *g;              // nmat * (mmax+1)

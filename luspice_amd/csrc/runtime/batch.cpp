@@ -80,19 +80,20 @@ void Batch::dfree(void *p)
 int Batch::alloc_krylov(int mm)
 {
     const int nc = (int)circ_.size();
-    for (void *p : {(void *)d_V_, (void *)d_Z_, (void *)d_partial_, (void *)d_partial2_, (void *)d_H_, (void *)d_cs_,
+    for (void *p : {(void *)d_V_, (void *)d_Z_, (void *)d_partial_, (void *)d_partial2_, (void *)d_folded_, (void *)d_H_, (void *)d_cs_,
                     (void *)d_sn_, (void *)d_g_, (void *)d_yv_})
         dfree(p);
     d_V_ = (double *)dalloc((size_t)(mm + 1) * ntot_ * 8);
     d_Z_ = (double *)dalloc((size_t)mm * ntot_ * 8);
     d_partial_ = (double *)dalloc((size_t)nchunks_ * (mm + 1) * 8);
     d_partial2_ = (double *)dalloc((size_t)nchunks_ * (mm + 1) * 8);
+    d_folded_ = (double *)dalloc((size_t)nc * (mm + 1) * 8);
     d_H_ = (double *)dalloc((size_t)nc * (mm + 1) * mm * 8);
     d_cs_ = (double *)dalloc((size_t)nc * mm * 8);
     d_sn_ = (double *)dalloc((size_t)nc * mm * 8);
     d_g_ = (double *)dalloc((size_t)nc * (mm + 1) * 8);
     d_yv_ = (double *)dalloc((size_t)nc * mm * 8);
-    if (!d_V_ || !d_Z_ || !d_partial_ || !d_partial2_ || !d_H_ || !d_cs_ || !d_sn_ || !d_g_ || !d_yv_)
+    if (!d_V_ || !d_Z_ || !d_partial_ || !d_partial2_ || !d_folded_ || !d_H_ || !d_cs_ || !d_sn_ || !d_g_ || !d_yv_)
         return LSP_E_ALLOC;
     mm_alloc_ = mm;
     return LSP_OK;
@@ -1024,9 +1025,18 @@ int Batch::upload_all()
         sbeg[nc] = nsblock_ = (int)sblock.size();
         d_sblock_ = upload(sblock);
         d_sbeg_ = upload(sbeg);
+        std::vector<int> each(nc + 1);
+        for (int m = 0; m <= nc; m++) each[m] = m;
+        sreads_ = creads_ = 0;
+        for (int m = 0; m < nc; m++) {
+            const long ch = cbeg[m + 1] - cbeg[m];
+            sreads_ += ch * (sbeg[m + 1] - sbeg[m]);
+            creads_ += ch * ch;
+        }
+        d_each_ = upload(each);
         d_spartial_ = (double *)dalloc((size_t)nsblock_ * kSpmvDots * 8);
         d_pnorm_ = (double *)dalloc((size_t)nchunks_ * 8);
-        if (!d_sblock_ || !d_sbeg_ || !d_spartial_ || !d_pnorm_) return LSP_E_ALLOC;
+        if (!d_sblock_ || !d_sbeg_ || !d_each_ || !d_spartial_ || !d_pnorm_) return LSP_E_ALLOC;
         rc = alloc_krylov(mm);
         if (rc) return rc;
         d_act_ = (int *)dalloc(nc * 4);
@@ -1122,6 +1132,10 @@ KrylovArgs Batch::kargs() const
     K.V = d_V_;
     K.w = d_w_;
     K.spartial = d_spartial_; K.partial = d_partial_; K.partial2 = d_partial2_; K.pnorm = d_pnorm_;
+    K.folded = d_folded_;
+    K.each = d_each_;
+    K.sreads = sreads_;
+    K.creads = creads_;
     K.H = d_H_; K.cs = d_cs_; K.sn = d_sn_; K.g = d_g_; K.yv = d_yv_;
     K.beta = d_beta_; K.nb = d_nb_; K.nact = d_nact_;
     K.act = d_act_; K.jfin = d_jfin_; K.conv = d_conv_; K.cycled = d_cycled_;

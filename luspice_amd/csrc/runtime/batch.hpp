@@ -140,12 +140,14 @@ struct DeviceArrays {
            *d_Z_ = nullptr;
     int2 *d_sblock_ = nullptr;           // (matrix, first slice) of the GMRES products' workgroups
     int *d_sbeg_ = nullptr;              // nmat+1 ranges of them per matrix
+    int *d_each_ = nullptr;              // nmat+1: 0, 1, 2, ..
+    long sreads_ = 0, creads_ = 0;       // KrylovArgs
     int nsblock_ = 0;
     long *d_voff_ = nullptr;
     int4 *d_chunks_ = nullptr;
     int *d_cbeg_ = nullptr;
     int nchunks_ = 0;
-    double *d_partial_ = nullptr, *d_partial2_ = nullptr, *d_spartial_ = nullptr, *d_pnorm_ = nullptr,
+    double *d_partial_ = nullptr, *d_partial2_ = nullptr, *d_spartial_ = nullptr, *d_pnorm_ = nullptr, *d_folded_ = nullptr,
            *d_H_ = nullptr, *d_cs_ = nullptr, *d_sn_ = nullptr, *d_g_ = nullptr, *d_yv_ = nullptr;
     int *d_act_ = nullptr, *d_conv_ = nullptr, *d_cycled_ = nullptr, *d_subset_ = nullptr;
     // what the host reads after a refactor or solve, in one block (StatusLayout)

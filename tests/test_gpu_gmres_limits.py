@@ -23,3 +23,33 @@ def test_no_cycle_leaves_x_at_zero(prec):
     x, rep = B.solve(np.zeros(c.n))
     assert rep["rc"] == 0 and rep["converged"] == 1 and not x.any(), rep
     B.close()
+
+
+@pytest.mark.parametrize("sizes,chunk", [((3000,), 1), ((3000, 333, 2500), 1), ((3000,), 2), ((3000,), 512)])
+@pytest.mark.parametrize("inner", [3, 40])
+def test_many_reduction_chunks(sizes, chunk, inner):
+    """Chunks of 1 and 2 rows: the parts of a sum are added up by a launch of
+    their own (9 and 2.25 million reads a sum at 3000 rows); 512 rows: by the
+    kernels that need them.  Residuals on the host from the caller's values: a
+    solve that reports convergence met 1e-9, and reported it to rounding."""
+    print("case: reduction chunks", sizes, chunk, inner, flush=True)
+    circ = [L.mna("sized", n=n, lr=0.02, seed=n) for n in sizes]
+    B = L.Batch(circ, chunk_rows=chunk, ir_inner=inner, ir_outer=60, factor_shift=1e-3)
+    for prec in ("fp32", "fp64"):
+        B.set_active(None)
+        assert B.refactor(prec)["rc"] == 0
+        rhs = np.concatenate([c.rhs for c in circ])
+        for mask in (None, [1] + [0] * (len(sizes) - 1)):
+            B.set_active(mask)
+            x, rep = B.solve(rhs)
+            assert rep["rc"] == 0 and rep["fallback"] == 0, rep
+            assert rep["inner_total"] >= 5, rep
+            o, worst = 0, 0.0
+            for i, c in enumerate(circ):
+                if mask is None or mask[i]:
+                    v = x[o:o + c.n]
+                    r = c.rhs - np.bincount(c.row, c.val * v[c.col], c.n)
+                    worst = max(worst, np.linalg.norm(r) / np.linalg.norm(c.rhs))
+                o += c.n
+            assert worst <= 1e-9 and abs(worst - rep["max_rel_res"]) <= 1e-12 + 0.1 * worst, (worst, rep)
+    B.close()
