@@ -212,7 +212,8 @@ hipError_t k_start(const KrylovArgs &K, const double *r, int cyc, double *hist, 
 hipError_t k_chunk_dots(const KrylovArgs &K, int nv, hipStream_t s);
 hipError_t k_orth(const KrylovArgs &K, int j, bool first, hipStream_t s);
 hipError_t k_basis(const KrylovArgs &K, int j, const UnsetArgs &U, hipStream_t s);
-hipError_t k_update(const KrylovArgs &K, const double *Z, double *x, const int *gate, hipStream_t s);
+// steps: the most a matrix's cycle had
+hipError_t k_update(const KrylovArgs &K, const double *Z, double *x, int steps, const int *gate, hipStream_t s);
 hipError_t k_zero_int(int *p, long n, hipStream_t s);
 hipError_t k_copy(const double *src, double *dst, long n, hipStream_t s);
 

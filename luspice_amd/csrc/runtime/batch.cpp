@@ -1642,7 +1642,7 @@ int Batch::gmres_ir(const double *d_bv, double *d_xv, int prec, const std::vecto
             // once and do nothing while a circuit is still iterating, so one
             // host wait per iteration serves both
             const int *gate = d_nact_ + nact_word(cyc, j + 1);
-            LSP_HIP(k_update(K, d_Z_, d_xv, gate, s), "update");
+            LSP_HIP(k_update(K, d_Z_, d_xv, j + 1, gate, s), "update");
             LSP_TRY(launch_residual(K, d_bv, d_xv, cyc + 1, false, gate));
             LSP_TRY(read_status(lay.ticks, lay.end));
             if (status<int>(lay.abort)[1]) return LSP_E_DEVICE;
@@ -2052,7 +2052,7 @@ int Batch::record_step(int prec)
     LSP_TRY(launch_residual(K, d_bv, d_xv, 0, true, nullptr));
     const int mg = std::min(K.mmax, graph_inner(prec));
     for (int j = 0; j < mg; j++) LSP_TRY(launch_inner(K, prec, j, d_nact_ + nact_word(0, j)));
-    LSP_HIP(k_update(K, d_Z_, d_xv, nullptr, s), "update");
+    LSP_HIP(k_update(K, d_Z_, d_xv, mg, nullptr, s), "update");
     LSP_TRY(launch_residual(K, d_bv, d_xv, 1, false, nullptr));
 #undef LSP_TRY
 #undef LSP_HIP

@@ -53,3 +53,33 @@ def test_many_reduction_chunks(sizes, chunk, inner):
                 o += c.n
             assert worst <= 1e-9 and abs(worst - rep["max_rel_res"]) <= 1e-12 + 0.1 * worst, (worst, rep)
     B.close()
+
+
+@pytest.mark.parametrize("inner", [64, 65, 130])
+@pytest.mark.parametrize("chunk", [0, 16])
+def test_long_cycles(inner, chunk):
+    """Cycles of at most and of more than 64 steps (back substitution by the
+    update itself or by a launch of its own), beside a circuit that takes few.
+    Residuals as above; the second circuit's solution within 1e-6 of its own
+    solve (the pass line of every solution test here)."""
+    print("case: long cycles", inner, chunk, flush=True)
+    circ = [L.mna("sized", n=n, lr=0.02, seed=n) for n in (1500, 300)]
+    B = L.Batch(circ, chunk_rows=chunk, ir_inner=inner, ir_outer=60, factor_shift=0.1)
+    assert B.refactor("fp64")["rc"] == 0
+    rhs = np.concatenate([c.rhs for c in circ])
+    x, rep = B.solve(rhs)
+    assert rep["rc"] == 0 and rep["fallback"] == 0, rep
+    assert rep["inner_total"] > inner, rep            # a full cycle of `inner` steps, then another
+    o, worst = 0, 0.0
+    for c in circ:
+        v = x[o:o + c.n]
+        r = c.rhs - np.bincount(c.row, c.val * v[c.col], c.n)
+        worst = max(worst, np.linalg.norm(r) / np.linalg.norm(c.rhs))
+        o += c.n
+    assert worst <= 1e-9 and abs(worst - rep["max_rel_res"]) <= 1e-12 + 0.1 * worst, (worst, rep)
+    A = L.Batch(circ[1])
+    assert A.refactor("fp64")["rc"] == 0
+    y, _ = A.solve(circ[1].rhs)
+    assert np.linalg.norm(x[circ[0].n:] - y) <= 1e-6 * np.linalg.norm(y)
+    A.close()
+    B.close()
