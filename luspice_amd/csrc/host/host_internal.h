@@ -174,6 +174,21 @@ struct LspLocalSolve {
 };
 void lsp_plan_local_solve(const LspPlan &P, bool forward, LspLocalSolve &S);
 
+// Whether a circuit's solves can be one workgroup's: the vector fits 64 KB of
+// LDS (the backward solve holds all n values), and L and U have an entry (lanes
+// without one read entry 0).
+constexpr int kLocalRows = 8192;
+bool lsp_local_solve_fits(const LspPlan &P);
+
+// A pair of solves of one circuit, and which circuits of a batch are solved by
+// one workgroup each (the others through the task queue).
+struct LspSolveLoad {
+    long tasks = 0, levels = 0;
+    bool fits = false;
+};
+LspSolveLoad lsp_solve_load(const LspPlan &P, const LspLocalSolve (&S)[2]);
+std::vector<char> lsp_choose_local(const std::vector<LspSolveLoad> &circ);
+
 // Ruiz equilibration scales: after `sweeps` sweeps, R A C has every row and
 // column maximum close to 1 (used to pivot on the scaled matrix).
 void lsp_ruiz_scales(int n, long nnz, const int *row, const int *col, const double *val, int sweeps,

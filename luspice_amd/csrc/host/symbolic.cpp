@@ -588,6 +588,58 @@ void lsp_plan_local_solve(const LspPlan &P, bool forward, LspLocalSolve &S)
     S.wave.push_back((int)(S.task.size() / 4));
 }
 
+bool lsp_local_solve_fits(const LspPlan &P)
+{
+    return P.n <= kLocalRows && P.tail_k0 > 0 && P.n_l > 0 && P.n_u > 0;
+}
+
+LspSolveLoad lsp_solve_load(const LspPlan &P, const LspLocalSolve (&S)[2])
+{
+    LspSolveLoad L;
+    L.tasks = (long)(P.fwd_task.size() + P.bwd_task.size());
+    L.fits = S[0].nlev + S[1].nlev > 0;
+    if (L.fits) {
+        L.levels = S[0].nlev + S[1].nlev;
+    } else {
+        for (const std::vector<int> *key : {&P.fwd_key, &P.bwd_key})
+            for (size_t t = 0; t < key->size(); t++) L.levels += t == 0 || (*key)[t] != (*key)[t - 1];
+    }
+    return L;
+}
+
+// Estimates of a pair of solves: one workgroup takes 0.64 us a level or 0.17 us a
+// task, whichever is more, 256 of them at a time; the queue 0.95 us a level of
+// the deepest circuit or 1 us per 200 tasks of all.  The two kinds run one after
+// the other, so it is all circuits that fit or none.  Measured on 130 batches
+// (one to 256 circuits of 100 to 8000 unknowns, copies and mixed sizes) the pair
+// chosen takes 0.2 % more than the faster one on average and 6 % at most.  Some of
+// them, one workgroup each / queue, fp32, us: one circuit of 1000 unknowns 115 /
+// 133, of 5000 262 / 215, of 8000 449 / 288; 36 copies of 8000 591 / 584, 64
+// 648 / 937; 24 circuits of 100 to 5000 291 / 232, 64 294 / 270, 128 324 / 342,
+// 256 345 / 515.  (A limit on each circuit's own tasks sent some to either kind:
+// those 24 and 64 took 381 and 423.)
+std::vector<char> lsp_choose_local(const std::vector<LspSolveLoad> &circ)
+{
+    double one = 0.0, sum = 0.0;
+    long levels[2] = {0, 0}, tasks[2] = {0, 0};          // of all circuits, of those that do not fit
+    for (const LspSolveLoad &C : circ) {
+        const double t = std::max(0.64 * (double)C.levels, 0.17 * (double)C.tasks);
+        if (C.fits) {
+            one = std::max(one, t);
+            sum += t;
+        }
+        for (int k = 0; k < (C.fits ? 1 : 2); k++) {
+            levels[k] = std::max(levels[k], C.levels);
+            tasks[k] += C.tasks;
+        }
+    }
+    auto queue = [&](int k) { return std::max(0.95 * (double)levels[k], 0.005 * (double)tasks[k]); };
+    const bool on = std::max(one, sum / 256.0) + queue(1) < queue(0);
+    std::vector<char> pick(circ.size(), 0);
+    for (size_t m = 0; m < circ.size(); m++) pick[m] = on && circ[m].fits;
+    return pick;
+}
+
 // ---------------------------------------------------------------------------
 // dense trailing block
 // ---------------------------------------------------------------------------

@@ -31,10 +31,6 @@ static_assert(kTriPacket == ::kTriPacketBase && kTriPacketLane == ::kTriPacketPe
               "packet layout of the plan and the solve kernel");
 static_assert(kLocalSolveWaves == ::kLocalWaves, "waves of a one-workgroup solve");
 
-// Circuits of at most this many unknowns may be solved by one workgroup each
-// (their vector is 64 KB of LDS).
-constexpr int kLocalRows = 8192;
-
 
 Batch::~Batch()
 {
@@ -294,8 +290,7 @@ static int build_circuit(CircuitHost &C, const lsp_circuit_in &in, const lsp_opt
         const double tden = opt.tail_density > 0 ? opt.tail_density : 0.5;
         if (tmax > 0 && lsp_plan_set_tail(C.plan, 64, tmax, tden) < 0) return LSP_E_STRUCTURE;
     }
-    // (the solves read entry 0 of L and U where a lane has none)
-    if (C.n <= kLocalRows && C.plan.tail_k0 > 0 && C.plan.n_l > 0 && C.plan.n_u > 0)
+    if (lsp_local_solve_fits(C.plan))
         for (int d = 0; d < 2; d++) lsp_plan_local_solve(C.plan, d == 0, C.local[d]);
     std::vector<int> rp, ci, rsrc;
     lsp_coo_to_csr(C.n, C.nnz, C.row.data(), C.col.data(), rp, ci, rsrc);
@@ -304,21 +299,12 @@ static int build_circuit(CircuitHost &C, const lsp_circuit_in &in, const lsp_opt
     return ir_level_lists(C);
 }
 
-// Which circuits' triangular solves are one workgroup's (localsolve.hip).  Per
-// pair of solves that takes 0.64 us a level or 0.16 us a task, whichever is
-// more; the task queue takes 0.95 us a level or, for all circuits together, 1 us
-// per 190 tasks.  Measured (fp64, us, one workgroup / queue): n = 200, 87 levels
-// and 124 tasks, 56 / 81; n = 1020, 88 and 285, 53 / 58; n = 4999, 160 and 1230,
-// 192 / 156; 512 circuits of 100 to 5000 unknowns, 165 000 tasks, 450 / 960.
 static void choose_local(std::vector<CircuitHost> &circ)
 {
-    auto tasks = [](const CircuitHost &C) { return (long)(C.plan.fwd_task.size() + C.plan.bwd_task.size()); };
-    long total = 0;
-    for (const CircuitHost &C : circ) total += tasks(C);
-    for (CircuitHost &C : circ) {
-        const long levels = C.local[0].nlev + C.local[1].nlev;
-        C.local_on = levels > 0 && tasks(C) <= std::max(6 * levels, total / 30);
-    }
+    std::vector<LspSolveLoad> load;
+    for (const CircuitHost &C : circ) load.push_back(lsp_solve_load(C.plan, C.local));
+    const std::vector<char> on = lsp_choose_local(load);
+    for (size_t m = 0; m < circ.size(); m++) circ[m].local_on = on[m];
 }
 
 template <typename T>
