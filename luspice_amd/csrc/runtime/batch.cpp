@@ -155,6 +155,9 @@ X *Batch::upload(const std::vector<X> &v)
     return d;
 }
 
+// Rows of a reduction chunk of the GMRES kernels.
+constexpr int kChunkRows = 512;
+
 // Results of at most this many bytes go to the host by export_kernel; a larger
 // one is a copy, whose rate counts more than its latency.
 constexpr size_t kStageBytes = 256 * 1024;
@@ -496,36 +499,45 @@ int Batch::set_active(const int *mask)
 // (an upper estimate used for admission; device_bytes() reports the actual).
 size_t Batch::estimate_device_bytes() const
 {
-    double n = 0, nnz = 0, slots = 0, rel = 0, deps = 0, local = 0, nlu = 0, sell = 0, slices = 0, T = 0, T2 = 0, lists = 0, tiles = 0;
-    double maxcol = 0;
     const double nc = (double)circ_.size();
+    const double m = std::max(1, opt_.ir_inner);
+    const int cr = opt_.chunk_rows > 0 ? opt_.chunk_rows : kChunkRows;
+    double n = 0, nnz = 0, slots = 0, rel = 0, nlu = 0, sell = 0, slices = 0, T = 0, T2 = 0, chunks = 0, blocks = 0;
+    double b = 0, maxcol = 0;
     for (const auto &C : circ_) {
         const LspPlan &P = C.plan;
         n += C.n; nnz += C.nnz; slots += (double)P.cp[C.n]; rel += (double)P.relp[C.n];
-        deps += (double)P.dep.size();
-        for (const LspLocalSolve &S : C.local) local += (double)(S.task.size() + S.rec.size() + S.wave.size());
         nlu += (double)(P.n_l + P.n_u); sell += (double)C.sell.slots; slices += C.sell.nslices;
         T += P.tail_T; T2 += (double)P.tail_T * P.tail_T;
-        const double nt = (P.tail_T + 63) / 64;                           // tiles, their packed copies and inverses
-        lists += 2 * nt * nt + P.tail_T / 4 + 8 * nt;
-        tiles += nt * nt + 2 * nt;
+        chunks += (C.n + cr - 1) / cr;
+        blocks += (C.sell.nslices + 3) / 4;
         maxcol = std::max(maxcol, (double)P.max_col);
+        b += 8.0 * (double)P.dep.size();
+        for (const LspLocalSolve &S : C.local) b += 4.0 * (double)(S.task.size() + S.rec.size() + S.wave.size());
+        b += 4.0 * (double)(P.fpk.size() + P.bpk.size() + P.twide.size() + C.flvp.size() + C.blvp.size());
+        b += 8.0 * (double)(P.fwd_task.size() + P.bwd_task.size());
+        // dense block: packed tiles, the panels' operands, flags, task lists
+        const double nt = (P.tail_T + 63) / 64;
+        b += 8.0 * 64 * 64 * (nt * nt + 2 * nt) + 4 * nt * nt + 16 * nt * nt + 8 * (0.27 * P.tail_T + 3);
+        b += 8 * ((double)P.cp[P.tail_k0] / kFillSlots + 1);               // unset fill
     }
-    const double m = std::max(1, opt_.ir_inner);
-    double b = 0;
-    b += 8 * (n + nc) + 4 * n + 8 * slots + 8 * nnz + 8 * deps;          // cp dp pos dst asrc aslot dep
+    b += 8 * (n + nc) + 4 * n + 8 * slots + 8 * nnz;                      // cp dp pos dst asrc aslot
     b += 8 * (n + nc) + 4 * nlu + 24 * n + 2 * rel;                       // lrp urp lci uci rowat q snend ru fcut bcut rel
-    b += 8 * (slices + nc) + 8 * n + 8 * sell;                            // SELL structure
-    b += 12 * n + 8 * nnz + 12 * sell;                                    // flags, values
-    b += 4 * local + 4 * nc;                                              // one-workgroup solves
+    b += 12 * n;                                                          // dpos, fused IR step's rows by level
+    b += 8 * (slices + nc) + 8 * n + 8 * sell + 8 * slices;               // SELL structure, slice tasks
+    b += 4 * n + 8 * nnz + 12 * sell;                                     // flags, values
     if (opt_.krylov_spmv == 2) b += 2 * sell;                              // FP16 SELL values
     b += 16 * nnz + 24 * n + 16 * (nc + 1);                               // Ruiz: row/col, scaled values, scales
     if (opt_.factor_shift > 0.0) b += 8 * n;                               // shifted diagonal entries
-    b += 16 * T + 8.0 * 64 * 64 * tiles;                                   // dense block work
-    b += (sizeof(FactorTask) + 16) * n + 8 * slices + 16 * n;             // task lists, row packets
-    b += 8 * lists + 8 * (slots / kFillSlots + nc);                       // dense-block and fill work lists
-    b += 64 * n + 8 * (2 * m + 1) * n;                                    // vectors, Krylov bases V and Z
+    b += 16 * T;                                                          // dense block columns and rows
+    b += sizeof(FactorTask) * n;                                          // refactor tasks
+    b += 80 * n + 8 * (2 * m + 1) * n;                                    // vectors, Krylov bases V and Z
+    b += 16 * chunks + (16 * (m + 1) + 8) * chunks + (8 + 8 * kSpmvDots) * blocks;   // reduction parts
+    b += 8 * nc * ((m + 1) * m + 2 * (m + 1) + 3 * m);                    // Hessenberg matrices and what goes with them
     b += (4 + 8) * (slots + nlu + n) + (8 + 4 + 8) * T2;                   // fp32 + fp64 factor sets
+    // descriptors (both sets, SELL, dense jobs), status and state words
+    b += nc * (2 * (sizeof(FactorDesc<double>) + sizeof(TriDesc<double>) + sizeof(IrDesc<double>) + sizeof(DenseJob)) +
+               3 * sizeof(SellDesc<double>) + 4 * kMstat + 128);
     if (maxcol > std::max(1, opt_.lds_cap)) b += 256.0 * 8 * 4 * maxcol * 8;   // global column scratch
     return (size_t)(1.05 * b) + (1u << 20);
 }
@@ -990,7 +1002,7 @@ int Batch::upload_all()
         std::vector<long> voff(nc);
         std::vector<int4> chunks;
         std::vector<int> cbeg(nc + 1, 0);
-        int cr = opt_.chunk_rows > 0 ? opt_.chunk_rows : 512;
+        const int cr = opt_.chunk_rows > 0 ? opt_.chunk_rows : kChunkRows;
         for (int m = 0; m < nc; m++) {
             voff[m] = circ_[m].voff;
             cbeg[m] = (int)chunks.size();
