@@ -2,11 +2,11 @@
 //
 // Conventions
 //   * wave64 everywhere: lane = threadIdx.x & 63, wave = threadIdx.x >> 6.
-//   * Cross-workgroup hand-off uses epoch-tagged flags: a producer stores
-//     flag[i] = epoch with release semantics at agent scope after its data
-//     stores; a consumer spins on an acquire load until flag[i] == epoch.
-//     Epochs increase per launch, so flags never need clearing.
-//   * Every spin is bounded: after kSpinLimit polls the waiter raises the
+//   * Cross-workgroup hand-off is by data stored and loaded coherently, seen
+//     either by an epoch-tagged flag (stored once the data is acknowledged;
+//     epochs increase per launch, so flags never need clearing) or by the
+//     values themselves (unset before the launch).
+//   * Every spin is bounded: after kRoundLimit polls the waiter raises the
 //     shared abort word, every other waiter sees it and leaves, and the kernel
 //     drains normally.  The host reports the abort as an error.
 #pragma once
@@ -37,31 +37,12 @@ template <typename T> __device__ __forceinline__ const LSP_GLOBAL T *gp(const T 
 }
 
 constexpr int kWave = 64;
-constexpr int kSpinLimit = 1 << 22;   // ~ seconds with s_sleep(1) between polls
 
 __device__ __forceinline__ int lane_id() { return threadIdx.x & (kWave - 1); }
 
-__device__ __forceinline__ int ld_acquire(const int *p)
-{
-    return __hip_atomic_load(gp(p), __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
-}
 __device__ __forceinline__ int ld_relaxed(const int *p)
 {
     return __hip_atomic_load(gp(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-// Read-modify-write probes are performed at the device coherence point, so a
-// flag written by a wave on another XCD is seen whatever a local cache holds.
-__device__ __forceinline__ int ld_coherent(int *p)
-{
-    return __hip_atomic_fetch_add(p, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void publish(int *p, int v)
-{
-    __hip_atomic_exchange(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void st_release(int *p, int v)
-{
-    __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ void st_relaxed(int *p, int v)
 {
@@ -266,14 +247,6 @@ __device__ __forceinline__ void wave_fence()
     __builtin_amdgcn_wave_barrier();
 }
 
-// Orders this wave's earlier LDS / global accesses before its later ones as
-// seen by other lanes of the same wave.
-__device__ __forceinline__ void wave_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-}
-
 // Wave-collective wait: every lane whose flag pointer is non-null waits until
 // *flag == epoch; returns true once all of them have seen it, false when the
 // wait was abandoned (round limit hit here, or the abort word raised
@@ -284,30 +257,18 @@ __device__ __forceinline__ void wave_sync()
 // per round (an acquire load would also invalidate the cache on every poll);
 // rounds back off exponentially up to ~1 us.  Hundreds of waves polling every
 // few hundred cycles with all lanes saturate the memory path the producers
-// need, and the factorization then crawls.  The caller issues one
-// acquire_fence() after a successful wait.
-
-__device__ __forceinline__ bool wave_wait(const int *flag, int epoch, int *abort_word,
-                                          int *dbg = nullptr, int who2 = -1, int max_backoff = 7)
+// need, and the factorization then crawls.  What the flags announce is stored and
+// loaded coherently, so no fence follows (see st_coherent).
+__device__ __forceinline__ bool wave_wait(const int *flag, int epoch, int *abort_word, int max_backoff)
 {
-    int seen = flag ? -1 : epoch;
     int ok = flag == nullptr;
     int backoff = 0;
     for (int round = 0;; round++) {
-        if (!ok) {
-            seen = ld_relaxed(flag);
-            ok = seen == epoch;
-        }
+        if (!ok) ok = ld_relaxed(flag) == epoch;
         if (__all(ok)) return true;
         if ((round & 15) == 15 && aborted(abort_word)) return false;
         if (round > kRoundLimit) {
-            if (!ok && atomicCAS(abort_word, 0, kErrSpin) == 0 && dbg) {
-                dbg[1] = seen;
-                dbg[2] = epoch;
-                dbg[3] = round;
-                dbg[4] = who2;
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-            }
+            if (!ok) atomicCAS(abort_word, 0, kErrSpin);
             return false;
         }
         for (int s = 0; s <= backoff; s++) __builtin_amdgcn_s_sleep(4);
@@ -412,12 +373,6 @@ __device__ __forceinline__ bool wave_wait_value(const double *p, double &v, int 
     return ok;
 }
 
-// Makes data published before the observed flags visible to this wave.
-__device__ __forceinline__ void acquire_fence()
-{
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-}
-
 // wave64 reductions (DPP / permute lowered by the compiler from shuffles)
 __device__ __forceinline__ double wave_sum(double v)
 {
@@ -458,13 +413,6 @@ __device__ __forceinline__ int splu_pivot_verdict(bool diag_pivot, double pv, do
     }
     if (pv > lmax * (1.0 + eps)) return 0;              // the unique maximum
     return pv < lmax * (1.0 - eps) ? 1 : 2;             // smaller, or a tie broken by reach order
-}
-
-__device__ __forceinline__ int wave_min_int(int v)
-{
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = min(v, __shfl_xor(v, off, kWave));
-    return v;
 }
 
 template <typename T> __device__ __forceinline__ double to_f64(T v) { return (double)v; }

@@ -432,8 +432,7 @@ __global__ void __launch_bounds__(256, 2) dense_lu_kernel(const DenseJob *jobs, 
             continue;
         }
         // the panel's triangle from the left, by groups of four rows
-        ok = ok && wave_wait(lane == 0 ? &ready[(size_t)q * (nt + 1)] : nullptr, epoch, abort_word, nullptr, -1,
-                             kSolveBackoff);
+        ok = ok && wave_wait(lane == 0 ? &ready[(size_t)q * (nt + 1)] : nullptr, epoch, abort_word, kSolveBackoff);
         if (ok) {
             const LSP_GLOBAL double *wp = gp(J.W) + (size_t)q * 2 * kTile + (low ? kTile : 0) + lk * kNb + li;
             double w[16][4];

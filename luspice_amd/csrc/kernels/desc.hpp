@@ -84,7 +84,6 @@ struct FactorDesc {
                             // columns whose pivot splu would not pick, columns
                             // too close to call, first of either, pad
     // dense trailing block (tail_T = 0: none, tail_k0 = n)
-    const int *tail_ds;     // tail_T: sparse dependencies of tail column c
     double *tail_S;         // tail_T^2 fp64 work block, column-major
     unsigned long long *tail_colmax;   // tail_T: max |L(i,c)| as bit patterns
     T *tail_F;              // tail_T^2 factor in storage precision (tail_S itself for fp64)
@@ -118,7 +117,7 @@ struct TriDesc {
     const int *tail_lcut;   // tail_T: end of the sparse part of L row tail_k0 + r
     int *tail_ctr;          // 4 ints: block ticket counter, exit counter, pad
     // one-workgroup solve, forward and backward: first task per wave, tasks
-    // and records of four ints each, levels (null: solved by the task queue)
+    // and records of four ints each, levels (of the circuits solved that way)
     const int *lwave[2], *ltask[2], *lrec[2];
     int lnlev[2];
     int n;
@@ -168,16 +167,6 @@ struct IrDesc {
     const int *brow, *blvp; // the same for the backward solve
     long voff;              // first entry of the circuit in the vector arenas
     int n, tail_k0, tail_T, nlv_f, nlv_b, pad_;
-};
-
-// Status words written by the persistent kernels.
-struct KStatus {
-    int abort_code;         // kErr* (0 = none)
-    int bad_pivot_count;    // columns whose pivot failed the tolerance test
-    int first_bad_pivot;    // smallest failing column (INT_MAX if none)
-    int first_singular;     // smallest column with a zero pivot (INT_MAX)
-    int bad_matrix;         // matrix index of the first failure (-1)
-    int pad_[3];
 };
 
 }  // namespace lsp

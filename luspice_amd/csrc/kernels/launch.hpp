@@ -195,8 +195,7 @@ hipError_t launch_solve_unset(const TriLaunch &L, long n, hipStream_t st);
 // spmv.hip
 template <typename V>
 hipError_t launch_sell_spmv(const SellDesc<V> *mats, const int2 *tasks, int ntask,
-                            const int64_t *voff, const double *x, double *y, const double *b,
-                            const int *active, hipStream_t st);
+                            const int64_t *voff, const double *x, double *y, hipStream_t st);
 hipError_t launch_csr_spmv(int n, const int *rowptr, const int *colidx, const double *values,
                            const double *x, double *y, hipStream_t st);
 hipError_t launch_csr_spmv_f32(int n, const int *rowptr, const int *colidx, const float *values,

@@ -10,9 +10,9 @@
 //   Reference layout: src/sellc_spmv.cu:170-257 (C = 32, one warp per slice,
 //   y returned in slice order and permuted on the host at
 //   bench/test_lu_gpu_f32.cu:196-199); here y is written straight to the
-//   original row through perm.  Value type V = double, float or __half,
+//   original row through perm.  Value type V = double or float (the products of
+//   GMRES, sell_block_kernel, also __half),
 //   accumulation always fp64 (src/mp/fp16_spmv.cu:50-59 pattern).
-//   With b != nullptr the kernel writes the residual b - A x instead.
 //   Batched: tasks are (matrix, slice) pairs over any number of matrices;
 //   vectors of matrix m start at voff[m] in the shared arenas.
 //
@@ -28,15 +28,13 @@ constexpr int kSpmvBatch = 8;           // slots of a row loaded per round
 template <typename V>
 __global__ void __launch_bounds__(256)
 sell_spmv_kernel(const SellDesc<V> *mats, const int2 *tasks, int ntask,
-                 const int64_t *voff, const double *x, double *y, const double *b,
-                 const int *active)
+                 const int64_t *voff, const double *x, double *y)
 {
     // the task index is wave-uniform: readfirstlane lets the task and its
     // descriptor come through scalar loads
     const int t = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
     if (t >= ntask) return;
     const int2 tk = tasks[t];
-    if (active && !active[tk.x]) return;
     const SellDesc<V> M = mats[tk.x];
     const int lane = lane_id();
     const int k = tk.y * kWave + lane;
@@ -46,7 +44,6 @@ sell_spmv_kernel(const SellDesc<V> *mats, const int2 *tasks, int ntask,
     const int len = M.rlen[k];
     const int64_t base = M.off[tk.y] + lane;
     const int row = M.perm[k];
-    const double bi = b ? b[vo + row] : 0.0;
     // kSpmvBatch slots per round: every value and column id of the round is
     // loaded, then every x entry, then the products are added in slot order
     // (the same sum as one slot at a time), so a row of up to kSpmvBatch
@@ -68,7 +65,7 @@ sell_spmv_kernel(const SellDesc<V> *mats, const int2 *tasks, int ntask,
         for (int u = 0; u < kSpmvBatch; u++)
             if (j0 + u < len) s += to_f64(v[u]) * xv[u];
     }
-    y[vo + row] = b ? bi - s : s;
+    y[vo + row] = s;
 }
 
 // The products of a GMRES cycle, one workgroup per four slices of one matrix;
@@ -199,24 +196,18 @@ __global__ void gather_cast_kernel(long count, const int *idx, const double *in,
 
 template <typename V>
 hipError_t launch_sell_spmv(const SellDesc<V> *mats, const int2 *tasks, int ntask,
-                            const int64_t *voff, const double *x, double *y, const double *b,
-                            const int *active, hipStream_t st)
+                            const int64_t *voff, const double *x, double *y, hipStream_t st)
 {
     if (ntask <= 0) return hipSuccess;
     const int blocks = (ntask + 3) / 4;
     hipLaunchKernelGGL(sell_spmv_kernel<V>, dim3(blocks), dim3(256), 0, st, mats, tasks, ntask,
-                       voff, x, y, b, active);
+                       voff, x, y);
     return hipGetLastError();
 }
 template hipError_t launch_sell_spmv<double>(const SellDesc<double> *, const int2 *, int,
-                                             const int64_t *, const double *, double *,
-                                             const double *, const int *, hipStream_t);
+                                             const int64_t *, const double *, double *, hipStream_t);
 template hipError_t launch_sell_spmv<float>(const SellDesc<float> *, const int2 *, int,
-                                            const int64_t *, const double *, double *,
-                                            const double *, const int *, hipStream_t);
-template hipError_t launch_sell_spmv<__half>(const SellDesc<__half> *, const int2 *, int,
-                                             const int64_t *, const double *, double *,
-                                             const double *, const int *, hipStream_t);
+                                            const int64_t *, const double *, double *, hipStream_t);
 
 hipError_t launch_csr_spmv(int n, const int *rowptr, const int *colidx, const double *values,
                            const double *x, double *y, hipStream_t st)

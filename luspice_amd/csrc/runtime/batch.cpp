@@ -351,7 +351,6 @@ int Batch::ensure_factor_set(FactorSet<T> &fs)
         F.done = d_done_ + C.o_n;
         F.mstat = d_mstat_ + kMstat * m;
         F.n = C.n;
-        F.tail_ds = d_tail_ds_ + C.o_t;
         F.tail_S = fs.tailS + C.o_t2;
         F.tail_colmax = d_colmax_ + C.o_t;
         F.tail_F = fs.tailF + C.o_t2;
@@ -529,9 +528,9 @@ size_t Batch::estimate_device_bytes() const
     if (opt_.krylov_spmv == 2) b += 2 * sell;                              // FP16 SELL values
     b += 16 * nnz + 24 * n + 16 * (nc + 1);                               // Ruiz: row/col, scaled values, scales
     if (opt_.factor_shift > 0.0) b += 8 * n;                               // shifted diagonal entries
-    b += 16 * T;                                                          // dense block columns and rows
+    b += 12 * T;                                                          // dense block columns and rows
     b += sizeof(FactorTask) * n;                                          // refactor tasks
-    b += 80 * n + 8 * (2 * m + 1) * n;                                    // vectors, Krylov bases V and Z
+    b += 72 * n + 8 * (2 * m + 1) * n;                                    // vectors, Krylov bases V and Z
     b += 16 * chunks + (16 * (m + 1) + 8) * chunks + (8 + 8 * kSpmvDots) * blocks;   // reduction parts
     b += 8 * nc * ((m + 1) * m + 2 * (m + 1) + 3 * m);                    // Hessenberg matrices and what goes with them
     b += (4 + 8) * (slots + nlu + n) + (8 + 4 + 8) * T2;                   // fp32 + fp64 factor sets
@@ -551,7 +550,7 @@ size_t Batch::device_bytes() const
 
 // Device phase: concatenates the circuits' structures and uploads them.
 // Also the second half of a rebuild (release_device first): the stream,
-// events, pinned words and the b / x arenas are kept.
+// pinned memory and the b / x arenas are kept.
 int Batch::upload_all()
 {
     if (circ_.empty() || uploaded_) return LSP_E_ARG;
@@ -729,12 +728,11 @@ int Batch::upload_all()
     }
     // dense trailing blocks, the jobs by falling order T
     {
-        std::vector<int> tds, tlc;
+        std::vector<int> tlc;
         d_colmax_ = (unsigned long long *)dalloc(nt_tot_ * sizeof(unsigned long long));
         std::vector<int> mat, order;
         for (int m = 0; m < nc; m++) {
             const LspPlan &P = circ_[m].plan;
-            tds.insert(tds.end(), P.tail_ds.begin(), P.tail_ds.end());
             tlc.insert(tlc.end(), P.tail_lcut.begin(), P.tail_lcut.end());
             if (P.tail_T > 0) mat.push_back(m);
         }
@@ -777,7 +775,6 @@ int Batch::upload_all()
         dgrid_.npivot = (int)H.pivot.size();
         dgrid_.ngather = (int)H.gather.size();
         dgrid_.ntrsv = (int)H.trsv.size();
-        d_tail_ds_ = upload(tds);
         d_tail_lcut_ = upload(tlc);
         d_tail_ctr_ = upload(std::vector<int>(4 * nc, 0));
         std::vector<int2> fill;
@@ -788,7 +785,7 @@ int Batch::upload_all()
         }
         d_fillchunk_ = upload(fill);
         nfillchunk_ = (int)fill.size();
-        if (!d_tail_ds_ || !d_tail_lcut_ || !d_tail_ctr_ || !d_fillchunk_ || !dgrid_.lu ||
+        if (!d_tail_lcut_ || !d_tail_ctr_ || !d_fillchunk_ || !dgrid_.lu ||
             !dgrid_.pivot || !dgrid_.gather || !dgrid_.trsv)
             return LSP_E_ALLOC;
     }
@@ -956,7 +953,7 @@ int Batch::upload_all()
             const size_t lds_cu = 160 * 1024;
             per_cu = (int)std::max<size_t>(1, std::min<size_t>(8, lds_cu / lds));
         }
-        // Waves beyond the widest dependency level only poll; size each
+        // Waves beyond the most tasks of one queue key only poll; size each
         // persistent grid to about twice that width (4 waves per block), but to
         // 128 blocks at least while there are tasks for them: a task held early
         // has its loads done when its turn comes (refactor of 200 unknowns 125
@@ -996,7 +993,7 @@ int Batch::upload_all()
         if (!d_b_) d_b_ = (double *)dalloc(ntot_ * 8);     // kept by a rebuild (with their contents)
         if (!d_x_) d_x_ = (double *)dalloc(ntot_ * 8);
         d_r_ = (double *)dalloc(ntot_ * 8); d_w_ = (double *)dalloc(ntot_ * 8);
-        d_z_ = (double *)dalloc(ntot_ * 8); d_t_ = (double *)dalloc(ntot_ * 8);
+        d_t_ = (double *)dalloc(ntot_ * 8);
         d_ty_ = (double *)dalloc(ntot_ * 8); d_tz_ = (double *)dalloc(ntot_ * 8);
         d_typ_ = (double *)dalloc(ntot_ * 8); d_tzp_ = (double *)dalloc(ntot_ * 8);
         std::vector<long> voff(nc);
@@ -1040,7 +1037,7 @@ int Batch::upload_all()
         d_act_ = (int *)dalloc(nc * 4);
         d_conv_ = (int *)dalloc(nc * 4); d_cycled_ = (int *)dalloc(nc * 4);
         d_subset_ = (int *)dalloc(nc * 4);
-        if (!d_b_ || !d_x_ || !d_r_ || !d_w_ || !d_z_ || !d_t_ || !d_ty_ || !d_tz_ || !d_typ_ || !d_tzp_ ||
+        if (!d_b_ || !d_x_ || !d_r_ || !d_w_ || !d_t_ || !d_ty_ || !d_tz_ || !d_typ_ || !d_tzp_ ||
             !d_voff_ || !d_chunks_ || !d_cbeg_ || !d_act_ || !d_conv_ || !d_cycled_ || !d_subset_)
             return LSP_E_ALLOC;
         if (!h_pin_) {
@@ -1065,7 +1062,7 @@ int Batch::upload_all()
 // Frees every device array of the batch except the b / x arenas (callers may
 // hold their addresses, and b carries the caller's right-hand sides) and
 // resets the derived sizes; upload_all() then rebuilds from circ_.  The
-// stream, events and pinned host words stay.
+// stream and pinned host memory stay.
 void Batch::release_device()
 {
     if (stream_) (void)hipStreamSynchronize(stream_);
@@ -1482,12 +1479,6 @@ int Batch::launch_trisolve_prec(int prec, const double *d_b, double *d_x, const 
     return LSP_E_ARG;
 }
 
-int Batch::launch_spmv64(const double *d_xv, double *d_y, const double *d_bv, const int *active)
-{
-    return check(launch_sell_spmv<double>(d_sdesc64_, d_stask_, nstask_, (const int64_t *)d_voff_,
-                                          d_xv, d_y, d_bv, active, stream_), "spmv");
-}
-
 int Batch::trisolve(const double *b, double *x, bool on_device)
 {
     if (cur_prec_ < 0) return LSP_E_ARG;
@@ -1543,10 +1534,11 @@ int Batch::spmv(const double *x, double *y, bool on_device, int prec)
         dy = d_w_;
     }
     if (prec == LSP_PREC_FP32)
-        rc = check(launch_sell_spmv<float>(d_sdesc32_, d_stask_, nstask_, (const int64_t *)d_voff_,
-                                           dx, dy, nullptr, nullptr, stream_), "spmv32");
+        rc = check(launch_sell_spmv<float>(d_sdesc32_, d_stask_, nstask_, (const int64_t *)d_voff_, dx, dy, stream_),
+                   "spmv32");
     else
-        rc = launch_spmv64(dx, dy, nullptr, nullptr);
+        rc = check(launch_sell_spmv<double>(d_sdesc64_, d_stask_, nstask_, (const int64_t *)d_voff_, dx, dy, stream_),
+                   "spmv");
     if (rc) return rc;
     return on_device ? finish() : fetch(d_w_, y);
 }

@@ -88,7 +88,7 @@ struct DeviceArrays {
     int *d_llist_ = nullptr;             // their circuits, most tasks first
     int nlocal_ = 0, local_rows_ = 0;    // count, most unknowns of one
     int *d_fpk_ = nullptr, *d_bpk_ = nullptr, *d_twide_ = nullptr;
-    double *d_tailW_ = nullptr, *d_tailP_ = nullptr;   // diagonal-block inverses, packed tiles
+    double *d_tailW_ = nullptr, *d_tailP_ = nullptr;   // diagonal blocks' operands, packed tiles
     // Ruiz equilibration (FP16 factor storage)
     int *d_arow_ = nullptr, *d_acol_ = nullptr;
     long *d_raoff_ = nullptr, *d_rvoff_ = nullptr;
@@ -106,8 +106,8 @@ struct DeviceArrays {
     int2 *d_fwtask_ = nullptr, *d_bwtask_ = nullptr, *d_stask_ = nullptr;
     long nslot_tot_ = 0, nl_tot_ = 0, nu_tot_ = 0, nsell_tot_ = 0;
     int nstask_ = 0;
-    int *d_ctr_ = nullptr;               // [0..1] factor, [2..3] fwd, [4..5] bwd
-    int *d_epoch_ = nullptr;             // epoch counters: [0] factor, [1] fwd, [2] bwd
+    int *d_ctr_ = nullptr;               // queue blocks (kQueueInts each): refactor, forward, backward, dense block
+    int *d_epoch_ = nullptr;             // epoch counters: [0] refactor, [1] dense block
     int *d_abort_ = nullptr;             // [0] factor, [1] trisolve (in the status block)
     int *d_mstat_ = nullptr;             // kMstat per circuit (in the status block)
     unsigned *d_exp_ = nullptr;          // workgroups done of a running export
@@ -118,9 +118,9 @@ struct DeviceArrays {
     long scratch_stride_ = 0;
     int fblocks_ = 0, tblocks_f_ = 0, tblocks_b_ = 0;
     int nq_f_ = 1, nq_t_ = 1;                          // queue counters: refactor, solves
-    long width_f_ = 0, width_tf_ = 0, width_tb_ = 0;   // widest merged level
+    long width_f_ = 0, width_tf_ = 0, width_tb_ = 0;   // most tasks of one key in the merged lists
     // dense trailing blocks
-    int *d_tail_ds_ = nullptr, *d_tail_lcut_ = nullptr, *d_tail_ctr_ = nullptr;
+    int *d_tail_lcut_ = nullptr, *d_tail_ctr_ = nullptr;
     unsigned long long *d_colmax_ = nullptr;
     int *d_dflag_ = nullptr;                   // per tile of every dense job: epoch of the launch that made it final
     std::vector<DenseJob> jobs_;               // without their work blocks (ensure_factor_set)
@@ -135,7 +135,7 @@ struct DeviceArrays {
     FactorSet<__half> f16_;
     // vectors and Krylov state
     double *d_b_ = nullptr, *d_x_ = nullptr, *d_r_ = nullptr, *d_w_ = nullptr,
-           *d_z_ = nullptr, *d_t_ = nullptr, *d_ty_ = nullptr, *d_tz_ = nullptr, *d_typ_ = nullptr,
+           *d_t_ = nullptr, *d_ty_ = nullptr, *d_tz_ = nullptr, *d_typ_ = nullptr,
            *d_tzp_ = nullptr, *d_V_ = nullptr,
            *d_Z_ = nullptr;
     int2 *d_sblock_ = nullptr;           // (matrix, first slice) of the GMRES products' workgroups
@@ -242,7 +242,6 @@ public:
     // unset: the solves' work values are to be set to the unset marker first
     int launch_trisolve_prec(int prec, const double *d_b, double *d_x, const int *active,
                              const int *d_nact = nullptr, bool unset = true);
-    int launch_spmv64(const double *d_x, double *d_y, const double *d_b, const int *active);
     hipStream_t stream() const { return stream_; }
     int cur_prec() const { return cur_prec_; }
     std::string last_error;

@@ -144,10 +144,10 @@ int main(int argc, char **argv)
     auto csr64 = [&]() { CK(lsp::launch_csr_spmv(n, d_rp, d_ci, d_v64, d_x, d_y64, 0)); };
     auto csr32 = [&]() { CK(lsp::launch_csr_spmv_f32(n, d_rp, d_ci, d_v32, d_x, d_y32, 0)); };
     auto sel64 = [&]() {
-        CK(lsp::launch_sell_spmv<double>(d_D64, d_tasks, S.nslices, d_voff, d_x, d_y64, nullptr, nullptr, 0));
+        CK(lsp::launch_sell_spmv<double>(d_D64, d_tasks, S.nslices, d_voff, d_x, d_y64, 0));
     };
     auto sel32 = [&]() {
-        CK(lsp::launch_sell_spmv<float>(d_D32, d_tasks, S.nslices, d_voff, d_x, d_y32, nullptr, nullptr, 0));
+        CK(lsp::launch_sell_spmv<float>(d_D32, d_tasks, S.nslices, d_voff, d_x, d_y32, 0));
     };
 
     // fp32 vs fp64 on the CSR path, and SELL against CSR (fp64: same per-row order)
