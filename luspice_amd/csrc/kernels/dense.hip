@@ -330,6 +330,7 @@ __global__ void __launch_bounds__(256, 2) dense_lu_kernel(const DenseJob *jobs, 
         const DenseJob J = jobs[tk.x];
         if (active && !active[J.mat]) continue;
         T *F = ((const FactorDesc<T> *)mats)[J.mat].tail_F;
+        double *S = ((const FactorDesc<T> *)mats)[J.mat].tail_S;
         const int ti = tk.y, tj = tk.z;
         const int q = min(ti, tj);
         const bool low = ti > tj;                       // a tile of L: (r, c) = (j, i)
@@ -348,7 +349,7 @@ __global__ void __launch_bounds__(256, 2) dense_lu_kernel(const DenseJob *jobs, 
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 const int r = r0 + 16 * x + 4 * e + lk;
-                const double v = gp(J.S)[rs * min(r, J.T - 1) + cs * min(c, J.T - 1)];
+                const double v = gp(S)[rs * min(r, J.T - 1) + cs * min(c, J.T - 1)];
                 acc[x][e] = r < J.T && c < J.T ? v : (ti == tj && r == c ? 1.0 : 0.0);
             }
         // operand tiles of product p: X left (rows r), Y right (columns c)
@@ -407,7 +408,7 @@ __global__ void __launch_bounds__(256, 2) dense_lu_kernel(const DenseJob *jobs, 
             // storage precision, and the column maxima of |L|
             auto put = [&](int r, int cc, double f) {
                 if (r < J.T && cc < J.T) {
-                    gp(J.S)[ld * cc + r] = f;
+                    gp(S)[ld * cc + r] = f;
                     if constexpr (sizeof(T) != 8) st_g(&F[ld * cc + r], from_f64<T>(f));
                 }
             };
@@ -472,7 +473,7 @@ __global__ void __launch_bounds__(256, 2) dense_lu_kernel(const DenseJob *jobs, 
                 am[4 * x + e] = in ? fabs(acc[x][e]) : 0.0;
                 if (in) {
                     const size_t at = rs * r + cs * c;
-                    gp(J.S)[at] = acc[x][e];
+                    gp(S)[at] = acc[x][e];
                     if constexpr (sizeof(T) != 8) st_g(&F[at], from_f64<T>(acc[x][e]));
                 }
             }
@@ -499,7 +500,7 @@ __global__ void __launch_bounds__(256) dense_pivot_kernel(const DenseJob *jobs, 
     const int c = tk.y * 256 + (int)threadIdx.x;
     if (c >= J.T || (active && !active[J.mat])) return;
     const FactorDesc<T> M = ((const FactorDesc<T> *)mats)[J.mat];
-    const double *Sc = J.S + (size_t)c * (size_t)J.T;
+    const double *Sc = M.tail_S + (size_t)c * (size_t)J.T;
     const int k = M.tail_k0 + c;
     const double piv = Sc[c];
     const double lmax = __longlong_as_double((long long)J.colmax[c]);

@@ -126,10 +126,9 @@ struct TriDesc {
     int pad_;
 };
 
-// One dense trailing block to factor (fp64 work, fixed pivot order), nt x nt
-// tiles of 64 x 64.
+// One dense trailing block to factor (fp64 work in FactorDesc::tail_S, T x T,
+// column-major; fixed pivot order), nt x nt tiles of 64 x 64.
 struct DenseJob {
-    double *S;              // T x T, column-major, leading dimension T
     double *P;              // nt * nt packed tiles: the final tiles of L and U as operands
     double *W;              // per panel 2 x 64 x 64: its diagonal block's factors as operands (dense.hip)
     unsigned long long *colmax;

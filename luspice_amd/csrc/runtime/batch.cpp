@@ -314,18 +314,22 @@ template <typename T>
 int Batch::ensure_factor_set(FactorSet<T> &fs)
 {
     if (fs.ready) return LSP_OK;
-    fs.val = (T *)dalloc(nslot_tot_ * sizeof(T));
-    fs.lrow = (T *)dalloc(nl_tot_ * sizeof(T));
-    fs.urow = (T *)dalloc(nu_tot_ * sizeof(T));
-    fs.diag = (T *)dalloc(ntot_ * sizeof(T));
-    // fp64 factors of the dense blocks stay where they were computed
-    fs.tailS = (double *)dalloc(nt2_tot_ * sizeof(double));
-    if constexpr (std::is_same<T, double>::value) fs.tailF = fs.tailS;
-    else fs.tailF = (T *)dalloc(nt2_tot_ * sizeof(T));
-    std::vector<DenseJob> jobs = jobs_;
-    for (DenseJob &J : jobs) J.S = fs.tailS + circ_[J.mat].o_t2;
-    fs.djobs = upload(jobs);
-    if (!fs.val || !fs.lrow || !fs.urow || !fs.diag || !fs.tailS || !fs.tailF || !fs.djobs) return LSP_E_ALLOC;
+    // One allocation: the first refactor waits for it.  fp64 factors of the dense
+    // blocks stay where they were computed.
+    constexpr bool in_place = std::is_same<T, double>::value;
+    const size_t t = sizeof(T);
+    const size_t len[6] = {nt2_tot_ * sizeof(double), in_place ? 0 : nt2_tot_ * t, nslot_tot_ * t, nl_tot_ * t,
+                           nu_tot_ * t, ntot_ * t};
+    size_t at[7] = {0};
+    for (int k = 0; k < 6; k++) at[k + 1] = at[k] + ((len[k] + 255) & ~(size_t)255);
+    char *p = (char *)dalloc(at[6]);
+    if (!p) return LSP_E_ALLOC;
+    fs.tailS = (double *)(p + at[0]);
+    fs.tailF = (T *)(p + at[in_place ? 0 : 1]);
+    fs.val = (T *)(p + at[2]);
+    fs.lrow = (T *)(p + at[3]);
+    fs.urow = (T *)(p + at[4]);
+    fs.diag = (T *)(p + at[5]);
     const int nc = (int)circ_.size();
     std::vector<FactorDesc<T>> fd(nc);
     std::vector<TriDesc<T>> td(nc);
@@ -731,6 +735,7 @@ int Batch::upload_all()
         std::vector<int> tlc;
         d_colmax_ = (unsigned long long *)dalloc(nt_tot_ * sizeof(unsigned long long));
         std::vector<int> mat, order;
+        std::vector<DenseJob> jobs;
         for (int m = 0; m < nc; m++) {
             const LspPlan &P = circ_[m].plan;
             tlc.insert(tlc.end(), P.tail_lcut.begin(), P.tail_lcut.end());
@@ -760,7 +765,7 @@ int Batch::upload_all()
             J.colmax = d_colmax_ + C.o_t;
             J.flag = d_dflag_ + ntile;
             J.mat = m;
-            jobs_.push_back(J);
+            jobs.push_back(J);
             order.push_back(J.T);
             ntile += (size_t)J.nt * J.nt;
             npanel += J.nt;
@@ -776,6 +781,7 @@ int Batch::upload_all()
         dgrid_.ngather = (int)H.gather.size();
         dgrid_.ntrsv = (int)H.trsv.size();
         d_tail_lcut_ = upload(tlc);
+        d_djobs_ = upload(jobs);
         d_tail_ctr_ = upload(std::vector<int>(4 * nc, 0));
         std::vector<int2> fill;
         for (int m = 0; m < nc; m++) {
@@ -785,7 +791,7 @@ int Batch::upload_all()
         }
         d_fillchunk_ = upload(fill);
         nfillchunk_ = (int)fill.size();
-        if (!d_tail_lcut_ || !d_tail_ctr_ || !d_fillchunk_ || !dgrid_.lu ||
+        if (!d_tail_lcut_ || !d_djobs_ || !d_tail_ctr_ || !d_fillchunk_ || !dgrid_.lu ||
             !dgrid_.pivot || !dgrid_.gather || !dgrid_.trsv)
             return LSP_E_ALLOC;
     }
@@ -1174,7 +1180,7 @@ int Batch::refactor_t(FactorSet<T> &fs, const int *d_active)
     rc = check(launch_refactor<T>(L, fblocks_, stream_), "refactor launch");
     if (!rc && njobs_) {
         // two 4-wave workgroups per CU (the kernel's register budget)
-        rc = check(launch_dense_lu<T>(fs.djobs, fs.fdesc, d_active, dgrid_, d_ctr_ + 3 * kQueueInts, d_epoch_ + 1,
+        rc = check(launch_dense_lu<T>(d_djobs_, fs.fdesc, d_active, dgrid_, d_ctr_ + 3 * kQueueInts, d_epoch_ + 1,
                                       d_abort_, d_ticks_ + kTickDense1, 2 * cu_count_, opt_.refactor_ptol, L.stol, stream_), "dense lu");
     }
     return rc;

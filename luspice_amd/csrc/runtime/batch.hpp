@@ -58,7 +58,6 @@ struct FactorSet {                       // per storage precision
     // factors that circuits outside its mask still solve with.
     double *tailS = nullptr;
     T *tailF = nullptr;
-    DenseJob *djobs = nullptr;           // device
     FactorDesc<T> *fdesc = nullptr;      // device
     TriDesc<T> *tdesc = nullptr;         // device
     IrDesc<T> *idesc = nullptr;          // device (fused IR step)
@@ -123,7 +122,7 @@ struct DeviceArrays {
     int *d_tail_lcut_ = nullptr, *d_tail_ctr_ = nullptr;
     unsigned long long *d_colmax_ = nullptr;
     int *d_dflag_ = nullptr;                   // per tile of every dense job: epoch of the launch that made it final
-    std::vector<DenseJob> jobs_;               // without their work blocks (ensure_factor_set)
+    DenseJob *d_djobs_ = nullptr;
     int njobs_ = 0;
     DenseGrid dgrid_;                          // work lists of the dense-block launches
     int2 *d_fillchunk_ = nullptr;              // (matrix, chunk) of the unset fill
