@@ -10,9 +10,10 @@
 // persistent launch walks every column of every matrix in the batch.
 //
 // Mapping to CDNA4
-//   * one wave64 per column task; tasks come from a global queue in an
-//     order that rises along every dependency, so a task only waits on tasks handed out earlier, which are held
-//     by running waves: the schedule cannot deadlock whatever the occupancy;
+//   * one wave64 per column task; tasks come from a global queue in an order
+//     that rises along every dependency, so a task only waits on tasks handed
+//     out earlier, which are held by running waves: the schedule cannot
+//     deadlock whatever the occupancy;
 //   * the column's working vector x (fp64) lives in LDS when it fits
 //     (cap doubles per wave), else in a per-wave global scratch slice;
 //   * a task is one record and a dependency one more, so a column's loads are
@@ -20,9 +21,9 @@
 //     flags and A's values; L), not ten through pointer arrays;
 //   * dependencies are fetched 64 at a time (one lane per dependency) and
 //     applied in order, by supernode segment, as soon as a leading group of
-//     their flags has been seen; inside the last run, by their values; rows below a segment are reached through
-//     16-bit local slot indices precomputed by the plan, so no search and no
-//     atomics touch x;
+//     their flags has been seen; inside the last run, by their values; rows
+//     below a segment are reached through 16-bit local slot indices precomputed
+//     by the plan, so no search and no atomics touch x;
 //   * the finished column's L part is stored with agent-coherent stores and
 //     the column's flag is published once they are acknowledged, so no L2
 //     write-back / invalidate is needed on either side;
@@ -429,9 +430,8 @@ __device__ void factor_column(const LSP_CONST FactorDesc<T> *M, const LSP_CONST 
                 if (lane >= ta && lane < tb) x[s0 + lane] = xc;
                 // rows below this part of the run: the run's later rows, then
                 // the rows of L(:, jl) through the map
-                // (about 32 loads in flight: a narrow part, such as the single
-                // column that ends a critical chain step, covers more rows
-                // per round trip)
+                // (a narrow part, such as a single column, covers more rows per
+                // round trip)
                 // (fp64 values: half the columns in flight per pass, for the
                 // register budget of 4 waves per SIMD)
                 constexpr int kB8 = sizeof(T) == 8 ? 4 : 8;

@@ -3,8 +3,8 @@
 //
 // Same solves as trisolve.hip, x = Q U^-1 L^-1 P b over the rows below the dense
 // block.  There every level of dependencies costs a hand-off through memory
-// (0.95 us: store, poll, sum, store) and every task a chain of loads (4 us on
-// one of 1024 waves); a circuit of 1000 to 5000 unknowns has 40 to 90 levels
+// (0.95 us: store, poll, sum, store; 2 to 4 us for the tasks of a large grid's
+// critical chain) and every task a chain of loads (4 us on one of 1024 waves); a circuit of 1000 to 5000 unknowns has 40 to 90 levels
 // and 150 to 800 tasks per solve.  Here the vector is in LDS, a level costs a
 // barrier and an LDS gather (0.64 us), and what a task reads from memory (its
 // header, its rows' records, their entries) is static, so it is loaded one task
@@ -12,7 +12,7 @@
 // to the waves in turn, so in a chain of one-task levels each wave has the time
 // of 16 levels for its loads.  What bounds it: instruction issue of the one CU
 // (0.16 us a task), so lone circuits with many tasks per level stay on the
-// queue (choose_local in the runtime).
+// queue (lsp_choose_local).
 //
 // Measured, pair of solves with the dense block's, queue -> here: 512 circuits
 // of 100 to 5000 unknowns 954 -> 463 us (fp32), 1032 -> 521 us (fp64); 17 circuits
