@@ -83,3 +83,22 @@ def test_long_cycles(inner, chunk):
     assert np.linalg.norm(x[circ[0].n:] - y) <= 1e-6 * np.linalg.norm(y)
     A.close()
     B.close()
+
+
+@pytest.mark.parametrize("prec", ["fp32", "fp64"])
+def test_many_reduction_chunks_in_a_graph(prec):
+    """The launches that add up the parts are recorded with the step: every
+    replay meets the residual line of the eager solve, eager work between them."""
+    print("case: reduction chunks in a graph", prec, flush=True)
+    c = L.mna("sized", n=3000, lr=0.02, seed=3)
+    B = L.Batch(c, chunk_rows=1)
+    for k in range(4):
+        B.set_rhs(c.rhs * (1.0 + k))
+        rr, sr = B.graph_step(prec)
+        assert rr["rc"] == 0 and sr["rc"] == 0 and sr["converged"] == 1, (rr, sr)
+        x = B.get_x() / (1.0 + k)
+        r = c.rhs - np.bincount(c.row, c.val * x[c.col], c.n)
+        assert np.linalg.norm(r) <= 1e-9 * np.linalg.norm(c.rhs)
+        y, se = B.solve(c.rhs)
+        assert se["rc"] == 0 and np.linalg.norm(x - y) <= 1e-6 * np.linalg.norm(y)
+    B.close()
